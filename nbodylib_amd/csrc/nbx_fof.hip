@@ -645,29 +645,53 @@ __device__ __forceinline__ void ball_walk(const DevTree &T, const double *q, boo
     }
 }
 
-__device__ __forceinline__ uint64_t morton_spread(uint64_t v) {
-    v &= 0x1fffffULL;
-    v = (v | (v << 32)) & 0x1f00000000ffffULL;
-    v = (v | (v << 16)) & 0x1f0000ff0000ffULL;
-    v = (v | (v << 8)) & 0x100f00f00f00f00fULL;
-    v = (v | (v << 4)) & 0x10c30c30c30c30c3ULL;
-    v = (v | (v << 2)) & 0x1249249249249249ULL;
-    return v;
-}
-__global__ __launch_bounds__(256) void k_morton_keys(const double *qx, const double *qy, const double *qz, int64_t m,
-                                                     double lo0, double lo1, double lo2, double s0, double s1,
-                                                     double s2, uint64_t *keys, int32_t *idx) {
+// Morton key of a point over the root box: the bits of its ND cell indices
+// interleaved, 21 a dimension in 3-D and 10 in 6-D (63 and 60 bits).  Points
+// outside the box take its border cells, NaN the lowest; the key only orders
+// the points.
+template <int ND>
+__global__ __launch_bounds__(256) void k_point_keys(DevTree T, PointCoords q, int64_t m, uint64_t *keys,
+                                                    int32_t *idx) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= m) return;
-    const double q[3] = {qx[i], qy[i], qz[i]}, lo[3] = {lo0, lo1, lo2}, sc[3] = {s0, s1, s2};
+    constexpr int BITS = ND == 3 ? 21 : 10;
+    const double top = (double)((1 << BITS) - 1);
+    cdptr rb = (cdptr)node_box(T, 1, ND);
     uint64_t key = 0;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const double t = fmin(fmax((q[d] - lo[d]) * sc[d], 0.0), 2097151.0);
-        key |= morton_spread((uint64_t)t) << (2 - d);
+    for (int d = 0; d < ND; ++d) {
+        const double ext = rb[ND + d] - rb[d];
+        const double t = ext > 0.0 ? (q.c[d][i] - rb[d]) * (top / ext) : 0.0;
+        const uint32_t cell = (uint32_t)fmin(fmax(t, 0.0), top);
+#pragma unroll
+        for (int b = 0; b < BITS; ++b) key |= (uint64_t)((cell >> b) & 1u) << (b * ND + (ND - 1 - d));
     }
     keys[i] = key;
     idx[i] = (int32_t)i;
+}
+
+static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+size_t nbx_point_order_bytes(int64_t m) {
+    size_t tb = 0;
+    nbx_sort_pairs_u64(nullptr, tb, nullptr, nullptr, nullptr, nullptr, m, nullptr);
+    return 2 * align256(sizeof(uint64_t) * m) + align256(sizeof(int32_t) * m) + tb;
+}
+
+hipError_t nbx_point_order(const DevTree &T, const PointCoords &q, int64_t m, int32_t *order, void *work,
+                           hipStream_t st) {
+    char *w = (char *)work;
+    uint64_t *keys = (uint64_t *)w, *keys2 = (uint64_t *)(w + align256(sizeof(uint64_t) * m));
+    int32_t *idx = (int32_t *)(w + 2 * align256(sizeof(uint64_t) * m));
+    void *tmp = w + 2 * align256(sizeof(uint64_t) * m) + align256(sizeof(int32_t) * m);
+    ProfScope ps("k_point_order", st);
+    if (T.nd == 6) hipLaunchKernelGGL(k_point_keys<6>, dim3(nblk(m)), dim3(256), 0, st, T, q, m, keys, idx);
+    else hipLaunchKernelGGL(k_point_keys<3>, dim3(nblk(m)), dim3(256), 0, st, T, q, m, keys, idx);
+    hipError_t e = hipGetLastError();
+    size_t tb = 0;
+    if (e == hipSuccess) e = nbx_sort_pairs_u64(nullptr, tb, keys, keys2, idx, order, m, st);
+    if (e == hipSuccess) e = nbx_sort_pairs_u64(tmp, tb, keys, keys2, idx, order, m, st);
+    return e;
 }
 
 template <int FILL>

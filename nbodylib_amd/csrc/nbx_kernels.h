@@ -76,7 +76,10 @@ struct KnnArgs {
     double *hout;       // as rho, or by ID with hout_by_id (nullable)
     int32_t hout_by_id;  // particle queries: hout[ID] rather than hout[slot]
     int32_t *err;       // set to 1 if a row has fewer than kh neighbours
-    const int32_t *qlist;  // nullable: query slots (FP64 re-run of mixed-form fallbacks)
+    // nullable: the queries in the order the waves take them -- slots (FP64
+    // re-run of mixed-form fallbacks, lists of particles) or, for position
+    // queries, their indices
+    const int32_t *qlist;
     // particle queries of a run of whole waves only: slots [64 wbeg, 64 (wbeg + wcnt)) (wcnt 0: every slot)
     int32_t wbeg, wcnt;
     int32_t row0;  // subtracted from the slot of a row written in the by-slot layout
@@ -135,10 +138,15 @@ struct BallManyArgs {
     const int32_t *order;  // positions in walk order (nullable: as given)
 };
 hipError_t nbx_launch_ball_many(const DevTree &T, const BallManyArgs &A, bool fill, hipStream_t st);
-// Morton keys (21 bits a dimension over the box lo + [0, 2^21 / s)) and
-// their indices, for ordering query positions along the space-filling curve
-__global__ void k_morton_keys(const double *qx, const double *qy, const double *qz, int64_t m, double lo0, double lo1,
-                              double lo2, double s0, double s1, double s2, uint64_t *keys, int32_t *idx);
+// Order of m query points (T.nd coordinates each) along the Morton curve over
+// the root box, so that a wave's 64 points are neighbours: order[0..m).
+// work: nbx_point_order_bytes(m) bytes of device memory.
+struct PointCoords {
+    const double *c[6];
+};
+size_t nbx_point_order_bytes(int64_t m);
+hipError_t nbx_point_order(const DevTree &T, const PointCoords &q, int64_t m, int32_t *order, void *work,
+                           hipStream_t st);
 
 // ------------------------------------------------------------------ smoothed velocities
 struct SmoothArgs {

@@ -324,7 +324,7 @@ __global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
     const int kh = A.kh;
     const int hc = heap_cap4(kh);
     const int nfill = hc - kh;  // filler entries, first after sorting
-    const bool listed = (QSRC != NBX_Q_POINTS) && A.qlist != nullptr;
+    const bool listed = A.qlist != nullptr;
     const int wend = A.wbeg + A.wcnt;
     const int nq = (QSRC == NBX_Q_POINTS || listed) ? A.m
                    : (A.wcnt > 0 && wend < (T.n + NBX_WAVE - 1) / NBX_WAVE ? wend * NBX_WAVE : T.n);
