@@ -82,6 +82,10 @@ struct Workspace {
         used = a + bytes;
         return (T *)(base + a);
     }
+    size_t left() const {
+        const size_t a = (used + 255) & ~(size_t)255;
+        return a < cap ? cap - a : 0;
+    }
 };
 
 // ------------------------------------------------------------------ profiling
@@ -502,17 +506,36 @@ struct ScratchLease {
 };
 
 // Bytes the fused kNN + density pass carves, in its order: densities by slot,
-// the error flag and, for the precision form, the fallback list and the
-// search scratch.
-static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed) {
+// the error flag, the fallback list (precision form) and the search scratch.
+// kh: entries the FP64 search keeps (0: its scratch not counted).
+static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed, int32_t kh) {
     Workspace dry = {nullptr, ~(size_t)0, 0};
     dry.carve<char>(sizeof(double) * t->n);
     dry.carve<char>(sizeof(int32_t));
     if (mixed) {
         dry.carve<char>(sizeof(int32_t) * (t->n + 1));
         dry.carve<char>(nbx_mixed_scratch_bytes(t->nd, k + 1));
+    } else if (kh > 0) {
+        dry.carve<char>(nbx_knn_scratch_bytes(t->nd, kh, NBX_Q_SLOTS, t->n));
     }
     return dry.used;
+}
+
+// The FP64 search with its scratch from ws (as much of it as is left), or
+// from the tree's kept scratch when ws is null.
+static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t st, Workspace *ws = nullptr) {
+    if (nq <= 0) return hipSuccess;
+    size_t need = nbx_knn_scratch_bytes(t->nd, A.kh, A.qsrc, nq);
+    std::unique_ptr<ScratchLease> lease;
+    if (!ws) {
+        lease.reset(new ScratchLease(t, need, st));
+        if (lease->err != hipSuccess) return lease->err;
+        ws = &lease->ws;
+    }
+    need = std::min(need, ws->left());
+    void *work = ws->carve<void>(need);
+    if (!work) return hipErrorInvalidValue;
+    return nbx_launch_knn(t->view(), A, nq, st, work, need);
 }
 
 // ------------------------------------------------------------------ precision form
@@ -637,7 +660,7 @@ extern "C" int nbx_knn_dev(nbx_tree *t, int32_t k, int32_t variant, int32_t layo
         if (d2_dev) HIPCK(nbx_launch_rows_fp64(t->view(), A.nn, d2_dev, k, layout, st));
         return NBX_OK;
     }
-    HIPCK(nbx_launch_knn(t->view(), A, nq, st));
+    HIPCK(run_plain(t, A, nq, st));
     return NBX_OK;
 }
 
@@ -688,7 +711,7 @@ extern "C" int nbx_knn_targets(nbx_tree *t, const int32_t *ids, int64_t m, int32
     A.qlist = dsl;
     A.m = (int32_t)m;
     A.list_rows = 1;
-    hipError_t e = nbx_launch_knn(t->view(), A, (int)m, nullptr);
+    hipError_t e = run_plain(t, A, (int)m, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e == hipSuccess) e = hipMemcpy(nn, dnn, sizeof(int32_t) * m * k, hipMemcpyDeviceToHost);
     if (e == hipSuccess && d2) e = hipMemcpy(d2, dd2, sizeof(double) * m * k, hipMemcpyDeviceToHost);
@@ -757,7 +780,7 @@ static int points_impl(nbx_tree *t, const double *q, int64_t m, int32_t k, bool 
     A.hout = dh;
     A.err = err;
     int32_t herr = 0;
-    hipError_t e = nbx_launch_knn(t->view(), A, (int)m, nullptr);
+    hipError_t e = run_plain(t, A, (int)m, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e == hipSuccess) e = hipMemcpy(&herr, err, sizeof(int32_t), hipMemcpyDeviceToHost);
     if (e == hipSuccess && nn) e = hipMemcpy(nn, dnn, sizeof(int32_t) * m * k, hipMemcpyDeviceToHost);
@@ -844,7 +867,7 @@ static int density_impl(nbx_tree *t, int32_t k, int32_t variant, int32_t nsearch
     if (ws) {
         if (A.dens == NBX_DO_VELPHYS) return fail(NBX_ERR_UNSUPPORTED, "no workspace form of this density");
     } else {
-        lease.reset(new ScratchLease(t, density_ws_bytes(t, k, mixed), st));
+        lease.reset(new ScratchLease(t, density_ws_bytes(t, k, mixed, A.kh), st));
         if (lease->err != hipSuccess) return hipfail(lease->err, "density scratch");
         ws = &lease->ws;
     }
@@ -864,7 +887,7 @@ static int density_impl(nbx_tree *t, int32_t k, int32_t variant, int32_t nsearch
     A.hout_by_id = 1;
     A.err = err;
     A.nn = nn_slot;
-    hipError_t e = mixed ? run_mixed(t, A, k, st, ws) : nbx_launch_knn(t->view(), A, (int)n, st);
+    hipError_t e = mixed ? run_mixed(t, A, k, st, ws) : run_plain(t, A, (int)n, st, ws);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, rho, t->perm, rho_id, n);
         e = hipGetLastError();
@@ -899,7 +922,10 @@ extern "C" int nbx_knn_density_dev(nbx_tree *t, int32_t k, int32_t *nn_by_slot_d
 // device.  Every call on a GPU shares that GPU's copy: it clears what must
 // start at zero itself (fill kernels), and calls that overlap on one GPU race.
 #define NBX_NOALLOC_BYTES ((size_t)256 << 20)
-static __device__ __align__(256) unsigned char scratch[NBX_NOALLOC_BYTES];
+// Past the bytes that limit the tree's size, room for the FP64 search's
+// smallest scratch (8 workgroups, 1.03 MiB at k > 64).
+#define NBX_NOALLOC_ARRAY (NBX_NOALLOC_BYTES + ((size_t)2 << 20))
+static __device__ __align__(256) unsigned char scratch[NBX_NOALLOC_ARRAY];
 #define NBX_MAX_DEVICES 64
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[NBX_MAX_DEVICES];  // per device: the address of `scratch` there
@@ -924,7 +950,8 @@ extern "C" int nbx_knn_density_noalloc(nbx_tree *t, int32_t k, int32_t *nn_by_sl
     if (k < 1 || k > heap_cap(t)) return fail(NBX_ERR_UNSUPPORTED, "k out of range");
     // the carves density_impl and run_mixed will make
     const int64_t n = t->n;
-    const size_t need = density_ws_bytes(t, k, mixed_ok(t, k));
+    // (the FP64 search runs with the scratch that is left, if less than its full need)
+    const size_t need = density_ws_bytes(t, k, mixed_ok(t, k), 0);
     if (need > NBX_NOALLOC_BYTES)
         return fail(NBX_ERR_UNSUPPORTED, "nbx_knn_density_noalloc: " + std::to_string(n) + " particles need " +
                                              std::to_string(need >> 20) + " MiB of scratch; the maximum is " +
@@ -932,7 +959,7 @@ extern "C" int nbx_knn_density_noalloc(nbx_tree *t, int32_t k, int32_t *nn_by_sl
     void *base = nullptr;
     int rc = noalloc_scratch(&base);
     if (rc) return rc;
-    Workspace ws = {(char *)base, NBX_NOALLOC_BYTES, 0};
+    Workspace ws = {(char *)base, NBX_NOALLOC_ARRAY, 0};
     return density_impl(t, k, NBX_DENS_SYMMETRIC, 0, rho_by_id_dev, h_by_id_dev, nn_by_slot_dev, (hipStream_t)stream,
                         nullptr, &ws);
 }
@@ -1116,7 +1143,7 @@ extern "C" int nbx_smooth_local_points(nbx_tree *t, const double *q, int64_t m, 
         }
         for (int d = 0; d < 3; ++d) K.q[d] = dq + d * m;
         K.nn = dnn;
-        if (e == hipSuccess) e = nbx_launch_knn(t->view(), K, (int)m, st);
+        if (e == hipSuccess) e = run_plain(t, K, (int)m, st);
         if (e == hipSuccess) {
             hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, st, rid, t->perm, n, rslot);
             hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, st, wid, t->perm, n, wslot);
@@ -1451,10 +1478,9 @@ static int sph_tree_impl(nbx_tree *t, int32_t k, int64_t block, const double *g_
     }
     // the search's temporaries, reused by every block
     Workspace ws = {nullptr, 0, 0};
-    if (mixed) {
-        ws.cap = 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1);
-        HIPCK(bufs.alloc(&ws.base, ws.cap));
-    }
+    ws.cap = mixed ? 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1)
+                   : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, block);
+    HIPCK(bufs.alloc(&ws.base, ws.cap));
     double *D[3] = {ds, ds ? ds + n : nullptr, ds ? ds + 2 * n : nullptr};
     for (int64_t r0 = 0; r0 < n; r0 += block) {
         const int64_t nr = std::min<int64_t>(block, n - r0);
@@ -1471,7 +1497,7 @@ static int sph_tree_impl(nbx_tree *t, int32_t k, int64_t block, const double *g_
         A.wcnt = (int32_t)((nr + NBX_WAVE - 1) / NBX_WAVE);
         A.row0 = (int32_t)r0;
         ws.used = 0;
-        hipError_t e = mixed ? run_mixed(t, A, k, st, &ws) : nbx_launch_knn(t->view(), A, A.wcnt * NBX_WAVE, st);
+        hipError_t e = mixed ? run_mixed(t, A, k, st, &ws) : run_plain(t, A, A.wcnt * NBX_WAVE, st, &ws);
         if (e == hipSuccess) e = nbx_launch_kth_last(X, t->perm, nbr, r0, nr, k, err, st);
         if (e == hipSuccess)
             e = adj ? nbx_launch_sph_adj_rows(X, t->mass, nbr, n, r0, nr, k, gs, D, ms, st)

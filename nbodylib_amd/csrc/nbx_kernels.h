@@ -87,7 +87,14 @@ struct KnnArgs {
     double band_rel;    // precision form: least relative half-width of the FP64 re-check band
 };
 
-hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st);
+// work (nullable): device memory of nbx_knn_scratch_bytes for the
+// per-workgroup scratch and the queue counters.  Fewer bytes, down to
+// nbx_knn_scratch_least, run fewer workgroups; without work the launcher
+// allocates on the stream.
+hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st, void *work = nullptr,
+                          size_t work_bytes = 0);
+size_t nbx_knn_scratch_bytes(int nd, int kh, int qsrc, int64_t nqueries);
+size_t nbx_knn_scratch_least(int nd, int kh);
 // work (nullable): device memory of at least nbx_mixed_scratch_bytes(nd, kh)
 // bytes for the per-workgroup scratch and the queue counters; without it the
 // launcher allocates them on the stream.

@@ -10,185 +10,168 @@
 // sibling leaves).  The wave walks the implicit tree once for all 64 lanes
 // (a node is opened when any lane's bound reaches it), so node boxes and
 // leaf particles arrive through the scalar cache as 64-byte s_load bursts
-// and are shared by the whole wave.  Each lane keeps its own 4-ary max-heap
-// of (d2, particle ID) in LDS -- the reference's PriorityQueue
-// (PriorityQueue.h:47-84), with three dependent levels instead of five for
-// k = 32 -- laid out [position][lane] so same-position accesses are
-// conflict-free.  A leaf is consumed in two phases: (1) all lanes test every
-// candidate against their current k-th distance, building a 32-bit accept
-// mask; (2) lanes insert their accepted candidates one at a time from an LDS
-// copy of the leaf with a branch-free root replacement, so the wave pays for
-// as many heap insertions as its busiest lane, not the sum over lanes.
+// and are shared by the whole wave.  A leaf is consumed in two phases: (1)
+// all lanes test every candidate against their current k-th distance,
+// building a 32-bit accept mask; (2) lanes insert their accepted candidates
+// one at a time from an LDS copy of the leaf, so the wave pays for as many
+// insertions as its busiest lane, not the sum over lanes.
+//
+// Kept entries.  Each lane keeps its kh smallest d2 in LDS, laid out
+// [position][lane] (conflict-free), in G groups of S positions, with every
+// group's largest value and its position in registers.  An insertion stores
+// over the largest kept value, reloads that one group and takes its maximum:
+// one store, S independent loads and about 60 VALU, with a single LDS round
+// trip.  The particles' slots go to a per-workgroup scratch block in device
+// memory (a store nothing waits for), so LDS holds 8 bytes per entry and 9
+// waves fit on a CU at k = 32.  The 4-ary heap of (d2, ID) pairs in LDS that
+// this replaced held 12 bytes per entry (6 waves per CU) and took three
+// dependent levels and about 135 VALU per insertion.  Measured, heap to
+// groups: k = 32 density of 2.1M clustered particles 10.7 -> 4.6 ms; 0.5M
+// particles k = 8 1.68 -> 0.88, k = 64 8.4 -> 4.1, k = 128 40 -> 12 ms; 6-D
+// k = 64 63 -> 28 ms.
+// The scratch is sized by the resident workgroups: the kernel is persistent
+// and takes waves of queries from its XCD's share through an atomic counter,
+// as the precision form does (nbx_mixed.hip).
 //
 // Exactness: distances are summed in the reference's order with no FMA
 // (this file is built with -ffp-contract=off); pruning uses box_lb, which is
 // never larger than a computed particle distance.  The neighbour set is the k
 // smallest (d2, ID) pairs: ties at the k-th distance go to the smaller ID
-// (the reference's choice there depends on its traversal order).
+// (the reference's choice there depends on its traversal order).  The search
+// itself evicts any of several equal d2; a lane remembers the smallest value
+// it discarded, and when that equals its final k-th distance a second walk
+// collects the particles at exactly that distance and keeps the smallest IDs.
+#include <atomic>
+
 #include "nbx_kernels.h"
 
-// Heap entries are (d2, particle ID) pairs ordered by d2, then ID; the ID is
-// carried in the heap so ties never need a lookup.  Empty entries are
-// (NBX_MAXVALUE, NBX_NOID); filler entries (-1, -1) pad the heap to a
-// capacity of 1 (mod 4) and, being smaller than every key, are never evicted.
-#define NBX_NOID 0x7fffffff
-
-// (da, ia) > (db, ib)
-__device__ __forceinline__ bool kgt(double da, int32_t ia, double db, int32_t ib) {
-    return da > db || (da == db && ia > ib);
+// v_max_f64 without the NaN canonicalisation fmax() adds: kept values are
+// never NaN (a NaN d2 fails every test that leads here).
+__device__ __forceinline__ double kmax(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
 
-#define HD(p) hd[(p) * NBX_WAVE + lane]
-#define HI(p) hid[(p) * NBX_WAVE + lane]
-
-// Heap capacity for kh kept entries: kh rounded up to 1 (mod 4), so every
-// parent of a full 4-ary heap has four children.
-__host__ __device__ __forceinline__ int heap_cap4(int kh) { return ((kh + 2) & ~3) + 1; }
-
-// Largest of four children (and its index 0..3).
-__device__ __forceinline__ void max4(const double *d, const int32_t *id, double &bd, int32_t &bi, int &bx) {
-    const bool s01 = kgt(d[1], id[1], d[0], id[0]), s23 = kgt(d[3], id[3], d[2], id[2]);
-    const double m01 = s01 ? d[1] : d[0], m23 = s23 ? d[3] : d[2];
-    const int32_t j01 = s01 ? id[1] : id[0], j23 = s23 ? id[3] : id[2];
-    const bool s = kgt(m23, j23, m01, j01);
-    bd = s ? m23 : m01;
-    bi = s ? j23 : j01;
-    bx = s ? (s23 ? 3 : 2) : (s01 ? 1 : 0);
-}
-
-// 4-ary max-heap, 0-based, children of p at 4p+1 .. 4p+4 (the reference's
-// PriorityQueue, PriorityQueue.h:47-84, with three dependent levels instead
-// of five for k = 32).  Replace the root of the full heap of hc entries by
-// (dv, iv) for the lanes with ins set and sift it down; the other lanes
-// rewrite the root with itself.  LV unrolled levels cover hc <= 85 (LV = 3)
-// or hc <= 341 (LV = 4) and nothing branches.  (kth, kid) is the root afterwards.
-template <int LV>
-__device__ __forceinline__ void heap_replace_root(double *hd, int32_t *hid, int lane, int hc, bool ins, double dn,
-                                                  int32_t in, double &kth, int32_t &kid) {
-    const double dv = ins ? dn : kth;
-    const int32_t iv = ins ? in : kid;
-    double td = dv;
-    int32_t ti = iv;
-    int p = 0;
-    bool go = ins;
-#pragma unroll
-    for (int lv = 0; lv < LV; ++lv) {
-        const int c = 4 * p + 1;
-        go = go && c < hc;
-        const int cc = go ? c : 1;
-        double d[4];
-        int32_t id[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) { d[u] = HD(cc + u); id[u] = HI(cc + u); }
-        double bd;
-        int32_t bi;
-        int bx;
-        max4(d, id, bd, bi, bx);
-        go = go && kgt(bd, bi, dv, iv);
-        HD(p) = go ? bd : dv;
-        HI(p) = go ? bi : iv;
-        if (lv == 0) { td = go ? bd : dv; ti = go ? bi : iv; }
-        p = go ? cc + bx : p;
-    }
-    HD(p) = dv;
-    HI(p) = iv;
-    kth = td;
-    kid = ti;
-}
-
-// Sift (dv, iv) down from the root of a heap of m <= hc entries; children
-// at positions >= m read as (-inf, min) and never outrank an entry.
-template <int LV>
-__device__ __forceinline__ void heap_sift_bounded(double *hd, int32_t *hid, int lane, int m, double dv, int32_t iv) {
-    int p = 0;
-    bool go = true;
-#pragma unroll
-    for (int lv = 0; lv < LV; ++lv) {
-        const int c = 4 * p + 1;
-        go = go && c < m;
-        const int cc = go ? c : 1;
-        double d[4];
-        int32_t id[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const double t = HD(cc + u);
-            const int32_t ti = HI(cc + u);
-            const bool in = cc + u < m;
-            d[u] = in ? t : -INFINITY;
-            id[u] = in ? ti : (int32_t)0x80000000;
-        }
-        double bd;
-        int32_t bi;
-        int bx;
-        max4(d, id, bd, bi, bx);
-        go = go && kgt(bd, bi, dv, iv);
-        HD(p) = go ? bd : dv;
-        HI(p) = go ? bi : iv;
-        p = go ? cc + bx : p;
-    }
-    HD(p) = dv;
-    HI(p) = iv;
-}
-
-// General sift from position p in a heap of size m (short selection of the
-// velocity density only).
-__device__ __forceinline__ void heap_sift(double *hd, int32_t *hid, int lane, int m, int p, double dv, int32_t iv) {
-    for (;;) {
-        int c = 4 * p + 1;
-        if (c >= m) break;
-        double dc = HD(c);
-        int32_t ic = HI(c);
-        int best = c;
-        for (int u = 1; u < 4; ++u) {
-            if (c + u < m && kgt(HD(c + u), HI(c + u), dc, ic)) { best = c + u; dc = HD(c + u); ic = HI(c + u); }
-        }
-        if (!kgt(dc, ic, dv, iv)) break;
-        HD(p) = dc;
-        HI(p) = ic;
-        p = best;
-    }
-    HD(p) = dv;
-    HI(p) = iv;
-}
-
-// Heap sort in place: positions 0..hc-1 ascending afterwards (fillers first).
-template <int LV>
-__device__ __forceinline__ void heap_sort(double *hd, int32_t *hid, int lane, int hc) {
-    for (int m = hc - 1; m > 0; --m) {
-        const double dt = HD(0), dm = HD(m);
-        const int32_t it = HI(0), im = HI(m);
-        HD(m) = dt;
-        HI(m) = it;
-        heap_sift_bounded<LV>(hd, hid, lane, m, dm, im);
-    }
-}
-
-// heap levels below the root that a capacity of KMAX entries needs
 template <int KMAX>
-struct HeapLv {
-    static constexpr int LV = KMAX <= 85 ? 3 : 4;
-    static_assert(KMAX <= 341, "four levels hold at most 341 entries");
+struct KShape {
+    static constexpr int G = KMAX <= 33 ? 3 : (KMAX <= 65 ? 5 : 11);
+    static constexpr int S = KMAX / G;
+    static_assert(G * S == KMAX, "groups must tile KMAX");
 };
+
+#define HD(p) hd[(p) * NBX_WAVE + lane]  // kept d2 (LDS); unused positions hold -1
+#define SL(p) sl[(p) * NBX_WAVE + lane]  // their slots (scratch)
+
+// Per-lane search state.  kth: the largest kept d2 (NBX_MAXVALUE while fewer
+// than kh are kept); gm, gp: each group's largest value and its position;
+// lost: the smallest d2 discarded so far that was equal to kth when discarded.
+template <int ND, int KMAX>
+struct KnnCtx {
+    double q[ND];
+    double kth, lost;
+    double gm[KShape<KMAX>::G];
+    int gp[KShape<KMAX>::G];
+    bool act, exz;
+    int fill;  // kh while nothing is kept and a whole leaf fits (wave-uniform), else 0
+};
+
+// Largest of the S values of group g and its (first) position.
+template <int KMAX>
+__device__ __forceinline__ void group_max(const double *hd, int lane, int base, double &m, int &at) {
+    constexpr int S = KShape<KMAX>::S;
+    double x[S];
+#pragma unroll
+    for (int u = 0; u < S; ++u) x[u] = HD(base + u);
+    m = x[0];
+#pragma unroll
+    for (int u = 1; u < S; ++u) m = kmax(m, x[u]);
+    uint32_t eq = 0;
+#pragma unroll
+    for (int u = S - 1; u >= 0; --u) eq = eq + eq + (x[u] == m ? 1u : 0u);
+    at = base + __builtin_ctz(eq);
+}
+
+template <int ND, int KMAX>
+__device__ __forceinline__ void knn_top(KnnCtx<ND, KMAX> &c) {
+    c.kth = c.gm[0];
+#pragma unroll
+    for (int g = 1; g < KShape<KMAX>::G; ++g) c.kth = kmax(c.kth, c.gm[g]);
+}
+
+// Store (d2, slot) over the largest kept value in the lanes with ins set;
+// the others store that value back, so only the slot's store branches.
+template <int ND, int KMAX>
+__device__ __forceinline__ void knn_replace(KnnCtx<ND, KMAX> &c, double *hd, int32_t *sl, int lane, bool ins,
+                                            double d2, int32_t slot) {
+    constexpr int G = KShape<KMAX>::G, S = KShape<KMAX>::S;
+    int g0 = 0, p = c.gp[0];
+#pragma unroll
+    for (int g = 1; g < G; ++g) {
+        const bool here = c.gm[g] == c.kth;
+        g0 = here ? g : g0;
+        p = here ? c.gp[g] : p;
+    }
+    HD(p) = ins ? d2 : c.kth;
+    if (ins) SL(p) = slot;
+    double m;
+    int at;
+    group_max<KMAX>(hd, lane, g0 * S, m, at);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        c.gm[g] = g0 == g ? m : c.gm[g];
+        c.gp[g] = g0 == g ? at : c.gp[g];
+    }
+    knn_top<ND, KMAX>(c);
+}
 
 template <int ND>
-struct LeafCtx {
-    double q[ND];
-    bool act;
-    bool exz;
-    double kth;   // root of the heap: the kh-th smallest (d2, ID) so far
-    int32_t kid;
-};
+__device__ __forceinline__ double knn_d2(const double *q, const double *cx, int j) {
+    double d2 = 0.0;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        const double t = q[d] - cx[d * NBX_LEAF + j];
+        d2 += t * t;
+    }
+    return d2;
+}
+
+// Insert one accepted candidate (j of the LDS copy) per lane.  TIE 0: the
+// search.  TIE 1: the candidate lies at exactly the k-th distance; entries at
+// that distance hold -(2 + ID) (see knn_ties), the largest ID is the lowest
+// value, and it gives way to a smaller ID.
+template <int ND, int KMAX, int TIE>
+__device__ __forceinline__ void knn_insert(const DevTree &T, KnnCtx<ND, KMAX> &c, double *hd, int32_t *sl,
+                                           const double *cx, int lane, int kh, int base, int j, bool has) {
+    if constexpr (TIE == 0) {
+        const double d2 = knn_d2<ND>(c.q, cx, j);
+        const bool in = has && d2 <= c.kth && (!c.exz || d2 > 0.0);
+        c.lost = in ? c.kth : c.lost;  // the evicted value, or d2 itself when equal
+        knn_replace<ND, KMAX>(c, hd, sl, lane, in && d2 < c.kth, d2, base + j);
+    } else {
+        const double mine = has ? -2.0 - (double)T.perm[base + j] : -1.0;
+        double lo = 0.0;
+        int at = 0;
+        for (int p = 0; p < kh; ++p) {
+            const double v = HD(p);
+            at = v < lo ? p : at;
+            lo = v < lo ? v : lo;
+        }
+        if (has && mine > lo) {
+            HD(at) = mine;
+            SL(at) = base + j;
+        }
+    }
+}
 
 // Consume one leaf for every active lane (two-phase insertion, see header).
-template <int ND, int LV>
-__device__ __forceinline__ void knn_leaf(const DevTree &T, int leaf, LeafCtx<ND> &c, double *hd, int32_t *hid,
-                                         double *cx, int32_t *cid, int lane, int hc) {
+template <int ND, int KMAX, int TIE>
+__device__ __forceinline__ void knn_leaf(const DevTree &T, const double *const (&X)[ND], int leaf,
+                                         KnnCtx<ND, KMAX> &c, double *hd, int32_t *sl, double *cx, int lane, int kh) {
     const int base = leaf * NBX_LEAF;
-    if (lane < NBX_LEAF) {
+    double st[ND];
 #pragma unroll
-        for (int d = 0; d < ND; ++d) cx[d * NBX_LEAF + lane] = T.x[d][base + lane];
-        cid[lane] = T.perm[base + lane];
-    }
+    for (int d = 0; d < ND; ++d) st[d] = X[d][base + (lane & (NBX_LEAF - 1))];
     uint32_t mask = 0;
     // candidates arrive in chunks through the scalar cache: 8 per dimension
     // (24 SGPR pairs) in 3-D, 4 in 6-D
@@ -199,86 +182,109 @@ __device__ __forceinline__ void knn_leaf(const DevTree &T, int leaf, LeafCtx<ND>
     for (int jj = 0; jj < NBX_LEAF; jj += CH) {
         dxc cv[ND];
 #pragma unroll
-        for (int d = 0; d < ND; ++d) cv[d] = *(cdcptr)(T.x[d] + base + jj);
+        for (int d = 0; d < ND; ++d) cv[d] = *(cdcptr)(X[d] + base + jj);
 #pragma unroll
         for (int u = 0; u < CH; ++u) {
             double d2 = 0.0;
 #pragma unroll
             for (int d = 0; d < ND; ++d) {
-                double t = c.q[d] - cv[d][u];
+                const double t = c.q[d] - cv[d][u];
                 d2 += t * t;
             }
-            // the query itself has d2 == 0: excluded by the d2 > 0 rule of
-            // the target search and kept by the position search, as in the
-            // reference (KDLeafNode.cxx:19-21, :123-124)
-            bool ok = (d2 <= c.kth) && (!c.exz || d2 > 0.0);
-            mask |= ok ? (1u << (jj + u)) : 0u;
+            mask = mask + mask + ((TIE ? d2 == c.kth : d2 <= c.kth) ? 1u : 0u);
         }
     }
+    mask = __builtin_bitreverse32(mask);  // candidate j was shifted in at bit 31 - j
     if (!c.act) mask = 0;
+    if (!ballot(mask != 0)) return;
+    if (lane < NBX_LEAF) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) cx[d * NBX_LEAF + lane] = st[d];
+    }
     __syncthreads();
-    while (ballot(mask != 0)) {
+    if (TIE == 0 && c.fill) {
+        // first leaf met with nothing kept: the accepted candidates take the
+        // positions in turn, and the group maxima are taken once at the end
+        c.fill = 0;
+        int cnt = 0;
+        for (int j = 0; j < NBX_LEAF; ++j) {
+            const double d2 = knn_d2<ND>(c.q, cx, j);
+            const bool in = ((mask >> j) & 1u) && d2 < c.kth && (!c.exz || d2 > 0.0);
+            if (in) {
+                HD(cnt) = d2;
+                SL(cnt) = base + j;
+            }
+            cnt += in ? 1 : 0;
+        }
+#pragma unroll
+        for (int g = 0; g < KShape<KMAX>::G; ++g)
+            group_max<KMAX>(hd, lane, g * KShape<KMAX>::S, c.gm[g], c.gp[g]);
+        knn_top<ND, KMAX>(c);
+        __syncthreads();
+        return;
+    }
+    // as many steps as the lane with the most candidates needs (a counted
+    // loop keeps the search state in place across steps)
+    int nit = __popc(mask);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) nit = max(nit, __shfl_xor(nit, off));
+    nit = __builtin_amdgcn_readfirstlane(nit);
+    for (int it = 0; it < nit; ++it) {
         const bool has = mask != 0;
         const int j = __builtin_ctz(mask | 0x80000000u);
         mask &= mask - 1;
-        double d2 = 0.0;
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            double t = c.q[d] - cx[d * NBX_LEAF + j];
-            d2 += t * t;
-        }
-        const int32_t id = cid[j];
-        heap_replace_root<LV>(hd, hid, lane, hc, has && kgt(c.kth, c.kid, d2, id), d2, id, c.kth, c.kid);
+        knn_insert<ND, KMAX, TIE>(T, c, hd, sl, cx, lane, kh, base, j, has);
     }
     __syncthreads();
 }
 
 // Uniform stackless depth-first walk of the heap-ordered tree.  The first
 // descent follows the ancestors of the wave's own leaf node (anc; -1 when
-// the queries are not tree particles or are image-shifted), so every heap
+// the queries are not tree particles or are image-shifted), so every lane
 // is filled from the query's own neighbourhood before anything else is
 // opened; below that children are taken nearest first from qc.  A node is
 // opened when any active lane has box_lb <= its current k-th distance.
 // State is uniform (SGPRs): node, depth and one "right child first" bit per
-// depth.
-template <int ND, int LV>
-__device__ __forceinline__ void knn_walk(const DevTree &T, LeafCtx<ND> &c, const float *qc, int anc, double *hd,
-                                         int32_t *hid, double *cx, int32_t *cid, int lane, int hc) {
-    const int D = T.depth;
+// depth; the tree's fields it reads are scalar values of their own (a field
+// read from the wide argument block in the loop would bring back the block).
+template <int ND, int KMAX, int TIE>
+__device__ __forceinline__ void knn_walk(const DevTree &T, KnnCtx<ND, KMAX> &c, const float *qc, int anc, double *hd,
+                                         int32_t *sl, double *cx, int lane, int kh) {
+    int D = T.depth, nleafp = T.nleafp;
+    const double *boxp = T.box;
+    const float *planep = T.plane;
+    asm volatile("" : "+s"(D), "+s"(nleafp), "+s"(boxp), "+s"(planep));
+    const double *X[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        X[d] = T.x[d];
+        asm volatile("" : "+s"(X[d]));
+    }
     int node = 1, dep = 0;
     uint64_t firstright = 0;
-    bool down = true;
     for (;;) {
-        if (down) {
-            cdptr bx = (cdptr)node_box(T, node, ND);
-            bool want = c.act && box_lb<ND>(c.q, bx) <= c.kth;
-            if (ballot(want)) {
-                if (dep == D) {
-                    knn_leaf<ND, LV>(T, node - T.nleafp, c, hd, hid, cx, cid, lane, hc);
-                    down = false;
-                } else {
-                    int c0 = 2 * node;
-                    int first = c0;
-                    if (anc >= 0 && (anc >> (D - dep)) == node) first = anc >> (D - dep - 1);
-                    else if (first_is_right<ND>(T, node, qc)) first = c0 + 1;
-                    dep += 1;
-                    if (first & 1) firstright |= (1ULL << dep);
-                    else firstright &= ~(1ULL << dep);
-                    node = first;
-                    continue;
-                }
+        cdptr bx = (cdptr)(boxp + (size_t)node * 2 * ND);
+        const bool want = c.act && box_lb<ND>(c.q, bx) <= c.kth;
+        if (ballot(want)) {
+            if (dep == D) {
+                knn_leaf<ND, KMAX, TIE>(T, X, node - nleafp, c, hd, sl, cx, lane, kh);
             } else {
-                down = false;
+                int first;
+                if (anc >= 0 && (anc >> (D - dep)) == node) first = anc >> (D - dep - 1);
+                else first = 2 * node + (first_is_right<ND>(planep, node, qc) ? 1 : 0);
+                dep += 1;
+                firstright = (firstright & ~(1ULL << dep)) | ((uint64_t)(first & 1) << dep);
+                node = first;
+                continue;
             }
         }
-        if (node == 1) break;
-        if ((uint64_t)(node & 1) == ((firstright >> dep) & 1ULL)) {
-            node ^= 1;  // the sibling always exists in the padded tree
-            down = true;
-        } else {
+        // climb to the next unvisited sibling (it always exists in the padded tree)
+        while (node != 1 && (uint64_t)(node & 1) != ((firstright >> dep) & 1ULL)) {
             node >>= 1;
             dep -= 1;
         }
+        if (node == 1) break;
+        node ^= 1;
     }
 }
 
@@ -312,18 +318,85 @@ __device__ __forceinline__ bool image_pass(int pass, const double *x0, const dou
     return uncond || kth > sqrt(sval);
 }
 
+
+// Rank of v among the kh kept values (positions past kh hold -1 and are not
+// counted): how many are smaller.
+template <int KMAX>
+__device__ __forceinline__ int knn_rank(const double *hd, int lane, int kh, const double (&x)[KMAX <= 65 ? KMAX : 1],
+                                        double v) {
+    int r = 0;
+    if constexpr (KMAX <= 65) {
+#pragma unroll
+        for (int p = 0; p < KMAX; ++p) r += x[p] < v ? 1 : 0;
+        r -= KMAX - kh;
+    } else {
+#pragma unroll 4
+        for (int p = 0; p < kh; ++p) r += HD(p) < v ? 1 : 0;
+    }
+    return r;
+}
+template <int KMAX>
+__device__ __forceinline__ void knn_load(const double *hd, int lane, double (&x)[KMAX <= 65 ? KMAX : 1]) {
+    if constexpr (KMAX <= 65) {
+#pragma unroll
+        for (int p = 0; p < KMAX; ++p) x[p] = HD(p);
+    }
+}
+// The kept entries in ascending order of (value, ID, position): slots (or
+// IDs; -1 for a missing one) to so, values to sd.  si: room for the IDs.
+template <int KMAX>
+__device__ __forceinline__ void knn_sort(const DevTree &T, const double *hd, const int32_t *sl, int32_t *so,
+                                         double *sd, int32_t *si, int lane, int kh, bool ids) {
+    auto put = [&](int p, double v, int r) {
+        int32_t e = -1;
+        if (v < NBX_MAXVALUE) {
+            e = SL(p);
+            if (ids) e = T.perm[e];
+        }
+        so[r * NBX_WAVE + lane] = e;
+        sd[r * NBX_WAVE + lane] = v;
+    };
+    double x[KMAX <= 65 ? KMAX : 1];
+    knn_load<KMAX>(hd, lane, x);
+    int sum = 0;
+    for (int p = 0; p < kh; ++p) {
+        const double v = HD(p);
+        const int r = knn_rank<KMAX>(hd, lane, kh, x, v);
+        sum += r;
+        put(p, v, r);
+    }
+    // equal values share a rank, which lowers the sum of the ranks; those
+    // lanes rank again with the IDs (on a lattice every lane)
+    if (sum != kh * (kh - 1) / 2) {
+        for (int p = 0; p < kh; ++p) si[p * NBX_WAVE + lane] = HD(p) < NBX_MAXVALUE ? T.perm[SL(p)] : 0;
+        for (int i = 0; i < kh; ++i) {
+            const double v = HD(i);
+            const int32_t id = si[i * NBX_WAVE + lane];
+            int r = 0;
+#pragma unroll 8
+            for (int p = 0; p < kh; ++p) {
+                const double w = HD(p);
+                const int32_t ip = si[p * NBX_WAVE + lane];
+                r += w < v || (w == v && (ip < id || (ip == id && p < i))) ? 1 : 0;
+            }
+            put(i, v, r);
+        }
+    }
+}
+
+// scratch of one workgroup, in 4-byte words: slots by position, the output
+// rows in ascending order (entries and their d2), IDs by position
+#define KNN_BLKW(KM) ((KM) * NBX_WAVE * 5)
+#define KNN_CTR_STRIDE 16  // XCD counters 64 bytes apart
+
+// One wave of 64 queries, wave index g.
 template <int ND, int KMAX, int QSRC>
-__global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
-    __shared__ double hd[KMAX * NBX_WAVE];
-    __shared__ int32_t hid[KMAX * NBX_WAVE];
-    __shared__ double cx[ND * NBX_LEAF];
-    __shared__ int32_t cid[NBX_LEAF];
-    __shared__ double racc[NBX_WAVE];  // symmetric scatter into the wave's own queries
-    const int lane = threadIdx.x;
-    const int g = xcd_wave(blockIdx.x, gridDim.x) + A.wbeg;
+__device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, double *hd, double *cx, int32_t *sl,
+                                         int g, int lane) {
+    int32_t *const so = sl + KMAX * NBX_WAVE;                  // sorted entries
+    double *const sd = (double *)(so + KMAX * NBX_WAVE);       // their d2
+    int32_t *const si = (int32_t *)(sd + KMAX * NBX_WAVE);     // IDs by position
     const int kh = A.kh;
-    const int hc = heap_cap4(kh);
-    const int nfill = hc - kh;  // filler entries, first after sorting
     const bool listed = A.qlist != nullptr;
     const int wend = A.wbeg + A.wcnt;
     const int nq = (QSRC == NBX_Q_POINTS || listed) ? A.m
@@ -340,39 +413,73 @@ __global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
 #pragma unroll
         for (int d = 0; d < ND; ++d) q0[d] = valid ? T.x[d][qi] : 0.0;
     }
-    // the fillers sit at the bottom of the heap array, where a 4-ary heap of
-    // empty entries stays valid with them as leaves
-    for (int p = 0; p < hc; ++p) {
-        const bool fill = p >= kh;
-        HD(p) = fill ? -1.0 : NBX_MAXVALUE;
-        HI(p) = fill ? -1 : NBX_NOID;
+    KnnCtx<ND, KMAX> c;
+#pragma unroll
+    for (int gr = 0; gr < KShape<KMAX>::G; ++gr) {
+        constexpr int S = KShape<KMAX>::S;
+        for (int u = 0; u < S; ++u) HD(gr * S + u) = gr * S + u < kh ? NBX_MAXVALUE : -1.0;
+        c.gm[gr] = gr * S < kh ? NBX_MAXVALUE : -1.0;
+        c.gp[gr] = gr * S;
     }
-    LeafCtx<ND> c;
     c.exz = (QSRC == NBX_Q_SLOTS) && A.excl_zero;
     c.kth = NBX_MAXVALUE;
-    c.kid = NBX_NOID;
+    c.lost = INFINITY;
+    c.fill = kh >= NBX_LEAF ? kh : 0;
     const int npass = (QSRC != NBX_Q_SLOTS && A.periodic) ? 8 : 1;
-    for (int pass = 0; pass < npass; ++pass) {
+    uint32_t passes = 0;  // image passes the lane took part in
+    auto pass_begin = [&](int pass, bool again, float(&qc)[ND]) -> bool {
 #pragma unroll
         for (int d = 0; d < ND; ++d) c.q[d] = q0[d];
         c.act = valid;
         if (pass > 0) {
             double xp[3];
-            c.act = valid && image_pass(pass, q0, A.period, c.kth, ND == 6, xp);
+            const bool take = image_pass(pass, q0, A.period, c.kth, ND == 6, xp);
+            c.act = valid && take;
             c.q[0] = xp[0]; c.q[1] = xp[1]; c.q[2] = xp[2];
         }
-        if (!ballot(c.act)) continue;
-        float qc[ND];
+        if (again) c.act = (passes >> pass) & 1u;
+        else passes |= c.act ? 1u << pass : 0u;
 #pragma unroll
         for (int d = 0; d < ND; ++d) qc[d] = (float)readfirst_d(c.q[d]);
-        const int anc = (pass == 0 && QSRC != NBX_Q_POINTS && !listed) ? T.nleafp + 2 * g : -1;
-        knn_walk<ND, HeapLv<KMAX>::LV>(T, c, qc, anc, hd, hid, cx, cid, lane, hc);
+        return ballot(c.act) != 0;
+    };
+    const int own_leaves = (QSRC != NBX_Q_POINTS && !listed) ? T.nleafp + 2 * g : -1;
+    for (int pass = 0; pass < npass; ++pass) {
+        float qc[ND];
+        if (!pass_begin(pass, false, qc)) continue;
+        knn_walk<ND, KMAX, 0>(T, c, qc, pass == 0 ? own_leaves : -1, hd, sl, cx, lane, kh);
     }
     const double kth = c.kth;
 
+    // Ties at the k-th distance: something equal to it was discarded, so the
+    // entries at that distance may not be the smallest IDs.  Those entries
+    // are emptied (to the value of an ID past all others), every particle at
+    // exactly that distance is met again, and the smallest IDs stay.
+    const bool tied = valid && c.lost == kth && kth < NBX_MAXVALUE;
+    if (ballot(tied)) {
+        const uint32_t taken = passes;
+        if (tied) {
+            for (int p = 0; p < kh; ++p)
+                if (HD(p) == kth) HD(p) = -2.0 - 2147483648.0;
+        }
+        passes = tied ? taken : 0u;
+        for (int pass = 0; pass < npass; ++pass) {
+            float qc[ND];
+            if (!pass_begin(pass, true, qc)) continue;
+            knn_walk<ND, KMAX, 1>(T, c, qc, pass == 0 ? own_leaves : -1, hd, sl, cx, lane, kh);
+        }
+        if (tied) {
+            for (int p = 0; p < kh; ++p)
+                if (HD(p) < -1.5) HD(p) = kth;
+        }
+    }
+    __syncthreads();
+
     // ------------------------------------------------------------ densities
     // Symmetric scatter: contributions to the wave's own 64 queries (slot
-    // runs only) are summed in LDS and flushed with one atomic per query.
+    // runs only) are summed in LDS (over the leaf copy) and flushed with one
+    // atomic per query.
+    double *const racc = cx;
     const bool sym = QSRC == NBX_Q_SLOTS && A.dens == NBX_DO_SYM;
     const bool own = sym && !listed;
     double racc_own = 0.0;
@@ -382,50 +489,44 @@ __global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
     // query are undefined there)
     if (A.dens != NBX_DO_NONE && valid &&
         (QSRC == NBX_Q_SLOTS || A.dens == NBX_DO_GATHER || (QSRC == NBX_Q_POINTS && A.dens == NBX_DO_VEL))) {
-        bool bad = false;
+        const bool bad = !(kth < NBX_MAXVALUE);  // fewer than kh neighbours
         if (A.dens == NBX_DO_VEL || A.dens == NBX_DO_VELPHYS) {
             // CalcVelDensity: |dv| of the Nsearch physical neighbours, the
             // Nsmooth smallest of them, h_v = max/2, sum W(|dv|/h_v) h_v^-3.
-            // The kh entries move to positions 0..kh-1 first (sorted order).
+            // |dv| takes the place of d2; the terms are summed in the order
+            // of (|dv|, ID).
             // (CalcVelDensityPosition: the query's velocity comes with it)
             const int ns = A.nsmooth;
             const bool pts = QSRC == NBX_Q_POINTS;
             const double qvx = pts ? A.qv[0][qi] : T.x[3][qi];
             const double qvy = pts ? A.qv[1][qi] : T.x[4][qi];
             const double qvz = pts ? A.qv[2][qi] : T.x[5][qi];
-            heap_sort<HeapLv<KMAX>::LV>(hd, hid, lane, hc);
-            for (int p = 0; p < kh; ++p) {
-                const int32_t id = HI(p + nfill);
-                if (id == NBX_NOID) { bad = true; break; }
-                const int32_t s = T.inv[id];
-                double vx = qvx - T.x[3][s], vy = qvy - T.x[4][s], vz = qvz - T.x[5][s];
-                HD(p) = sqrt(vx * vx + vy * vy + vz * vz);
-                HI(p) = id;
-            }
             if (!bad) {
-                for (int p = (ns - 2) / 4; p >= 0; --p) heap_sift(hd, hid, lane, ns, p, HD(p), HI(p));
-                for (int p = ns; p < kh; ++p) {
-                    const double dv = HD(p);
-                    const int32_t iv = HI(p);
-                    if (kgt(HD(0), HI(0), dv, iv)) heap_sift(hd, hid, lane, ns, 0, dv, iv);
+                for (int p = 0; p < kh; ++p) {
+                    const int32_t s = SL(p);
+                    double vx = qvx - T.x[3][s], vy = qvy - T.x[4][s], vz = qvz - T.x[5][s];
+                    HD(p) = sqrt(vx * vx + vy * vy + vz * vz);
                 }
-                double hv = 0.5 * HD(0);
-                double norm = 1.0 / pow(hv, 3.0);
+                knn_sort<KMAX>(T, hd, sl, so, sd, si, lane, kh, false);
+                const double hv = 0.5 * sd[(ns - 1) * NBX_WAVE + lane];
+                const double norm = 1.0 / pow(hv, 3.0);
+                // CalcVelDensityWithPhysDensity (KDCalcSmoothQuantities.cxx:428-466):
+                // each term times W(r_ij / h) h^-3 / rho_i * m_i, with
+                // h = d2 of the Nsearch-th neighbour / 2 (no square root)
+                const bool phys = A.dens == NBX_DO_VELPHYS;
+                const double hp = 0.5 * kth;
+                const double pnorm = phys ? 1.0 / pow(hp, 3.0) : 0.0;
+                const double rhoi = phys ? A.rho_in[qi] : 1.0, mi = phys ? T.mass[qi] : 0.0;
                 double den = 0.0;
-                if (A.dens == NBX_DO_VEL) {
-                    for (int p = 0; p < ns; ++p) den = den + wsm_at(HD(p), hv, T.kern, T.kernres) * norm;
-                } else {
-                    // CalcVelDensityWithPhysDensity (KDCalcSmoothQuantities.cxx:428-466):
-                    // each term times W(r_ij / h) h^-3 / rho_i * m_i, with
-                    // h = d2 of the Nsearch-th neighbour / 2 (no square root)
-                    const double hp = 0.5 * kth;
-                    const double pnorm = 1.0 / pow(hp, 3.0);
-                    const double rhoi = A.rho_in[qi], mi = T.mass[qi];
-                    for (int p = 0; p < ns; ++p) {
-                        const int32_t s = T.inv[HI(p)];
+                for (int p = 0; p < ns; ++p) {
+                    const double v = sd[p * NBX_WAVE + lane];
+                    const double vW = wsm_at(v, hv, T.kern, T.kernres) * norm;
+                    if (!phys) {
+                        den = den + vW;
+                    } else {
+                        const int32_t s = so[p * NBX_WAVE + lane];
                         double dx = T.x[0][qi] - T.x[0][s], dy = T.x[1][qi] - T.x[1][s], dz = T.x[2][qi] - T.x[2][s];
                         double r = sqrt(dx * dx + dy * dy + dz * dz);
-                        double vW = wsm_at(HD(p), hv, T.kern, T.kernres) * norm;
                         double W = wsm_at(r, hp, T.kern, T.kernres) * pnorm;
                         den = den + vW * (W / rhoi * mi);
                     }
@@ -434,41 +535,45 @@ __global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
                 if (A.hout) A.hout[A.hout_by_id ? T.perm[qi] : qi] = hv;
             }
         } else {
-            double hi = 0.5 * sqrt(kth);
-            double norm = 1.0 / pow(hi, (double)ND);
+            const double hi = 0.5 * sqrt(kth);
+            const double norm = 1.0 / pow(hi, (double)ND);
             const double mi = QSRC == NBX_Q_SLOTS ? T.mass[qi] : 0.0;
+            // Wsm's lookup with the table step's division as a product; r/h
+            // stays a division, so the k-th neighbour's is exactly 2 and it
+            // takes the table's last entry, as in the reference
+            const double ck = 0.5 * (T.kernres - 1), top = (double)(T.kernres - 1);
             double acc = 0.0;
             // entries in groups of 8 so their slot/mass gathers are in flight
-            // together; summed in heap-position order
-            for (int p0 = 0; p0 < hc; p0 += 8) {
-                int32_t idv[8], sv[8];
+            // together; summed in position order
+            for (int p0 = 0; p0 < kh; p0 += 8) {
+                int32_t sv[8];
                 double dv[8], mv[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const bool in = p0 + u < hc;
-                    idv[u] = in ? HI(p0 + u) : -1;
-                    dv[u] = in ? HD(p0 + u) : 0.0;
+                    const bool in = p0 + u < kh;
+                    dv[u] = in ? HD(p0 + u) : NBX_MAXVALUE;
+                    sv[u] = dv[u] < NBX_MAXVALUE ? SL(p0 + u) : 0;
                 }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) sv[u] = (idv[u] >= 0 && idv[u] != NBX_NOID) ? T.inv[idv[u]] : 0;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) mv[u] = T.mass[sv[u]];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const int32_t id = idv[u];
-                    if (id < 0) continue;  // filler or past the end
-                    if (id == NBX_NOID) { bad = true; continue; }
+                    if (!(dv[u] < NBX_MAXVALUE)) continue;  // past the end, or missing
                     const int32_t s = sv[u];
-                    double W = wsm_at(sqrt(dv[u]), hi, T.kern, T.kernres);
+                    const double fi = sqrt(dv[u]) / hi * ck;
+                    double W = T.kern[T.kernres - 1];
+                    if (fi < top) {
+                        const int i = (int)fi;
+                        W = T.kern[i] + (T.kern[i + 1] - T.kern[i]) * (fi - (double)i);
+                    }
                     if (A.dens == NBX_DO_SYM) {
-                        double Wij = 0.5 * W * norm;
+                        const double Wij = 0.5 * W * norm;
                         acc = acc + Wij * mv[u];
                         const uint32_t r = (uint32_t)(s - g * NBX_WAVE);
                         if (own && r < NBX_WAVE) atomicAdd(&racc[r], Wij * mi);
                         else unsafeAtomicAdd(A.rho + s, Wij * mi);
                     } else {
-                        double Wij = W * norm;
-                        acc += Wij * mv[u];
+                        acc += W * norm * mv[u];
                     }
                 }
             }
@@ -482,12 +587,13 @@ __global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
     if (sym && valid) unsafeAtomicAdd(A.rho + qi, racc_own + (own ? racc[lane] : 0.0));
 
     // ------------------------------------------------------------ outputs
+    // (rows of the search only: the velocity densities ask for none)
     if (A.nn == nullptr && A.d2 == nullptr) return;
-    // (the velocity density sorted already and reused the entries)
-    if (valid && A.dens != NBX_DO_VEL && A.dens != NBX_DO_VELPHYS) heap_sort<HeapLv<KMAX>::LV>(hd, hid, lane, hc);
+    const bool ids = QSRC == NBX_Q_POINTS || A.layout == 0;
+    if (valid) knn_sort<KMAX>(T, hd, sl, so, sd, si, lane, kh, ids);
     __syncthreads();
     const int kout = A.kout;
-    const int off = ((A.drop == NBX_DROP_SMALLEST) ? 1 : 0) + ((A.dens == NBX_DO_VEL || A.dens == NBX_DO_VELPHYS) ? 0 : nfill);
+    const int off = (A.drop == NBX_DROP_SMALLEST) ? 1 : 0;
     const int total = NBX_WAVE * kout;
     for (int e = lane; e < total; e += NBX_WAVE) {
         int r = e / kout, t = e - r * kout;
@@ -500,39 +606,123 @@ __global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A) {
         else if (listed && A.list_rows) row = lr;
         else if (A.layout == 1) row = qr - A.row0;
         else row = T.perm[qr];
-        const int32_t id = hid[(t + off) * NBX_WAVE + r];
-        if (A.nn) {
-            int32_t v = -1;
-            if (id != NBX_NOID) v = (QSRC == NBX_Q_POINTS || A.layout == 0) ? id : T.inv[id];
-            A.nn[row * kout + t] = v;
+        if (A.nn) A.nn[row * kout + t] = so[(t + off) * NBX_WAVE + r];
+        if (A.d2) A.d2[row * kout + t] = sd[(t + off) * NBX_WAVE + r];
+    }
+    __syncthreads();  // the scratch is written again by the next wave of queries
+}
+
+// Persistent kernel, one wave per workgroup: workgroup b stays on XCD
+// (b mod 8), takes waves of queries from that XCD's contiguous share through
+// its counter, then from the other shares in turn, and owns one scratch
+// block.  Every ticket names one wave; a workgroup exits when all eight
+// counters have passed their shares' ends.
+template <int ND, int KMAX, int QSRC>
+__global__ __launch_bounds__(64) void k_knn(DevTree T, KnnArgs A, int nw, int32_t *scratch, int32_t *ctr) {
+    __shared__ double hd[KMAX * NBX_WAVE];
+    __shared__ double cx[ND * NBX_LEAF];  // leaf copy; then the symmetric scatter
+    static_assert(ND * NBX_LEAF >= NBX_WAVE, "the scatter lies over the leaf copy");
+    const int lane = threadIdx.x;
+    int32_t *sl = scratch + (size_t)blockIdx.x * KNN_BLKW(KMAX);
+    // in a VGPR pair: a scalar base would be spilled and reloaded per store
+    asm volatile("" : "+v"(sl));
+    const int x = blockIdx.x & 7, q8 = nw >> 3, r8 = nw & 7;
+    for (int s = 0; s < 8; ++s) {
+        const int y = (x + s) & 7;
+        const int ybeg = y * q8 + (y < r8 ? y : r8), ycnt = q8 + (y < r8 ? 1 : 0);
+        for (;;) {
+            int t = 0;
+            if (lane == 0) t = atomicAdd(ctr + y * KNN_CTR_STRIDE, 1);
+            t = __builtin_amdgcn_readfirstlane(t);
+            if (t >= ycnt) break;
+            knn_task<ND, KMAX, QSRC>(T, A, hd, cx, sl, A.wbeg + ybeg + t, lane);
         }
-        if (A.d2) A.d2[row * kout + t] = hd[(t + off) * NBX_WAVE + r];
     }
 }
 
-template <int ND, int KMAX>
-static void launch_q(const DevTree &T, const KnnArgs &A, int blocks, hipStream_t st) {
-    if (A.qsrc == NBX_Q_SLOTS)
-        hipLaunchKernelGGL((k_knn<ND, KMAX, NBX_Q_SLOTS>), dim3(blocks), dim3(NBX_WAVE), 0, st, T, A);
-    else if (A.qsrc == NBX_Q_PERIODIC)
-        hipLaunchKernelGGL((k_knn<ND, KMAX, NBX_Q_PERIODIC>), dim3(blocks), dim3(NBX_WAVE), 0, st, T, A);
-    else
-        hipLaunchKernelGGL((k_knn<ND, KMAX, NBX_Q_POINTS>), dim3(blocks), dim3(NBX_WAVE), 0, st, T, A);
+// Resident workgroups of one instance over the device, a multiple of 8.
+template <int ND, int KMAX, int QSRC>
+static int knn_resident() {
+    static std::atomic<int> grid{0};
+    int g = grid.load();
+    if (g == 0) {
+        int dev = 0, ncu = 0, per = 0;
+        if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+        if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) ncu = 256;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn<ND, KMAX, QSRC>, NBX_WAVE, 0) != hipSuccess ||
+            per <= 0)
+            per = 1;
+        g = (per * ncu) & ~7;
+        g = g < 8 ? 8 : g;
+        grid.store(g);
+    }
+    return g;
 }
 
-hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st) {
-    int blocks = (nqueries + NBX_WAVE - 1) / NBX_WAVE;
-    if (blocks == 0) return hipSuccess;
-    ProfScope ps(A.qlist ? "k_knn_fallback" : "k_knn_fp64", st);
-    if (T.nd == 6) {
-        if (A.kh <= 65) launch_q<6, 65>(T, A, blocks, st);
-        else if (A.kh <= 129) launch_q<6, 129>(T, A, blocks, st);
-        else return hipErrorInvalidValue;
+static int knn_kmax(int kh) { return kh <= 33 ? 33 : (kh <= 65 ? 65 : 132); }
+static const size_t KNN_CTR_BYTES = 8 * KNN_CTR_STRIDE * sizeof(int32_t);
+
+// f<ND, KMAX, QSRC>() of the instance that serves kh kept entries on T.nd
+#define KNN_DISPATCH(nd, km, qsrc, F)                                                           \
+    ((nd) == 6 ? ((km) <= 65 ? KNN_DISPATCH_Q(6, 65, qsrc, F) : KNN_DISPATCH_Q(6, 132, qsrc, F)) \
+               : ((km) <= 33   ? KNN_DISPATCH_Q(3, 33, qsrc, F)                                  \
+                  : (km) <= 65 ? KNN_DISPATCH_Q(3, 65, qsrc, F)                                  \
+                               : KNN_DISPATCH_Q(3, 132, qsrc, F)))
+#define KNN_DISPATCH_Q(ND, KM, qsrc, F)                             \
+    ((qsrc) == NBX_Q_SLOTS      ? F(ND, KM, NBX_Q_SLOTS)            \
+     : (qsrc) == NBX_Q_PERIODIC ? F(ND, KM, NBX_Q_PERIODIC) : F(ND, KM, NBX_Q_POINTS))
+
+// workgroups for nw waves: no more than are resident (or than there are waves)
+static int knn_grid(int nd, int kh, int qsrc, int64_t nw) {
+#define KNN_F(ND, KM, Q) knn_resident<ND, KM, Q>()
+    const int res = KNN_DISPATCH(nd, knn_kmax(kh), qsrc, KNN_F);
+#undef KNN_F
+    const int64_t want = (nw + 7) & ~(int64_t)7;
+    return (int)(want < res ? want : res);
+}
+static size_t knn_block_bytes(int nd, int kh) {
+    const int km = nd == 6 && kh <= 65 ? 65 : knn_kmax(kh);
+    return (size_t)KNN_BLKW(km) * sizeof(int32_t);
+}
+
+size_t nbx_knn_scratch_bytes(int nd, int kh, int qsrc, int64_t nqueries) {
+    const int64_t nw = (nqueries + NBX_WAVE - 1) / NBX_WAVE;
+    return KNN_CTR_BYTES + (size_t)knn_grid(nd, kh, qsrc, nw) * knn_block_bytes(nd, kh);
+}
+size_t nbx_knn_scratch_least(int nd, int kh) { return KNN_CTR_BYTES + 8 * knn_block_bytes(nd, kh); }
+
+template <int ND, int KMAX, int QSRC>
+static void knn_start(const DevTree &T, const KnnArgs &A, int grid, int nw, int32_t *scr, int32_t *ctr,
+                      hipStream_t st) {
+    hipLaunchKernelGGL((k_knn<ND, KMAX, QSRC>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, nw, scr, ctr);
+}
+
+hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st, void *work,
+                          size_t work_bytes) {
+    const int nw = (nqueries + NBX_WAVE - 1) / NBX_WAVE;
+    if (nw == 0) return hipSuccess;
+    if (A.kh < 1 || A.kh > 129) return hipErrorInvalidValue;
+    int grid = knn_grid(T.nd, A.kh, A.qsrc, nw);
+    const size_t blk = knn_block_bytes(T.nd, A.kh);
+    void *mem = work;
+    if (mem) {
+        // as many workgroups as the scratch given has blocks for
+        if (work_bytes < nbx_knn_scratch_least(T.nd, A.kh)) return hipErrorInvalidValue;
+        const size_t fit = (work_bytes - KNN_CTR_BYTES) / blk;
+        if (fit < (size_t)grid) grid = (int)fit & ~7;
     } else {
-        if (A.kh <= 33) launch_q<3, 33>(T, A, blocks, st);
-        else if (A.kh <= 65) launch_q<3, 65>(T, A, blocks, st);
-        else if (A.kh <= 129) launch_q<3, 129>(T, A, blocks, st);
-        else return hipErrorInvalidValue;
+        const hipError_t e = hipMallocAsync(&mem, KNN_CTR_BYTES + (size_t)grid * blk, st);
+        if (e != hipSuccess) return e;
     }
-    return hipGetLastError();
+    int32_t *ctr = (int32_t *)mem, *scr = (int32_t *)((char *)mem + KNN_CTR_BYTES);
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, ctr, 0, (int64_t)(8 * KNN_CTR_STRIDE));
+    {
+        ProfScope ps(A.qsrc != NBX_Q_POINTS && A.qlist ? "k_knn_fallback" : "k_knn_fp64", st);
+#define KNN_F(ND, KM, Q) knn_start<ND, KM, Q>(T, A, grid, nw, scr, ctr, st)
+        KNN_DISPATCH(T.nd, knn_kmax(A.kh), A.qsrc, KNN_F);
+#undef KNN_F
+    }
+    const hipError_t e = hipGetLastError();
+    if (!work) hipFreeAsync(mem, st);
+    return e;
 }

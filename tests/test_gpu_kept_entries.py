@@ -1,0 +1,79 @@
+"""FP64 search at the edges of its kept-entry groups (33, 65 and 129 entries)
+and where ties cross the k-th distance: rows equal the (d2, ID)-sorted brute
+force entry by entry."""
+import numpy as np
+import pytest
+
+import oracle
+from nbodylib_amd import datagen
+
+pytestmark = pytest.mark.gpu
+
+KS = [1, 2, 31, 32, 33, 34, 64, 65, 66, 128, 129]
+
+
+def _rows(q, pos, k, target):
+    """(d2, ID)-sorted rows; target: d2 == 0 is no neighbour."""
+    d = np.zeros((len(q), len(pos)))
+    for c in range(3):
+        d += (q[:, c][:, None] - pos[:, c][None, :]) ** 2
+    if target:
+        d[d == 0.0] = np.inf
+    ids = np.lexsort((np.broadcast_to(np.arange(len(pos)), d.shape), d), axis=1)[:, :k]
+    return ids, np.take_along_axis(d, ids, 1)
+
+
+def _lattice(g):
+    ax = np.arange(g) + 0.5
+    p = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3)
+    return p[np.random.default_rng(g).permutation(len(p))]  # IDs in no spatial order
+
+
+@pytest.mark.parametrize("k", KS)
+@pytest.mark.parametrize("kind", ["clustered", "lattice"])
+def test_rows_exact(gpu, kind, k):
+    import nbodylib_amd as nb
+
+    pos = _lattice(9) if kind == "lattice" else datagen.clustered(911, 1.0, nhalo=4, seed=5)[0]
+    print(f"kept entries {kind} n={len(pos)} k={k}", flush=True)
+    t = nb.KDTree(pos, kerntype=nb.KSPH)
+    nn, d2 = t.FindNearest(k)
+    ids, dd = _rows(pos, pos, k, True)
+    assert np.array_equal(d2, dd) and np.array_equal(nn, ids)
+    # positions: particles (found at d2 = 0), lattice cell centres, far outside
+    q = np.concatenate([pos[:70], pos[:40] + 0.5, pos[:5] + 1e3])
+    nn, d2 = t.FindNearestPosPoints(q, k)
+    ids, dd = _rows(q, pos, k, False)
+    assert np.array_equal(d2, dd) and np.array_equal(nn, ids)
+
+
+@pytest.mark.parametrize("k", [6, 7, 32, 64, 128])
+def test_periodic_lattice(gpu, k):
+    import nbodylib_amd as nb
+
+    pos = _lattice(8)
+    print(f"periodic lattice k={k}", flush=True)
+    t = nb.KDTree(pos, kerntype=nb.KSPH, period=8.0)
+    nn, d2 = t.FindNearest(k)
+    bi, bd = oracle.knn_brute(pos, k, mode=1, period=8.0)
+    assert np.array_equal(d2, bd) and np.array_equal(np.sort(nn, 1), np.sort(bi, 1))
+
+
+def test_coinciding_particles(gpu):
+    """More particles at one point than are kept: the smallest IDs stay, and a
+    target search, which skips them all, reports the others."""
+    import nbodylib_amd as nb
+
+    rng = np.random.default_rng(8)
+    pos = rng.random((600, 3))
+    pos[rng.permutation(600)[:90]] = 0.25
+    t = nb.KDTree(pos, kerntype=nb.KSPH)
+    q = np.concatenate([np.full((3, 3), 0.25), pos[:66]])
+    for k in (20, 40):
+        print(f"coinciding k={k}", flush=True)
+        nn, d2 = t.FindNearestPosPoints(q, k)
+        ids, dd = _rows(q, pos, k, False)
+        assert np.array_equal(d2, dd) and np.array_equal(nn, ids)
+        nn, d2 = t.FindNearest(k)
+        ids, dd = _rows(pos, pos, k, True)
+        assert np.array_equal(d2, dd) and np.array_equal(nn, ids)
