@@ -310,10 +310,12 @@ int nbx_sph_density_adjoint_dev(const double *pos_dev, const double *mass_dev, c
 /* The same forward and adjoint over the tree's own neighbour lists, with no
  * list of all n kept: each particle's k nearest under CalcDensity's search
  * (KDCalcSmoothQuantities.cxx:227: self and d2 == 0 excluded, no period) are
- * recomputed for one block of block_rows tree slots at a time (rounded up
- * to a multiple of 1024; <= 0 takes every slot at once) into a buffer of
- * block_rows * k * 4 bytes and consumed there.  The list memory is that
- * buffer instead of n * k * 4 bytes.  TPHYS trees, either form (the
+ * found again.  The forward sums them in the search and keeps no list
+ * (block_rows is not read).  The adjoint finds them for one block of
+ * block_rows tree slots at a time (rounded up to a multiple of 1024; <= 0
+ * takes every slot at once) into a buffer of block_rows * k * 4 bytes and
+ * consumes them there.  The list memory is that buffer instead of
+ * n * k * 4 bytes.  TPHYS trees, either form (the
  * precision form's neighbour sets are the plain form's).  All by ID, device
  * pointers: rho_by_id, h_by_id (nullable), g_by_id = dL/drho, dpos_by_id
  * (3*n SoA) and dmass_by_id, the last two written (not accumulated). */

@@ -17,20 +17,6 @@
 // atomics (LDS ones for particles of the same block).
 #include "nbx_kernels.h"
 
-// Cubic spline without branches: with t = max(2 - q, 0), s = max(1 - q, 0),
-// W = t^3/4 - s^3 (= 1 - 1.5q^2 + 0.75q^3 on [0,1], (2-q)^3/4 on [1,2], 0
-// beyond) and W' = -0.75 t^2 + 3 s^2.
-__device__ __forceinline__ double w_cubic(double q) {
-    const double t = fmax(2.0 - q, 0.0), s = fmax(1.0 - q, 0.0);
-    return 0.25 * t * t * t - s * s * s;
-}
-__device__ __forceinline__ double dw_cubic(double q) {
-    const double t = fmax(2.0 - q, 0.0), s = fmax(1.0 - q, 0.0);
-    return -0.75 * t * t + 3.0 * s * s;
-}
-
-#define SIGMA3 0.31830988618379067154  // 1/pi
-
 // Contributions to particles of the same 1024-particle block (most of them
 // when the arrays are in tree order) are summed in LDS and flushed with one
 // atomic per particle and component; the rest go straight to HBM.
@@ -59,7 +45,7 @@ __global__ __launch_bounds__(ADJ_B) void k_sph_fwd(const double *__restrict__ X,
         const double h = 0.5 * sqrt(dx * dx + dy * dy + dz * dz);
         if (hout) hout[i] = h;
         const double ih = 1.0 / h;
-        const double norm = 0.5 * SIGMA3 * ih * ih * ih;
+        const double norm = 0.5 * NBX_SIGMA3 * ih * ih * ih;
         for (int j0 = 0; j0 < k; j0 += ADJ_G) {
             int64_t qv[ADJ_G];
             double rv[ADJ_G], mv[ADJ_G];
@@ -130,16 +116,16 @@ __global__ __launch_bounds__(ADJ_B) void k_sph_adj(const double *__restrict__ X,
                 const double r = sqrt(ex * ex + ey * ey + ez * ez);
                 const double qq = r * ih;
                 const double W = w_cubic(qq), dW = dw_cubic(qq);
-                const double w = 0.5 * SIGMA3 * W * ih3;
+                const double w = 0.5 * NBX_SIGMA3 * W * ih3;
                 const double a = gi * mv[u] + gv[u] * mi;
                 const uint64_t lr = (uint64_t)(q - i0);
                 const bool loc = lr < ADJ_B;
                 if (loc) atomicAdd(&lm[lr], w * gi);
                 else unsafeAtomicAdd(dmass + q, w * gi);
                 gm += w * gv[u];
-                Hs += a * (-0.5 * SIGMA3 * (qq * dW + 3.0 * W) * ih4);
+                Hs += a * (-0.5 * NBX_SIGMA3 * (qq * dW + 3.0 * W) * ih4);
                 if (r > 0.0) {
-                    const double f = a * 0.5 * SIGMA3 * dW * ih4 / r;
+                    const double f = a * 0.5 * NBX_SIGMA3 * dW * ih4 / r;
                     gx += f * ex;
                     gy += f * ey;
                     gz += f * ez;
@@ -212,45 +198,4 @@ hipError_t nbx_launch_sph_adj(const double *pos, const double *mass, const int32
     const double *X[3] = {pos, pos + n, pos + 2 * n};
     double *D[3] = {dpos, dpos + n, dpos + 2 * n};
     return nbx_launch_sph_adj_rows(X, mass, nbr, n, 0, n, k, g, D, dmass, st);
-}
-
-// Move each row's k-th neighbour -- its largest (d2, ID), the one that sets
-// h -- into the last column (rows of slots from a search whose rows are not
-// in exact FP64 order).  d2 summed x -> z without FMA, as the search's.
-// A row with fewer than k neighbours (entries -1, possible when exact
-// duplicates are excluded) raises *err and its missing entries become the
-// row's own slot, so no later pass reads outside the arrays.
-__global__ void k_kth_last(const double *__restrict__ X, const double *__restrict__ Y, const double *__restrict__ Z,
-                           const int32_t *__restrict__ perm, int32_t *nbr, int64_t r0, int64_t nr, int k,
-                           int32_t *err) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nr) return;
-    const int64_t i = r0 + r;
-    int32_t *row = nbr + r * k;
-    const double xi = X[i], yi = Y[i], zi = Z[i];
-    int best = 0;
-    double bd = -1.0;
-    int32_t bid = -1;
-    for (int j = 0; j < k; ++j) {
-        if (row[j] < 0) {
-            row[j] = (int32_t)i;
-            atomicOr(err, 1);
-        }
-        const int32_t s = row[j];
-        const double ex = xi - X[s], ey = yi - Y[s], ez = zi - Z[s];
-        const double d = ex * ex + ey * ey + ez * ez;
-        const int32_t id = perm[s];
-        if (d > bd || (d == bd && id > bid)) { best = j; bd = d; bid = id; }
-    }
-    const int32_t tmp = row[k - 1];
-    row[k - 1] = row[best];
-    row[best] = tmp;
-}
-
-hipError_t nbx_launch_kth_last(const double *const *X, const int32_t *perm, int32_t *nbr, int64_t r0, int64_t nr, int k,
-                               int32_t *err, hipStream_t st) {
-    const int blocks = (int)((nr + 255) / 256);
-    if (!blocks) return hipSuccess;
-    hipLaunchKernelGGL(k_kth_last, dim3(blocks), dim3(256), 0, st, X[0], X[1], X[2], perm, nbr, r0, nr, k, err);
-    return hipGetLastError();
 }

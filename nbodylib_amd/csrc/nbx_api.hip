@@ -651,13 +651,8 @@ extern "C" int nbx_knn_dev(nbx_tree *t, int32_t k, int32_t variant, int32_t layo
     A.d2 = d2_dev;
     hipStream_t st = (hipStream_t)stream;
     if (mixed_ok(t, k) && A.qsrc == NBX_Q_SLOTS && A.kh == k) {
-        // FP32 search; when distances are asked for, the rows' FP64 d2 and
-        // their FP64 order come from a row pass over the selected entries
-        DevBufs bufs(st);
-        if (d2_dev && !A.nn) HIPCK(bufs.alloc(&A.nn, sizeof(int32_t) * (size_t)t->n * k));
-        A.d2 = nullptr;
+        // rows in key order, or with d2 in (d2, ID) order
         HIPCK(run_mixed(t, A, k, st));
-        if (d2_dev) HIPCK(nbx_launch_rows_fp64(t->view(), A.nn, d2_dev, k, layout, st));
         return NBX_OK;
     }
     HIPCK(run_plain(t, A, nq, st));
@@ -1440,78 +1435,26 @@ extern "C" int nbx_ball_mark(nbx_tree *t, const double *x, int64_t exclude_id, d
 // ------------------------------------------------------------------ differentiation form over the tree
 // The frozen list is the tree's own: each particle's k nearest under
 // CalcDensity's search (KDCalcSmoothQuantities.cxx:227; self and d2 = 0
-// excluded, no period), recomputed for one block of tree slots at a time
-// into a buffer of that block and consumed there, so no list of all n is
-// kept.  Forward and adjoint are row-separable (every row adds its own
-// terms), so the blocks sum to the whole.  Work runs in slot order on the
-// tree's sorted coordinates; results are scattered back by ID.
-static int sph_tree_impl(nbx_tree *t, int32_t k, int64_t block, const double *g_id, double *rho_id, double *h_id,
-                         double *dpos_id, double *dmass_id, hipStream_t st) {
+// excluded, no period).  Work runs in slot order on the tree's sorted
+// coordinates; results are scattered back by ID.
+static int sph_tree_check(nbx_tree *t, int32_t k) {
     if (!t) return fail(NBX_ERR_ARG, "NULL tree");
     if (t->nd != 3 || t->tvel) return fail(NBX_ERR_UNSUPPORTED, "the differentiation form needs a TPHYS tree");
-    const bool mixed = mixed_ok(t, k);
     if (k < 2 || k > heap_cap(t)) return fail(NBX_ERR_UNSUPPORTED, "k out of range");
-    const int64_t n = t->n;
-    if (n <= k) return fail(NBX_ERR_SEARCH, "fewer than k + 1 particles");
-    if (block <= 0) block = n;
-    block = (block + 1023) / 1024 * 1024;  // whole waves and whole 1024-row windows
-    if (block > n) block = (n + 1023) / 1024 * 1024;
-    DevBufs bufs(st);
-    int32_t *nbr = nullptr, *err = nullptr;
-    HIPCK(bufs.alloc(&nbr, sizeof(int32_t) * (size_t)block * k));
-    HIPCK(bufs.alloc(&err, sizeof(int32_t)));
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, err, 0, (int64_t)1);
-    const double *X[3] = {t->xs[0], t->xs[1], t->xs[2]};
-    double *rs = nullptr, *hs = nullptr, *gs = nullptr, *ds = nullptr, *ms = nullptr;
-    const bool adj = g_id != nullptr;
-    if (adj) {
-        HIPCK(bufs.alloc(&gs, sizeof(double) * n));
-        HIPCK(bufs.alloc(&ds, sizeof(double) * 3 * n));
-        HIPCK(bufs.alloc(&ms, sizeof(double) * n));
-        hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, st, g_id, t->perm, n, gs);
-        hipLaunchKernelGGL(k_fill_f64, dim3(nblk(3 * n)), dim3(256), 0, st, ds, 0.0, 3 * n);
-        hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, ms, 0.0, n);
-    } else {
-        HIPCK(bufs.alloc(&rs, sizeof(double) * n));
-        if (h_id) HIPCK(bufs.alloc(&hs, sizeof(double) * n));
-        hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, rs, 0.0, n);
-    }
-    // the search's temporaries, reused by every block
-    Workspace ws = {nullptr, 0, 0};
-    ws.cap = mixed ? 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1)
-                   : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, block);
-    HIPCK(bufs.alloc(&ws.base, ws.cap));
-    double *D[3] = {ds, ds ? ds + n : nullptr, ds ? ds + 2 * n : nullptr};
-    for (int64_t r0 = 0; r0 < n; r0 += block) {
-        const int64_t nr = std::min<int64_t>(block, n - r0);
-        KnnArgs A;
-        memset(&A, 0, sizeof(A));
-        A.qsrc = NBX_Q_SLOTS;
-        A.excl_zero = 1;
-        A.kh = k;
-        A.kout = k;
-        A.layout = NBX_LAYOUT_BY_SLOT;
-        A.dens = NBX_DO_NONE;
-        A.nn = nbr;
-        A.wbeg = (int32_t)(r0 / NBX_WAVE);
-        A.wcnt = (int32_t)((nr + NBX_WAVE - 1) / NBX_WAVE);
-        A.row0 = (int32_t)r0;
-        ws.used = 0;
-        hipError_t e = mixed ? run_mixed(t, A, k, st, &ws) : run_plain(t, A, A.wcnt * NBX_WAVE, st, &ws);
-        if (e == hipSuccess) e = nbx_launch_kth_last(X, t->perm, nbr, r0, nr, k, err, st);
-        if (e == hipSuccess)
-            e = adj ? nbx_launch_sph_adj_rows(X, t->mass, nbr, n, r0, nr, k, gs, D, ms, st)
-                    : nbx_launch_sph_fwd_rows(X, t->mass, nbr, n, r0, nr, k, rs, hs, st);
-        if (e != hipSuccess) return hipfail(e, "differentiation form");
-    }
-    if (adj) {
-        for (int c = 0; c < 3; ++c)
-            hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, ds + c * n, t->perm, dpos_id + c * n, n);
-        hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, ms, t->perm, dmass_id, n);
-    } else {
-        hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, rs, t->perm, rho_id, n);
-        if (h_id) hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, hs, t->perm, h_id, n);
-    }
+    if (t->n <= k) return fail(NBX_ERR_SEARCH, "fewer than k + 1 particles");
+    return NBX_OK;
+}
+static KnnArgs sph_tree_search(int32_t k) {
+    KnnArgs A;
+    memset(&A, 0, sizeof(A));
+    A.qsrc = NBX_Q_SLOTS;
+    A.excl_zero = 1;
+    A.kh = k;
+    A.kout = k;
+    A.layout = NBX_LAYOUT_BY_SLOT;
+    return A;
+}
+static int sph_tree_end(const int32_t *err, hipStream_t st) {
     int32_t herr = 0;
     HIPCK(hipGetLastError());
     HIPCK(hipMemcpyAsync(&herr, err, sizeof(int32_t), hipMemcpyDeviceToHost, st));
@@ -1520,16 +1463,97 @@ static int sph_tree_impl(nbx_tree *t, int32_t k, int64_t block, const double *g_
     return NBX_OK;
 }
 
+// Forward: the density is summed in the search itself, so no list is made
+// and one launch covers every row: 1M particles at k = 32 take 1.38 ms in
+// kernels.  With each 256K-row block's list written, its k-th neighbour moved
+// last and a density kernel reading it back they took 3.7 ms.
+static int sph_tree_fwd(nbx_tree *t, int32_t k, double *rho_id, double *h_id, hipStream_t st) {
+    const int rc = sph_tree_check(t, k);
+    if (rc) return rc;
+    const int64_t n = t->n;
+    const bool mixed = mixed_ok(t, k);
+    ScratchLease lease(t, density_ws_bytes(t, k, mixed, k), st);
+    if (lease.err != hipSuccess) return hipfail(lease.err, "differentiation form scratch");
+    double *rs = lease.ws.carve<double>(sizeof(double) * n);
+    int32_t *err = lease.ws.carve<int32_t>(sizeof(int32_t));
+    if (!rs || !err) return fail(NBX_ERR_ARG, "scratch too small");
+    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, rs, 0.0, n);
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, err, 0, (int64_t)1);
+    KnnArgs A = sph_tree_search(k);
+    A.dens = NBX_DO_SPLINE;
+    A.rho = rs;
+    A.hout = h_id;
+    A.hout_by_id = 1;
+    A.err = err;
+    const hipError_t e = mixed ? run_mixed(t, A, k, st, &lease.ws) : run_plain(t, A, (int)n, st, &lease.ws);
+    if (e != hipSuccess) return hipfail(e, "differentiation form");
+    hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, rs, t->perm, rho_id, n);
+    return sph_tree_end(err, st);
+}
+
+// Adjoint: the list is recomputed for one block of tree slots at a time into
+// a buffer of that block and consumed there, so no list of all n is kept.
+// It is row-separable (every row adds its own terms), so the blocks sum to
+// the whole.
+static int sph_tree_adj(nbx_tree *t, int32_t k, int64_t block, const double *g_id, double *dpos_id, double *dmass_id,
+                        hipStream_t st) {
+    const int rc = sph_tree_check(t, k);
+    if (rc) return rc;
+    const int64_t n = t->n;
+    const bool mixed = mixed_ok(t, k);
+    if (block <= 0) block = n;
+    block = (block + 1023) / 1024 * 1024;  // whole waves and whole 1024-row windows
+    if (block > n) block = (n + 1023) / 1024 * 1024;
+    DevBufs bufs(st);
+    int32_t *nbr = nullptr, *err = nullptr;
+    double *gs = nullptr, *ds = nullptr, *ms = nullptr;
+    HIPCK(bufs.alloc(&nbr, sizeof(int32_t) * (size_t)block * k));
+    HIPCK(bufs.alloc(&err, sizeof(int32_t)));
+    HIPCK(bufs.alloc(&gs, sizeof(double) * n));
+    HIPCK(bufs.alloc(&ds, sizeof(double) * 3 * n));
+    HIPCK(bufs.alloc(&ms, sizeof(double) * n));
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, err, 0, (int64_t)1);
+    hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, st, g_id, t->perm, n, gs);
+    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(3 * n)), dim3(256), 0, st, ds, 0.0, 3 * n);
+    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, ms, 0.0, n);
+    // the search's temporaries, reused by every block
+    Workspace ws = {nullptr, 0, 0};
+    ws.cap = mixed ? 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1)
+                   : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, block);
+    HIPCK(bufs.alloc(&ws.base, ws.cap));
+    const double *X[3] = {t->xs[0], t->xs[1], t->xs[2]};
+    double *D[3] = {ds, ds + n, ds + 2 * n};
+    for (int64_t r0 = 0; r0 < n; r0 += block) {
+        const int64_t nr = std::min<int64_t>(block, n - r0);
+        KnnArgs A = sph_tree_search(k);
+        A.nn = nbr;
+        A.exact_rows = 1;  // the k-th neighbour, which sets h, comes last
+        A.miss_self = 1;   // no entry points outside the arrays
+        A.err = err;
+        A.wbeg = (int32_t)(r0 / NBX_WAVE);
+        A.wcnt = (int32_t)((nr + NBX_WAVE - 1) / NBX_WAVE);
+        A.row0 = (int32_t)r0;
+        ws.used = 0;
+        hipError_t e = mixed ? run_mixed(t, A, k, st, &ws) : run_plain(t, A, A.wcnt * NBX_WAVE, st, &ws);
+        if (e == hipSuccess) e = nbx_launch_sph_adj_rows(X, t->mass, nbr, n, r0, nr, k, gs, D, ms, st);
+        if (e != hipSuccess) return hipfail(e, "differentiation form");
+    }
+    for (int c = 0; c < 3; ++c)
+        hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, ds + c * n, t->perm, dpos_id + c * n, n);
+    hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, ms, t->perm, dmass_id, n);
+    return sph_tree_end(err, st);
+}
+
 extern "C" int nbx_sph_density_fwd_tree_dev(nbx_tree *t, int32_t k, int64_t block_rows, double *rho_by_id_dev,
                                             double *h_by_id_dev, void *stream) {
     if (!rho_by_id_dev) return fail(NBX_ERR_ARG, "NULL output");
-    return sph_tree_impl(t, k, block_rows, nullptr, rho_by_id_dev, h_by_id_dev, nullptr, nullptr, (hipStream_t)stream);
+    (void)block_rows;  // no list is made
+    return sph_tree_fwd(t, k, rho_by_id_dev, h_by_id_dev, (hipStream_t)stream);
 }
 extern "C" int nbx_sph_density_adjoint_tree_dev(nbx_tree *t, int32_t k, int64_t block_rows, const double *g_by_id_dev,
                                                 double *dpos_by_id_dev, double *dmass_by_id_dev, void *stream) {
     if (!g_by_id_dev || !dpos_by_id_dev || !dmass_by_id_dev) return fail(NBX_ERR_ARG, "NULL argument");
-    return sph_tree_impl(t, k, block_rows, g_by_id_dev, nullptr, nullptr, dpos_by_id_dev, dmass_by_id_dev,
-                         (hipStream_t)stream);
+    return sph_tree_adj(t, k, block_rows, g_by_id_dev, dpos_by_id_dev, dmass_by_id_dev, (hipStream_t)stream);
 }
 
 // ------------------------------------------------------------------ differentiation form

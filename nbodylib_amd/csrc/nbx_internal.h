@@ -198,6 +198,20 @@ __device__ __forceinline__ double wsm_at(double rij, double hi, const double *ke
     return kern[i] + (kern[i + 1] - kern[i]) * (r - delta * i) / delta;
 }
 
+// The analytic cubic spline of the differentiation form (WSPH,
+// SmoothingKernels.h:32-37), without branches: with t = max(2 - q, 0), s =
+// max(1 - q, 0), W = t^3/4 - s^3 (= 1 - 1.5q^2 + 0.75q^3 on [0,1], (2-q)^3/4
+// on [1,2], 0 beyond) and W' = -0.75 t^2 + 3 s^2.
+#define NBX_SIGMA3 0.31830988618379067154  // its 3-D norm, 1/pi
+__device__ __forceinline__ double w_cubic(double q) {
+    const double t = fmax(2.0 - q, 0.0), s = fmax(1.0 - q, 0.0);
+    return 0.25 * t * t * t - s * s * s;
+}
+__device__ __forceinline__ double dw_cubic(double q) {
+    const double t = fmax(2.0 - q, 0.0), s = fmax(1.0 - q, 0.0);
+    return -0.75 * t * t + 3.0 * s * s;
+}
+
 // Lock-free union-find over slots (hook the larger root under the smaller).
 //
 // A parent pointer only ever points to a smaller slot of the same set, and

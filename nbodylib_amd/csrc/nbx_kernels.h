@@ -50,6 +50,7 @@ hipError_t nbx_sort_pairs_u64(void *temp, size_t &temp_bytes, uint64_t *kin, uin
 #define NBX_DO_GATHER 2  // CalcDensityParticle: W m_j gathered
 #define NBX_DO_VEL 3     // CalcVelDensity
 #define NBX_DO_VELPHYS 4  // CalcVelDensityWithPhysDensity: CalcVelDensity weighted by W(r) m_i / rho_i
+#define NBX_DO_SPLINE 5  // the differentiation form's forward: 1/2 W scattered to both ends, analytic spline (3-D)
 // Output drop rule for the k+1 periodic search
 #define NBX_DROP_NONE 0
 #define NBX_DROP_SMALLEST 1
@@ -75,7 +76,7 @@ struct KnnArgs {
     double *rho;        // by slot (density); by query row for position queries
     double *hout;       // as rho, or by ID with hout_by_id (nullable)
     int32_t hout_by_id;  // particle queries: hout[ID] rather than hout[slot]
-    int32_t *err;       // set to 1 if a row has fewer than kh neighbours
+    int32_t *err;       // set to 1 if a row has fewer than kh neighbours (densities, miss_self)
     // nullable: the queries in the order the waves take them -- slots (FP64
     // re-run of mixed-form fallbacks, lists of particles) or, for position
     // queries, their indices
@@ -84,6 +85,8 @@ struct KnnArgs {
     int32_t wbeg, wcnt;
     int32_t row0;  // subtracted from the slot of a row written in the by-slot layout
     int32_t list_rows;  // with qlist: row r of the output is the query qlist[r]
+    int32_t exact_rows;  // precision form: rows in ascending (d2, ID) order (always so when d2 is given)
+    int32_t miss_self;   // particle queries: a missing entry becomes the row's own slot and sets *err
     double band_rel;    // precision form: least relative half-width of the FP64 re-check band
 };
 
@@ -101,11 +104,6 @@ size_t nbx_knn_scratch_least(int nd, int kh);
 hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double *ext, int32_t *fallback_list,
                                 int32_t *fallback_count, hipStream_t st, void *work = nullptr, size_t work_bytes = 0);
 size_t nbx_mixed_scratch_bytes(int nd, int kh);
-// FP64 d2 of every entry of the n rows nn (by ID, layout 0, or by slot,
-// layout 1) written by the precision-form kernel, rows re-sorted ascending
-// by (d2, ID); k <= 64.
-hipError_t nbx_launch_rows_fp64(const DevTree &T, int32_t *nn, double *d2, int k, int layout, hipStream_t st);
-
 // ------------------------------------------------------------------ FOF
 // Link rule of a FOF run: pairs link when their value is below lim.  Plain
 // FOF: d2 against b^2.  FOFCriterion with FOF3d / FOF6d: the comparator's sum
@@ -206,11 +204,6 @@ hipError_t nbx_launch_sph_fwd_rows(const double *const *X, const double *mass, c
 hipError_t nbx_launch_sph_adj_rows(const double *const *X, const double *mass, const int32_t *nbr, int64_t n,
                                    int64_t r0, int64_t nr, int k, const double *g, double *const *D, double *dmass,
                                    hipStream_t st);
-// Each row's largest (d2, ID) neighbour moved into its last column; rows
-// with a missing entry (-1) set *err and have it replaced by their own slot.
-hipError_t nbx_launch_kth_last(const double *const *X, const int32_t *perm, int32_t *nbr, int64_t r0, int64_t nr, int k,
-                               int32_t *err, hipStream_t st);
-
 // ------------------------------------------------------------------ profiling
 struct ProfScope {
     hipStream_t st;

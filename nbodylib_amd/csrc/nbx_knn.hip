@@ -480,7 +480,8 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
     // runs only) are summed in LDS (over the leaf copy) and flushed with one
     // atomic per query.
     double *const racc = cx;
-    const bool sym = QSRC == NBX_Q_SLOTS && A.dens == NBX_DO_SYM;
+    const bool spline = ND == 3 && QSRC == NBX_Q_SLOTS && A.dens == NBX_DO_SPLINE;
+    const bool sym = QSRC == NBX_Q_SLOTS && (A.dens == NBX_DO_SYM || spline);
     const bool own = sym && !listed;
     double racc_own = 0.0;
     if (own) racc[lane] = 0.0;
@@ -536,7 +537,8 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
             }
         } else {
             const double hi = 0.5 * sqrt(kth);
-            const double norm = 1.0 / pow(hi, (double)ND);
+            const double ih = 1.0 / hi;
+            const double norm = spline ? NBX_SIGMA3 * ih * ih * ih : 1.0 / pow(hi, (double)ND);
             const double mi = QSRC == NBX_Q_SLOTS ? T.mass[qi] : 0.0;
             // Wsm's lookup with the table step's division as a product; r/h
             // stays a division, so the k-th neighbour's is exactly 2 and it
@@ -560,13 +562,18 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
                 for (int u = 0; u < 8; ++u) {
                     if (!(dv[u] < NBX_MAXVALUE)) continue;  // past the end, or missing
                     const int32_t s = sv[u];
-                    const double fi = sqrt(dv[u]) / hi * ck;
-                    double W = T.kern[T.kernres - 1];
-                    if (fi < top) {
-                        const int i = (int)fi;
-                        W = T.kern[i] + (T.kern[i + 1] - T.kern[i]) * (fi - (double)i);
+                    double W;
+                    if (spline) {
+                        W = w_cubic(sqrt(dv[u]) * ih);
+                    } else {
+                        const double fi = sqrt(dv[u]) / hi * ck;
+                        W = T.kern[T.kernres - 1];
+                        if (fi < top) {
+                            const int i = (int)fi;
+                            W = T.kern[i] + (T.kern[i + 1] - T.kern[i]) * (fi - (double)i);
+                        }
                     }
-                    if (A.dens == NBX_DO_SYM) {
+                    if (sym) {
                         const double Wij = 0.5 * W * norm;
                         acc = acc + Wij * mv[u];
                         const uint32_t r = (uint32_t)(s - g * NBX_WAVE);
@@ -577,7 +584,7 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
                     }
                 }
             }
-            if (A.dens == NBX_DO_SYM) racc_own = acc;
+            if (sym) racc_own = acc;
             else A.rho[qi] = acc;
             if (A.hout) A.hout[A.hout_by_id ? T.perm[qi] : qi] = hi;
         }
@@ -590,6 +597,14 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
     // (rows of the search only: the velocity densities ask for none)
     if (A.nn == nullptr && A.d2 == nullptr) return;
     const bool ids = QSRC == NBX_Q_POINTS || A.layout == 0;
+    if (A.miss_self && valid && !(kth < NBX_MAXVALUE)) {
+        atomicOr(A.err, 1);
+        for (int p = 0; p < kh; ++p)
+            if (!(HD(p) < NBX_MAXVALUE)) {
+                HD(p) = 0.5 * NBX_MAXVALUE;
+                SL(p) = qi;
+            }
+    }
     if (valid) knn_sort<KMAX>(T, hd, sl, so, sd, si, lane, kh, ids);
     __syncthreads();
     const int kout = A.kout;

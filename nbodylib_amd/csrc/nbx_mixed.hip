@@ -44,6 +44,9 @@
 // carries a storage error proportional to its leaf's size, which in
 // clustered data can reach 1e-5 of the neighbour distance); the search --
 // every candidate test and heap operation -- stays in FP32.
+#include <algorithm>
+#include <atomic>
+
 #include "nbx_kernels.h"
 
 typedef float fx8 __attribute__((ext_vector_type(8)));
@@ -589,9 +592,22 @@ __device__ __forceinline__ int verify_walk(const DevTree &T, const double *q, bo
 #define SKC(p) kb[(p) * NBX_WAVE + lane]
 #define SLB(p) slb[(p) * NBX_WAVE + lane]
 
+// What an instance does with the neighbours it found.  Instances of their
+// own, because code in the table instance changes its register allocation.
+//  * EXACT orders the rows before they leave LDS and computes d2 as they are
+//    written, coalesced.  A kernel that read the rows back, one thread per
+//    row, and sorted them in per-thread arrays (scratch memory) took 1.53 ms
+//    for 1M rows of 20; here they cost under 0.1 ms.
+//  * SPLINE sums the differentiation form's forward over the neighbours while
+//    their slots are in LDS, so no list is written or read.
+#define MX_TABLE 0   // the table densities, rows in key order
+#define MX_EXACT 1   // no density; rows in ascending (d2, ID) order, with d2 when asked for
+#define MX_SPLINE 2  // the analytic-spline symmetric density (NBX_DO_SPLINE), no rows
+
 // One wave of 64 consecutive queries (tree order), wave index g.
-// k = kh - 1 neighbours; A.dens: NBX_DO_NONE / NBX_DO_SYM / NBX_DO_GATHER.
-template <int ND, int KMAX>
+// k = kh - 1 neighbours; A.dens: NBX_DO_NONE / NBX_DO_SYM / NBX_DO_GATHER, or
+// as MODE says.
+template <int ND, int KMAX, int MODE>
 __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, const double *ext, int32_t *fb_list,
                                          int32_t *fb_count, uint32_t *hk, float *cx, double *racc, uint32_t *sl,
                                          uint32_t *slb, uint32_t *skc, int g, int lane) {
@@ -827,16 +843,22 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
     // Symmetric scatter: contributions to the wave's own 64 queries (about
     // half of all neighbour entries) are summed in LDS and flushed with one
     // atomic per query; the rest go straight to HBM.
-    const bool sym = A.dens == NBX_DO_SYM;
+    const bool sym = MODE == MX_SPLINE || (MODE == MX_TABLE && A.dens == NBX_DO_SYM);
     double racc_own = 0.0;
-    const bool dens_here = ok && A.dens != NBX_DO_NONE;
+    const bool dens_here = MODE != MX_EXACT && ok && A.dens != NBX_DO_NONE;
     if (sym) racc[lane] = 0.0;
     __syncthreads();
     if (dens_here) {
         // weights from FP64 distances of the k selected neighbours (the FP32
         // offsets carry a storage error proportional to the leaf size)
         const double hi = 0.5 * sqrt(Dk);
-        const double norm = 1.0 / pow(hi, (double)ND);
+        double norm, ih = 0.0;
+        if constexpr (MODE == MX_SPLINE) {
+            ih = 1.0 / hi;
+            norm = 0.5 * NBX_SIGMA3 * ih * ih * ih;
+        } else {
+            norm = 1.0 / pow(hi, (double)ND);
+        }
         const double mi = T.mass[qi];
         // the table lookup of Wsm (KDCalcSmoothQuantities.cxx:12-15) with
         // its division by the table step turned into a product: index
@@ -861,16 +883,20 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
             for (int u = 0; u < MX_DB; ++u) {
                 if (p0 + u >= k) break;
                 const int32_t s = sv[u];
-                const double fi = sqrt(d2v[u]) / hi * ck;
                 double W;
-                if (!(fi < (double)(kres - 1))) {
-                    W = T.kern[kres - 1];
+                if constexpr (MODE == MX_SPLINE) {
+                    W = w_cubic(sqrt(d2v[u]) * ih);
                 } else {
-                    const int i = (int)fi;
-                    W = T.kern[i] + (T.kern[i + 1] - T.kern[i]) * (fi - (double)i);
+                    const double fi = sqrt(d2v[u]) / hi * ck;
+                    if (!(fi < (double)(kres - 1))) {
+                        W = T.kern[kres - 1];
+                    } else {
+                        const int i = (int)fi;
+                        W = T.kern[i] + (T.kern[i + 1] - T.kern[i]) * (fi - (double)i);
+                    }
                 }
                 if (sym) {
-                    double Wij = 0.5 * W * norm;
+                    const double Wij = MODE == MX_SPLINE ? W * norm : 0.5 * W * norm;
                     acc = acc + Wij * mv[u];
                     const uint32_t r = (uint32_t)(s - g * NBX_WAVE);
                     if (r < NBX_WAVE) atomicAdd(&racc[r], Wij * mi);
@@ -888,7 +914,45 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
     if (sym && valid) unsafeAtomicAdd(A.rho + qi, racc_own + racc[lane]);
 
     // ---------------------------------------------------------------- outputs
-    if (A.nn == nullptr) return;
+    if constexpr (MODE == MX_SPLINE) return;
+    if (A.nn == nullptr && (MODE != MX_EXACT || A.d2 == nullptr)) return;
+    if constexpr (MODE == MX_EXACT) {
+        // The entries come in key order, which departs from (d2, ID) order
+        // only between neighbouring keys.  Passes that carry the larger of
+        // two neighbours along run until one changes nothing (one or two
+        // passes; as many as a shell has members on a lattice).
+        auto slot_put = [&](int p, int32_t s) {
+            if constexpr (GT) SKC(p) = (uint32_t)s;
+            else SLB(p) = (uint32_t)s;
+        };
+        for (bool again = ok; ballot(again);) {
+            if (again) {
+                again = false;
+                int32_t sc = slot_final(0);
+                double dc = d64<ND>(T, c.q, sc);
+                for (int p0 = 1; p0 < k; p0 += MX_DB) {
+                    int32_t sv[MX_DB];
+                    double dv[MX_DB];
+#pragma unroll
+                    for (int u = 0; u < MX_DB; ++u) {
+                        sv[u] = p0 + u < k ? slot_final(p0 + u) : qi;
+                        dv[u] = d64<ND>(T, c.q, sv[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < MX_DB; ++u) {
+                        if (p0 + u >= k) break;
+                        bool below = dv[u] < dc;
+                        if (dv[u] == dc) below = T.perm[sv[u]] < T.perm[sc];
+                        slot_put(p0 + u - 1, below ? sv[u] : sc);
+                        sc = below ? sc : sv[u];
+                        dc = below ? dc : dv[u];
+                        again |= below;
+                    }
+                }
+                slot_put(k - 1, sc);
+            }
+        }
+    }
     const uint64_t okm = ballot(ok);
     __syncthreads();
     // entry e = lane + 64 i of the wave's rows is row r = e / k, column
@@ -914,7 +978,15 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
         if constexpr (GT) s = (int32_t)hk[t * NBX_WAVE + r];  // decoded above
         else s = (int32_t)slb[t * NBX_WAVE + r];
         int64_t row = A.layout == 1 ? qr - A.row0 : T.perm[qr];
-        A.nn[row * k + t] = A.layout == 1 ? s : T.perm[s];
+        if (MODE != MX_EXACT || A.nn) A.nn[row * k + t] = A.layout == 1 ? s : T.perm[s];
+        if constexpr (MODE == MX_EXACT) {
+            if (A.d2) {
+                double q[ND];
+#pragma unroll
+                for (int d = 0; d < ND; ++d) q[d] = T.x[d][qr];
+                A.d2[row * k + t] = d64<ND>(T, q, s);
+            }
+        }
     }
 }
 
@@ -934,7 +1006,7 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
 // scratch words per workgroup: 16-bit handles and the visit table, and for
 // KMAX > 33 the slots and keys in ascending order
 #define MX_BLKW(KM) ((KM) * (NBX_WAVE / 2) + MX_V + ((KM) <= 33 ? 0 : 2 * (KM) * NBX_WAVE))
-template <int ND, int KMAX>
+template <int ND, int KMAX, int MODE>
 __global__ __launch_bounds__(64) void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list,
                                                    int32_t *fb_count, uint32_t *scratch, int32_t *ctr) {
     __shared__ uint32_t hk[KMAX * NBX_WAVE];
@@ -962,7 +1034,7 @@ __global__ __launch_bounds__(64) void k_knn_mixed(DevTree T, KnnArgs A, const do
             if (lane == 0) t = atomicAdd(ctr + y * MX_CTR_STRIDE, 1);
             t = __builtin_amdgcn_readfirstlane(__shfl(t, 0));
             if (t >= ycnt) break;
-            mix_task<ND, KMAX>(T, A, ext, fb_list, fb_count, hk, cx, racc, sl, slb, skc, A.wbeg + ybeg + t, lane);
+            mix_task<ND, KMAX, MODE>(T, A, ext, fb_list, fb_count, hk, cx, racc, sl, slb, skc, A.wbeg + ybeg + t, lane);
         }
     }
 }
@@ -974,30 +1046,41 @@ __global__ void k_mx_zero(int32_t *p, int cnt) {
 
 // Resident workgroups of one instance over the device, a multiple of 8
 // (every XCD gets workgroups) and at least 8.
-template <int ND, int KMAX>
+template <int ND, int KMAX, int MODE>
 static int mx_grid() {
-    static int grid = 0;
-    if (grid == 0) {
+    static std::atomic<int> grid{0};
+    if (grid.load() == 0) {
         int dev = 0, ncu = 0, per = 0;
         if (hipGetDevice(&dev) != hipSuccess) dev = 0;
         if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) ncu = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn_mixed<ND, KMAX>, NBX_WAVE, 0) != hipSuccess ||
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn_mixed<ND, KMAX, MODE>, NBX_WAVE, 0) != hipSuccess ||
             per <= 0)
             per = 8;
         const int gsz = (per * ncu) & ~7;
-        grid = gsz < 8 ? 8 : gsz;
+        grid.store(gsz < 8 ? 8 : gsz);
     }
-    return grid;
+    return grid.load();
 }
 
-static int mx_launch_grid(int nd, int km) {
-    return nd == 3 ? (km == 33 ? mx_grid<3, 33>() : mx_grid<3, 65>())
-                   : (km == 33 ? mx_grid<6, 33>() : mx_grid<6, 65>());
+template <int ND, int KMAX>
+static int mx_grid_mode(int mode) {
+    if constexpr (ND == 3)
+        if (mode == MX_SPLINE) return mx_grid<ND, KMAX, MX_SPLINE>();
+    return mode == MX_EXACT ? mx_grid<ND, KMAX, MX_EXACT>() : mx_grid<ND, KMAX, MX_TABLE>();
+}
+static int mx_launch_grid(int nd, int km, int mode) {
+    return nd == 3 ? (km == 33 ? mx_grid_mode<3, 33>(mode) : mx_grid_mode<3, 65>(mode))
+                   : (km == 33 ? mx_grid_mode<6, 33>(mode) : mx_grid_mode<6, 65>(mode));
+}
+static int mx_mode(const KnnArgs &A) {
+    return A.dens == NBX_DO_SPLINE ? MX_SPLINE : (A.exact_rows || A.d2 ? MX_EXACT : MX_TABLE);
 }
 
 size_t nbx_mixed_scratch_bytes(int nd, int kh) {
     const int km = kh <= 33 ? 33 : 65;
-    return (size_t)mx_launch_grid(nd, km) * MX_BLKW(km) * sizeof(uint32_t) + 8 * MX_CTR_STRIDE * sizeof(int32_t);
+    int g = 0;  // enough for any instance
+    for (int mode = 0; mode < 3; ++mode) g = std::max(g, mx_launch_grid(nd, km, mode));
+    return (size_t)g * MX_BLKW(km) * sizeof(uint32_t) + 8 * MX_CTR_STRIDE * sizeof(int32_t);
 }
 
 hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double *ext, int32_t *fallback_list,
@@ -1007,7 +1090,11 @@ hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double
     if ((T.nd != 3 && T.nd != 6) || A.kh > 65 || A.kh < 2 || !T.kernf || !T.org || !T.boxf || !ext)
         return hipErrorInvalidValue;
     const int km = A.kh <= 33 ? 33 : 65;
-    const int grid = mx_launch_grid(T.nd, km);
+    const int mode = mx_mode(A);
+    // densities and exact rows do not come together; the spline is 3-D
+    if ((mode == MX_EXACT && A.dens != NBX_DO_NONE) || (mode == MX_SPLINE && (T.nd != 3 || A.nn || A.d2)))
+        return hipErrorInvalidValue;
+    const int grid = mx_launch_grid(T.nd, km, mode);
     const size_t nscr = (size_t)grid * MX_BLKW(km);
     const size_t need = nscr * sizeof(uint32_t) + 8 * MX_CTR_STRIDE * sizeof(int32_t);
     void *mem = work;
@@ -1023,76 +1110,20 @@ hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double
     hipLaunchKernelGGL(k_mx_zero, dim3(1), dim3(8 * MX_CTR_STRIDE), 0, st, ctr, 8 * MX_CTR_STRIDE);
     {
         ProfScope ps("k_knn_mixed", st);
-#define MIXL(ND, KM)                                                                                            \
-    hipLaunchKernelGGL((k_knn_mixed<ND, KM>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, ext, fallback_list, \
+#define MIXL(ND, KM, MODE)                                                                                       \
+    hipLaunchKernelGGL((k_knn_mixed<ND, KM, MODE>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, ext, fallback_list, \
                        fallback_count, scr, ctr)
         if (T.nd == 3) {
-            if (km == 33) MIXL(3, 33);
-            else MIXL(3, 65);
+            if (mode == MX_TABLE) { if (km == 33) MIXL(3, 33, MX_TABLE); else MIXL(3, 65, MX_TABLE); }
+            else if (mode == MX_EXACT) { if (km == 33) MIXL(3, 33, MX_EXACT); else MIXL(3, 65, MX_EXACT); }
+            else { if (km == 33) MIXL(3, 33, MX_SPLINE); else MIXL(3, 65, MX_SPLINE); }
         } else {
-            if (km == 33) MIXL(6, 33);
-            else MIXL(6, 65);
+            if (mode == MX_TABLE) { if (km == 33) MIXL(6, 33, MX_TABLE); else MIXL(6, 65, MX_TABLE); }
+            else { if (km == 33) MIXL(6, 33, MX_EXACT); else MIXL(6, 65, MX_EXACT); }
         }
 #undef MIXL
     }
     e = hipGetLastError();
     if (!work) hipFreeAsync(mem, st);
     return e;
-}
-
-// FP64 distances for rows written by the precision-form kernel, whose rows
-// are in FP32 key order: each row's entries get their FP64 d2 (summed over
-// the dimensions in order, no FMA, as every FP64 distance here) and are
-// sorted ascending by (d2, ID) -- the LoadNN order of the FP64 form
-// (KDFindNearest.cxx:11-24) with ties to the smaller ID.  Rows and entries
-// are by ID (layout 0) or by slot (layout 1).  One thread per row.
-template <int ND, int KM>
-__global__ __launch_bounds__(256) void k_rows_fp64(DevTree T, int32_t *nn, double *d2, int k, int layout) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= T.n) return;
-    const int32_t qs = layout == 0 ? T.inv[r] : (int32_t)r;
-    double q[ND];
-#pragma unroll
-    for (int d = 0; d < ND; ++d) q[d] = T.x[d][qs];
-    double dv[KM];
-    int32_t iv[KM], ev[KM];
-    int32_t *row = nn + r * k;
-    for (int j = 0; j < k; ++j) {
-        const int32_t e = row[j];
-        // a missing neighbour (-1) keeps d2 = MAXVALUE and sorts last
-        const bool miss = e < 0;
-        const int32_t s = miss ? 0 : (layout == 0 ? T.inv[e] : e);
-        const double v = miss ? NBX_MAXVALUE : d64<ND>(T, q, s);
-        const int32_t id = miss ? 0x7fffffff : (layout == 0 ? e : T.perm[e]);
-        // insertion into the sorted prefix (the rows come nearly sorted)
-        int p = j;
-        while (p > 0 && (dv[p - 1] > v || (dv[p - 1] == v && iv[p - 1] > id))) {
-            dv[p] = dv[p - 1];
-            iv[p] = iv[p - 1];
-            ev[p] = ev[p - 1];
-            --p;
-        }
-        dv[p] = v;
-        iv[p] = id;
-        ev[p] = e;
-    }
-    for (int j = 0; j < k; ++j) {
-        row[j] = ev[j];
-        d2[r * k + j] = dv[j];
-    }
-}
-
-hipError_t nbx_launch_rows_fp64(const DevTree &T, int32_t *nn, double *d2, int k, int layout, hipStream_t st) {
-    if (T.n == 0) return hipSuccess;
-    if (k < 1 || k > 64) return hipErrorInvalidValue;
-    const int blocks = (int)((T.n + 255) / 256);
-    ProfScope ps("k_rows_fp64", st);
-    if (T.nd == 3) {
-        if (k <= 32) hipLaunchKernelGGL((k_rows_fp64<3, 32>), dim3(blocks), dim3(256), 0, st, T, nn, d2, k, layout);
-        else hipLaunchKernelGGL((k_rows_fp64<3, 64>), dim3(blocks), dim3(256), 0, st, T, nn, d2, k, layout);
-    } else {
-        if (k <= 32) hipLaunchKernelGGL((k_rows_fp64<6, 32>), dim3(blocks), dim3(256), 0, st, T, nn, d2, k, layout);
-        else hipLaunchKernelGGL((k_rows_fp64<6, 64>), dim3(blocks), dim3(256), 0, st, T, nn, d2, k, layout);
-    }
-    return hipGetLastError();
 }

@@ -1,6 +1,7 @@
-"""FP64 search at the edges of its kept-entry groups (33, 65 and 129 entries)
-and where ties cross the k-th distance: rows equal the (d2, ID)-sorted brute
-force entry by entry."""
+"""Searches at the edges of their kept-entry groups (33, 65 and 129 entries) and
+where ties cross the k-th distance: rows equal the (d2, ID)-sorted brute force
+entry by entry.  The forward density summed in the search equals the one over
+the same lists."""
 import numpy as np
 import pytest
 
@@ -31,15 +32,21 @@ def _lattice(g):
 
 @pytest.mark.parametrize("k", KS)
 @pytest.mark.parametrize("kind", ["clustered", "lattice"])
-def test_rows_exact(gpu, kind, k):
+@pytest.mark.parametrize("form", ["plain", "mixed"])
+def test_rows_exact(gpu, form, kind, k):
     import nbodylib_amd as nb
 
     pos = _lattice(9) if kind == "lattice" else datagen.clustered(911, 1.0, nhalo=4, seed=5)[0]
-    print(f"kept entries {kind} n={len(pos)} k={k}", flush=True)
-    t = nb.KDTree(pos, kerntype=nb.KSPH)
+    print(f"kept entries {form} {kind} n={len(pos)} k={k}", flush=True)
+    t = nb.KDTree(pos, kerntype=nb.KSPH, form=nb.FORM_PLAIN if form == "plain" else nb.FORM_MIXED)
     nn, d2 = t.FindNearest(k)
     ids, dd = _rows(pos, pos, k, True)
     assert np.array_equal(d2, dd) and np.array_equal(nn, ids)
+    if form == "mixed":  # by slot: the same rows through the tree order
+        order = t.order()
+        ns, ds = t.FindNearest(k, layout=nb.LAYOUT_BY_SLOT)
+        assert np.array_equal(ds, dd[order]) and np.array_equal(order[ns], ids[order])
+        return
     # positions: particles (found at d2 = 0), lattice cell centres, far outside
     q = np.concatenate([pos[:70], pos[:40] + 0.5, pos[:5] + 1e3])
     nn, d2 = t.FindNearestPosPoints(q, k)
@@ -77,3 +84,28 @@ def test_coinciding_particles(gpu):
         nn, d2 = t.FindNearest(k)
         ids, dd = _rows(pos, pos, k, True)
         assert np.array_equal(d2, dd) and np.array_equal(nn, ids)
+
+
+@pytest.mark.parametrize("k", [2, 31, 32, 33, 64, 65, 129])
+@pytest.mark.parametrize("form", ["plain", "mixed"])
+def test_forward_in_search(gpu, form, k):
+    """Sums of k own and as many scattered terms as a particle is a neighbour
+    to: a few hundred roundings of 1.1e-16 each, in any order."""
+    import torch
+
+    import nbodylib_amd as nb
+    from nbodylib_amd.device import DeviceTree, sph_density
+
+    n = 1500
+    print(f"forward in search {form} k={k}", flush=True)
+    pos = torch.tensor(datagen.clustered(n, 1.0, nhalo=5, seed=k)[0].T.copy(), device="cuda")
+    m = torch.tensor(datagen.lognormal_masses(n, k), device="cuda")
+    t = DeviceTree(pos, mass=m, kerntype=nb.KSPH, form=nb.FORM_PLAIN if form == "plain" else nb.FORM_MIXED)
+    nn = torch.empty((n, k), dtype=torch.int32, device="cuda")
+    d2 = torch.empty((n, k), dtype=torch.float64, device="cuda")
+    t.knn(k, nn, d2, layout=nb.LAYOUT_BY_ID)
+    ro, ho = sph_density(pos, m, nn)
+    rho, h = torch.empty_like(ro), torch.empty_like(ho)
+    t.sph_density(k, rho, h, block_rows=1024)
+    assert torch.equal(h, ho)
+    assert float((rho / ro - 1.0).abs().max()) < 1e-12
