@@ -211,10 +211,37 @@ struct MixSrc {
     const float *xf[ND == 6 ? 6 : 1];
 };
 
+// What a leaf visit reads in 6-D, loaded a leaf ahead: this lane's candidate,
+// and the leaf's origin.
+struct MixPre {
+    float st[6];
+    double o[6];
+};
+__device__ __forceinline__ void mix_load(const MixSrc<6> &S, int leaf, int lane, MixPre &p) {
+#pragma unroll
+    for (int d = 0; d < 6; ++d) p.st[d] = S.xf[d][leaf * NBX_LEAF + (lane & (NBX_LEAF - 1))];
+    const double2 *op = (const double2 *)(S.org + (size_t)leaf * 6);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const double2 v = op[i];
+        p.o[2 * i] = v.x;
+        p.o[2 * i + 1] = v.y;
+    }
+}
+
+// 6-D: a query in LDS, 8 floats: its coordinates and its threshold (two
+// 16-byte accesses)
+#define MX_QW 8
+__device__ __forceinline__ void mix_put_query(float *qb, int at, const float *q, float th) {
+    float4 *p = (float4 *)qb + 2 * at;
+    p[0] = make_float4(q[0], q[1], q[2], q[3]);
+    p[1] = make_float4(q[4], q[5], th, 0.0f);
+}
+
 template <int ND, int KMAX>
 __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<ND> &c, bool want,
                                          uint32_t *hk, uint32_t *sl, float *cx, int lane,
-                                         uint32_t (&gm)[GShape<KMAX>::G]) {
+                                         uint32_t (&gm)[GShape<KMAX>::G], const MixPre &pre) {
     const int base = leaf * NBX_LEAF;
     // A kept candidate is stored as a 16-bit handle, its leaf's visit number
     // << 5 | its index in the leaf; the wave's visit table (vt, right after
@@ -228,7 +255,7 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
         c.nvis += 1;
     }
     // candidate (lane mod 32) of this leaf: the tested point in phase 1 and
-    // this lane's part of the LDS copy used in phase 2
+    // this lane's part of the LDS copy used in phase 2 (6-D: loaded ahead)
     float st[ND];
     if constexpr (ND == 3) {
         const float4 v = S.xq[base + (lane & (NBX_LEAF - 1))];
@@ -237,13 +264,13 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
         st[2] = v.z;
     } else {
 #pragma unroll
-        for (int d = 0; d < ND; ++d) st[d] = S.xf[d][base + (lane & (NBX_LEAF - 1))];
+        for (int d = 0; d < ND; ++d) st[d] = pre.st[d];
     }
     // query relative to this leaf's centre, rounded once to FP32
     const double *o = S.org + (size_t)leaf * ND;
     float qv[ND];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) qv[d] = (float)(c.q[d] - ((cdptr)o)[d]);
+    for (int d = 0; d < ND; ++d) qv[d] = (float)(c.q[d] - (ND == 6 ? pre.o[d] : ((cdptr)o)[d]));
     const float th = __uint_as_float(c.root);
     uint32_t mask = 0u;
     if constexpr (ND == 3) {
@@ -289,45 +316,38 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
         mask = __builtin_bitreverse32(mask);
     } else {
         // Phase 1, transposed: the lanes that want this leaf put their query
-        // offsets and thresholds in LDS (qb, tb, which alias cx), and each
-        // step tests two of them against the 32 candidates, one candidate per
-        // lane; the ballot's halves are the two queries' accept masks,
-        // selected into the owning lanes' mask register.  Lanes that do not
-        // want the leaf have no candidate in it: their FP64 bound already
-        // exceeds their largest kept key.
+        // offsets and thresholds in LDS (over cx), and each step tests two of
+        // them against the 32 candidates, one candidate per lane; the
+        // ballot's halves are the two queries' accept masks, left in LDS for
+        // their lanes.  Lanes that do not want the leaf have no candidate in
+        // it: their bound already exceeds their largest kept key.
         const uint64_t wm = ballot(want);
         const int nwq = __popcll(wm);
-        float *qb = cx;
-        float *tb = cx + ND * NBX_WAVE;
-        if (want) {
-            const int wr = __builtin_amdgcn_mbcnt_hi((uint32_t)(wm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)wm, 0u));
-#pragma unroll
-            for (int d = 0; d < ND; ++d) qb[d * NBX_WAVE + wr] = qv[d];
-            tb[wr] = th;
+        const int wr = __builtin_amdgcn_mbcnt_hi((uint32_t)(wm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)wm, 0u));
+        if (want) mix_put_query(cx, wr, qv, th);
+        if ((nwq & 1) && lane == 0) {
+            // an odd count's last step tests a second query that passes nothing
+            const float none[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            mix_put_query(cx, nwq, none, -1.0f);
         }
         __syncthreads();
-        uint64_t wrest = wm;  // wanting lanes not yet given a mask, in rank order
+        const float4 *qm = (const float4 *)cx + 2 * (lane >> 5);
+        uint32_t *mb = (uint32_t *)(cx + MX_QW * NBX_WAVE);
         for (int it = 0; it < nwq; it += 2) {
-            const int qs = it + (lane >> 5);
-            const int qc = qs < nwq ? qs : it;
-            float t = qb[qc] - st[0];
-            float dd = t * t;
-#pragma unroll
-            for (int d = 1; d < ND; ++d) {
-                t = qb[d * NBX_WAVE + qc] - st[d];
-                dd = __builtin_fmaf(t, t, dd);
-            }
-            const uint64_t pm = ballot(qs < nwq && dd <= tb[qc]);
-            const int l0 = (int)__builtin_ctzll(wrest);
-            wrest &= wrest - 1;
-            mask = lane == l0 ? (uint32_t)pm : mask;
-            if (it + 1 < nwq) {
-                const int l1 = (int)__builtin_ctzll(wrest);
-                wrest &= wrest - 1;
-                mask = lane == l1 ? (uint32_t)(pm >> 32) : mask;
-            }
+            const float4 a = qm[2 * it], b = qm[2 * it + 1];
+            const float t0 = a.x - st[0], t1 = a.y - st[1], t2 = a.z - st[2], t3 = a.w - st[3], t4 = b.x - st[4],
+                        t5 = b.y - st[5];
+            float dd = t0 * t0;
+            dd = __builtin_fmaf(t1, t1, dd);
+            dd = __builtin_fmaf(t2, t2, dd);
+            dd = __builtin_fmaf(t3, t3, dd);
+            dd = __builtin_fmaf(t4, t4, dd);
+            dd = __builtin_fmaf(t5, t5, dd);
+            const uint64_t pm = ballot(dd <= b.z);
+            if (lane == 0) *(uint64_t *)(mb + it) = pm;
         }
         __syncthreads();
+        mask = want ? mb[wr] : 0u;
     }
     if (c.self >= base && c.self < base + NBX_LEAF) mask &= ~(1u << (c.self - base));
     if (!c.act) mask = 0;
@@ -408,6 +428,133 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
     __syncthreads();
 }
 
+// The 8 nodes three levels below an opened node, tested at once (6-D).  A
+// wave of 64 queries opens about 600 leaves there, each wanted by 10 of them
+// on average, so testing one node at a time for all 64 lanes spends 2500 box
+// tests, each behind a load of its own, mostly on lanes that ruled the node
+// out above.  Here the lanes that want the node are compacted into LDS and
+// each step tests 8 of them against the 8 boxes, one pair per lane; the 7
+// planes that order them are evaluated one per lane.  The tests use the
+// bounds from before the first of the 8 is entered, so they never miss one
+// that the walk by single nodes opens.
+// Measured on 2.1M particles, k = 64: 51.9 -> 42.4 ms with the leaves under a
+// height-3 node tested so, 39.2 with the queries and masks of this test and
+// of the leaf scan in 16-byte LDS rows, 37.1 with the height-3 nodes under a
+// height-6 node tested the same way and the leaf data loaded a leaf ahead
+// (308,000 -> 273,000 VALU per wave over the last two).  It still waits for
+// half its cycles: 18.9 KB of LDS a wave leave 2 waves per SIMD.
+// order: the 8 in visiting order, 3 bits each; todo: bit i set when the i-th
+// of that order is open; returns the lane's own mask, by child.
+template <int ND>
+__device__ __forceinline__ uint32_t mix_test8(const float *boxp, const float *planep, int node, int height, float th,
+                                              const float *q32, const float *qc, int anc, bool want, float *cx,
+                                              int lane, uint32_t &order, uint32_t &todo) {
+    const int l8 = lane & 7;
+    // the box of this lane's child
+    const float4 *bp = (const float4 *)(boxp + (size_t)(8 * node + l8) * 2 * ND);
+    float bx[2 * ND];
+#pragma unroll
+    for (int i = 0; i < ND / 2; ++i) {
+        const float4 v = bp[i];
+        bx[4 * i] = v.x;
+        bx[4 * i + 1] = v.y;
+        bx[4 * i + 2] = v.z;
+        bx[4 * i + 3] = v.w;
+    }
+    // which half comes first: bit 0 the node's, bits 1-2 its children's,
+    // bits 3-6 its grandchildren's
+    uint32_t right;
+    {
+        const int lv = l8 == 0 ? 0 : (l8 < 3 ? 1 : 2);
+        const int nid = (node << lv) + (l8 == 7 ? 0 : l8 + 1 - (1 << lv));
+        const float4 *pp = (const float4 *)(planep + (size_t)nid * 8);
+        const float4 p0 = pp[0], p1 = pp[1];
+        float s = __builtin_fmaf(p0.x, qc[0], 0.0f);
+        s = __builtin_fmaf(p0.y, qc[1], s);
+        s = __builtin_fmaf(p0.z, qc[2], s);
+        s = __builtin_fmaf(p0.w, qc[3], s);
+        s = __builtin_fmaf(p1.x, qc[4], s);
+        s = __builtin_fmaf(p1.y, qc[5], s);
+        bool r = s > p1.z;
+        if ((anc >> (height - lv)) == nid) r = (anc >> (height - 1 - lv)) & 1;  // the wave's own leaves first
+        right = (uint32_t)ballot(r) & 0x7fu;
+    }
+    const uint64_t wm = ballot(want);
+    const int nwq = __popcll(wm);
+    const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(wm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)wm, 0u));
+    if (want) mix_put_query(cx, rank, q32, th);
+    __syncthreads();
+    // the step's ballot holds 8 bits per query: byte r of mb is the mask of
+    // the query with rank r
+    uint8_t *mb = (uint8_t *)(cx + MX_QW * NBX_WAVE);
+    const float4 *qm = (const float4 *)cx;
+    uint64_t any = 0;
+    for (int it = 0; it < nwq; it += 8) {
+        const int qs = it + (lane >> 3);
+        const int q = qs < nwq ? qs : it;
+        const float4 a = qm[2 * q], b = qm[2 * q + 1];
+        const float x[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
+        float s = 0.0f;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {  // box_lb32
+            const float t = fmaxf(bx[d] - x[d], x[d] - bx[ND + d]);
+            const float tl = fmaxf(__builtin_fmaf(t, 1.0f - 0x1p-20f, -0x1p-20f * fabsf(x[d])), 0.0f);
+            s = __builtin_fmaf(tl, tl, s);
+        }
+        const uint64_t pm = ballot(qs < nwq && s <= b.z);
+        if (lane == 0) *(uint64_t *)(mb + it) = pm;
+        any |= pm;
+    }
+    __syncthreads();
+    const uint32_t mine = want ? mb[rank] : 0u;
+    uint32_t open = (uint32_t)(any | (any >> 32));
+    open |= open >> 16;
+    open = (open | (open >> 8)) & 0xffu;
+    uint32_t od = 0, td = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t a = (uint32_t)(i >> 2) ^ (right & 1u);
+        const uint32_t b = 2u * a + (((uint32_t)(i >> 1) & 1u) ^ ((right >> (1u + a)) & 1u));
+        const uint32_t l = 2u * b + (((uint32_t)i & 1u) ^ ((right >> (3u + b)) & 1u));
+        od |= l << (3 * i);
+        td |= ((open >> l) & 1u) << i;
+    }
+    order = __builtin_amdgcn_readfirstlane(od);
+    todo = __builtin_amdgcn_readfirstlane(td);
+    return mine;
+}
+__device__ __forceinline__ int mix_next8(uint32_t order, uint32_t todo) {
+    return (int)((order >> (3 * __builtin_ctz(todo))) & 7u);
+}
+
+// An opened node of height 3: its leaves, each loaded while the one before
+// it is consumed.
+template <int ND, int KMAX>
+__device__ __forceinline__ void mix_sub8(const MixSrc<ND> &S, const float *boxp, const float *planep, int node,
+                                         int nleafp, MixCtx<ND> &c, const float *q32, const float *qc, int anc,
+                                         bool want, uint32_t *hk, uint32_t *sl, float *cx, int lane,
+                                         uint32_t (&gm)[GShape<KMAX>::G]) {
+    uint32_t order, todo;
+    const uint32_t mine = mix_test8<ND>(boxp, planep, node, 3, __uint_as_float(c.root), q32, qc, anc, want, cx, lane,
+                                        order, todo);
+    if (!todo) return;
+    const int leaf0 = 8 * node - nleafp;
+    int l = mix_next8(order, todo);
+    MixPre pre;
+    mix_load(S, leaf0 + l, lane, pre);
+    for (;;) {
+        todo &= todo - 1;
+        const int ln = todo ? mix_next8(order, todo) : l;
+        MixPre nxt;
+        mix_load(S, leaf0 + ln, lane, nxt);
+        if (c.nvis >= MX_V) return;  // visit table full: lanes fall back
+        mix_leaf<ND, KMAX>(S, leaf0 + l, c, (mine >> l) & 1u, hk, sl, cx, lane, gm, pre);
+        if (!todo) return;
+        l = ln;
+        pre = nxt;
+    }
+}
+
 // Stackless depth-first walk: the ancestor of the wave's own leaves first,
 // else the child nearer to the wave's first query; firstright[dep] records
 // which child was entered first at each depth.  Two loop forms visit the
@@ -456,7 +603,7 @@ __device__ __forceinline__ void mix_walk(const DevTree &T, const double *ext, Mi
             if (ballot(want)) {
                 if (dep == D) {
                     if (c.nvis >= MX_V) break;  // visit table full: lanes fall back
-                    mix_leaf<ND, KMAX>(S, node - nleafp, c, want, hk, sl, cx, lane, gm);
+                    mix_leaf<ND, KMAX>(S, node - nleafp, c, want, hk, sl, cx, lane, gm, MixPre());
                 } else {
                     int first;
                     if ((anc >> (D - dep)) == node) first = anc >> (D - dep - 1);
@@ -482,8 +629,27 @@ __device__ __forceinline__ void mix_walk(const DevTree &T, const double *ext, Mi
                 const bool want = box_lb32<ND>(q32, bx) <= __uint_as_float(c.root);
                 if (ballot(want)) {
                     if (dep == D) {
+                        // trees of fewer than 8 leaves only: the rest end in mix_sub8
                         if (c.nvis >= MX_V) break;  // visit table full: lanes fall back
-                        mix_leaf<ND, KMAX>(S, node - nleafp, c, want, hk, sl, cx, lane, gm);
+                        MixPre pre;
+                        mix_load(S, node - nleafp, lane, pre);
+                        mix_leaf<ND, KMAX>(S, node - nleafp, c, want, hk, sl, cx, lane, gm, pre);
+                        down = false;
+                    } else if (dep == D - 3 || dep == D - 6) {
+                        // height 3, or height 6: the height-3 nodes under it in turn
+                        uint32_t order = 0, todo = 1, mine = want ? 1u : 0u;
+                        const int n0 = dep == D - 6 ? 8 * node : node;
+                        if (dep == D - 6)
+                            mine = mix_test8<ND>(boxp, planep, node, 6, __uint_as_float(c.root), q32, qc, anc, want, cx,
+                                                 lane, order, todo);
+                        while (todo) {
+                            const int l = mix_next8(order, todo);
+                            todo &= todo - 1;
+                            mix_sub8<ND, KMAX>(S, boxp, planep, n0 + l, nleafp, c, q32, qc, anc, (mine >> l) & 1u, hk, sl,
+                                               cx, lane, gm);
+                            if (c.nvis >= MX_V) break;
+                        }
+                        if (c.nvis >= MX_V) break;
                         down = false;
                     } else {
                         const int c0 = 2 * node;
@@ -1006,16 +1172,18 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
 // scratch words per workgroup: 16-bit handles and the visit table, and for
 // KMAX > 33 the slots and keys in ascending order
 #define MX_BLKW(KM) ((KM) * (NBX_WAVE / 2) + MX_V + ((KM) <= 33 ? 0 : 2 * (KM) * NBX_WAVE))
+// (6-D, k <= 32: LDS allows 15 waves per CU, so the registers are held to the
+// 128 that four waves per SIMD leave)
 template <int ND, int KMAX, int MODE>
-__global__ __launch_bounds__(64) void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list,
+__global__ __launch_bounds__(64, ND == 6 && KMAX == 33 ? 4 : 1) void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list,
                                                    int32_t *fb_count, uint32_t *scratch, int32_t *ctr) {
     __shared__ uint32_t hk[KMAX * NBX_WAVE];
     // one buffer for three uses at different times: the leaf copy (phase 2),
-    // the compacted queries and masks (phase 1) and the symmetric scatter into
-    // the wave's own queries (density)
-    constexpr int UB1 = ND == 3 ? 0 : ND * NBX_WAVE + NBX_WAVE;  // transposed phase 1 (6-D only)
+    // the compacted queries and their masks (6-D node tests and phase 1) and
+    // the symmetric scatter into the wave's own queries (density)
+    constexpr int UB1 = ND == 3 ? 0 : (MX_QW + 1) * NBX_WAVE;
     constexpr int UBN = UB1 > ND * NBX_LEAF + 2 * NBX_WAVE ? UB1 : ND * NBX_LEAF + 2 * NBX_WAVE;
-    __shared__ __attribute__((aligned(8))) float ub[UBN];
+    __shared__ __attribute__((aligned(16))) float ub[UBN];
     float *cx = ub;
     double *racc = (double *)(ub + ND * NBX_LEAF);
     const int lane = threadIdx.x;

@@ -109,3 +109,26 @@ def test_forward_in_search(gpu, form, k):
     t.sph_density(k, rho, h, block_rows=1024)
     assert torch.equal(h, ho)
     assert float((rho / ro - 1.0).abs().max()) < 1e-12
+
+
+@pytest.mark.parametrize("n", [20, 33, 65, 129, 256, 257, 1000, 2048, 2049, 4097, 9000])
+@pytest.mark.parametrize("k", [8, 32, 64])
+def test_phase_rows_by_tree_height(gpu, n, k):
+    """6-D precision form: trees below, at and above the heights (3 and 6) from
+    which nodes are tested eight at a time."""
+    import nbodylib_amd as nb
+
+    k = min(k, n - 2)
+    print(f"phase rows n={n} k={k}", flush=True)
+    x, v, _ = datagen.clustered(n, 1.0, nhalo=4, seed=n, with_vel=True)
+    v = v / v.std()
+    t = nb.KDTree(x, vel=v, treetype=nb.TPHS, aniso=-1, kerntype=nb.KSPH, form=nb.FORM_MIXED)
+    nn, d2 = t.FindNearestPhase(k)
+    ph = np.concatenate([x, v], 1)
+    for a in range(0, n, 1500):
+        d = np.zeros((len(ph[a:a + 1500]), n))
+        for c in range(6):
+            d += (ph[a:a + 1500, c][:, None] - ph[:, c][None, :]) ** 2
+        d[d == 0.0] = np.inf
+        assert np.array_equal(d2[a:a + 1500], np.sort(d, 1)[:, :k])
+        assert np.array_equal(np.take_along_axis(d, nn[a:a + 1500].astype(np.int64), 1), d2[a:a + 1500])
