@@ -1506,23 +1506,18 @@ static int sph_tree_adj(nbx_tree *t, int32_t k, int64_t block, const double *g_i
     if (block > n) block = (n + 1023) / 1024 * 1024;
     DevBufs bufs(st);
     int32_t *nbr = nullptr, *err = nullptr;
-    double *gs = nullptr, *ds = nullptr, *ms = nullptr;
+    char *work = nullptr;
     HIPCK(bufs.alloc(&nbr, sizeof(int32_t) * (size_t)block * k));
     HIPCK(bufs.alloc(&err, sizeof(int32_t)));
-    HIPCK(bufs.alloc(&gs, sizeof(double) * n));
-    HIPCK(bufs.alloc(&ds, sizeof(double) * 3 * n));
-    HIPCK(bufs.alloc(&ms, sizeof(double) * n));
+    HIPCK(bufs.alloc(&work, nbx_sph_work_size(n)));
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, err, 0, (int64_t)1);
-    hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, st, g_id, t->perm, n, gs);
-    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(3 * n)), dim3(256), 0, st, ds, 0.0, 3 * n);
-    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, ms, 0.0, n);
+    const double *X[3] = {t->xs[0], t->xs[1], t->xs[2]};
+    nbx_sph_adj_begin(X, t->mass, nullptr, n, g_id, t->perm, work, st);
     // the search's temporaries, reused by every block
     Workspace ws = {nullptr, 0, 0};
     ws.cap = mixed ? 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1)
                    : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, block);
     HIPCK(bufs.alloc(&ws.base, ws.cap));
-    const double *X[3] = {t->xs[0], t->xs[1], t->xs[2]};
-    double *D[3] = {ds, ds + n, ds + 2 * n};
     for (int64_t r0 = 0; r0 < n; r0 += block) {
         const int64_t nr = std::min<int64_t>(block, n - r0);
         KnnArgs A = sph_tree_search(k);
@@ -1535,12 +1530,11 @@ static int sph_tree_adj(nbx_tree *t, int32_t k, int64_t block, const double *g_i
         A.row0 = (int32_t)r0;
         ws.used = 0;
         hipError_t e = mixed ? run_mixed(t, A, k, st, &ws) : run_plain(t, A, A.wcnt * NBX_WAVE, st, &ws);
-        if (e == hipSuccess) e = nbx_launch_sph_adj_rows(X, t->mass, nbr, n, r0, nr, k, gs, D, ms, st);
         if (e != hipSuccess) return hipfail(e, "differentiation form");
+        ProfScope ps("k_sph_adj", st);
+        nbx_sph_adj_rows(nbr, nullptr, n, r0, nr, k, work, st);
     }
-    for (int c = 0; c < 3; ++c)
-        hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, ds + c * n, t->perm, dpos_id + c * n, n);
-    hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, ms, t->perm, dmass_id, n);
+    nbx_sph_adj_end(t->inv, n, dpos_id, dmass_id, work, st);
     return sph_tree_end(err, st);
 }
 
@@ -1574,5 +1568,36 @@ extern "C" int nbx_sph_density_adjoint_dev(const double *pos, const double *mass
     hipLaunchKernelGGL(k_fill_f64, dim3(nblk(3 * n)), dim3(256), 0, st, dpos, 0.0, 3 * n);
     hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, dmass, 0.0, n);
     HIPCK(nbx_launch_sph_adj(pos, mass, nbr, n, k, g, dpos, dmass, st));
+    return NBX_OK;
+}
+
+// The same with the rows in a spatial order (for arrays in no such order).
+extern "C" int64_t nbx_sph_work_bytes(int64_t n) { return n < 1 ? 0 : (int64_t)nbx_sph_work_size(n); }
+extern "C" int nbx_sph_list_check_dev(const int32_t *nbr, int64_t n, int32_t k, int64_t *stats, void *stream) {
+    if (!nbr || !stats) return fail(NBX_ERR_ARG, "NULL argument");
+    if (n < 1 || k < 1) return fail(NBX_ERR_ARG, "bad sizes");
+    HIPCK(nbx_launch_sph_list_check(nbr, n, k, stats, (hipStream_t)stream));
+    return NBX_OK;
+}
+extern "C" int nbx_sph_order_dev(const double *pos, int64_t n, int32_t *order, void *work, void *stream) {
+    if (!pos || !order || !work) return fail(NBX_ERR_ARG, "NULL argument");
+    if (n < 1 || n > INT32_MAX) return fail(NBX_ERR_ARG, "bad sizes");
+    HIPCK(nbx_launch_sph_order(pos, n, order, work, (hipStream_t)stream));
+    return NBX_OK;
+}
+extern "C" int nbx_sph_density_fwd_ordered_dev(const double *pos, const double *mass, const int32_t *nbr,
+                                               const int32_t *order, int64_t n, int32_t k, double *rho, double *h,
+                                               void *work, void *stream) {
+    if (!pos || !mass || !nbr || !rho || !work) return fail(NBX_ERR_ARG, "NULL argument");
+    if (n < 1 || n > INT32_MAX || k < 1) return fail(NBX_ERR_ARG, "bad sizes");
+    HIPCK(nbx_launch_sph_fwd_ordered(pos, mass, nbr, order, n, k, rho, h, work, (hipStream_t)stream));
+    return NBX_OK;
+}
+extern "C" int nbx_sph_density_adjoint_ordered_dev(const double *pos, const double *mass, const int32_t *nbr,
+                                                   const int32_t *order, int64_t n, int32_t k, const double *g,
+                                                   double *dpos, double *dmass, void *work, void *stream) {
+    if (!pos || !mass || !nbr || !g || !dpos || !dmass || !work) return fail(NBX_ERR_ARG, "NULL argument");
+    if (n < 1 || n > INT32_MAX || k < 1) return fail(NBX_ERR_ARG, "bad sizes");
+    HIPCK(nbx_launch_sph_adj_ordered(pos, mass, nbr, order, n, k, g, dpos, dmass, work, (hipStream_t)stream));
     return NBX_OK;
 }

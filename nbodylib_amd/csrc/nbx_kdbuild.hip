@@ -663,3 +663,9 @@ done:
 #undef KDCK
     return e;
 }
+
+hipError_t nbx_sort_pairs_u32(void *temp, size_t &temp_bytes, uint32_t *kin, uint32_t *kout, int32_t *vin,
+                              int32_t *vout, int64_t n, int bits, hipStream_t st) {
+    return rocprim::radix_sort_pairs(temp, temp_bytes, kin, kout, vin, vout, (unsigned int)n, 0, (unsigned)bits, st,
+                                     false);
+}

@@ -38,6 +38,8 @@ __global__ void k_boxf(const double *box, float *boxf, int64_t count, int nd);
 hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleafp, int32_t *order, hipStream_t st);
 hipError_t nbx_sort_pairs_u64(void *temp, size_t &temp_bytes, uint64_t *kin, uint64_t *kout, int32_t *vin,
                               int32_t *vout, int64_t n, hipStream_t st);
+hipError_t nbx_sort_pairs_u32(void *temp, size_t &temp_bytes, uint32_t *kin, uint32_t *kout, int32_t *vin,
+                              int32_t *vout, int64_t n, int bits, hipStream_t st);  // keys below 2^bits
 
 // ------------------------------------------------------------------ kNN
 // Query source
@@ -197,13 +199,31 @@ hipError_t nbx_launch_sph_fwd(const double *pos, const double *mass, const int32
                               double *h, hipStream_t st);
 hipError_t nbx_launch_sph_adj(const double *pos, const double *mass, const int32_t *nbr, int64_t n, int k,
                               const double *g, double *dpos, double *dmass, hipStream_t st);
-// The same over rows [r0, r0 + nr) of n particles, row i of the list at
-// nbr[(i - r0) k]; X[3] / D[3] are the coordinate / gradient arrays of all n.
-hipError_t nbx_launch_sph_fwd_rows(const double *const *X, const double *mass, const int32_t *nbr, int64_t n,
-                                   int64_t r0, int64_t nr, int k, double *rho, double *h, hipStream_t st);
-hipError_t nbx_launch_sph_adj_rows(const double *const *X, const double *mass, const int32_t *nbr, int64_t n,
-                                   int64_t r0, int64_t nr, int k, const double *g, double *const *D, double *dmass,
-                                   hipStream_t st);
+// A stored list over particles in an order of their own.  list_check: smallest
+// and largest entry and the number of entries within their row's block of
+// 1024 (stats: 3 int64 of device memory).  order: a permutation that brings
+// spatial neighbours together (work: nbx_sph_work_size).  The ordered forward
+// and adjoint take the rows in that order (null: as they lie); both outputs
+// are written.
+hipError_t nbx_launch_sph_list_check(const int32_t *nbr, int64_t n, int k, int64_t *stats, hipStream_t st);
+size_t nbx_sph_work_size(int64_t n);
+hipError_t nbx_launch_sph_order(const double *pos, int64_t n, int32_t *order, void *work, hipStream_t st);
+hipError_t nbx_launch_sph_fwd_ordered(const double *pos, const double *mass, const int32_t *nbr, const int32_t *order,
+                                      int64_t n, int k, double *rho, double *h, void *work, hipStream_t st);
+hipError_t nbx_launch_sph_adj_ordered(const double *pos, const double *mass, const int32_t *nbr, const int32_t *order,
+                                      int64_t n, int k, const double *g, double *dpos, double *dmass, void *work,
+                                      hipStream_t st);
+
+// The adjoint in parts, for lists made a block at a time: begin packs the
+// particles (cotangents g at gidx) and clears the sums, rows adds the rows
+// [r0, r0 + nr) (row r0 at nbr[0]; with an order: all rows), end writes the
+// sums of rank[i] to i.
+void nbx_sph_adj_begin(const double *const *X, const double *mass, const int32_t *order, int64_t n, const double *g,
+                       const int32_t *gidx, void *work, hipStream_t st);
+void nbx_sph_adj_rows(const int32_t *nbr, const int32_t *order, int64_t n, int64_t r0, int64_t nr, int k, void *work,
+                      hipStream_t st);
+void nbx_sph_adj_end(const int32_t *rank, int64_t n, double *dpos, double *dmass, void *work, hipStream_t st);
+
 // ------------------------------------------------------------------ profiling
 struct ProfScope {
     hipStream_t st;
