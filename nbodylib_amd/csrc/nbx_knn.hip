@@ -540,10 +540,6 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
             const double ih = 1.0 / hi;
             const double norm = spline ? NBX_SIGMA3 * ih * ih * ih : 1.0 / pow(hi, (double)ND);
             const double mi = QSRC == NBX_Q_SLOTS ? T.mass[qi] : 0.0;
-            // Wsm's lookup with the table step's division as a product; r/h
-            // stays a division, so the k-th neighbour's is exactly 2 and it
-            // takes the table's last entry, as in the reference
-            const double ck = 0.5 * (T.kernres - 1), top = (double)(T.kernres - 1);
             double acc = 0.0;
             // entries in groups of 8 so their slot/mass gathers are in flight
             // together; summed in position order
@@ -562,17 +558,8 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
                 for (int u = 0; u < 8; ++u) {
                     if (!(dv[u] < NBX_MAXVALUE)) continue;  // past the end, or missing
                     const int32_t s = sv[u];
-                    double W;
-                    if (spline) {
-                        W = w_cubic(sqrt(dv[u]) * ih);
-                    } else {
-                        const double fi = sqrt(dv[u]) / hi * ck;
-                        W = T.kern[T.kernres - 1];
-                        if (fi < top) {
-                            const int i = (int)fi;
-                            W = T.kern[i] + (T.kern[i + 1] - T.kern[i]) * (fi - (double)i);
-                        }
-                    }
+                    const double r = sqrt(dv[u]);
+                    const double W = spline ? w_cubic(r * ih) : wsm_at(r, hi, T.kern, T.kernres);
                     if (sym) {
                         const double Wij = 0.5 * W * norm;
                         acc = acc + Wij * mv[u];
