@@ -117,7 +117,7 @@ __device__ __forceinline__ bool fof_surely(double v, const FofLink &L) {
 }
 
 template <int ND, int MT>
-__device__ __forceinline__ double fof_lb(const double *q, cdptr b, const FofLink &L) {
+__device__ __forceinline__ double fof_lb_box(const double *q, const double (&b)[2 * ND], const FofLink &L) {
     double t2[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
@@ -127,7 +127,7 @@ __device__ __forceinline__ double fof_lb(const double *q, cdptr b, const FofLink
     return fof_bval<ND, MT>(t2, L);
 }
 template <int ND, int MT>
-__device__ __forceinline__ double fof_ub(const double *q, cdptr b, const FofLink &L) {
+__device__ __forceinline__ double fof_ub(const double *q, const double (&b)[2 * ND], const FofLink &L) {
     double t2[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
@@ -136,6 +136,23 @@ __device__ __forceinline__ double fof_ub(const double *q, cdptr b, const FofLink
         t2[d] = (a2 > c2) ? a2 : c2;
     }
     return fof_bval<ND, MT>(t2, L);
+}
+// Both bounds between two boxes, lower (lb) and upper (ub), the first box in
+// registers.
+template <int ND, int MT>
+__device__ __forceinline__ void fof_bounds(const double (&a)[2 * ND], const double (&b)[2 * ND], const FofLink &L,
+                                           double &lb, double &ub) {
+    double l2[ND], u2[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        const double u = b[ND + d] - a[d], v = a[ND + d] - b[d];
+        const double m = u > v ? u : v;
+        u2[d] = m * m;
+        const double g = fmax(fmax(b[d] - a[ND + d], a[d] - b[ND + d]), 0.0);
+        l2[d] = g * g;
+    }
+    lb = fof_bval<ND, MT>(l2, L);
+    ub = fof_bval<ND, MT>(u2, L);
 }
 template <int ND, int MT>
 __device__ __forceinline__ double fof_bbub(cdptr a, cdptr b, const FofLink &L) {
@@ -231,25 +248,122 @@ __device__ __forceinline__ uint32_t fof_scan_few(const DevTree &T, int base, con
     return pair ? own : 0u;
 }
 // Largest count of wanting lanes for which the leaf is scanned by
-// fof_scan_few: the measured crossover with the scan by lanes on 3-D trees;
-// on 6-D trees, where a leaf is wanted by 6 lanes on average, every count
-// (measured faster throughout).
+// fof_scan_few.  3-D: past 24 the scan by lanes takes as few steps (limits of
+// 12, 24, 40 and 64 measured 2.86, 2.82, 2.91 and 2.93 ms on 16.8M); 6-D,
+// where a leaf is wanted by 6 lanes on average: every count.
 template <int ND>
 __device__ __forceinline__ constexpr int fof_few_max() { return ND == 6 ? NBX_WAVE : 24; }
 
+// Lanes of one set from which on their links to a leaf are joined together, a
+// candidate per lane: below it each lane makes its own, one after another.
+#define FOF_SHARE 3
+
+// The candidates of one leaf that the position q of each lane with pair set
+// (pm: their ballot) links to: bit j for slot base + j.
+template <int ND, int MT>
+__device__ __forceinline__ uint32_t fof_scan(const DevTree &T, int base, const double *q, bool pair, uint64_t pm,
+                                             const FofLink &L) {
+    if (__builtin_popcountll(pm) <= fof_few_max<ND>()) return fof_scan_few<ND, MT>(T, base, q, pair, pm, L);
+    uint32_t mask = 0, unsure = 0;
+    // the scan by lanes: candidates arrive as 64-byte (3-D) or 32-byte
+    // (6-D) scalar-load chunks per dimension (padding slots are 1e300
+    // away and never link)
+    constexpr int CH = ND == 6 ? 4 : 8;
+    typedef double dxc __attribute__((ext_vector_type(CH)));
+    typedef const __attribute__((address_space(4))) dxc *cdcptr;
+#pragma unroll
+    for (int jj = 0; jj < NBX_LEAF; jj += CH) {
+        dxc cv[ND];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) cv[d] = *(cdcptr)(T.x[d] + base + jj);
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+            double t2[ND];
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                const double t = q[d] - cv[d][u];
+                t2[d] = t * t;
+            }
+            // decisions are shifted in as they are made (a bit per candidate
+            // held in scalar masks until the end would spill them all); the
+            // comparators' values inside the reciprocal band are decided
+            // with the divisions after the scan, or at once in the 6-D
+            // persistent kernel (each the measured better form)
+            bool near;
+            if constexpr (MT == 0) {
+                near = fof_val<ND, MT>(t2, L) < L.lim;
+            } else if constexpr (ND == 3) {
+                const double v = fof_val_fast<ND, MT>(t2, L);
+                near = v < NBX_FOF_BAND_LO;
+                unsure = unsure + unsure + ((v >= NBX_FOF_BAND_LO && v < NBX_FOF_BAND_HI) ? 1u : 0u);
+            } else {
+                const double v = fof_val_fast<ND, MT>(t2, L);
+                near = v < NBX_FOF_BAND_LO;
+                const bool uns = v >= NBX_FOF_BAND_LO && v < NBX_FOF_BAND_HI;
+                if (ballot(uns) && uns) near = fof_val<ND, MT>(t2, L) < 1.0;
+            }
+            mask = mask + mask + (near ? 1u : 0u);
+        }
+    }
+    if constexpr (MT != 0 && ND == 3) {
+        // unsure holds candidate j at bit 31 - j, as mask does here
+        if (ballot(unsure != 0)) {
+            uint32_t um = unsure;
+            while (um) {
+                const int b = 31 - __builtin_clz(um);
+                um &= ~(1u << b);
+                const int32_t cs = base + (31 - b);
+                double t2[ND];
+#pragma unroll
+                for (int d = 0; d < ND; ++d) {
+                    const double t = q[d] - T.x[d][cs];
+                    t2[d] = t * t;
+                }
+                if (fof_val<ND, MT>(t2, L) < 1.0) mask |= 1u << b;
+            }
+        }
+    }
+    // candidate j was shifted in at bit 31 - j
+    mask = __builtin_bitreverse32(mask);
+    return pair ? mask : 0u;
+}
+
+// A lane's rq is a slot of its particle's set (a former root as a rule, so
+// finds from it are short), and lanes with equal rq are in one set.  Joins the
+// sets of the lanes with has set to slot t's (uniform): of the lanes that
+// share the first one's rq only that one makes the union, and all of them
+// take its result.
+__device__ __forceinline__ void fof_join(int32_t *P, bool has, int32_t t, int32_t &rq) {
+    const uint64_t m = ballot(has);
+    if (!m) return;
+    const int lead = __builtin_ctzll(m);
+    const int32_t r0 = __builtin_amdgcn_readlane(rq, lead);
+    const bool same = rq == r0;
+    if (has && (!same || (int)threadIdx.x == lead)) rq = uf_union_r(P, rq, t);
+    const int32_t r1 = __builtin_amdgcn_readlane(rq, lead);
+    if (same) rq = r1;
+}
+
 // Links from the (possibly image-shifted) position q to the particles of one
 // leaf.  act is the lane's own bound test for the leaf: a lane whose bound
-// rules out every link takes no part.  A leaf that is internally connected
-// needs one union with any particle it links to; otherwise every link is a
-// union (in the first pass only toward larger slots: the pair is met from
-// both sides).  rq is a hint for the root of qi (any former root of its
-// set), kept across unions so each find starts near the top.
+// rules out every link takes no part.  bx, lconn, pb: the leaf's box, whether
+// it is internally connected and its first slot's parent, read when it was
+// found open.  A leaf that is internally connected needs one union with any
+// particle it links to; otherwise every link joins two sets (in the first pass only links toward
+// larger slots: the pair is met from both sides).
+// Unions wait on chains of dependent loads, so what counts is how many a wave
+// makes one after another.  Made by each lane for each of its links they were
+// 286 per wave of the 16.8M clustered set, as many in turn as the busiest
+// lane has links; but the lanes mostly share one set, and what a set links to
+// needs one union per candidate, all 32 at once (FOF_SHARE).  With that,
+// fof_own and fof_join, the linking kernel went from 7.6 to 4.4 ms and
+// snapshots of 2M particles from 1.27 to 0.57 ms.
 template <int PASS0, int ND, int MT>
 __device__ __forceinline__ void fof_leaf(const DevTree &T, int leaf, const double *q, bool act, int32_t qi,
-                                         const FofLink &L, int32_t *P, const uint8_t *conn, int32_t &rq) {
+                                         const double (&bx)[2 * ND], bool lconn, int32_t pb, const FofLink &L,
+                                         int32_t *P, int32_t &rq) {
     const int base = leaf * NBX_LEAF;
-    const bool lconn = conn[T.nleafp + leaf];
-    cdptr bx = (cdptr)node_box(T, T.nleafp + leaf, ND);
+    const int lane = threadIdx.x;  // one wave per workgroup
     const bool encl = act && lconn && fof_surely<MT>(fof_ub<ND, MT>(q, bx, L), L);
     // The members of a connected leaf are one set (from the pre-pass, or
     // joined by the shortcut that flagged it before the pass ends), so once
@@ -257,121 +371,137 @@ __device__ __forceinline__ void fof_leaf(const DevTree &T, int leaf, const doubl
     // of it and neither scans the leaf nor makes a union; in dense regions
     // most visits to connected leaves are such.  A stale parent only misses
     // the skip, since sets only merge.
-    const int32_t pb = lconn ? P[base] : -1;
     const bool joined = lconn && (pb == rq || base == rq);
-    if (encl && !joined) rq = uf_union_r(P, rq, base);
+    fof_join(P, encl && !joined, base, rq);
     const bool pair = act && !encl && !joined;
     const uint64_t pm = ballot(pair);
     if (!pm) return;
-    uint32_t mask = 0;
-    if (__builtin_popcountll(pm) <= fof_few_max<ND>()) {
-        mask = fof_scan_few<ND, MT>(T, base, q, pair, pm, L);
-    } else {
-        uint32_t unsure = 0;
-        // the scan by lanes: candidates arrive as 64-byte (3-D) or 32-byte
-        // (6-D) scalar-load chunks per dimension (padding slots are 1e300
-        // away and never link)
-        constexpr int CH = ND == 6 ? 4 : 8;
-        typedef double dxc __attribute__((ext_vector_type(CH)));
-        typedef const __attribute__((address_space(4))) dxc *cdcptr;
-#pragma unroll
-        for (int jj = 0; jj < NBX_LEAF; jj += CH) {
-            dxc cv[ND];
-#pragma unroll
-            for (int d = 0; d < ND; ++d) cv[d] = *(cdcptr)(T.x[d] + base + jj);
-#pragma unroll
-            for (int u = 0; u < CH; ++u) {
-                double t2[ND];
-#pragma unroll
-                for (int d = 0; d < ND; ++d) {
-                    const double t = q[d] - cv[d][u];
-                    t2[d] = t * t;
-                }
-                // decisions are shifted in as they are made (a bit per candidate
-                // held in scalar masks until the end would spill them all); the
-                // comparators' values inside the reciprocal band are decided
-                // with the divisions after the scan, or at once in the 6-D
-                // persistent kernel (each the measured better form)
-                bool near;
-                if constexpr (MT == 0) {
-                    near = fof_val<ND, MT>(t2, L) < L.lim;
-                } else if constexpr (ND == 3) {
-                    const double v = fof_val_fast<ND, MT>(t2, L);
-                    near = v < NBX_FOF_BAND_LO;
-                    unsure = unsure + unsure + ((v >= NBX_FOF_BAND_LO && v < NBX_FOF_BAND_HI) ? 1u : 0u);
-                } else {
-                    const double v = fof_val_fast<ND, MT>(t2, L);
-                    near = v < NBX_FOF_BAND_LO;
-                    const bool uns = v >= NBX_FOF_BAND_LO && v < NBX_FOF_BAND_HI;
-                    if (ballot(uns) && uns) near = fof_val<ND, MT>(t2, L) < 1.0;
-                }
-                mask = mask + mask + (near ? 1u : 0u);
-            }
-        }
-        if constexpr (MT != 0 && ND == 3) {
-            // unsure holds candidate j at bit 31 - j, as mask does here
-            if (ballot(unsure != 0)) {
-                uint32_t um = unsure;
-                while (um) {
-                    const int b = 31 - __builtin_clz(um);
-                    um &= ~(1u << b);
-                    const int32_t cs = base + (31 - b);
-                    double t2[ND];
-#pragma unroll
-                    for (int d = 0; d < ND; ++d) {
-                        const double t = q[d] - T.x[d][cs];
-                        t2[d] = t * t;
-                    }
-                    if (fof_val<ND, MT>(t2, L) < 1.0) mask |= 1u << b;
-                }
-            }
-        }
-        // candidate j was shifted in at bit 31 - j
-        mask = __builtin_bitreverse32(mask);
-    }
+    uint32_t mask = fof_scan<ND, MT>(T, base, q, pair, pm, L);
     // Never the query itself; in the first pass, in a leaf not internally
-    // connected, only candidates at larger slots (the pair is met from both
-    // sides).
+    // connected, only candidates at larger slots (the wave's own leaves are
+    // not scanned here then, so these are all or none).
     const int qrel = qi - base;
-    const uint32_t self = (qrel >= 0 && qrel < NBX_LEAF) ? (1u << qrel) : 0u;
-    const uint32_t above = qrel < 0 ? ~0u : (qrel >= NBX_LEAF - 1 ? 0u : (~0u << (qrel + 1)));
-    mask &= (PASS0 && !lconn) ? above : ~self;
-    if (!pair) mask = 0;
-    if (!ballot(mask != 0)) return;
-    // The leaf's parents, read once with ordinary loads.  A candidate whose
-    // parent is the lane's root hint rq (a former root of its set) is
-    // already in that set, because sets only ever merge, so its link needs
-    // no union.  A stale parent costs only the skip.
-    __shared__ int32_t par[NBX_LEAF];
-    const int ln = threadIdx.x;  // one wave per workgroup
-    if (ln < NBX_LEAF) par[ln] = base + ln < T.n ? P[base + ln] : -1;
-    __syncthreads();
+    if (!PASS0) mask &= (qrel >= 0 && qrel < NBX_LEAF) ? ~(1u << qrel) : ~0u;
+    else if (!lconn && qrel >= 0) mask = 0;
+    uint64_t rest = ballot(mask != 0);
+    if (!rest) return;
     if (lconn) {
         // one link joins the whole leaf; the union goes through the first
         // slot, whose chain to the root is the shortest
-        if (mask) {
-            const int j = __builtin_ctz(mask);
-            if (par[j] != rq && par[0] != rq && base != rq) rq = uf_union_r(P, rq, base);
+        fof_join(P, mask != 0, base, rq);
+        return;
+    }
+    // The leaf's parents, read once with ordinary loads.  A candidate whose
+    // parent is rq is in that set already, because sets only ever merge, so
+    // its link needs no union.  A stale parent costs only the skip.
+    __shared__ int32_t par[NBX_LEAF];
+    const int32_t pc = lane < NBX_LEAF && base + lane < T.n ? P[base + lane] : -1;
+    if (lane < NBX_LEAF) par[lane] = pc;
+    __syncthreads();
+    bool alone = false;  // this lane's links are left to itself
+    while (rest) {
+        // the lanes that share the next one's rq
+        const int32_t r0 = __builtin_amdgcn_readlane(rq, __builtin_ctzll(rest));
+        const uint64_t same = ballot(rq == r0);
+        const uint64_t now = rest & same;
+        rest &= ~same;
+        if (__builtin_popcountll(now) < FOF_SHARE) {
+            alone = alone || ((now >> lane) & 1u);
+            continue;
         }
-    } else {
-        while (mask) {
-            const int j = __builtin_ctz(mask);
-            mask &= mask - 1;
-            if (par[j] == rq) continue;
-            rq = uf_union_r(P, rq, base + j);
+        // what any of them links to joins their set, a candidate per lane
+        uint32_t all = ((now >> lane) & 1u) ? mask : 0u;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) all |= (uint32_t)__shfl_xor((int)all, off);
+        const bool mine = lane < NBX_LEAF && ((all >> lane) & 1u) && pc != r0;
+        int32_t r = r0;
+        if (mine) r = uf_union_r(P, r0, base + lane);
+        const uint64_t made = ballot(mine);
+        if (made) {
+            const int32_t r1 = __builtin_amdgcn_readlane(r, __builtin_ctzll(made));
+            if (rq == r0) rq = r1;
         }
+    }
+    if (!alone) mask = 0;
+    while (mask) {
+        const int j = __builtin_ctz(mask);
+        mask &= mask - 1;
+        if (par[j] == rq) continue;
+        rq = uf_union_r(P, rq, base + j);
     }
     __syncthreads();
 }
 
+// The links among the wave's own particles (its two leaves), first pass.  The
+// components of the 64 particles are found in registers, by flooding from
+// each one's lowest lane through the lanes' link masks, and every other lane
+// then makes one union with its component's lowest particle.
+template <int ND, int MT>
+__device__ __forceinline__ void fof_own(const DevTree &T, const double *q, bool valid, int32_t qi, int g,
+                                        const double (&gb)[2 * ND], const FofLink &L, int32_t *P, int32_t &rq) {
+    const int lane = threadIdx.x;
+    const uint64_t vm = ballot(valid);
+    double lb, ub;
+    fof_bounds<ND, MT>(gb, gb, L, lb, ub);
+    uint64_t adj = vm;
+    if (!fof_surely<MT>(ub, L)) {
+        adj = 0;
+#pragma unroll 1
+        for (int h = 0; h < 2; ++h) {
+            if (!((vm >> (32 * h)) & 1u)) break;
+            // a particle of the other leaf only where its bound allows a link
+            const cdptr lb = (cdptr)node_box(T, T.nleafp + 2 * g + h, ND);
+            double lx[2 * ND];
+#pragma unroll
+            for (int d = 0; d < 2 * ND; ++d) lx[d] = lb[d];
+            const bool in = valid && ((lane >> 5) == h || fof_maybe<MT>(fof_lb_box<ND, MT>(q, lx, L), L));
+            adj |= (uint64_t)fof_scan<ND, MT>(T, g * NBX_WAVE + h * NBX_LEAF, q, in, ballot(in), L) << (32 * h);
+        }
+    }
+    adj &= ~(1ULL << lane);
+    uint64_t rest = ballot(valid && adj != 0);  // the others have no link here
+    int lead = lane;
+    while (rest) {
+        const int first = __builtin_ctzll(rest);
+        uint64_t comp = 1ULL << first, was;
+        do {
+            was = comp;
+            comp |= ballot((adj & comp) != 0) & vm;
+        } while (comp != was);
+        if ((comp >> lane) & 1u) lead = first;
+        rest &= ~comp;
+    }
+    if (valid && lead != lane) rq = uf_union_r(P, qi, g * NBX_WAVE + lead);
+    // one hint per component: that of its highest lane
+    for (uint64_t left = ballot(valid && lead != lane); left;) {
+        const int top = 63 - __builtin_clzll(left);
+        const int ld = __builtin_amdgcn_readlane(lead, top);
+        const uint64_t comp = ballot(lead == ld);
+        const int32_t r = __builtin_amdgcn_readlane(rq, top);
+        if (lead == ld) rq = r;
+        left &= ~comp;
+    }
+}
+
+// The walk.  The linking length never shrinks, so which nodes matter is a
+// question for the wave's box, and 64 nodes answer it at once: an opened node
+// has its 64 descendants six levels below tested, one per lane, against the
+// box of the wave's particles, and the ballots are the open ones and those
+// joined whole.  A wave of the 16.8M clustered set made 142 box tests one
+// after another, each behind a load of its own and for all 64 lanes, which
+// was most of its instructions; it now makes about 8 of these steps.  FOF6d
+// of 1.5M particles 1.13 -> 0.60 ms; 3-D FOF of 16.8M 8.3 -> 7.6 ms, the rest
+// of it unions (below).
+// Below a node of height 6 the descendants are leaves, and each open one goes
+// to fof_leaf with the lanes whose own bound allows a link.
+// gb: box of the lanes' positions; stk: LDS for the open masks of up to
+// FOF_STK levels.
+#define FOF_STK 6
 template <int PASS0, int ND, int MT>
 __device__ __forceinline__ void fof_walk(const DevTree &T, const double *q, bool act, int32_t qi, int g,
-                                         const FofLink &L, int32_t *P, uint8_t *conn, int32_t &rq) {
-    const int D = T.depth;
-    // the wave's own 64 particles form the parent of leaves 2g, 2g+1 (or the
-    // single leaf when the tree has one)
-    const int gnode = D >= 1 ? (T.nleafp + 2 * g) >> 1 : 1;
-    cdptr gb = (cdptr)node_box(T, gnode, ND);
+                                         const double (&gb)[2 * ND], const FofLink &L, int32_t *P, uint8_t *conn,
+                                         uint64_t *stk, int32_t &rq) {
+    const int lane = threadIdx.x;
     // In the first pass a node whose slots all lie below the wave's first
     // slot need not be entered.  Each of its links with a wave particle is
     // also met from the lower particle's wave, whose walk reaches the wave's
@@ -379,52 +509,114 @@ __device__ __forceinline__ void fof_walk(const DevTree &T, const double *q, bool
     // there): the pair's computed distance is the same from both sides,
     // fl(a - b) = -fl(b - a), and each route that side can take (scan,
     // enclosure of a connected leaf, wave-node shortcut) puts the pair in
-    // one set.  On a 6-D tree every such node is skipped; on a 3-D tree
-    // only such leaves, because there the wave-node shortcuts met in the
-    // lower subtrees join dense regions in fewer unions than their pairs'
-    // links do (the measured better form for each).  sh is the node's
-    // height, so its leaves are [node << sh, (node + 1) << sh) in heap
-    // order.
+    // one set.  On a 6-D tree every such node is skipped; on a 3-D tree only
+    // such leaves, because there the nodes joined whole in the lower subtrees
+    // save their pairs' own links in dense regions (the measured better form
+    // for each).
     const int lfirst = T.nleafp + 2 * g;
-    int node = 1, sh = D;
-    bool down = true;
+    const int first = T.depth % 6;
+    int sp = 0, height = T.depth;
+    uint32_t node = 1;  // the opened node
+    int step = height == 0 ? 0 : (first ? first : 6);
+    uint64_t todo = 0;   // its open descendants `step` levels below, at `height` after the expansion
+    uint32_t base = 0;   // the first of them
+    bool expand = true;
     for (;;) {
-        if (down && PASS0 && (ND == 6 || sh == 0) && ((node + 1) << sh) <= lfirst) down = false;
-        if (down) {
-            cdptr bx = (cdptr)node_box(T, node, ND);
-            bool want = act && fof_maybe<MT>(fof_lb<ND, MT>(q, bx, L), L);
-            if (ballot(want)) {
-                if (PASS0 && fof_surely<MT>(fof_bbub<ND, MT>(gb, bx, L), L)) {
-                    // every wave particle links to every particle of the node:
-                    // wave and node form one component
-                    const int32_t nfirst = node_first(T, node);
-                    if (act) rq = uf_union_r(P, rq, nfirst);
-                    if (!conn[node]) {
-                        const int32_t nlast = node_end(T, node);
-                        for (int32_t s = nfirst + 1 + threadIdx.x; s < nlast; s += NBX_WAVE) uf_union(P, s, nfirst);
-                        conn[node] = 1;
-                    }
-                    down = false;
-                } else if (node >= T.nleafp) {
-                    fof_leaf<PASS0, ND, MT>(T, node - T.nleafp, q, want, qi, L, P, conn, rq);
-                    down = false;
-                } else {
-                    node = 2 * node;
-                    --sh;
-                    continue;
+        if (expand) {
+            height -= step;
+            base = node << step;
+            const bool mine = lane < (1 << step);
+            const uint32_t child = base + (mine ? lane : 0);
+            double bx[2 * ND];
+            const double2 *bp = (const double2 *)node_box(T, (int)child, ND);
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                const double2 v = bp[i];
+                bx[2 * i] = v.x;
+                bx[2 * i + 1] = v.y;
+            }
+            double lb, ub;
+            fof_bounds<ND, MT>(gb, bx, L, lb, ub);
+            bool open = mine && fof_maybe<MT>(lb, L);
+            if (PASS0 && (ND == 6 || height == 0)) open = open && (int)((child + 1) << height) > lfirst;
+            if (PASS0 && height == 0) open = open && ((int)child >> 1) != (lfirst >> 1);  // done by fof_own
+            bool whole = PASS0 && mine && fof_surely<MT>(ub, L);
+            if (ND == 6 || !PASS0) whole = whole && open;
+            const uint64_t wh = ballot(whole);
+            todo = ballot(open && !whole);
+            if (wh) {
+                // every wave particle links to every particle of these nodes:
+                // wave and nodes form one component
+                const int32_t w0 = node_first(T, (int)(base + (uint32_t)__builtin_ctzll(wh)));
+                fof_join(P, act, w0, rq);
+                if (whole) {
+                    const int32_t nf = node_first(T, (int)child);
+                    uf_union(P, nf, w0);
                 }
-            } else {
-                down = false;
+                uint64_t loose = ballot(whole && !conn[child]);
+                while (loose) {
+                    const uint32_t c = base + (uint32_t)__builtin_ctzll(loose);
+                    loose &= loose - 1;
+                    const int32_t nf = node_first(T, (int)c), ne = node_end(T, (int)c);
+                    for (int32_t s = nf + 1 + lane; s < ne; s += NBX_WAVE) uf_union(P, s, nf);
+                    conn[c] = 1;
+                }
+            }
+            if (height == 0) {
+                // the leaves' flags and first parents together, not one
+                // load behind another
+                const bool op = (todo >> lane) & 1u;
+                const bool cf = op && conn[child];
+                const int32_t p0 = cf ? P[((int)child - T.nleafp) * NBX_LEAF] : -1;
+                const uint64_t cm = ballot(cf);
+                while (todo) {
+                    const int i = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    double lx[2 * ND];  // the leaf's box, from the lane that tested it
+#pragma unroll
+                    for (int d = 0; d < 2 * ND; ++d) lx[d] = lane_d(bx[d], i);
+                    const bool want = act && fof_maybe<MT>(fof_lb_box<ND, MT>(q, lx, L), L);
+                    if (!ballot(want)) continue;
+                    fof_leaf<PASS0, ND, MT>(T, (int)(base + (uint32_t)i) - T.nleafp, q, want, qi, lx, (cm >> i) & 1u,
+                                            __builtin_amdgcn_readlane(p0, i), L, P, rq);
+                }
             }
         }
-        if (node == 1) break;
-        if (!(node & 1)) {
-            node ^= 1;
-            down = true;
-        } else {
-            node >>= 1;
-            ++sh;
+        if (!todo) {
+            if (sp == 0) break;
+            --sp;  // back to the level above
+            todo = uniform64(stk[2 * sp]);
+            const uint64_t at = uniform64(stk[2 * sp + 1]);
+            base = (uint32_t)at;
+            height = (int)(at >> 32);
+            expand = false;
+            continue;
         }
+        node = base + (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        if (lane == 0) {
+            stk[2 * sp] = todo;
+            stk[2 * sp + 1] = ((uint64_t)height << 32) | base;
+        }
+        ++sp;
+        step = 6;
+        expand = true;
+    }
+}
+
+// Box of the positions of the lanes with act set (at least one).
+template <int ND>
+__device__ __forceinline__ void fof_wave_box(const double *q, bool act, double (&b)[2 * ND]) {
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        double lo = act ? q[d] : INFINITY, hi = act ? q[d] : -INFINITY;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, off));
+            hi = fmax(hi, __shfl_xor(hi, off));
+        }
+        b[d] = readfirst_d(lo);
+        b[ND + d] = readfirst_d(hi);
     }
 }
 
@@ -439,7 +631,11 @@ __device__ __forceinline__ void fof_task(const DevTree &T, const FofArgs &A, uin
     for (int d = 0; d < ND; ++d) q0[d] = valid ? T.x[d][qi] : 0.0;
     int32_t rq = valid ? qi : 0;
     const FofLink L = A.link;
-    fof_walk<1, ND, MT>(T, q0, valid, qi, g, L, A.parent, conn, rq);
+    __shared__ uint64_t stk[2 * FOF_STK];
+    double gb[2 * ND];
+    fof_wave_box<ND>(q0, valid, gb);
+    fof_own<ND, MT>(T, q0, valid, qi, g, gb, L, A.parent, rq);
+    fof_walk<1, ND, MT>(T, q0, valid, qi, g, gb, L, A.parent, conn, stk, rq);
     if (!A.periodic) return;
     // FOFSearchBallPeriodic: image toward the far wall when b^2 > s^2;
     // FOFSearchCriterionPeriodic: every image, left to the walk's bounds
@@ -465,18 +661,12 @@ __device__ __forceinline__ void fof_task(const DevTree &T, const FofArgs &A, uin
         }
         bool act = valid && (MT != 0 || L.lim > sval * sval);
         if (!ballot(act)) continue;
-        fof_walk<0, ND, MT>(T, xp, act, qi, g, L, A.parent, conn, rq);
+        fof_wave_box<ND>(xp, act, gb);
+        fof_walk<0, ND, MT>(T, xp, act, qi, g, gb, L, A.parent, conn, stk, rq);
     }
 }
 
-// Linking kernel for 3-D trees: one wave per workgroup in launch order, so
-// the hardware deals consecutive waves round robin to the XCDs.
-template <int ND, int MT>
-__global__ __launch_bounds__(64) void k_fof_waves(DevTree T, FofArgs A, uint8_t *conn) {
-    fof_task<ND, MT>(T, A, conn, blockIdx.x);
-}
-
-// Persistent linking kernel for 6-D trees, one wave per workgroup.  Workgroup b stays on
+// Persistent linking kernel, one wave per workgroup.  Workgroup b stays on
 // XCD (b mod 8) and takes waves from that XCD's contiguous share of the tree
 // order through the XCD's counter, so the nodes and leaves a neighbourhood's
 // waves share are fetched into one XCD's L2; once its share is drained it
@@ -484,9 +674,14 @@ __global__ __launch_bounds__(64) void k_fof_waves(DevTree T, FofArgs A, uint8_t 
 // shares' unequal cost (dense halos).  Every ticket names one wave, so every
 // wave runs once; a workgroup exits when all eight counters are past their
 // shares' ends.
+// Against one workgroup per wave in launch order: 2.7 and 4.4 ms on 16.8M
+// clustered particles, 0.46 and 0.57 ms on 2M (the order that won while the
+// walk was a serial chain of box tests: 10.2 against 11.1 ms).  Registers are
+// held to 5 waves per SIMD in 3-D and 4 in 6-D: 2.80 -> 2.69 ms and FOF6d of
+// 1.5M 0.63 -> 0.59 ms; one wave more spills (2.75 and 1.04 ms).
 #define FOF_CTR_STRIDE 16  // XCD counters 64 bytes apart
 template <int ND, int MT>
-__global__ __launch_bounds__(64) void k_fof(DevTree T, FofArgs A, uint8_t *conn, int32_t *ctr) {
+__global__ __launch_bounds__(64, ND == 3 ? 5 : 4) void k_fof(DevTree T, FofArgs A, uint8_t *conn, int32_t *ctr) {
     const int nw = (T.n + NBX_WAVE - 1) / NBX_WAVE;
     const int x = blockIdx.x & 7, q8 = nw >> 3, r8 = nw & 7;
     for (int s = 0; s < 8; ++s) {
@@ -519,20 +714,39 @@ static int fof_grid() {
     return grid;
 }
 
-// Group sizes and smallest member IDs.  Neighbouring slots mostly share a
-// root, so the lanes whose root equals the first active lane's are summed
-// in the wave and counted with one atomic pair; the rest count alone.
+// Group sizes and smallest member IDs, begun with each root's own share, so
+// that a particle alone (half of a clustered set) costs no atomic.
+__global__ __launch_bounds__(256) void k_fof_begin(const int32_t *P, int64_t n, const int32_t *perm, int32_t *cnt,
+                                                   int32_t *minid, int32_t *ng) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i == 0) *ng = 0;
+    if (i >= n) return;
+    if (P[i] == i) {
+        cnt[i] = 1;
+        minid[i] = perm[i];
+    }
+}
+// Every particle's root, stored as its parent (no links are made any more;
+// the find stores nothing on its way, so no stale grandparent can follow).
+// Neighbouring slots mostly share a root, so the lanes whose root equals the
+// first such lane's are summed in the wave and counted with one atomic pair;
+// the rest count alone.
 __global__ __launch_bounds__(256) void k_fof_compress(int32_t *P, int64_t n, const int32_t *perm, int32_t *cnt,
-                                                        int32_t *minid) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+                                                      int32_t *minid) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool in = i < n;
-    const int32_t r = in ? uf_find(P, (int32_t)i) : -1;
-    const int32_t id = in ? perm[i] : 0x7fffffff;
-    const uint64_t act = ballot(in);
+    int32_t r = in ? P[i] : -1;
+    if (in) {
+        for (int32_t up = uf_load_cached(P, r); up != r; up = uf_load_cached(P, r)) r = up;
+    }
+    const bool add = in && r != i;
+    if (add) P[i] = r;
+    const uint64_t act = ballot(add);
     if (!act) return;
+    const int32_t id = add ? perm[i] : 0x7fffffff;
     const int lead = __builtin_ctzll(act);
     const int32_t r0 = __shfl(r, lead);
-    const bool same = in && r == r0;
+    const bool same = add && r == r0;
     const uint64_t m = ballot(same);
     int32_t mn = same ? id : 0x7fffffff;
 #pragma unroll
@@ -541,25 +755,37 @@ __global__ __launch_bounds__(256) void k_fof_compress(int32_t *P, int64_t n, con
         atomicAdd(cnt + r0, (int32_t)__popcll(m));
         atomicMin(minid + r0, mn);
     }
-    if (in && !same) {
+    if (add && !same) {
         atomicAdd(cnt + r, 1);
         atomicMin(minid + r, id);
     }
 }
-__global__ __launch_bounds__(256) void k_fof_store_root(int32_t *P, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    P[i] = uf_find(P, (int32_t)i);
-}
+// Groups of at least minnum members; every other root's label is 0.  A block
+// takes FOF_COLLECT particles and one atomic for its groups (an atomic per
+// group on one counter took 165 us of 16.8M particles' 19,000 groups).
+#define FOF_COLLECT 4096
 __global__ __launch_bounds__(256) void k_fof_collect(const int32_t *P, const int32_t *cnt, const int32_t *minid,
-                                                       int64_t n, int32_t minnum, uint64_t *keys, int32_t *vals,
-                                                       int32_t *ng) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    if (P[i] != i || cnt[i] < minnum) return;
-    int32_t at = atomicAdd(ng, 1);
-    keys[at] = ((uint64_t)(0xffffffffu - (uint32_t)cnt[i]) << 32) | (uint32_t)minid[i];
-    vals[at] = (int32_t)i;
+                                                     int64_t n, int32_t minnum, uint64_t *keys, int32_t *vals,
+                                                     int32_t *lab, int32_t *ng) {
+    __shared__ int32_t found, at0;
+    __shared__ int32_t who[FOF_COLLECT];
+    if (threadIdx.x == 0) found = 0;
+    __syncthreads();
+    const int64_t i0 = (int64_t)blockIdx.x * FOF_COLLECT;
+    for (int t = threadIdx.x; t < FOF_COLLECT; t += 256) {
+        const int64_t i = i0 + t;
+        if (i >= n || P[i] != i) continue;
+        if (cnt[i] >= minnum) who[atomicAdd(&found, 1)] = (int32_t)i;
+        else lab[i] = 0;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) at0 = atomicAdd(ng, found);
+    __syncthreads();
+    for (int t = threadIdx.x; t < found; t += 256) {
+        const int32_t i = who[t];
+        keys[at0 + t] = ((uint64_t)(0xffffffffu - (uint32_t)cnt[i]) << 32) | (uint32_t)minid[i];
+        vals[at0 + t] = i;
+    }
 }
 __global__ __launch_bounds__(256) void k_fof_rank(const int32_t *vals, int64_t ng, int32_t *lab) {
     int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -751,19 +977,12 @@ static void launch_fof_t(const DevTree &T, const FofArgs &A, uint8_t *conn, hipS
                                A.parent, conn, 1, T.nleafp - 1);
     }
     ProfScope ps("k_fof_link", st);
-    if (ND == 3) {
-        // measured on 16.8M clustered particles: 10.2 ms per call in this
-        // order, 11.1 ms with the XCD shares below (before the skip of
-        // joined leaves); on the 6-D set the other way round (FOF6d 15.3 ms
-        // with the shares, 17.0 ms in this order)
-        hipLaunchKernelGGL((k_fof_waves<ND, MT>), dim3((T.n + NBX_WAVE - 1) / NBX_WAVE), dim3(NBX_WAVE), 0, st, T, A,
-                           conn);
-        return;
-    }
     // the XCD queue counters sit after the node flags, 64-byte aligned
     int32_t *ctr = (int32_t *)(((uintptr_t)(conn + 2 * (int64_t)T.nleafp) + 63) & ~(uintptr_t)63);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, ctr, 0, (int64_t)(8 * FOF_CTR_STRIDE));
-    hipLaunchKernelGGL((k_fof<ND, MT>), dim3(fof_grid<ND, MT>()), dim3(NBX_WAVE), 0, st, T, A, conn, ctr);
+    const int nw = (T.n + NBX_WAVE - 1) / NBX_WAVE, res = fof_grid<ND, MT>();
+    const int grid = nw < res ? (nw + 7) & ~7 : res;
+    hipLaunchKernelGGL((k_fof<ND, MT>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, conn, ctr);
 }
 
 // Bytes of the parent array, node flags and queue counters that
@@ -824,18 +1043,14 @@ hipError_t nbx_fof_canonical(const DevTree &T, int32_t *P, int32_t minnum, int32
     void *tmp = wb + W.off[8];
     hipError_t e = hipSuccess;
 #define CK(x) do { e = (x); if (e != hipSuccess) return e; } while (0)
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(n)), dim3(256), 0, st, cnt, 0, n);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(n)), dim3(256), 0, st, minid, 0x7fffffff, n);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(n)), dim3(256), 0, st, lab, 0, n);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, ng, 0, (int64_t)1);
     {
         ProfScope ps("k_fof_finish", st);
+        hipLaunchKernelGGL(k_fof_begin, dim3(nblk(n)), dim3(256), 0, st, P, n, T.perm, cnt, minid, ng);
         hipLaunchKernelGGL(k_fof_compress, dim3(nblk(n)), dim3(256), 0, st, P, n, T.perm, cnt, minid);
-        hipLaunchKernelGGL(k_fof_store_root, dim3(nblk(n)), dim3(256), 0, st, P, n);
     }
     {
-        hipLaunchKernelGGL(k_fof_collect, dim3(nblk(n)), dim3(256), 0, st, P, cnt, minid, n, minnum > 1 ? minnum : 1,
-                           keys, vals, ng);
+        hipLaunchKernelGGL(k_fof_collect, dim3((unsigned)((n + FOF_COLLECT - 1) / FOF_COLLECT)), dim3(256), 0, st, P, cnt,
+                           minid, n, minnum > 1 ? minnum : 1, keys, vals, lab, ng);
         int32_t hng = 0;
         CK(hipMemcpyAsync(&hng, ng, sizeof(int32_t), hipMemcpyDeviceToHost, st));
         CK(hipStreamSynchronize(st));

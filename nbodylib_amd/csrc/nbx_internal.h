@@ -183,6 +183,21 @@ __device__ __forceinline__ double readfirst_d(double v) {
     return u.d;
 }
 
+// lane i's value (i uniform)
+__device__ __forceinline__ double lane_d(double v, int i) {
+    union { double d; int32_t i[2]; } u;
+    u.d = v;
+    u.i[0] = __builtin_amdgcn_readlane(u.i[0], i);
+    u.i[1] = __builtin_amdgcn_readlane(u.i[1], i);
+    return u.d;
+}
+// a value all lanes hold, in scalar registers
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // Wsm, KDCalcSmoothQuantities.cxx:12-15: linear interpolation in the table,
 // indexed as (int)(r/h*0.5*(kernres-1)).  Past the table's end (r/h >= 2,
 // which CalcVelDensityWithPhysDensity's h without a square root reaches) the
