@@ -26,6 +26,11 @@
  * per possible group of minnum members) and is freed by
  * nbx_tree_destroy.  Calls on one tree from several threads or streams take
  * turns with the block; each waits on the device for the previous one's use.
+ *
+ * Device memory kept by the library: blocks given back by trees and calls are
+ * kept for later ones, at most 1/64 of the device's memory in all (4.5 GiB of
+ * 288); what exceeds that is freed, and everything kept is freed when an
+ * allocation fails.
  */
 #ifndef NBX_H
 #define NBX_H
@@ -96,9 +101,9 @@ int nbx_tree_create(const nbx_params *p, const double *pos, const double *vel, c
 int nbx_tree_create_dev(const nbx_params *p, const double *pos_dev, const double *vel_dev, const double *mass_dev,
                         int64_t n, void *stream, nbx_tree **out);
 /* Replaces KDTree::~KDTree (KDTree.cxx:1340-1356); caller-side reorder is the
- * shim's job.  The tree's arrays go back with hipFree, which waits for work
- * still running on the device, so no launch on any stream may still be using
- * the tree. */
+ * shim's job.  Waits for work still running on the device (as hipFree does),
+ * so no launch on any stream may still be using the tree.  Its memory is kept
+ * for the next tree (see below) or freed. */
 int nbx_tree_destroy(nbx_tree *t);
 /* slot -> ID map (host array of n).  The C++ shim uses it to reorder the
  * caller's Particle array as the reference does in BuildNodes. */

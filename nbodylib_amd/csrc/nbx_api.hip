@@ -41,31 +41,141 @@ static int hipfail(hipError_t e, const char *where) {
 extern "C" const char *nbx_last_error(void) { return g_err.c_str(); }
 extern "C" int nbx_host_fail(int code, const char *msg) { return fail(code, msg); }
 
-// Temporary device buffers of one host call, freed when the call returns on
-// any path (the HIPCK early returns included).  Constructed with a stream, it
-// allocates and frees in that stream's order (hipMallocAsync / hipFreeAsync).
+// ------------------------------------------------------------------ device memory
+// Blocks given back are kept, per device, for the next need of their size
+// class: a 2M-particle snapshot's tree and FOF took 6.0 ms, 4.3 of them in 12
+// hipMalloc, 12 hipFree and as many stream-ordered calls that mapped and
+// unmapped fresh memory, and takes 1.86 ms with one block per tree and blocks
+// kept.
+//  * Bounded: at most 1/64 of the device's memory is kept (4.5 GiB of 288);
+//    past that the oldest blocks are freed, and larger blocks are never kept.
+//    When an allocation fails every kept block is freed and it is tried again.
+//  * Streams: a block goes back with an event recorded on the stream that last
+//    used it, and the next user's stream waits for that event.
+//  * Threads: one mutex around the lists.
+// Nothing here is called under stream capture (every caller synchronises).
+struct KeptBlock {
+    void *p;
+    size_t bytes;
+    hipEvent_t used;
+};
+#define NBX_MAX_DEVICES 64
+struct KeptBlocks {
+    std::mutex mu;
+    std::vector<KeptBlock> free[NBX_MAX_DEVICES];  // oldest first
+    size_t total[NBX_MAX_DEVICES] = {};
+    size_t limit[NBX_MAX_DEVICES] = {};
+};
+static KeptBlocks &kept_blocks() {
+    static KeptBlocks *k = new KeptBlocks;  // never destroyed: trees may outlive static objects
+    return *k;
+}
+static size_t block_class(size_t bytes) {
+    size_t b = 4096;
+    while (b < bytes) b <<= 1;
+    const size_t step = b >= (1 << 16) ? b >> 3 : b;  // eighths of a power of two from 64 KiB on
+    return (bytes + step - 1) / step * step;
+}
+static void drop_block(KeptBlocks &k, int dev, size_t i) {
+    const KeptBlock b = k.free[dev][i];
+    k.free[dev].erase(k.free[dev].begin() + i);
+    k.total[dev] -= b.bytes;
+    hipEventSynchronize(b.used);
+    hipEventDestroy(b.used);
+    hipFree(b.p);
+}
+// *got bytes (at least need) at *p, for work on st from now on
+static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) {
+    *p = nullptr;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const size_t bytes = block_class(need);
+    if (dev >= 0 && dev < NBX_MAX_DEVICES) {
+        KeptBlocks &k = kept_blocks();
+        std::lock_guard<std::mutex> lk(k.mu);
+        std::vector<KeptBlock> &f = k.free[dev];
+        size_t best = f.size();
+        for (size_t i = 0; i < f.size(); ++i)  // the smallest that fits, the latest of equals
+            if (f[i].bytes >= bytes && f[i].bytes <= bytes + bytes / 2 && (best == f.size() || f[i].bytes <= f[best].bytes))
+                best = i;
+        if (best < f.size()) {
+            const KeptBlock b = f[best];
+            e = hipStreamWaitEvent(st, b.used, 0);
+            if (e != hipSuccess) return e;
+            f.erase(f.begin() + best);
+            k.total[dev] -= b.bytes;
+            hipEventDestroy(b.used);
+            *p = b.p;
+            *got = b.bytes;
+            return hipSuccess;
+        }
+    }
+    e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && dev >= 0 && dev < NBX_MAX_DEVICES) {
+        (void)hipGetLastError();
+        KeptBlocks &k = kept_blocks();
+        {
+            std::lock_guard<std::mutex> lk(k.mu);
+            while (!k.free[dev].empty()) drop_block(k, dev, 0);
+        }
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) *p = nullptr;
+    *got = bytes;
+    return e;
+}
+// st: the stream of the block's last use
+static void block_put(void *p, size_t bytes, hipStream_t st) {
+    if (!p) return;
+    int dev = 0;
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) == hipSuccess) dev = at.device;
+    else dev = -1;
+    hipEvent_t ev = nullptr;
+    if (dev >= 0 && dev < NBX_MAX_DEVICES) {
+        KeptBlocks &k = kept_blocks();
+        std::lock_guard<std::mutex> lk(k.mu);
+        if (k.limit[dev] == 0) {
+            size_t all = 0;
+            k.limit[dev] = hipDeviceTotalMem(&all, dev) == hipSuccess && all >= 64 ? all / 64 : 1;
+        }
+        if (bytes <= k.limit[dev] && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) {
+            if (hipEventRecord(ev, st) == hipSuccess) {
+                while (k.total[dev] + bytes > k.limit[dev]) drop_block(k, dev, 0);
+                k.free[dev].push_back({p, bytes, ev});
+                k.total[dev] += bytes;
+                return;
+            }
+            hipEventDestroy(ev);
+        }
+    }
+    hipFree(p);  // waits for work that still uses it
+}
+
+// Temporary device buffers of one host call, for work on one stream; given
+// back when the call returns on any path (the HIPCK early returns included).
 struct DevBufs {
-    std::vector<void *> held;
-    bool ordered = false;  // stream-ordered allocations on st
-    hipStream_t st = nullptr;
-    DevBufs() = default;
-    explicit DevBufs(hipStream_t s) : ordered(true), st(s) {}
+    struct Held {
+        void *p;
+        size_t bytes;
+    };
+    std::vector<Held> held;
+    hipStream_t st;
+    explicit DevBufs(hipStream_t s = nullptr) : st(s) {}
     DevBufs(const DevBufs &) = delete;
     DevBufs &operator=(const DevBufs &) = delete;
     template <class T>
     hipError_t alloc(T **ptr, size_t bytes) {
-        *ptr = nullptr;
-        const size_t b = bytes > 0 ? bytes : 1;
-        hipError_t e = ordered ? hipMallocAsync((void **)ptr, b, st) : hipMalloc((void **)ptr, b);
-        if (e == hipSuccess) held.push_back((void *)*ptr);
-        else *ptr = nullptr;
+        void *p = nullptr;
+        size_t got = 0;
+        const hipError_t e = block_get(bytes > 0 ? bytes : 1, st, &p, &got);
+        if (e == hipSuccess) held.push_back({p, got});
+        *ptr = (T *)p;
         return e;
     }
     ~DevBufs() {
-        for (void *x : held) {
-            if (ordered) hipFreeAsync(x, st);
-            else hipFree(x);
-        }
+        for (const Held &x : held) block_put(x.p, x.bytes, st);
     }
 };
 
@@ -180,6 +290,8 @@ struct nbx_tree {
     // tree.  One call holds it at a time (scr_mu); scr_done is recorded on
     // the holder's stream after its last use, and the next holder's stream
     // waits for it.
+    char *mem = nullptr;  // the arrays above, one block
+    size_t mem_bytes = 0;
     std::mutex scr_mu;
     char *scr = nullptr;
     size_t scr_cap = 0;
@@ -250,19 +362,10 @@ static inline int nblk(int64_t n, int b = 256) { return (int)((n + b - 1) / b); 
 
 static void free_tree(nbx_tree *t) {
     if (!t) return;
-    for (int d = 0; d < 6; ++d) { if (t->xs[d]) hipFree(t->xs[d]); if (t->xf[d]) hipFree(t->xf[d]); }
-    if (t->mass) hipFree(t->mass);
-    if (t->perm) hipFree(t->perm);
-    if (t->inv) hipFree(t->inv);
-    if (t->box) hipFree(t->box);
-    if (t->boxf) hipFree(t->boxf);
-    if (t->plane) hipFree(t->plane);
-    if (t->org) hipFree(t->org);
-    if (t->kern) hipFree(t->kern);
-    if (t->kernf) hipFree(t->kernf);
-    if (t->ext) hipFree(t->ext);
-    if (t->xq) hipFree(t->xq);
-    if (t->scr) hipFree(t->scr);
+    // no stream may still be using the tree (hipFree used to wait for that)
+    if (t->mem || t->scr) hipDeviceSynchronize();
+    block_put(t->mem, t->mem_bytes, nullptr);
+    block_put(t->scr, t->scr_cap, nullptr);
     if (t->scr_done) hipEventDestroy(t->scr_done);
     delete t;
 }
@@ -275,49 +378,63 @@ static int build_tree(nbx_tree *t, const double *pos, const double *vel, const d
     for (int d = 0; d < 3; ++d) c[d] = pos + d * n;
     for (int d = 0; d < 3; ++d) c[3 + d] = vel ? vel + d * n : nullptr;
 
-    // coordinates must be finite (a NaN or inf has no place in a split)
-    {
-        const int nb = 1024;
-        double *part = nullptr;
-        DevBufs pb(st);
-        HIPCK(pb.alloc(&part, sizeof(double) * 2 * nb * nd));
-        for (int d = 0; d < nd; ++d)
-            hipLaunchKernelGGL(k_bbox, dim3(nb), dim3(256), 0, st, c[d], n, part + 2 * nb * d);
-        std::vector<double> hp(2 * nb * nd);
-        HIPCK(hipMemcpyAsync(hp.data(), part, sizeof(double) * hp.size(), hipMemcpyDeviceToHost, st));
-        HIPCK(hipStreamSynchronize(st));
-        for (int d = 0; d < nd; ++d) {
-            double mn = INFINITY, mx = -INFINITY;
-            for (int b = 0; b < nb; ++b) { mn = std::min(mn, hp[2 * nb * d + 2 * b]); mx = std::max(mx, hp[2 * nb * d + 2 * b + 1]); }
-            if (!std::isfinite(mn) || !std::isfinite(mx)) return fail(NBX_ERR_ARG, "non-finite coordinates");
-        }
-    }
     // implicit heap-ordered tree over the leaves padded to a power of two
     t->nleaf = (int32_t)((n + NBX_LEAF - 1) / NBX_LEAF);
     t->nleafp = 1;
     t->depth = 0;
     while (t->nleafp < t->nleaf) { t->nleafp <<= 1; t->depth++; }
     t->nnodes = 2 * (int64_t)t->nleafp;
-    int32_t *order = nullptr;
-    DevBufs ob(st);  // order is freed (stream-ordered) when build_tree returns
-    HIPCK(ob.alloc(&order, sizeof(int32_t) * n));
+    DevBufs bufs(st);  // given back when build_tree returns
+    char *work = nullptr;
+    const size_t kd_bytes = nbx_kd_order_bytes(nd, n, t->nleafp);
+    Workspace ws = {nullptr, 0, 0};
+    ws.cap = 256 + sizeof(double) * 2 * nd * (NBX_BBOX_BLOCKS + 1) + 256 + sizeof(int32_t) * n + 256 + kd_bytes;
+    HIPCK(bufs.alloc(&work, ws.cap));
+    ws.base = work;
+    double *part = ws.carve<double>(sizeof(double) * 2 * nd * (NBX_BBOX_BLOCKS + 1));
+    int32_t *order = ws.carve<int32_t>(sizeof(int32_t) * n);
+    void *kd = ws.carve<void>(kd_bytes);
+    // coordinates must be finite (an inf has no place in a split)
+    {
+        double rb[12];
+        double *box = part + 2 * nd * NBX_BBOX_BLOCKS;
+        CoordPtrs cp;
+        for (int d = 0; d < nd; ++d) cp.c[d] = c[d];
+        const int nb = (int)std::min<int64_t>(NBX_BBOX_BLOCKS, (n + 2047) / 2048);
+        hipLaunchKernelGGL(k_bbox, dim3(nb, nd), dim3(256), 0, st, cp, n, part);
+        hipLaunchKernelGGL(k_bbox_end, dim3(nd), dim3(256), 0, st, part, nb, box);
+        HIPCK(hipMemcpyAsync(rb, box, sizeof(double) * 2 * nd, hipMemcpyDeviceToHost, st));
+        HIPCK(hipStreamSynchronize(st));
+        for (int d = 0; d < 2 * nd; ++d)
+            if (!std::isfinite(rb[d])) return fail(NBX_ERR_ARG, "non-finite coordinates");
+    }
     {
         ProfScope ps("k_build_kdorder", st);
-        HIPCK(nbx_kd_order(c, nd, n, t->nleafp, order, st));
+        HIPCK(nbx_kd_order(c, nd, n, t->nleafp, order, kd, st));
     }
     const int64_t npad = (n + NBX_LEAF - 1) / NBX_LEAF * NBX_LEAF;
-    for (int d = 0; d < ncoord; ++d) HIPCK(hipMalloc((void **)&t->xs[d], sizeof(double) * npad));
-    HIPCK(hipMalloc((void **)&t->mass, sizeof(double) * npad));
-    HIPCK(hipMalloc((void **)&t->perm, sizeof(int32_t) * npad));
-    HIPCK(hipMalloc((void **)&t->inv, sizeof(int32_t) * n));
-    HIPCK(hipMalloc((void **)&t->box, sizeof(double) * 2 * nd * (size_t)t->nnodes));
-    HIPCK(hipMalloc((void **)&t->plane, sizeof(float) * (nd == 6 ? 8 : 4) * (size_t)t->nleafp));
-    if (t->p.form == NBX_FORM_MIXED) {
-        HIPCK(hipMalloc((void **)&t->org, sizeof(double) * nd * (size_t)t->nleaf));
-        HIPCK(hipMalloc((void **)&t->ext, sizeof(double) * (size_t)t->nleaf));
-        if (nd == 3) HIPCK(hipMalloc((void **)&t->xq, sizeof(float4) * npad));
-        else for (int d = 0; d < nd; ++d) HIPCK(hipMalloc((void **)&t->xf[d], sizeof(float) * npad));
+    const bool mixed = t->p.form == NBX_FORM_MIXED;
+    make_kernel(nd, t->p.kerntype, t->kernres, t->kernnorm, t->hkern);
+    // the tree's arrays, carved from one block: the first pass sizes it
+    for (int pass = 0; pass < 2; ++pass) {
+        Workspace w = {t->mem, pass ? t->mem_bytes : ~(size_t)0, 0};
+        for (int d = 0; d < ncoord; ++d) t->xs[d] = w.carve<double>(sizeof(double) * npad);
+        t->mass = w.carve<double>(sizeof(double) * npad);
+        t->perm = w.carve<int32_t>(sizeof(int32_t) * npad);
+        t->inv = w.carve<int32_t>(sizeof(int32_t) * n);
+        t->box = w.carve<double>(sizeof(double) * 2 * nd * (size_t)t->nnodes);
+        t->plane = w.carve<float>(sizeof(float) * (nd == 6 ? 8 : 4) * (size_t)t->nleafp);
+        t->kern = w.carve<double>((sizeof(double) + sizeof(float)) * t->kernres);  // and the FP32 table after it
+        if (mixed) {
+            t->boxf = w.carve<float>(sizeof(float) * 2 * nd * (size_t)t->nnodes);
+            t->org = w.carve<double>(sizeof(double) * nd * (size_t)t->nleaf);
+            t->ext = w.carve<double>(sizeof(double) * (size_t)t->nleaf);
+            if (nd == 3) t->xq = w.carve<float4>(sizeof(float4) * npad);
+            else for (int d = 0; d < nd; ++d) t->xf[d] = w.carve<float>(sizeof(float) * npad);
+        }
+        if (pass == 0) HIPCK(block_get(w.used, st, (void **)&t->mem, &t->mem_bytes));
     }
+    t->kernf = (float *)(t->kern + t->kernres);
     {
         ProfScope ps("k_build_gather", st);
         GatherArgs g;
@@ -352,33 +469,29 @@ static int build_tree(nbx_tree *t, const double *pos, const double *vel, const d
                                1 << dep, 1 << dep, nd);
     }
     HIPCK(hipGetLastError());
-    if (t->p.form == NBX_FORM_MIXED) {
-        // FP32 node boxes for the precision form's walk, when every
-        // coordinate lies within 1e30 (the bound its FP32 node test assumes;
-        // otherwise the precision-form calls run the FP64 kernel)
-        double rb[12];
+    double rb[12];
+    if (mixed) {
+        // FP32 node boxes for the precision form's walk
+        const int64_t cnt = 2 * nd * (int64_t)t->nnodes;
+        hipLaunchKernelGGL(k_boxf, dim3(nblk(cnt)), dim3(256), 0, st, t->box, t->boxf, cnt, nd);
+        HIPCK(hipGetLastError());
         HIPCK(hipMemcpyAsync(rb, t->box + 2 * nd, sizeof(double) * 2 * nd, hipMemcpyDeviceToHost, st));
-        HIPCK(hipStreamSynchronize(st));
+    }
+    // kernel table, FP64 and FP32 in one copy
+    std::vector<char> tab((sizeof(double) + sizeof(float)) * t->kernres);
+    memcpy(tab.data(), t->hkern.data(), sizeof(double) * t->kernres);
+    float *tf = (float *)(tab.data() + sizeof(double) * t->kernres);
+    for (int i = 0; i < t->kernres; ++i) tf[i] = (float)t->hkern[i];
+    HIPCK(hipMemcpyAsync(t->kern, tab.data(), tab.size(), hipMemcpyHostToDevice, st));
+    HIPCK(hipStreamSynchronize(st));
+    if (mixed) {
+        // they serve when every coordinate lies within 1e30 (the bound the
+        // FP32 node test assumes; otherwise the precision-form calls run the
+        // FP64 kernel)
         bool fits = true;
         for (int d = 0; d < 2 * nd; ++d) fits = fits && fabs(rb[d]) <= 1e30;
-        if (fits) {
-            const int64_t cnt = 2 * nd * (int64_t)t->nnodes;
-            HIPCK(hipMalloc((void **)&t->boxf, sizeof(float) * cnt));
-            hipLaunchKernelGGL(k_boxf, dim3(nblk(cnt)), dim3(256), 0, st, t->box, t->boxf, cnt, nd);
-            HIPCK(hipGetLastError());
-        }
+        if (!fits) t->boxf = nullptr;
     }
-    // kernel table
-    make_kernel(nd, t->p.kerntype, t->kernres, t->kernnorm, t->hkern);
-    HIPCK(hipMalloc((void **)&t->kern, sizeof(double) * t->kernres));
-    HIPCK(hipMemcpyAsync(t->kern, t->hkern.data(), sizeof(double) * t->kernres, hipMemcpyHostToDevice, st));
-    {
-        std::vector<float> kf(t->hkern.begin(), t->hkern.end());
-        HIPCK(hipMalloc((void **)&t->kernf, sizeof(float) * t->kernres));
-        HIPCK(hipMemcpyAsync(t->kernf, kf.data(), sizeof(float) * t->kernres, hipMemcpyHostToDevice, st));
-        HIPCK(hipStreamSynchronize(st));
-    }
-    HIPCK(hipStreamSynchronize(st));
     return NBX_OK;
 }
 
@@ -486,14 +599,13 @@ struct ScratchLease {
             if (t->scr) {
                 if (t->scr_recorded) err = hipEventSynchronize(t->scr_done);
                 if (err != hipSuccess) return;
-                hipFree(t->scr);
+                block_put(t->scr, t->scr_cap, st);
                 t->scr = nullptr;
                 t->scr_cap = 0;
                 t->scr_recorded = false;
             }
-            err = hipMalloc((void **)&t->scr, need);
-            if (err != hipSuccess) { t->scr = nullptr; return; }
-            t->scr_cap = need;
+            err = block_get(need, st, (void **)&t->scr, &t->scr_cap);
+            if (err != hipSuccess) { t->scr = nullptr; t->scr_cap = 0; return; }
         }
         if (t->scr_recorded) err = hipStreamWaitEvent(st, t->scr_done, 0);
         if (err == hipSuccess) ws = {t->scr, t->scr_cap, 0};
@@ -525,6 +637,11 @@ static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed, int32_t
 // from the tree's kept scratch when ws is null.
 static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t st, Workspace *ws = nullptr) {
     if (nq <= 0) return hipSuccess;
+    // under capture the launcher allocates for itself, as part of the graph: a
+    // replay must not meet later calls in the tree's block
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (!ws && st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+        return nbx_launch_knn(t->view(), A, nq, st);
     size_t need = nbx_knn_scratch_bytes(t->nd, A.kh, A.qsrc, nq);
     std::unique_ptr<ScratchLease> lease;
     if (!ws) {
@@ -921,7 +1038,6 @@ extern "C" int nbx_knn_density_dev(nbx_tree *t, int32_t k, int32_t *nn_by_slot_d
 // smallest scratch (8 workgroups, 1.03 MiB at k > 64).
 #define NBX_NOALLOC_ARRAY (NBX_NOALLOC_BYTES + ((size_t)2 << 20))
 static __device__ __align__(256) unsigned char scratch[NBX_NOALLOC_ARRAY];
-#define NBX_MAX_DEVICES 64
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[NBX_MAX_DEVICES];  // per device: the address of `scratch` there
 

@@ -13,14 +13,8 @@
 #include "nbx_kernels.h"
 
 // ---------------------------------------------------------------- bounding box
-__global__ __launch_bounds__(256) void k_bbox(const double *__restrict__ c, int64_t n, double *__restrict__ part) {
+__device__ __forceinline__ void bbox_block(double mn, double mx, double *out) {
     __shared__ double smn[256], smx[256];
-    double mn = 1.0 / 0.0, mx = -1.0 / 0.0;
-    for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        double v = c[i];
-        mn = v < mn ? v : mn;
-        mx = v > mx ? v : mx;
-    }
     smn[threadIdx.x] = mn;
     smx[threadIdx.x] = mx;
     __syncthreads();
@@ -32,9 +26,28 @@ __global__ __launch_bounds__(256) void k_bbox(const double *__restrict__ c, int6
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = smn[0];
-        part[2 * blockIdx.x + 1] = smx[0];
+        out[0] = smn[0];
+        out[1] = smx[0];
     }
+}
+__global__ __launch_bounds__(256) void k_bbox(CoordPtrs c, int64_t n, double *__restrict__ part) {
+    const double *__restrict__ x = c.c[blockIdx.y];
+    double mn = 1.0 / 0.0, mx = -1.0 / 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        double v = x[i];
+        mn = v < mn ? v : mn;
+        mx = v > mx ? v : mx;
+    }
+    bbox_block(mn, mx, part + 2 * ((int64_t)blockIdx.y * NBX_BBOX_BLOCKS + blockIdx.x));
+}
+__global__ __launch_bounds__(256) void k_bbox_end(const double *__restrict__ part, int nb, double *__restrict__ box) {
+    const double *p = part + 2 * (int64_t)blockIdx.x * NBX_BBOX_BLOCKS;
+    double mn = 1.0 / 0.0, mx = -1.0 / 0.0;
+    for (int b = threadIdx.x; b < nb; b += 256) {
+        mn = fmin(mn, p[2 * b]);
+        mx = fmax(mx, p[2 * b + 1]);
+    }
+    bbox_block(mn, mx, box + 2 * blockIdx.x);
 }
 
 // ---------------------------------------------------------------- gather

@@ -563,48 +563,72 @@ __global__ __launch_bounds__(KD_LT) void k_kd_local(KdState S, int64_t n, int lb
 
 static inline int nblk(int64_t n, int b = KD_T) { return (int)((n + b - 1) / b); }
 
-hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleafp, int32_t *order, hipStream_t st) {
+// The build's temporaries: IDs and keys in the current and the next order,
+// and for the global levels their nodes' extents, pivots, counts and
+// histograms and the blocks' counts and prefixes.
+struct KdWork {
+    KdState S;
+    uint32_t *ext, *pre, *hist;
+    int32_t *need;
+    uint8_t *dsel;
+    uint64_t *blk, *bpre;
+    int ltot, lblk;
+    bool global;
+    int64_t nsegmax;
+    size_t total;
+    KdWork(void *base, int nd, int64_t n, int32_t nleafp) {
+        ltot = 0;  // log2 of the padded slot span
+        while (((int64_t)1 << ltot) < (int64_t)nleafp * NBX_LEAF) ++ltot;
+        int lloc = 0;
+        while ((1 << lloc) < KD_LOCAL) ++lloc;
+        lblk = ltot < lloc ? ltot : lloc;
+        global = ltot > lblk;
+        // the most nodes any global level has (its node ranges are 2 * KD_LOCAL)
+        nsegmax = global ? ((int64_t)1 << (ltot - lblk - 1)) : 1;
+        size_t at = 0;
+        auto carve = [&](size_t b) {
+            char *p = (char *)base + at;
+            at += (b + 255) & ~(size_t)255;
+            return (void *)p;
+        };
+        memset(&S, 0, sizeof(S));
+        S.id = (int32_t *)carve(sizeof(int32_t) * n);
+        for (int d = 0; d < nd; ++d) S.key[d] = (uint32_t *)carve(sizeof(uint32_t) * n);
+        if (global) {
+            const int64_t nb = (n + KD_LOCAL - 1) / KD_LOCAL;
+            S.id2 = (int32_t *)carve(sizeof(int32_t) * n);
+            for (int d = 0; d < nd; ++d) S.key2[d] = (uint32_t *)carve(sizeof(uint32_t) * n);
+            ext = (uint32_t *)carve(sizeof(uint32_t) * 2 * nd * nsegmax);
+            pre = (uint32_t *)carve(sizeof(uint32_t) * nsegmax);
+            need = (int32_t *)carve(sizeof(int32_t) * nsegmax);
+            dsel = (uint8_t *)carve((size_t)nsegmax);
+            hist = (uint32_t *)carve(sizeof(uint32_t) * 256 * nsegmax);
+            blk = (uint64_t *)carve(sizeof(uint64_t) * nb);
+            bpre = (uint64_t *)carve(sizeof(uint64_t) * nb);
+        }
+        total = at;
+    }
+};
+size_t nbx_kd_order_bytes(int nd, int64_t n, int32_t nleafp) { return KdWork(nullptr, nd, n, nleafp).total; }
+
+hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleafp, int32_t *order, void *work,
+                        hipStream_t st) {
     if (n <= 0) return hipSuccess;
     if (nd != 3 && nd != 6) return hipErrorInvalidValue;
-    int ltot = 0;  // log2 of the padded slot span
-    while (((int64_t)1 << ltot) < (int64_t)nleafp * NBX_LEAF) ++ltot;
-    int lloc = 0;
-    while ((1 << lloc) < KD_LOCAL) ++lloc;
-    const int lblk = ltot < lloc ? ltot : lloc;
-    const bool global = ltot > lblk;
-    // the most nodes any global level has (its node ranges are 2 * KD_LOCAL)
-    const int64_t nsegmax = global ? ((int64_t)1 << (ltot - lblk - 1)) : 1;
-
-    KdState Sh;
-    memset(&Sh, 0, sizeof(Sh));
+    KdWork W(work, nd, n, nleafp);
+    KdState &Sh = W.S;
+    const int ltot = W.ltot, lblk = W.lblk;
+    uint32_t *ext = W.ext, *pre = W.pre, *hist = W.hist;
+    int32_t *need = W.need;
+    uint8_t *dsel = W.dsel;
+    uint64_t *blk = W.blk, *bpre = W.bpre;
     KdCoords C;
     memset(&C, 0, sizeof(C));
     for (int d = 0; d < nd; ++d) C.c[d] = c[d];
-    hipError_t e = hipSuccess;
-    uint32_t *ext = nullptr, *pre = nullptr, *hist = nullptr;
-    int32_t *need = nullptr;
-    uint8_t *dsel = nullptr;
-    uint64_t *blk = nullptr, *bpre = nullptr;
-#define KDCK(x)                          \
-    do {                                 \
-        e = (x);                         \
-        if (e != hipSuccess) goto done;  \
-    } while (0)
-    KDCK(hipMallocAsync((void **)&Sh.id, sizeof(int32_t) * n, st));
-    for (int d = 0; d < nd; ++d) KDCK(hipMallocAsync((void **)&Sh.key[d], sizeof(uint32_t) * n, st));
     hipLaunchKernelGGL(k_kd_init, dim3(nblk(n)), dim3(KD_T), 0, st, C, nd, n, Sh);
-    if (global) {
+    if (W.global) {
         const int nb = nblk(n, KD_LOCAL);
-        KDCK(hipMallocAsync((void **)&Sh.id2, sizeof(int32_t) * n, st));
-        for (int d = 0; d < nd; ++d) KDCK(hipMallocAsync((void **)&Sh.key2[d], sizeof(uint32_t) * n, st));
-        KDCK(hipMallocAsync((void **)&ext, sizeof(uint32_t) * 2 * nd * nsegmax, st));
-        KDCK(hipMallocAsync((void **)&pre, sizeof(uint32_t) * nsegmax, st));
-        KDCK(hipMallocAsync((void **)&need, sizeof(int32_t) * nsegmax, st));
-        KDCK(hipMallocAsync((void **)&dsel, (size_t)nsegmax, st));
-        KDCK(hipMallocAsync((void **)&hist, sizeof(uint32_t) * 256 * nsegmax, st));
-        hipLaunchKernelGGL(k_kd_zero, dim3(nblk(256 * nsegmax)), dim3(KD_T), 0, st, hist, (int64_t)256 * nsegmax);
-        KDCK(hipMallocAsync((void **)&blk, sizeof(uint64_t) * nb, st));
-        KDCK(hipMallocAsync((void **)&bpre, sizeof(uint64_t) * nb, st));
+        hipLaunchKernelGGL(k_kd_zero, dim3(nblk(256 * W.nsegmax)), dim3(KD_T), 0, st, hist, (int64_t)256 * W.nsegmax);
         // root extents; deeper levels get theirs from the previous move
         hipLaunchKernelGGL(k_kd_ext_init, dim3(nblk(nd)), dim3(KD_T), 0, st, ext, (int64_t)nd);
         if (nd == 3)
@@ -645,23 +669,7 @@ hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleaf
         else
             hipLaunchKernelGGL(k_kd_local<6>, dim3((unsigned)nb), dim3(KD_LT), 0, st, Sh, n, lblk, order);
     }
-    e = hipGetLastError();
-done:
-    if (Sh.id) hipFreeAsync(Sh.id, st);
-    if (Sh.id2) hipFreeAsync(Sh.id2, st);
-    for (int d = 0; d < 6; ++d) {
-        if (Sh.key[d]) hipFreeAsync(Sh.key[d], st);
-        if (Sh.key2[d]) hipFreeAsync(Sh.key2[d], st);
-    }
-    if (ext) hipFreeAsync(ext, st);
-    if (pre) hipFreeAsync(pre, st);
-    if (need) hipFreeAsync(need, st);
-    if (dsel) hipFreeAsync(dsel, st);
-    if (hist) hipFreeAsync(hist, st);
-    if (blk) hipFreeAsync(blk, st);
-    if (bpre) hipFreeAsync(bpre, st);
-#undef KDCK
-    return e;
+    return hipGetLastError();
 }
 
 hipError_t nbx_sort_pairs_u32(void *temp, size_t &temp_bytes, uint32_t *kin, uint32_t *kout, int32_t *vin,

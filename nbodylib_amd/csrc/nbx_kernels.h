@@ -27,7 +27,14 @@ struct GatherArgs {
     float4 *xq;    // precision form, 3-D: the offsets and fl(fl(fl(x^2) + y^2) + z^2) interleaved
 };
 
-__global__ void k_bbox(const double *c, int64_t n, double *part);
+// Smallest and largest value of each coordinate array: blocks' shares (grid
+// blocks x arrays), then box[2 d], box[2 d + 1].
+#define NBX_BBOX_BLOCKS 1024
+struct CoordPtrs {
+    const double *c[6];
+};
+__global__ void k_bbox(CoordPtrs c, int64_t n, double *part);
+__global__ void k_bbox_end(const double *part, int nb, double *box);
 __global__ void k_gather_leaf(GatherArgs a);
 __global__ void k_leafbox_pad(double *box, int32_t nleaf, int32_t nleafp, int nd);
 __global__ void k_levelbox(double *box, float *plane, int32_t first, int32_t count, int nd);
@@ -35,7 +42,10 @@ __global__ void k_boxf(const double *box, float *boxf, int64_t count, int nd);
 
 // order (slot -> ID) of the implicit kd tree: midpoint splits along the
 // widest dimension of every node (nbx_kdbuild.hip)
-hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleafp, int32_t *order, hipStream_t st);
+// (work: nbx_kd_order_bytes of device memory)
+size_t nbx_kd_order_bytes(int nd, int64_t n, int32_t nleafp);
+hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleafp, int32_t *order, void *work,
+                        hipStream_t st);
 hipError_t nbx_sort_pairs_u64(void *temp, size_t &temp_bytes, uint64_t *kin, uint64_t *kout, int32_t *vin,
                               int32_t *vout, int64_t n, hipStream_t st);
 hipError_t nbx_sort_pairs_u32(void *temp, size_t &temp_bytes, uint32_t *kin, uint32_t *kout, int32_t *vin,
