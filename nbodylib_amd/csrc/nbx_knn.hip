@@ -238,11 +238,11 @@ __device__ __forceinline__ void knn_leaf(const DevTree &T, const double *const (
     __syncthreads();
 }
 
-// Uniform stackless depth-first walk of the heap-ordered tree.  The first
-// descent follows the ancestors of the wave's own leaf node (anc; -1 when
-// the queries are not tree particles or are image-shifted), so every lane
-// is filled from the query's own neighbourhood before anything else is
-// opened; below that children are taken nearest first from qc.  A node is
+// Uniform stackless depth-first walk of the heap-ordered tree.  It starts at
+// the wave's own leaf node (anc; -1 when the queries are not tree particles or
+// are image-shifted: then at the root), so every lane is filled from the
+// query's own neighbourhood before anything else is opened; elsewhere
+// children are taken nearest first from qc.  A node is
 // opened when any active lane has box_lb <= its current k-th distance.
 // State is uniform (SGPRs): node, depth and one "right child first" bit per
 // depth; the tree's fields it reads are scalar values of their own (a field
@@ -262,6 +262,13 @@ __device__ __forceinline__ void knn_walk(const DevTree &T, KnnCtx<ND, KMAX> &c, 
     }
     int node = 1, dep = 0;
     uint64_t firstright = 0;
+    if (anc >= 0) {
+        // nothing is kept yet, so every node down to the wave's own leaf is
+        // open: start there, the path's bits saying which child went first
+        node = anc;
+        dep = D;
+        firstright = (uint64_t)(__builtin_bitreverse32((uint32_t)anc) >> (31 - D)) & ~1ULL;
+    }
     for (;;) {
         cdptr bx = (cdptr)(boxp + (size_t)node * 2 * ND);
         const bool want = c.act && box_lb<ND>(c.q, bx) <= c.kth;
@@ -269,9 +276,7 @@ __device__ __forceinline__ void knn_walk(const DevTree &T, KnnCtx<ND, KMAX> &c, 
             if (dep == D) {
                 knn_leaf<ND, KMAX, TIE>(T, X, node - nleafp, c, hd, sl, cx, lane, kh);
             } else {
-                int first;
-                if (anc >= 0 && (anc >> (D - dep)) == node) first = anc >> (D - dep - 1);
-                else first = 2 * node + (first_is_right<ND>(planep, node, qc) ? 1 : 0);
+                const int first = 2 * node + (first_is_right<ND>(planep, node, qc) ? 1 : 0);
                 dep += 1;
                 firstright = (firstright & ~(1ULL << dep)) | ((uint64_t)(first & 1) << dep);
                 node = first;

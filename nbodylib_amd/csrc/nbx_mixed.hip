@@ -229,13 +229,21 @@ __device__ __forceinline__ void mix_load(const MixSrc<6> &S, int leaf, int lane,
     }
 }
 
-// 6-D: a query in LDS, 8 floats: its coordinates and its threshold (two
-// 16-byte accesses)
-#define MX_QW 8
+// A query in LDS for a transposed test: its coordinates and its threshold, 4
+// floats in 3-D and 8 in 6-D (16-byte accesses), at most MX_QMAX of them
+// (even, so that an odd count has room for one that passes nothing).
+#define MX_FEW 24  // 3-D: wanting lanes up to which a leaf is scanned transposed (see mix_leaf)
+#define MX_QW(ND) ((ND) == 6 ? 8 : 4)
+#define MX_QMAX(ND) ((ND) == 6 ? NBX_WAVE : MX_FEW + 2)
+template <int ND>
 __device__ __forceinline__ void mix_put_query(float *qb, int at, const float *q, float th) {
-    float4 *p = (float4 *)qb + 2 * at;
-    p[0] = make_float4(q[0], q[1], q[2], q[3]);
-    p[1] = make_float4(q[4], q[5], th, 0.0f);
+    float4 *p = (float4 *)qb + (MX_QW(ND) / 4) * at;
+    if constexpr (ND == 6) {
+        p[0] = make_float4(q[0], q[1], q[2], q[3]);
+        p[1] = make_float4(q[4], q[5], th, 0.0f);
+    } else {
+        p[0] = make_float4(q[0], q[1], q[2], th);
+    }
 }
 
 template <int ND, int KMAX>
@@ -273,7 +281,9 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
     for (int d = 0; d < ND; ++d) qv[d] = (float)(c.q[d] - (ND == 6 ? pre.o[d] : ((cdptr)o)[d]));
     const float th = __uint_as_float(c.root);
     uint32_t mask = 0u;
-    if constexpr (ND == 3) {
+    const uint64_t wm = ballot(want);
+    const int nwq = __popcll(wm);
+    if (ND == 3 && nwq > MX_FEW) {
         // Phase 1: every lane tests the 32 candidates, read in 64-byte scalar
         // loads, in the expanded form
         //     w + 2 qv.p >= |p|^2,  w = th + m - |qv|^2
@@ -320,30 +330,38 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
         // them against the 32 candidates, one candidate per lane; the
         // ballot's halves are the two queries' accept masks, left in LDS for
         // their lanes.  Lanes that do not want the leaf have no candidate in
-        // it: their bound already exceeds their largest kept key.
-        const uint64_t wm = ballot(want);
-        const int nwq = __popcll(wm);
+        // it: their bound already exceeds their largest kept key.  In 6-D
+        // always; in 3-D, where the scan by lanes takes 200 VALU and 57% of
+        // the leaves are wanted by at most 16 lanes, up to MX_FEW of them:
+        // 16.8M particles, k = 32, 18.58 ms without, 17.89 up to 12, 17.83
+        // up to 24, 17.91 up to 32, 18.06 up to 48.
         const int wr = __builtin_amdgcn_mbcnt_hi((uint32_t)(wm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)wm, 0u));
-        if (want) mix_put_query(cx, wr, qv, th);
+        if (want) mix_put_query<ND>(cx, wr, qv, th);
         if ((nwq & 1) && lane == 0) {
             // an odd count's last step tests a second query that passes nothing
             const float none[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-            mix_put_query(cx, nwq, none, -1.0f);
+            mix_put_query<ND>(cx, nwq, none, -1.0f);
         }
         __syncthreads();
-        const float4 *qm = (const float4 *)cx + 2 * (lane >> 5);
-        uint32_t *mb = (uint32_t *)(cx + MX_QW * NBX_WAVE);
+        constexpr int Q4 = MX_QW(ND) / 4;
+        const float4 *qm = (const float4 *)cx + Q4 * (lane >> 5);
+        uint32_t *mb = (uint32_t *)(cx + MX_QW(ND) * MX_QMAX(ND));
         for (int it = 0; it < nwq; it += 2) {
-            const float4 a = qm[2 * it], b = qm[2 * it + 1];
-            const float t0 = a.x - st[0], t1 = a.y - st[1], t2 = a.z - st[2], t3 = a.w - st[3], t4 = b.x - st[4],
-                        t5 = b.y - st[5];
+            const float4 a = qm[Q4 * it];
+            const float t0 = a.x - st[0], t1 = a.y - st[1], t2 = a.z - st[2];
             float dd = t0 * t0;
             dd = __builtin_fmaf(t1, t1, dd);
             dd = __builtin_fmaf(t2, t2, dd);
-            dd = __builtin_fmaf(t3, t3, dd);
-            dd = __builtin_fmaf(t4, t4, dd);
-            dd = __builtin_fmaf(t5, t5, dd);
-            const uint64_t pm = ballot(dd <= b.z);
+            float lim = a.w;
+            if constexpr (ND == 6) {
+                const float4 b = qm[Q4 * it + 1];
+                const float t3 = a.w - st[3], t4 = b.x - st[4], t5 = b.y - st[5];
+                dd = __builtin_fmaf(t3, t3, dd);
+                dd = __builtin_fmaf(t4, t4, dd);
+                dd = __builtin_fmaf(t5, t5, dd);
+                lim = b.z;
+            }
+            const uint64_t pm = ballot(dd <= lim);
             if (lane == 0) *(uint64_t *)(mb + it) = pm;
         }
         __syncthreads();
@@ -406,10 +424,10 @@ __device__ __forceinline__ void mix_leaf(const MixSrc<ND> &S, int leaf, MixCtx<N
     }
     // as many steps as the lane with the most candidates needs (a counted
     // loop keeps the kept-key state in place across steps)
-    int nit = __popc(mask);
+    const int nmine = __popc(mask);
+    int nit = 0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) nit = max(nit, __shfl_xor(nit, off));
-    nit = __builtin_amdgcn_readfirstlane(nit);
+    for (int b = 32; b > 0; b >>= 1) nit += ballot(nmine >= nit + b) ? b : 0;
     for (int it = 0; it < nit; ++it) {
         const bool has = mask != 0;
         const int j = __builtin_ctz(mask | 0x80000000u);
@@ -482,11 +500,11 @@ __device__ __forceinline__ uint32_t mix_test8(const float *boxp, const float *pl
     const uint64_t wm = ballot(want);
     const int nwq = __popcll(wm);
     const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(wm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)wm, 0u));
-    if (want) mix_put_query(cx, rank, q32, th);
+    if (want) mix_put_query<ND>(cx, rank, q32, th);
     __syncthreads();
     // the step's ballot holds 8 bits per query: byte r of mb is the mask of
     // the query with rank r
-    uint8_t *mb = (uint8_t *)(cx + MX_QW * NBX_WAVE);
+    uint8_t *mb = (uint8_t *)(cx + MX_QW(ND) * NBX_WAVE);
     const float4 *qm = (const float4 *)cx;
     uint64_t any = 0;
     for (int it = 0; it < nwq; it += 8) {
@@ -594,8 +612,12 @@ __device__ __forceinline__ void mix_walk(const DevTree &T, const double *ext, Mi
             asm volatile("" : "+v"(S.xf[d]));
         }
     }
-    int node = 1, dep = 0;
-    uint64_t firstright = 0;
+    // The walk starts where the first descent ends: every node on the way to
+    // the wave's own leaf is open (nothing is kept yet), and its child toward
+    // the leaf goes first.  Bit d of firstright is that child's last bit at
+    // depth d, the path's bits from the root down.
+    int node = anc, dep = D;
+    uint64_t firstright = (uint64_t)(__builtin_bitreverse32((uint32_t)anc) >> (31 - D)) & ~1ULL;
     if constexpr (ND == 3) {
         for (;;) {
             cfptr bx = (cfptr)(boxp + (size_t)node * 2 * ND);
@@ -605,9 +627,7 @@ __device__ __forceinline__ void mix_walk(const DevTree &T, const double *ext, Mi
                     if (c.nvis >= MX_V) break;  // visit table full: lanes fall back
                     mix_leaf<ND, KMAX>(S, node - nleafp, c, want, hk, sl, cx, lane, gm, MixPre());
                 } else {
-                    int first;
-                    if ((anc >> (D - dep)) == node) first = anc >> (D - dep - 1);
-                    else first = 2 * node + (first_is_right<ND>(planep, node, qc) ? 1 : 0);
+                    const int first = 2 * node + (first_is_right<ND>(planep, node, qc) ? 1 : 0);
                     dep += 1;
                     firstright = (firstright & ~(1ULL << dep)) | ((uint64_t)(first & 1) << dep);
                     node = first;
@@ -622,6 +642,13 @@ __device__ __forceinline__ void mix_walk(const DevTree &T, const double *ext, Mi
             node ^= 1;
         }
     } else {
+        if (D >= 6) {  // (below the node of height 6 in mix_test8's order)
+            node = anc >> 6;
+            dep = D - 6;
+        } else if (D >= 3) {
+            node = anc >> 3;
+            dep = D - 3;
+        }
         bool down = true;
         for (;;) {
             if (down) {
@@ -652,13 +679,7 @@ __device__ __forceinline__ void mix_walk(const DevTree &T, const double *ext, Mi
                         if (c.nvis >= MX_V) break;
                         down = false;
                     } else {
-                        const int c0 = 2 * node;
-                        int first = c0;
-                        if (anc >= 0 && (anc >> (D - dep)) == node) {
-                            first = anc >> (D - dep - 1);
-                        } else if (first_is_right<ND>(planep, node, qc)) {
-                            first = c0 + 1;
-                        }
+                        const int first = 2 * node + (first_is_right<ND>(planep, node, qc) ? 1 : 0);
                         dep += 1;
                         if (first & 1) firstright |= (1ULL << dep);
                         else firstright &= ~(1ULL << dep);
@@ -1181,7 +1202,7 @@ __global__ __launch_bounds__(64, ND == 6 && KMAX == 33 ? 4 : 1) void k_knn_mixed
     // one buffer for three uses at different times: the leaf copy (phase 2),
     // the compacted queries and their masks (6-D node tests and phase 1) and
     // the symmetric scatter into the wave's own queries (density)
-    constexpr int UB1 = ND == 3 ? 0 : (MX_QW + 1) * NBX_WAVE;
+    constexpr int UB1 = (MX_QW(ND) + 1) * MX_QMAX(ND);
     constexpr int UBN = UB1 > ND * NBX_LEAF + 2 * NBX_WAVE ? UB1 : ND * NBX_LEAF + 2 * NBX_WAVE;
     __shared__ __attribute__((aligned(16))) float ub[UBN];
     float *cx = ub;
