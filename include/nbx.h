@@ -350,7 +350,8 @@ int nbx_sph_density_adjoint_tree_dev(nbx_tree *t, int32_t k, int64_t block_rows,
                                      double *dpos_by_id_dev, double *dmass_by_id_dev, void *stream);
 
 /* Precision-form statistics of the last kNN/density call on this tree:
- * queries whose FP32 certificate failed and were recomputed in FP64. */
+ * queries searched in FP64, those whose FP32 certificate failed, or all of
+ * them where the whole call runs in FP64 because that is faster. */
 int nbx_tree_last_fallbacks(const nbx_tree *t, int64_t *fallbacks);
 
 /* Per-kernel timing with HIP events recorded on the launch stream.  When on,

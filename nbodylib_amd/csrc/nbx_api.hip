@@ -628,7 +628,7 @@ static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed, int32_t
         dry.carve<char>(sizeof(int32_t) * (t->n + 1));
         dry.carve<char>(nbx_mixed_scratch_bytes(t->nd, k + 1));
     } else if (kh > 0) {
-        dry.carve<char>(nbx_knn_scratch_bytes(t->nd, kh, NBX_Q_SLOTS, t->n));
+        dry.carve<char>(nbx_knn_scratch_bytes(t->nd, kh, NBX_Q_SLOTS, false, t->n));
     }
     return dry.used;
 }
@@ -637,12 +637,14 @@ static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed, int32_t
 // from the tree's kept scratch when ws is null.
 static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t st, Workspace *ws = nullptr) {
     if (nq <= 0) return hipSuccess;
+    const bool listed = A.qsrc != NBX_Q_POINTS && A.qlist;
+    size_t need = nbx_knn_scratch_bytes(t->nd, A.kh, A.qsrc, listed, nq);
+    if (need == 0) return nbx_launch_knn(t->view(), A, nq, st);
     // under capture the launcher allocates for itself, as part of the graph: a
     // replay must not meet later calls in the tree's block
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (!ws && st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
         return nbx_launch_knn(t->view(), A, nq, st);
-    size_t need = nbx_knn_scratch_bytes(t->nd, A.kh, A.qsrc, nq);
     std::unique_ptr<ScratchLease> lease;
     if (!ws) {
         lease.reset(new ScratchLease(t, need, st));
@@ -656,6 +658,17 @@ static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t s
 }
 
 // ------------------------------------------------------------------ precision form
+// Which precision-form searches run on the FP64 kernel with a wave per query
+// (nbx_knn_wave.hip), whose neighbour sets, exact rows and densities are the
+// same.  Rows in key order come from the FP32 kernel alone.  Measured in ms,
+// FP32 lanes / FP64 waves: densities at k = 32 of 4096 particles 0.31 / 0.023,
+// 131072 0.44 / 0.26, 524288 0.74 / 1.02; k = 64 of 1M 3.7 / 2.7, rows 4.2 /
+// 2.1; 6-D at k = 32 524288 4.98 / 3.86, 1M 8.4 / 8.4, k = 64 18.2 / 11.3.
+static bool mixed_by_waves(const nbx_tree *t, const KnnArgs &A, int k, int64_t nq) {
+    if (A.nn && !A.d2 && !A.exact_rows) return false;
+    return k > 32 || nq <= (t->nd == 6 ? 1048576 : 262144);
+}
+
 // FP32 search with the FP64 certificate; queries whose certificate fails are
 // re-run by the FP64 kernel from a list, so results equal the plain form's
 // neighbour sets.  A.dens / A.rho / A.nn / A.layout as for nbx_launch_knn.
@@ -666,6 +679,17 @@ static hipError_t run_mixed(nbx_tree *t, KnnArgs A, int k, hipStream_t st, Works
     // the fallback list holds at most the queries of the launch
     const int64_t nfb = A.wcnt > 0 ? std::min<int64_t>(n, (int64_t)A.wcnt * NBX_WAVE) : n;
     const size_t mbytes = nbx_mixed_scratch_bytes(t->nd, k + 1);
+    const int64_t nq = A.wcnt > 0 ? std::min<int64_t>((int64_t)A.wcnt * NBX_WAVE, n - (int64_t)A.wbeg * NBX_WAVE) : n;
+    const bool waves = mixed_by_waves(t, A, k, nq);
+    KnnArgs F = A;  // the FP64 search of the same queries
+    F.qsrc = NBX_Q_SLOTS;
+    F.kh = k;
+    F.kout = k;
+    F.excl_zero = 1;
+    if (waves && !ws) {
+        t->last_fallbacks.store(nq);
+        return nbx_launch_knn(t->view(), F, (int)nq, st);
+    }
     std::unique_ptr<ScratchLease> lease;
     if (!ws) {
         Workspace dry = {nullptr, ~(size_t)0, 0};
@@ -678,6 +702,10 @@ static hipError_t run_mixed(nbx_tree *t, KnnArgs A, int k, hipStream_t st, Works
     int32_t *fb = ws->carve<int32_t>(sizeof(int32_t) * (nfb + 1));
     void *mwork = ws->carve<void>(mbytes);
     if (!fb || !mwork) return hipErrorInvalidValue;
+    if (waves) {  // (scratch that is too small is refused either way)
+        t->last_fallbacks.store(nq);
+        return nbx_launch_knn(t->view(), F, (int)nq, st);
+    }
     hipError_t e = hipSuccess;
     int32_t *cnt = fb + nfb;
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, cnt, 0, (int64_t)1);
@@ -691,11 +719,6 @@ static hipError_t run_mixed(nbx_tree *t, KnnArgs A, int k, hipStream_t st, Works
     if (e == hipSuccess) e = hipMemcpyAsync(&hc, cnt, sizeof(int32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e == hipSuccess && hc > 0) {
-        KnnArgs F = A;
-        F.qsrc = NBX_Q_SLOTS;
-        F.kh = k;
-        F.kout = k;
-        F.excl_zero = 1;
         F.qlist = fb;
         F.m = hc;
         F.wbeg = F.wcnt = 0;
@@ -1632,7 +1655,7 @@ static int sph_tree_adj(nbx_tree *t, int32_t k, int64_t block, const double *g_i
     // the search's temporaries, reused by every block
     Workspace ws = {nullptr, 0, 0};
     ws.cap = mixed ? 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1)
-                   : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, block);
+                   : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, false, block);
     HIPCK(bufs.alloc(&ws.base, ws.cap));
     for (int64_t r0 = 0; r0 < n; r0 += block) {
         const int64_t nr = std::min<int64_t>(block, n - r0);

@@ -293,3 +293,33 @@ __device__ __forceinline__ void uf_union(int32_t *P, int32_t a, int32_t b) {
         if (a == b || uf_hook(P, a, b)) return;
     }
 }
+
+// Image point and test for periodic pass p (1..7), DistFunc.h:326-355 and
+// KDSplitNode.cxx:1119-1148: 1-D images need sqrt(Top) > s, the 2-D and 3-D
+// ones compare Top (a squared distance) with s (a distance), as the
+// reference does.  Phase-space searches take every image (:1153-1179).
+__device__ __forceinline__ bool image_pass(int pass, const double *x0, const double *per, double kth, bool uncond,
+                                           double *xp) {
+    const bool u0 = pass == 1 || pass == 4 || pass == 5 || pass == 7;
+    const bool u1 = pass == 2 || pass == 4 || pass == 6 || pass == 7;
+    const bool u2 = pass == 3 || pass == 5 || pass == 6 || pass == 7;
+    const bool use[3] = {u0, u1, u2};
+    double sval = 0.0, s1 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        xp[k] = x0[k];
+        if (use[k]) {
+            if (x0[k] < per[k] / 2.0) {
+                xp[k] = x0[k] + per[k];
+                sval += x0[k] * x0[k];
+                s1 = x0[k];
+            } else {
+                xp[k] = x0[k] - per[k];
+                sval += xp[k] * xp[k];
+                s1 = -xp[k];
+            }
+        }
+    }
+    if (pass <= 3) return uncond || sqrt(kth) > s1;
+    return uncond || kth > sqrt(sval);
+}

@@ -103,13 +103,16 @@ struct KnnArgs {
 };
 
 // work (nullable): device memory of nbx_knn_scratch_bytes for the
-// per-workgroup scratch and the queue counters.  Fewer bytes, down to
-// nbx_knn_scratch_least, run fewer workgroups; without work the launcher
-// allocates on the stream.
+// per-workgroup scratch and the queue counters (0: the search needs none).
+// Fewer bytes, down to eight workgroups' worth, run fewer workgroups; without
+// work the launcher allocates on the stream.
 hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st, void *work = nullptr,
                           size_t work_bytes = 0);
-size_t nbx_knn_scratch_bytes(int nd, int kh, int qsrc, int64_t nqueries);
-size_t nbx_knn_scratch_least(int nd, int kh);
+size_t nbx_knn_scratch_bytes(int nd, int kh, int qsrc, bool listed, int64_t nqueries);
+// The same, one query per wave; nbx_launch_knn takes it where nbx_knn_by_waves
+// says so.
+hipError_t nbx_launch_knn_wave(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st);
+bool nbx_knn_by_waves(int nd, int kh, int qsrc, bool listed, int64_t nqueries);
 // work (nullable): device memory of at least nbx_mixed_scratch_bytes(nd, kh)
 // bytes for the per-workgroup scratch and the queue counters; without it the
 // launcher allocates them on the stream.

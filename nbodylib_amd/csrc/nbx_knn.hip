@@ -26,9 +26,10 @@
 // waves fit on a CU at k = 32.  The 4-ary heap of (d2, ID) pairs in LDS that
 // this replaced held 12 bytes per entry (6 waves per CU) and took three
 // dependent levels and about 135 VALU per insertion.  Measured, heap to
-// groups: k = 32 density of 2.1M clustered particles 10.7 -> 4.6 ms; 0.5M
-// particles k = 8 1.68 -> 0.88, k = 64 8.4 -> 4.1, k = 128 40 -> 12 ms; 6-D
-// k = 64 63 -> 28 ms.
+// groups: 0.5M clustered particles k = 8 1.68 -> 0.88 ms; with room for 18
+// entries instead of 33, 16 waves on a CU, 2.1M 2.54 -> 1.79, 8.4M 9.9 -> 6.7
+// ms.  More entries, lists, positions and 6-D trees are searched with a wave
+// per query.
 // The scratch is sized by the resident workgroups: the kernel is persistent
 // and takes waves of queries from its XCD's share through an atomic counter,
 // as the precision form does (nbx_mixed.hip).
@@ -55,7 +56,7 @@ __device__ __forceinline__ double kmax(double a, double b) {
 
 template <int KMAX>
 struct KShape {
-    static constexpr int G = KMAX <= 33 ? 3 : (KMAX <= 65 ? 5 : 11);
+    static constexpr int G = 3;
     static constexpr int S = KMAX / G;
     static_assert(G * S == KMAX, "groups must tile KMAX");
 };
@@ -175,7 +176,7 @@ __device__ __forceinline__ void knn_leaf(const DevTree &T, const double *const (
     uint32_t mask = 0;
     // candidates arrive in chunks through the scalar cache: 8 per dimension
     // (24 SGPR pairs) in 3-D, 4 in 6-D
-    constexpr int CH = ND == 6 ? 4 : 8;
+    constexpr int CH = 8;
     typedef double dxc __attribute__((ext_vector_type(CH)));
     typedef const __attribute__((address_space(4))) dxc *cdcptr;
 #pragma unroll
@@ -293,60 +294,6 @@ __device__ __forceinline__ void knn_walk(const DevTree &T, KnnCtx<ND, KMAX> &c, 
     }
 }
 
-// Image point and test for periodic pass p (1..7), DistFunc.h:326-355 and
-// KDSplitNode.cxx:1119-1148: 1-D images need sqrt(Top) > s, the 2-D and 3-D
-// ones compare Top (a squared distance) with s (a distance), as the
-// reference does.  Phase-space searches take every image (:1153-1179).
-__device__ __forceinline__ bool image_pass(int pass, const double *x0, const double *per, double kth, bool uncond,
-                                           double *xp) {
-    const bool u0 = pass == 1 || pass == 4 || pass == 5 || pass == 7;
-    const bool u1 = pass == 2 || pass == 4 || pass == 6 || pass == 7;
-    const bool u2 = pass == 3 || pass == 5 || pass == 6 || pass == 7;
-    const bool use[3] = {u0, u1, u2};
-    double sval = 0.0, s1 = 0.0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        xp[k] = x0[k];
-        if (use[k]) {
-            if (x0[k] < per[k] / 2.0) {
-                xp[k] = x0[k] + per[k];
-                sval += x0[k] * x0[k];
-                s1 = x0[k];
-            } else {
-                xp[k] = x0[k] - per[k];
-                sval += xp[k] * xp[k];
-                s1 = -xp[k];
-            }
-        }
-    }
-    if (pass <= 3) return uncond || sqrt(kth) > s1;
-    return uncond || kth > sqrt(sval);
-}
-
-
-// Rank of v among the kh kept values (positions past kh hold -1 and are not
-// counted): how many are smaller.
-template <int KMAX>
-__device__ __forceinline__ int knn_rank(const double *hd, int lane, int kh, const double (&x)[KMAX <= 65 ? KMAX : 1],
-                                        double v) {
-    int r = 0;
-    if constexpr (KMAX <= 65) {
-#pragma unroll
-        for (int p = 0; p < KMAX; ++p) r += x[p] < v ? 1 : 0;
-        r -= KMAX - kh;
-    } else {
-#pragma unroll 4
-        for (int p = 0; p < kh; ++p) r += HD(p) < v ? 1 : 0;
-    }
-    return r;
-}
-template <int KMAX>
-__device__ __forceinline__ void knn_load(const double *hd, int lane, double (&x)[KMAX <= 65 ? KMAX : 1]) {
-    if constexpr (KMAX <= 65) {
-#pragma unroll
-        for (int p = 0; p < KMAX; ++p) x[p] = HD(p);
-    }
-}
 // The kept entries in ascending order of (value, ID, position): slots (or
 // IDs; -1 for a missing one) to so, values to sd.  si: room for the IDs.
 template <int KMAX>
@@ -361,12 +308,16 @@ __device__ __forceinline__ void knn_sort(const DevTree &T, const double *hd, con
         so[r * NBX_WAVE + lane] = e;
         sd[r * NBX_WAVE + lane] = v;
     };
-    double x[KMAX <= 65 ? KMAX : 1];
-    knn_load<KMAX>(hd, lane, x);
+    double x[KMAX];
+#pragma unroll
+    for (int p = 0; p < KMAX; ++p) x[p] = HD(p);
     int sum = 0;
     for (int p = 0; p < kh; ++p) {
         const double v = HD(p);
-        const int r = knn_rank<KMAX>(hd, lane, kh, x, v);
+        // how many are smaller (positions past kh hold -1 and are not counted)
+        int r = kh - KMAX;
+#pragma unroll
+        for (int u = 0; u < KMAX; ++u) r += x[u] < v ? 1 : 0;
         sum += r;
         put(p, v, r);
     }
@@ -402,22 +353,13 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
     double *const sd = (double *)(so + KMAX * NBX_WAVE);       // their d2
     int32_t *const si = (int32_t *)(sd + KMAX * NBX_WAVE);     // IDs by position
     const int kh = A.kh;
-    const bool listed = A.qlist != nullptr;
     const int wend = A.wbeg + A.wcnt;
-    const int nq = (QSRC == NBX_Q_POINTS || listed) ? A.m
-                   : (A.wcnt > 0 && wend < (T.n + NBX_WAVE - 1) / NBX_WAVE ? wend * NBX_WAVE : T.n);
-    const int gi = g * NBX_WAVE + lane;
-    const bool valid = gi < nq;
-    const int qi = listed ? (valid ? A.qlist[gi] : 0) : gi;
+    const int nq = A.wcnt > 0 && wend < (T.n + NBX_WAVE - 1) / NBX_WAVE ? wend * NBX_WAVE : T.n;
+    const int qi = g * NBX_WAVE + lane;
+    const bool valid = qi < nq;
     double q0[ND];
-    if (QSRC == NBX_Q_POINTS) {
-        // phase points (ND = 6) bring their velocities in qv
 #pragma unroll
-        for (int d = 0; d < ND; ++d) q0[d] = valid ? (d < 3 ? A.q[d][qi] : A.qv[d - 3][qi]) : 0.0;
-    } else {
-#pragma unroll
-        for (int d = 0; d < ND; ++d) q0[d] = valid ? T.x[d][qi] : 0.0;
-    }
+    for (int d = 0; d < ND; ++d) q0[d] = valid ? T.x[d][qi] : 0.0;
     KnnCtx<ND, KMAX> c;
 #pragma unroll
     for (int gr = 0; gr < KShape<KMAX>::G; ++gr) {
@@ -448,7 +390,7 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
         for (int d = 0; d < ND; ++d) qc[d] = (float)readfirst_d(c.q[d]);
         return ballot(c.act) != 0;
     };
-    const int own_leaves = (QSRC != NBX_Q_POINTS && !listed) ? T.nleafp + 2 * g : -1;
+    const int own_leaves = T.nleafp + 2 * g;
     for (int pass = 0; pass < npass; ++pass) {
         float qc[ND];
         if (!pass_begin(pass, false, qc)) continue;
@@ -481,32 +423,25 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
     __syncthreads();
 
     // ------------------------------------------------------------ densities
-    // Symmetric scatter: contributions to the wave's own 64 queries (slot
-    // runs only) are summed in LDS (over the leaf copy) and flushed with one
+    // Symmetric scatter: contributions to the wave's own 64 queries are summed in LDS (over the leaf copy) and flushed with one
     // atomic per query.
     double *const racc = cx;
     const bool spline = ND == 3 && QSRC == NBX_Q_SLOTS && A.dens == NBX_DO_SPLINE;
     const bool sym = QSRC == NBX_Q_SLOTS && (A.dens == NBX_DO_SYM || spline);
-    const bool own = sym && !listed;
     double racc_own = 0.0;
-    if (own) racc[lane] = 0.0;
+    if (sym) racc[lane] = 0.0;
     __syncthreads();
     // position queries take the gather forms only (mass and slot of the
     // query are undefined there)
-    if (A.dens != NBX_DO_NONE && valid &&
-        (QSRC == NBX_Q_SLOTS || A.dens == NBX_DO_GATHER || (QSRC == NBX_Q_POINTS && A.dens == NBX_DO_VEL))) {
+    if (A.dens != NBX_DO_NONE && valid && (QSRC == NBX_Q_SLOTS || A.dens == NBX_DO_GATHER)) {
         const bool bad = !(kth < NBX_MAXVALUE);  // fewer than kh neighbours
         if (A.dens == NBX_DO_VEL || A.dens == NBX_DO_VELPHYS) {
             // CalcVelDensity: |dv| of the Nsearch physical neighbours, the
             // Nsmooth smallest of them, h_v = max/2, sum W(|dv|/h_v) h_v^-3.
             // |dv| takes the place of d2; the terms are summed in the order
             // of (|dv|, ID).
-            // (CalcVelDensityPosition: the query's velocity comes with it)
             const int ns = A.nsmooth;
-            const bool pts = QSRC == NBX_Q_POINTS;
-            const double qvx = pts ? A.qv[0][qi] : T.x[3][qi];
-            const double qvy = pts ? A.qv[1][qi] : T.x[4][qi];
-            const double qvz = pts ? A.qv[2][qi] : T.x[5][qi];
+            const double qvx = T.x[3][qi], qvy = T.x[4][qi], qvz = T.x[5][qi];
             if (!bad) {
                 for (int p = 0; p < kh; ++p) {
                     const int32_t s = SL(p);
@@ -569,7 +504,7 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
                         const double Wij = 0.5 * W * norm;
                         acc = acc + Wij * mv[u];
                         const uint32_t r = (uint32_t)(s - g * NBX_WAVE);
-                        if (own && r < NBX_WAVE) atomicAdd(&racc[r], Wij * mi);
+                        if (r < NBX_WAVE) atomicAdd(&racc[r], Wij * mi);
                         else unsafeAtomicAdd(A.rho + s, Wij * mi);
                     } else {
                         acc += W * norm * mv[u];
@@ -583,12 +518,12 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
         if (bad) atomicOr(A.err, 1);
     }
     __syncthreads();
-    if (sym && valid) unsafeAtomicAdd(A.rho + qi, racc_own + (own ? racc[lane] : 0.0));
+    if (sym && valid) unsafeAtomicAdd(A.rho + qi, racc_own + racc[lane]);
 
     // ------------------------------------------------------------ outputs
     // (rows of the search only: the velocity densities ask for none)
     if (A.nn == nullptr && A.d2 == nullptr) return;
-    const bool ids = QSRC == NBX_Q_POINTS || A.layout == 0;
+    const bool ids = A.layout == 0;
     if (A.miss_self && valid && !(kth < NBX_MAXVALUE)) {
         atomicOr(A.err, 1);
         for (int p = 0; p < kh; ++p)
@@ -606,13 +541,7 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
         int r = e / kout, t = e - r * kout;
         int qr = g * NBX_WAVE + r;
         if (qr >= nq) break;
-        const int lr = qr;
-        if (listed) qr = A.qlist[qr];
-        int64_t row;
-        if (QSRC == NBX_Q_POINTS) row = qr;
-        else if (listed && A.list_rows) row = lr;
-        else if (A.layout == 1) row = qr - A.row0;
-        else row = T.perm[qr];
+        const int64_t row = A.layout == 1 ? qr - A.row0 : T.perm[qr];
         if (A.nn) A.nn[row * kout + t] = so[(t + off) * NBX_WAVE + r];
         if (A.d2) A.d2[row * kout + t] = sd[(t + off) * NBX_WAVE + r];
     }
@@ -666,42 +595,33 @@ static int knn_resident() {
     return g;
 }
 
-static int knn_kmax(int kh) { return kh <= 33 ? 33 : (kh <= 65 ? 65 : 132); }
-static const size_t KNN_CTR_BYTES = 8 * KNN_CTR_STRIDE * sizeof(int32_t);
+// Which kernel serves a search.  A lane per query shares each node and leaf
+// among 64 neighbours and wins for few kept entries over many queries; a wave
+// per query (nbx_knn_wave.hip) keeps its entries in registers and needs few
+// queries to fill the device.  Measured in ms, lanes / waves: 0.5M clustered
+// particles k = 8 0.70 / 0.61, periodic 0.73 / 0.81, density 0.69 / 0.78; 2.1M
+// k = 8 1.79 / 2.25, k = 20 3.79 / 2.90, k = 32 4.70 / 3.30; 8.4M k = 8 density
+// 6.4 / 12.2, k = 32 16.8 / 16.8.  Below 262144 queries the lanes leave CUs
+// idle (131072, k = 8: 0.30 / 0.15).
+#define KNN_KM 18
+bool nbx_knn_by_waves(int nd, int kh, int qsrc, bool listed, int64_t nqueries) {
+    return nd == 6 || kh > KNN_KM || qsrc == NBX_Q_POINTS || listed || nqueries <= 262144;
+}
 
-// f<ND, KMAX, QSRC>() of the instance that serves kh kept entries on T.nd
-#define KNN_DISPATCH(nd, km, qsrc, F)                                                           \
-    ((nd) == 6 ? ((km) <= 65 ? KNN_DISPATCH_Q(6, 65, qsrc, F) : KNN_DISPATCH_Q(6, 132, qsrc, F)) \
-               : ((km) <= 33   ? KNN_DISPATCH_Q(3, 33, qsrc, F)                                  \
-                  : (km) <= 65 ? KNN_DISPATCH_Q(3, 65, qsrc, F)                                  \
-                               : KNN_DISPATCH_Q(3, 132, qsrc, F)))
-#define KNN_DISPATCH_Q(ND, KM, qsrc, F)                             \
-    ((qsrc) == NBX_Q_SLOTS      ? F(ND, KM, NBX_Q_SLOTS)            \
-     : (qsrc) == NBX_Q_PERIODIC ? F(ND, KM, NBX_Q_PERIODIC) : F(ND, KM, NBX_Q_POINTS))
+static const size_t KNN_CTR_BYTES = 8 * KNN_CTR_STRIDE * sizeof(int32_t);
+static const size_t KNN_BLOCK_BYTES = (size_t)KNN_BLKW(KNN_KM) * sizeof(int32_t);
 
 // workgroups for nw waves: no more than are resident (or than there are waves)
-static int knn_grid(int nd, int kh, int qsrc, int64_t nw) {
-#define KNN_F(ND, KM, Q) knn_resident<ND, KM, Q>()
-    const int res = KNN_DISPATCH(nd, knn_kmax(kh), qsrc, KNN_F);
-#undef KNN_F
+static int knn_grid(int qsrc, int64_t nw) {
+    const int res = qsrc == NBX_Q_PERIODIC ? knn_resident<3, KNN_KM, NBX_Q_PERIODIC>()
+                                           : knn_resident<3, KNN_KM, NBX_Q_SLOTS>();
     const int64_t want = (nw + 7) & ~(int64_t)7;
     return (int)(want < res ? want : res);
 }
-static size_t knn_block_bytes(int nd, int kh) {
-    const int km = nd == 6 && kh <= 65 ? 65 : knn_kmax(kh);
-    return (size_t)KNN_BLKW(km) * sizeof(int32_t);
-}
 
-size_t nbx_knn_scratch_bytes(int nd, int kh, int qsrc, int64_t nqueries) {
-    const int64_t nw = (nqueries + NBX_WAVE - 1) / NBX_WAVE;
-    return KNN_CTR_BYTES + (size_t)knn_grid(nd, kh, qsrc, nw) * knn_block_bytes(nd, kh);
-}
-size_t nbx_knn_scratch_least(int nd, int kh) { return KNN_CTR_BYTES + 8 * knn_block_bytes(nd, kh); }
-
-template <int ND, int KMAX, int QSRC>
-static void knn_start(const DevTree &T, const KnnArgs &A, int grid, int nw, int32_t *scr, int32_t *ctr,
-                      hipStream_t st) {
-    hipLaunchKernelGGL((k_knn<ND, KMAX, QSRC>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, nw, scr, ctr);
+size_t nbx_knn_scratch_bytes(int nd, int kh, int qsrc, bool listed, int64_t nqueries) {
+    if (nbx_knn_by_waves(nd, kh, qsrc, listed, nqueries)) return 0;
+    return KNN_CTR_BYTES + (size_t)knn_grid(qsrc, (nqueries + NBX_WAVE - 1) / NBX_WAVE) * KNN_BLOCK_BYTES;
 }
 
 hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st, void *work,
@@ -709,25 +629,27 @@ hipError_t nbx_launch_knn(const DevTree &T, const KnnArgs &A, int nqueries, hipS
     const int nw = (nqueries + NBX_WAVE - 1) / NBX_WAVE;
     if (nw == 0) return hipSuccess;
     if (A.kh < 1 || A.kh > 129) return hipErrorInvalidValue;
-    int grid = knn_grid(T.nd, A.kh, A.qsrc, nw);
-    const size_t blk = knn_block_bytes(T.nd, A.kh);
+    const bool listed = A.qsrc != NBX_Q_POINTS && A.qlist;
+    if (nbx_knn_by_waves(T.nd, A.kh, A.qsrc, listed, nqueries)) return nbx_launch_knn_wave(T, A, nqueries, st);
+    int grid = knn_grid(A.qsrc, nw);
     void *mem = work;
     if (mem) {
         // as many workgroups as the scratch given has blocks for
-        if (work_bytes < nbx_knn_scratch_least(T.nd, A.kh)) return hipErrorInvalidValue;
-        const size_t fit = (work_bytes - KNN_CTR_BYTES) / blk;
+        if (work_bytes < KNN_CTR_BYTES + 8 * KNN_BLOCK_BYTES) return hipErrorInvalidValue;
+        const size_t fit = (work_bytes - KNN_CTR_BYTES) / KNN_BLOCK_BYTES;
         if (fit < (size_t)grid) grid = (int)fit & ~7;
     } else {
-        const hipError_t e = hipMallocAsync(&mem, KNN_CTR_BYTES + (size_t)grid * blk, st);
+        const hipError_t e = hipMallocAsync(&mem, KNN_CTR_BYTES + (size_t)grid * KNN_BLOCK_BYTES, st);
         if (e != hipSuccess) return e;
     }
     int32_t *ctr = (int32_t *)mem, *scr = (int32_t *)((char *)mem + KNN_CTR_BYTES);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, ctr, 0, (int64_t)(8 * KNN_CTR_STRIDE));
     {
-        ProfScope ps(A.qsrc != NBX_Q_POINTS && A.qlist ? "k_knn_fallback" : "k_knn_fp64", st);
-#define KNN_F(ND, KM, Q) knn_start<ND, KM, Q>(T, A, grid, nw, scr, ctr, st)
-        KNN_DISPATCH(T.nd, knn_kmax(A.kh), A.qsrc, KNN_F);
-#undef KNN_F
+        ProfScope ps("k_knn_fp64", st);
+        if (A.qsrc == NBX_Q_PERIODIC)
+            hipLaunchKernelGGL((k_knn<3, KNN_KM, NBX_Q_PERIODIC>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, nw, scr, ctr);
+        else
+            hipLaunchKernelGGL((k_knn<3, KNN_KM, NBX_Q_SLOTS>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, nw, scr, ctr);
     }
     const hipError_t e = hipGetLastError();
     if (!work) hipFreeAsync(mem, st);

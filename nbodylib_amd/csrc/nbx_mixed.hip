@@ -1271,15 +1271,12 @@ static int mx_grid() {
     return grid.load();
 }
 
-template <int ND, int KMAX>
-static int mx_grid_mode(int mode) {
-    if constexpr (ND == 3)
-        if (mode == MX_SPLINE) return mx_grid<ND, KMAX, MX_SPLINE>();
-    return mode == MX_EXACT ? mx_grid<ND, KMAX, MX_EXACT>() : mx_grid<ND, KMAX, MX_TABLE>();
-}
+// (more than 33 kept entries: rows in key order only, see mixed_by_waves)
 static int mx_launch_grid(int nd, int km, int mode) {
-    return nd == 3 ? (km == 33 ? mx_grid_mode<3, 33>(mode) : mx_grid_mode<3, 65>(mode))
-                   : (km == 33 ? mx_grid_mode<6, 33>(mode) : mx_grid_mode<6, 65>(mode));
+    if (km == 65) return nd == 3 ? mx_grid<3, 65, MX_TABLE>() : mx_grid<6, 65, MX_TABLE>();
+    if (nd == 3 && mode == MX_SPLINE) return mx_grid<3, 33, MX_SPLINE>();
+    if (mode == MX_EXACT) return nd == 3 ? mx_grid<3, 33, MX_EXACT>() : mx_grid<6, 33, MX_EXACT>();
+    return nd == 3 ? mx_grid<3, 33, MX_TABLE>() : mx_grid<6, 33, MX_TABLE>();
 }
 static int mx_mode(const KnnArgs &A) {
     return A.dens == NBX_DO_SPLINE ? MX_SPLINE : (A.exact_rows || A.d2 ? MX_EXACT : MX_TABLE);
@@ -1300,8 +1297,8 @@ hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double
         return hipErrorInvalidValue;
     const int km = A.kh <= 33 ? 33 : 65;
     const int mode = mx_mode(A);
-    // densities and exact rows do not come together; the spline is 3-D
-    if ((mode == MX_EXACT && A.dens != NBX_DO_NONE) || (mode == MX_SPLINE && (T.nd != 3 || A.nn || A.d2)))
+    // densities and exact rows do not come together; the spline is 3-D; both keep at most 33
+    if ((mode != MX_TABLE && km > 33) || (mode == MX_EXACT && A.dens != NBX_DO_NONE) || (mode == MX_SPLINE && (T.nd != 3 || A.nn || A.d2)))
         return hipErrorInvalidValue;
     const int grid = mx_launch_grid(T.nd, km, mode);
     const size_t nscr = (size_t)grid * MX_BLKW(km);
@@ -1323,12 +1320,14 @@ hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double
     hipLaunchKernelGGL((k_knn_mixed<ND, KM, MODE>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, ext, fallback_list, \
                        fallback_count, scr, ctr)
         if (T.nd == 3) {
-            if (mode == MX_TABLE) { if (km == 33) MIXL(3, 33, MX_TABLE); else MIXL(3, 65, MX_TABLE); }
-            else if (mode == MX_EXACT) { if (km == 33) MIXL(3, 33, MX_EXACT); else MIXL(3, 65, MX_EXACT); }
-            else { if (km == 33) MIXL(3, 33, MX_SPLINE); else MIXL(3, 65, MX_SPLINE); }
+            if (km == 65) MIXL(3, 65, MX_TABLE);
+            else if (mode == MX_TABLE) MIXL(3, 33, MX_TABLE);
+            else if (mode == MX_EXACT) MIXL(3, 33, MX_EXACT);
+            else MIXL(3, 33, MX_SPLINE);
         } else {
-            if (mode == MX_TABLE) { if (km == 33) MIXL(6, 33, MX_TABLE); else MIXL(6, 65, MX_TABLE); }
-            else { if (km == 33) MIXL(6, 33, MX_EXACT); else MIXL(6, 65, MX_EXACT); }
+            if (km == 65) MIXL(6, 65, MX_TABLE);
+            else if (mode == MX_TABLE) MIXL(6, 33, MX_TABLE);
+            else MIXL(6, 33, MX_EXACT);
         }
 #undef MIXL
     }
