@@ -23,8 +23,12 @@
 //    entries took six times as many (0.5M queries, k = 32: 1.54 ms, and 0.77
 //    with keys).
 //  * No scratch, no counters: a call is one launch.
-// Vector issue bounds it: 0.84k instructions a query at k = 32 in 3-D, of
-// which the merges are about half, 93% of the cycles busy.
+// Vector issue bounds it: about 0.85k instructions a query at k = 32 in 3-D, of
+// which the merges are about half, 95% of the cycles busy.  So the common path
+// is kept short (the last few open nodes are taken without a minimum, a group's
+// leaves share one scalar base address, padding needs no test of its own and
+// the query's own entry is sorted out after something was accepted): 6-D, 0.5M,
+// k = 64 5.68 -> 5.4 ms.
 // Measured, a lane per query -> this: 4096 particles, k = 32, periodic 266 ->
 // 27 us; 100k positions among 1M particles 6.17 -> 0.59 ms; 2.1M clustered
 // particles, density at k = 32 4.5 -> 4.2 ms; 0.5M particles k = 64 3.8 ->
@@ -348,10 +352,9 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
     int sp = 0, height = T.depth, step = first;
     uint32_t node = 1, base = 0, key = ~0u;
     bool expand = true;
-    // nearest open descendant (its lane), which is then marked taken; -1: none
+    // nearest of the descendants (its lane), which is then marked taken
     auto take = [&]() -> int {
         const uint32_t m = wave_umin(key);
-        if (m > k.lim) return -1;
         if (key == m) key = ~0u;
         return (int)(m & 63u);
     };
@@ -360,7 +363,7 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
             height -= step;
             base = node << step;
             const bool mine = lane < (1 << step);
-            const double2 *bp = (const double2 *)node_box(T, (int)(base + (mine ? lane : 0)), ND);
+            const double2 *bp = (const double2 *)node_box(T, (int)base, ND) + (mine ? lane * ND : 0);
             double bx[2 * ND];
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
@@ -379,43 +382,50 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
         }
         if (height == 0) {
             // the four nearest open leaves, two particles per lane
-            const int i0 = take();
-            if (i0 >= 0) {
-                int li = i0;
-                bool has = lane < 16;
+            uint64_t open = ballot(key <= k.lim);
+            if (open) {
+                int li = 0;
+                uint64_t has = ~0ULL;  // the lanes with a leaf, 16 for each
+                const int nopen = __builtin_popcountll(open);
+                if (nopen <= 4) {  // all of them, in any order
+                    if (key <= k.lim) key = ~0u;
+                    has >>= 64 - 16 * nopen;
 #pragma unroll
-                for (int j = 1; j < 4; ++j) {
-                    const int i = take();
-                    if (i < 0) break;
-                    const bool mine = lane >> 4 == j;
-                    li = mine ? i : li;
-                    has |= mine;
+                    for (int j = 0; j < 4; ++j) {
+                        if (!open) break;
+                        li = lane >> 4 == j ? __builtin_ctzll(open) : li;
+                        open &= open - 1;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int i = take();
+                        li = lane >> 4 == j ? i : li;
+                    }
                 }
-                const int32_t sl = ((int)base + li - T.nleafp) * NBX_LEAF + 2 * (lane & 15);
+                const int32_t s0 = ((int)base - T.nleafp) * NBX_LEAF;  // the first of the 64 leaves
+                const uint32_t ls = (uint32_t)(li * NBX_LEAF + 2 * (lane & 15));
+                const int32_t sl = s0 + (int32_t)ls;
                 double d2[2] = {0.0, 0.0};
 #pragma unroll
                 for (int d = 0; d < ND; ++d) {
-                    const double2 x = *(const double2 *)(T.x[d] + sl);
+                    const double2 x = *(const double2 *)((const char *)(T.x[d] + s0) + ls * 8u);
                     const double t0 = q[d] - x.x, t1 = q[d] - x.y;
                     d2[0] += t0 * t0;
                     d2[1] += t1 * t1;
                 }
-                uint64_t acc[2];
+                // (padding slots lie at 1e300, so their d2 is infinite)
+                uint64_t acc[2] = {ballot(d2[0] <= k.kth) & has, ballot(d2[1] <= k.kth) & has};
+                if (!(acc[0] | acc[1])) continue;
+                const int2 ids = *(const int2 *)((const char *)(T.perm + s0) + ls * 4u);
+                const int32_t id[2] = {ids.x, ids.y};
+                // equally far as the last kept: only a smaller ID counts; the
+                // query itself has d2 == 0
                 int cnt = 0;
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    // (the query itself has d2 == 0)
-                    acc[p] = ballot(has & (d2[p] <= k.kth) & (sl + p < T.n) & (!exz | (d2[p] > 0.0)));
-                    cnt += __builtin_popcountll(acc[p]);
-                }
-                if (cnt == 0) continue;
-                const int2 ids = *(const int2 *)(T.perm + sl);
-                const int32_t id[2] = {ids.x, ids.y};
-                // (equally far from the last kept: only a smaller ID counts)
-                cnt = 0;
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    acc[p] &= ballot((d2[p] < k.kth) | (id[p] < k.kid));
+                    acc[p] &= ballot(d2[p] < k.kth) | ballot(id[p] < k.kid);
+                    if (exz) acc[p] &= ballot(d2[p] > 0.0);
                     cnt += __builtin_popcountll(acc[p]);
                 }
                 if (cnt < WV_MERGE) {
@@ -452,8 +462,11 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
                 continue;
             }
         } else {
-            const int i = take();
-            if (i >= 0) {
+            const uint64_t open = ballot(key <= k.lim);
+            if (open) {
+                int i = __builtin_ctzll(open);
+                if (open & (open - 1)) i = take();
+                else if (lane == i) key = ~0u;
                 sh.stk[sp][lane] = key;
                 ++sp;
                 node = base + (uint32_t)i;
