@@ -1102,17 +1102,12 @@ extern "C" int nbx_knn_density_noalloc(nbx_tree *t, int32_t k, int32_t *nn_by_sl
 // pass gives neighbour rows by slot and rho, then the smoothing kernels run
 // over those rows.  A caller's rho (the reference's densityset = 1), means
 // (meanvelset = 1) or dispersions (veldispset = 1) replace computed ones.
-// Host arrays by ID: rows of ncomp values -> [ncomp][n] by slot on the device.
-static hipError_t upload_rows(const nbx_tree *t, const double *rows, int ncomp, double *tmp, double *by_slot) {
-    const int64_t n = t->n;
-    std::vector<double> soa((size_t)ncomp * n);
-    for (int64_t i = 0; i < n; ++i)
-        for (int c = 0; c < ncomp; ++c) soa[(size_t)c * n + i] = rows[ncomp * i + c];
-    hipError_t e = hipMemcpy(tmp, soa.data(), sizeof(double) * ncomp * n, hipMemcpyHostToDevice);
-    for (int c = 0; c < ncomp && e == hipSuccess; ++c)
-        hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, nullptr, tmp + c * n, t->perm, n,
-                           by_slot + c * n);
-    return e;
+// Host arrays by ID: rows of ncomp values -> [n][w] by slot on the device.
+static hipError_t upload_rows(const nbx_tree *t, const double *rows, int ncomp, double *tmp, int w, double *by_slot) {
+    const hipError_t e = hipMemcpy(tmp, rows, sizeof(double) * ncomp * t->n, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_smooth_in, dim3(nblk(t->n)), dim3(256), 0, nullptr, tmp, t->perm, t->n, w, ncomp, by_slot);
+    return hipGetLastError();
 }
 
 static int smooth_impl(nbx_tree *t, int32_t k, const double *rho_by_id, const double *mean_in, const double *disp_in,
@@ -1126,41 +1121,45 @@ static int smooth_impl(nbx_tree *t, int32_t k, const double *rho_by_id, const do
     const bool need_disp = disp_out || moments;
     hipStream_t st = nullptr;
     int32_t *nn = nullptr;
-    double *rid = nullptr, *rslot = nullptr, *mean = nullptr, *disp = nullptr, *mom = nullptr, *buf = nullptr;
+    double *rid = nullptr, *hid = nullptr, *mean = nullptr, *disp = nullptr, *mom = nullptr, *buf = nullptr;
+    SmoothRec *rec = nullptr;
     HIPCK(bufs.alloc(&nn, sizeof(int32_t) * (size_t)n * k));
     HIPCK(bufs.alloc(&rid, sizeof(double) * n));
-    HIPCK(bufs.alloc(&rslot, sizeof(double) * n));
-    HIPCK(bufs.alloc(&mean, sizeof(double) * 3 * n));
-    if (need_disp) HIPCK(bufs.alloc(&disp, sizeof(double) * 9 * n));
-    if (moments) HIPCK(bufs.alloc(&mom, sizeof(double) * 6 * n));
+    HIPCK(bufs.alloc(&hid, sizeof(double) * n));
+    HIPCK(bufs.alloc(&rec, sizeof(SmoothRec) * n));
+    HIPCK(bufs.alloc(&mean, sizeof(double4) * n));
+    if (need_disp) HIPCK(bufs.alloc(&disp, sizeof(SmoothSum) * n));
+    if (moments) HIPCK(bufs.alloc(&mom, sizeof(SmoothSum) * n));
     HIPCK(bufs.alloc(&buf, sizeof(double) * 9 * n));
-    int rc = density_impl(t, k, NBX_DENS_SYMMETRIC, 0, rid, nullptr, nn, st);
+    int rc = density_impl(t, k, NBX_DENS_SYMMETRIC, 0, rid, hid, nn, st);
     hipError_t e = hipSuccess;
     if (rc == NBX_OK) {
         if (rho_by_id) e = hipMemcpy(rid, rho_by_id, sizeof(double) * n, hipMemcpyHostToDevice);
-        if (e == hipSuccess) hipLaunchKernelGGL(k_gather_by_id, dim3(nblk(n)), dim3(256), 0, st, rid, t->perm, n, rslot);
+        if (e == hipSuccess) hipLaunchKernelGGL(k_smooth_pack, dim3(nblk(n)), dim3(256), 0, st, t->view(), rid, hid, rec);
         if (e == hipSuccess) {
-            if (mean_in) e = upload_rows(t, mean_in, 3, buf, mean);
-            else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(3 * n)), dim3(256), 0, st, mean, 0.0, 3 * n);
+            if (mean_in) e = upload_rows(t, mean_in, 3, buf, 4, mean);
+            else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(4 * n)), dim3(256), 0, st, mean, 0.0, 4 * n);
         }
         if (e == hipSuccess && need_disp) {
-            if (disp_in) e = upload_rows(t, disp_in, 9, buf, disp);
-            else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(9 * n)), dim3(256), 0, st, disp, 0.0, 9 * n);
+            if (disp_in) e = upload_rows(t, disp_in, 9, buf, 8, disp);
+            else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(8 * n)), dim3(256), 0, st, disp, 0.0, 8 * n);
         }
         if (e == hipSuccess && moments)
-            hipLaunchKernelGGL(k_fill_f64, dim3(nblk(6 * n)), dim3(256), 0, st, mom, 0.0, 6 * n);
+            hipLaunchKernelGGL(k_fill_f64, dim3(nblk(8 * n)), dim3(256), 0, st, mom, 0.0, 8 * n);
         if (e == hipSuccess) {
-            SmoothArgs A = {nn, k, rslot, mean, disp, moments ? mom : nullptr, moments ? mom + 3 * n : nullptr};
+            SmoothArgs A = {nn, k, rec, (double4 *)mean, (SmoothSum *)disp, (SmoothSum *)mom};
             e = nbx_launch_smooth(t->view(), A, mean_in == nullptr, need_disp && disp_in == nullptr, st);
         }
         struct Out {
-            double *dev;
-            int ncomp;
+            const double *dev;
+            int w, from0, ncomp;
             double *host;
-        } outs[4] = {{mean, 3, mean_out}, {disp, 9, disp_out}, {mom, 3, skew_out}, {mom + 3 * n, 3, kurt_out}};
+        } outs[4] = {{mean, 4, 0, 3, mean_out}, {disp, 8, 0, 9, disp_out}, {mom, 8, 0, 3, skew_out},
+                     {mom, 8, 3, 3, kurt_out}};
         for (const Out &o : outs) {
             if (e != hipSuccess || !o.host) continue;
-            hipLaunchKernelGGL(k_smooth_out, dim3(nblk(n)), dim3(256), 0, st, o.dev, t->perm, n, o.ncomp, buf);
+            hipLaunchKernelGGL(k_smooth_out, dim3(nblk(n)), dim3(256), 0, st, o.dev, t->perm, n, o.w, o.from0, o.ncomp,
+                               buf);
             e = hipMemcpy(o.host, buf, sizeof(double) * o.ncomp * n, hipMemcpyDeviceToHost);
         }
         if (e != hipSuccess) rc = hipfail(e, "smoothed velocities");

@@ -169,17 +169,25 @@ hipError_t nbx_point_order(const DevTree &T, const PointCoords &q, int64_t m, in
                            hipStream_t st);
 
 // ------------------------------------------------------------------ smoothed velocities
+struct SmoothRec {
+    double4 x, v;  // position and mass / density; velocity and h
+};
+struct SmoothSum {
+    double c[8];  // dispersion: xx xy xz yy yz zz; moments: skewness, kurtosis
+};
+#define SM_DIAG(d) ((d) * (7 - (d)) / 2)  // xx, yy, zz
 struct SmoothArgs {
     const int32_t *nn;  // n x k neighbour slots, rows by slot
     int32_t k;
-    const double *rho;  // densities by slot
-    double *mean;       // smoothed velocity by slot, [3][n]; zeroed by the caller
-    double *disp;       // dispersion by slot, [9][n] (upper triangle used) or null; zeroed by the caller
-    double *skew;       // skewness by slot, [3][n], or null; zeroed by the caller
-    double *kurt;       // kurtosis by slot, [3][n] (with skew); zeroed by the caller
+    const SmoothRec *rec;  // by slot
+    double4 *mean;         // smoothed velocity by slot; zeroed by the caller, as the sums below
+    SmoothSum *disp;       // dispersion by slot, or null
+    SmoothSum *mom;        // moments by slot, or null
 };
+__global__ void k_smooth_pack(DevTree T, const double *rho_by_id, const double *h_by_id, SmoothRec *rec);
+__global__ void k_smooth_in(const double *rows, const int32_t *perm, int64_t n, int w, int ncomp, double *out);
 // with_mean / with_disp: compute those first (else A.mean / A.disp hold the
-// caller's); the moments run when A.skew is set.
+// caller's); the moments run when A.mom is set.
 hipError_t nbx_launch_smooth(const DevTree &T, const SmoothArgs &A, bool with_mean, bool with_disp, hipStream_t st);
 // Local mean / dispersion of a per-particle scalar (gather form): row r of
 // nn holds the k neighbours of query r, whose coordinates are q (position
@@ -197,7 +205,7 @@ struct LocalArgs {
     double *disp;           // by row, nullable
 };
 hipError_t nbx_launch_smooth_local(const DevTree &T, const LocalArgs &A, hipStream_t st);
-__global__ void k_smooth_out(const double *in, const int32_t *perm, int64_t n, int ncomp, double *out);
+__global__ void k_smooth_out(const double *in, const int32_t *perm, int64_t n, int w, int from0, int ncomp, double *out);
 __global__ void k_gather_by_id(const double *by_id, const int32_t *perm, int64_t n, double *by_slot);
 
 // ------------------------------------------------------------------ small kernels
