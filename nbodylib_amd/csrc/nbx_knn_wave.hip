@@ -485,10 +485,10 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
 }
 
 template <int ND, int E, int QSRC>
-__global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int nq) {
+__global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int first) {
     __shared__ WvShared<E> sh;
     const int lane = threadIdx.x;
-    const int g = xcd_wave(blockIdx.x, gridDim.x);
+    const int g = first + xcd_wave(blockIdx.x, gridDim.x);
     const int kh = A.kh;
     const bool listed = A.qlist != nullptr;
     const int qi = listed ? A.qlist[g] : A.wbeg * NBX_WAVE + g;
@@ -640,14 +640,19 @@ __global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int nq) {
     }
 }
 
+// A launch holds fewer than 2^32 threads, hence the runs of queries.
+#define WV_RUN (1 << 25)
 template <int ND, int E>
 static void wave_start(const DevTree &T, const KnnArgs &A, int nq, hipStream_t st) {
-    if (A.qsrc == NBX_Q_SLOTS)
-        hipLaunchKernelGGL((k_knn_wave<ND, E, NBX_Q_SLOTS>), dim3(nq), dim3(NBX_WAVE), 0, st, T, A, nq);
-    else if (A.qsrc == NBX_Q_PERIODIC)
-        hipLaunchKernelGGL((k_knn_wave<ND, E, NBX_Q_PERIODIC>), dim3(nq), dim3(NBX_WAVE), 0, st, T, A, nq);
-    else
-        hipLaunchKernelGGL((k_knn_wave<ND, E, NBX_Q_POINTS>), dim3(nq), dim3(NBX_WAVE), 0, st, T, A, nq);
+    for (int64_t q0 = 0; q0 < nq; q0 += WV_RUN) {
+        const dim3 grid((unsigned)std::min<int64_t>(WV_RUN, nq - q0));
+        if (A.qsrc == NBX_Q_SLOTS)
+            hipLaunchKernelGGL((k_knn_wave<ND, E, NBX_Q_SLOTS>), grid, dim3(NBX_WAVE), 0, st, T, A, (int)q0);
+        else if (A.qsrc == NBX_Q_PERIODIC)
+            hipLaunchKernelGGL((k_knn_wave<ND, E, NBX_Q_PERIODIC>), grid, dim3(NBX_WAVE), 0, st, T, A, (int)q0);
+        else
+            hipLaunchKernelGGL((k_knn_wave<ND, E, NBX_Q_POINTS>), grid, dim3(NBX_WAVE), 0, st, T, A, (int)q0);
+    }
 }
 
 hipError_t nbx_launch_knn_wave(const DevTree &T, const KnnArgs &A, int nqueries, hipStream_t st) {
