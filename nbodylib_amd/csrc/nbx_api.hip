@@ -720,7 +720,6 @@ static hipError_t run_mixed(nbx_tree *t, KnnArgs A, int k, hipStream_t st, Works
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e == hipSuccess && hc > 0) {
         F.qlist = fb;
-        F.m = hc;
         F.wbeg = F.wcnt = 0;
         e = nbx_launch_knn(T, F, hc, st);
     }
@@ -844,7 +843,6 @@ extern "C" int nbx_knn_targets(nbx_tree *t, const int32_t *ids, int64_t m, int32
     A.nn = dnn;
     A.d2 = dd2;
     A.qlist = dsl;
-    A.m = (int32_t)m;
     A.list_rows = 1;
     hipError_t e = run_plain(t, A, (int)m, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -881,27 +879,9 @@ static int points_impl(nbx_tree *t, const double *q, int64_t m, int32_t k, bool 
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, nullptr, err, 0, (int64_t)1);
     KnnArgs A;
     memset(&A, 0, sizeof(A));
-    // A wave walks the tree once for its 64 points, so they are taken in
-    // Morton order: for 100k unordered positions over 1M clustered particles
-    // (k = 32) the call takes 9.5 ms so, 158 ms in the given order; keys and
-    // sort are 0.08 ms of it.  A single wave's worth stays as given.
-    if (m > NBX_WAVE) {
-        int32_t *order = nullptr;
-        char *tmp = nullptr;
-        PointCoords pc = {};
-        for (int d = 0; d < 3; ++d) {
-            pc.c[d] = dq + d * m;
-            pc.c[3 + d] = dqv ? dqv + d * m : nullptr;  // read on 6-D trees, whose points have velocities
-        }
-        HIPCK(bufs.alloc(&order, sizeof(int32_t) * m));
-        HIPCK(bufs.alloc(&tmp, nbx_point_order_bytes(m)));
-        HIPCK(nbx_point_order(t->view(), pc, m, order, tmp, nullptr));
-        A.qlist = order;
-    }
     A.qsrc = NBX_Q_POINTS;
     A.kh = k;
     A.kout = k;
-    A.m = (int32_t)m;
     A.periodic = periodic && t->p.periodic && t->n > t->p.bucket_size;
     for (int d = 0; d < 3; ++d) { A.period[d] = t->p.period[d]; A.q[d] = dq + d * m; }
     A.nn = dnn;
@@ -1265,15 +1245,6 @@ extern "C" int nbx_smooth_local_points(nbx_tree *t, const double *q, int64_t m, 
         K.qsrc = NBX_Q_POINTS;
         K.kh = k;
         K.kout = k;
-        K.m = (int32_t)m;
-        if (m > NBX_WAVE) {  // as in points_impl
-            int32_t *order = nullptr;
-            char *tmp = nullptr;
-            if (e == hipSuccess) e = bufs.alloc(&order, sizeof(int32_t) * m);
-            if (e == hipSuccess) e = bufs.alloc(&tmp, nbx_point_order_bytes(m));
-            if (e == hipSuccess) e = nbx_point_order(t->view(), PointCoords{{dq, dq + m, dq + 2 * m}}, m, order, tmp, st);
-            K.qlist = order;
-        }
         for (int d = 0; d < 3; ++d) K.q[d] = dq + d * m;
         K.nn = dnn;
         if (e == hipSuccess) e = run_plain(t, K, (int)m, st);

@@ -871,16 +871,14 @@ __device__ __forceinline__ void ball_walk(const DevTree &T, const double *q, boo
     }
 }
 
-// Morton key of a point over the root box: the bits of its ND cell indices
-// interleaved, 21 a dimension in 3-D and 10 in 6-D (63 and 60 bits).  Points
-// outside the box take its border cells, NaN the lowest; the key only orders
-// the points.
-template <int ND>
+// Morton key of a point over the root box: the bits of its cell indices
+// interleaved, 21 a dimension.  Points outside the box take its border cells,
+// NaN the lowest; the key only orders the points.
 __global__ __launch_bounds__(256) void k_point_keys(DevTree T, PointCoords q, int64_t m, uint64_t *keys,
                                                     int32_t *idx) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= m) return;
-    constexpr int BITS = ND == 3 ? 21 : 10;
+    constexpr int ND = 3, BITS = 21;
     const double top = (double)((1 << BITS) - 1);
     cdptr rb = (cdptr)node_box(T, 1, ND);
     uint64_t key = 0;
@@ -911,8 +909,7 @@ hipError_t nbx_point_order(const DevTree &T, const PointCoords &q, int64_t m, in
     int32_t *idx = (int32_t *)(w + 2 * align256(sizeof(uint64_t) * m));
     void *tmp = w + 2 * align256(sizeof(uint64_t) * m) + align256(sizeof(int32_t) * m);
     ProfScope ps("k_point_order", st);
-    if (T.nd == 6) hipLaunchKernelGGL(k_point_keys<6>, dim3(nblk(m)), dim3(256), 0, st, T, q, m, keys, idx);
-    else hipLaunchKernelGGL(k_point_keys<3>, dim3(nblk(m)), dim3(256), 0, st, T, q, m, keys, idx);
+    hipLaunchKernelGGL(k_point_keys, dim3(nblk(m)), dim3(256), 0, st, T, q, m, keys, idx);
     hipError_t e = hipGetLastError();
     size_t tb = 0;
     if (e == hipSuccess) e = nbx_sort_pairs_u64(nullptr, tb, keys, keys2, idx, order, m, st);

@@ -77,7 +77,6 @@ struct KnnArgs {
     int32_t layout;     // NBX_LAYOUT_BY_ID / BY_SLOT
     int32_t dens;       // NBX_DO_*
     int32_t nsmooth;    // velocity density
-    int32_t m;          // external points
     int32_t periodic;
     double period[3];
     const double *q[3];  // external points (SoA)
@@ -158,11 +157,10 @@ struct BallManyArgs {
     const int32_t *order;  // positions in walk order (nullable: as given)
 };
 hipError_t nbx_launch_ball_many(const DevTree &T, const BallManyArgs &A, bool fill, hipStream_t st);
-// Order of m query points (T.nd coordinates each) along the Morton curve over
-// the root box, so that a wave's 64 points are neighbours: order[0..m).
+// Order of m query points along the Morton curve over the root box, so that a wave's 64 points are neighbours: order[0..m).
 // work: nbx_point_order_bytes(m) bytes of device memory.
 struct PointCoords {
-    const double *c[6];
+    const double *c[3];
 };
 size_t nbx_point_order_bytes(int64_t m);
 hipError_t nbx_point_order(const DevTree &T, const PointCoords &q, int64_t m, int32_t *order, void *work,
