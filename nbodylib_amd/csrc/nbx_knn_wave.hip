@@ -358,6 +358,20 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
         if (key == m) key = ~0u;
         return (int)(m & 63u);
     };
+    int staged = 0;  // accepted entries in sh that are not kept yet
+    auto flush = [&]() {
+        if (staged < WV_MERGE) {
+            __syncthreads();
+            for (int j = 0; j < staged; ++j)
+                wv_insert(k, readfirst_d(sh.d[j]), __builtin_amdgcn_readfirstlane(sh.id[j]),
+                          __builtin_amdgcn_readfirstlane(sh.slot[j]), lane);
+            __syncthreads();
+        } else {
+            wv_merge(k, staged, kh, sh, lane);
+        }
+        wv_kth(k, kh);
+        staged = 0;
+    };
     for (;;) {
         if (expand) {
             height -= step;
@@ -421,33 +435,13 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
                 const int32_t id[2] = {ids.x, ids.y};
                 // equally far as the last kept: only a smaller ID counts; the
                 // query itself has d2 == 0
-                int cnt = 0;
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
                     acc[p] &= ballot(d2[p] < k.kth) | ballot(id[p] < k.kid);
                     if (exz) acc[p] &= ballot(d2[p] > 0.0);
-                    cnt += __builtin_popcountll(acc[p]);
-                }
-                if (cnt < WV_MERGE) {
-#pragma unroll
-                    for (int p = 0; p < 2; ++p)
-                        for (uint64_t m = acc[p]; m; m &= m - 1) {
-                            const int j = __builtin_ctzll(m);
-                            wv_insert(k, lane_d(d2[p], j), __builtin_amdgcn_readlane(id[p], j),
-                                      __builtin_amdgcn_readlane(sl, j) + p, lane);
-                        }
-                    if (cnt) wv_kth(k, kh);
-                    continue;
-                }
-                int staged = 0;
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    if (p > 0 && staged + __builtin_popcountll(acc[p]) > NBX_WAVE) {
-                        wv_merge(k, staged, kh, sh, lane);
-                        wv_kth(k, kh);
-                        staged = 0;
-                        acc[p] &= ballot(before(d2[p], id[p], k.kth, k.kid));
-                    }
+                    const int cnt = __builtin_popcountll(acc[p]);
+                    if (cnt == 0) continue;
+                    if (staged + cnt > NBX_WAVE) flush();
                     if ((acc[p] >> lane) & 1ULL) {
                         const int at = staged + __builtin_amdgcn_mbcnt_hi((uint32_t)(acc[p] >> 32),
                                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)acc[p], 0));
@@ -455,10 +449,9 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
                         sh.id[at] = id[p];
                         sh.slot[at] = sl + p;
                     }
-                    staged += __builtin_popcountll(acc[p]);
+                    staged += cnt;
                 }
-                wv_merge(k, staged, kh, sh, lane);
-                wv_kth(k, kh);
+                if (staged) flush();
                 continue;
             }
         } else {
