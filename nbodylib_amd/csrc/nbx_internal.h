@@ -121,31 +121,6 @@ __device__ __forceinline__ double box_ub(const double *q, cdptr b) {
     }
     return s;
 }
-// Upper bound on the squared distance between any point of box a and any
-// point of box b (monotone for the same reason).
-template <int ND>
-__device__ __forceinline__ double boxbox_ub(cdptr a, cdptr b) {
-    double s = 0.0;
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-        double u = b[ND + d] - a[d], v = a[ND + d] - b[d];
-        double m = u > v ? u : v;
-        s += m * m;
-    }
-    return s;
-}
-template <int ND>
-__device__ __forceinline__ double boxbox_lb(cdptr a, cdptr b) {
-    double s = 0.0;
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-        double t = 0.0;
-        if (a[ND + d] < b[d]) t = b[d] - a[ND + d];
-        else if (b[ND + d] < a[d]) t = a[d] - b[ND + d];
-        s += t * t;
-    }
-    return s;
-}
 
 // Which child of internal node p to descend first, seen from the uniform
 // point qc: the one whose box centre is nearer (a heuristic for the visiting
@@ -157,10 +132,6 @@ __device__ __forceinline__ bool first_is_right(const float *plane, int p, const 
 #pragma unroll
     for (int d = 0; d < ND; ++d) s = __builtin_fmaf(pl[d], qc[d], s);
     return s > pl[ND];
-}
-template <int ND>
-__device__ __forceinline__ bool first_is_right(const DevTree &T, int p, const float *qc) {
-    return first_is_right<ND>(T.plane, p, qc);
 }
 
 // Workgroups of a launch are dealt round-robin to the 8 XCDs (workgroup b

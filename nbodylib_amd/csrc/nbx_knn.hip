@@ -175,7 +175,7 @@ __device__ __forceinline__ void knn_leaf(const DevTree &T, const double *const (
     for (int d = 0; d < ND; ++d) st[d] = X[d][base + (lane & (NBX_LEAF - 1))];
     uint32_t mask = 0;
     // candidates arrive in chunks through the scalar cache: 8 per dimension
-    // (24 SGPR pairs) in 3-D, 4 in 6-D
+    // (24 SGPR pairs)
     constexpr int CH = 8;
     typedef double dxc __attribute__((ext_vector_type(CH)));
     typedef const __attribute__((address_space(4))) dxc *cdcptr;
@@ -431,8 +431,7 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
     double racc_own = 0.0;
     if (sym) racc[lane] = 0.0;
     __syncthreads();
-    // position queries take the gather forms only (mass and slot of the
-    // query are undefined there)
+    // image-shifted queries take the gather forms only
     if (A.dens != NBX_DO_NONE && valid && (QSRC == NBX_Q_SLOTS || A.dens == NBX_DO_GATHER)) {
         const bool bad = !(kth < NBX_MAXVALUE);  // fewer than kh neighbours
         if (A.dens == NBX_DO_VEL || A.dens == NBX_DO_VELPHYS) {

@@ -573,8 +573,9 @@ __device__ __forceinline__ void mix_sub8(const MixSrc<ND> &S, const float *boxp,
     }
 }
 
-// Stackless depth-first walk: the ancestor of the wave's own leaves first,
-// else the child nearer to the wave's first query; firstright[dep] records
+// Stackless depth-first walk, begun at the wave's own leaf (3-D) or its
+// ancestor three or six levels up (6-D): elsewhere the child nearer to the
+// wave's first query comes first; firstright[dep] records
 // which child was entered first at each depth.  Two loop forms visit the
 // nodes in the same order; the compiler schedules them differently, and the
 // measured faster one is used for each dimensionality (3-D: climb to the
@@ -1216,8 +1217,9 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
 // (6-D, k <= 32: LDS allows 15 waves per CU, so the registers are held to the
 // 128 that four waves per SIMD leave)
 template <int ND, int KMAX, int MODE>
-__global__ __launch_bounds__(64, ND == 6 && KMAX == 33 ? 4 : 1) void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list,
-                                                   int32_t *fb_count, uint32_t *scratch, int32_t *ctr) {
+__global__ __launch_bounds__(64, ND == 6 && KMAX == 33 ? 4 : 1)
+void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list, int32_t *fb_count, uint32_t *scratch,
+                 int32_t *ctr) {
     __shared__ uint32_t hk[KMAX * NBX_WAVE];
     // one buffer for three uses at different times: the leaf copy (phase 2),
     // the compacted queries and their masks (6-D node tests and phase 1) and
