@@ -125,44 +125,113 @@ __global__ __launch_bounds__(KD_T) void k_kd_ext(KdState S, int64_t n, int lseg,
     }
 }
 
-// Split dimension (largest extent) and the left count of every node; the
-// radix select state starts with prefix 0 and rank = left count.
-__global__ __launch_bounds__(KD_T) void k_kd_dims(const uint32_t *__restrict__ ext, int nd, int64_t n, int lseg,
-                                                  int64_t nseg, uint8_t *__restrict__ dsel, uint32_t *__restrict__ pre,
-                                                  int32_t *__restrict__ need) {
-    int64_t s = (int64_t)blockIdx.x * KD_T + threadIdx.x;
-    if (s >= nseg) return;
-    const int64_t a = s << lseg;
-    if (a >= n) return;
-    int best = 0;
-    float bext = -1.0f;
-    for (int d = 0; d < nd; ++d) {
-        const float e = fdekey(ext[(s * nd + d) * 2 + 1]) - fdekey(ext[(s * nd + d) * 2]);
-        if (e > bext) {
-            bext = e;
-            best = d;
-        }
+// Radix select of the split coordinate's median.  A level's state before digit
+// d (d = 0 the highest; 4: the finished pivot) is pre[d], the digits found so
+// far, and need[d], the rank left among the keys that have them; hist[d] counts
+// digit d of those keys.  A launch counts one digit, and its blocks first take
+// the step from the digit before by themselves, each for its own node, the
+// node's first block noting it for the launches to come.  (Steps in launches of
+// their own, and others for the dimensions and for clearing, made 14 launches
+// per level; these are 7.  On 2M particles a launch is mostly its start and
+// end: FOF of a new snapshot 1.85 -> 1.76 ms.)
+struct KdSel {
+    uint8_t *dsel;   // split dimension
+    uint32_t *pre;   // [5][nsegmax]
+    int32_t *need;   // [5][nsegmax]
+    uint32_t *hist;  // [4][nsegmax][256]
+    int64_t nsegmax;
+};
+struct KdStep {
+    uint32_t pre;
+    int32_t need, dim;
+};
+
+// One wave: the digit whose bin holds the rank left, four bins per lane and a
+// wave prefix sum.
+__device__ __forceinline__ void kd_step(const KdSel &Q, int64_t s, int d, KdStep &to) {
+    const int lane = threadIdx.x & 63;
+    const uint4 v = *(const uint4 *)(Q.hist + ((d - 1) * Q.nsegmax + s) * 256 + 4 * lane);
+    const uint32_t c4 = v.x + v.y + v.z + v.w;
+    uint32_t inc = c4;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)inc, off);
+        if (lane >= off) inc += y;
     }
-    dsel[s] = (uint8_t)best;
-    pre[s] = 0u;
-    const int64_t m = min(a + ((int64_t)1 << (lseg - 1)), n);
-    need[s] = (int32_t)(m - a);
+    const uint32_t exc = inc - c4;
+    const uint32_t r = (uint32_t)Q.need[(d - 1) * Q.nsegmax + s];
+    const uint64_t bm = ballot(exc < r && r <= inc);
+    const int L = bm ? __builtin_ctzll(bm) : 63;
+    if (lane == L) {
+        uint32_t rr = r - exc;
+        int b = 4 * lane;
+        if (rr > v.x) {
+            rr -= v.x;
+            ++b;
+            if (rr > v.y) {
+                rr -= v.y;
+                ++b;
+                if (rr > v.z) {
+                    rr -= v.z;
+                    ++b;
+                }
+            }
+        }
+        to.pre = Q.pre[(d - 1) * Q.nsegmax + s] | ((uint32_t)b << (32 - 8 * d));
+        to.need = (int32_t)rr;
+        to.dim = Q.dsel[s];
+    }
 }
 
-// Radix select pass: histogram of the 8-bit digit at `sh` of the split keys
-// whose higher digits equal the node's prefix.
-__global__ __launch_bounds__(KD_T) void k_kd_hist(KdState S, int64_t n, int lseg, int sh,
-                                                  const uint8_t *__restrict__ dsel, const uint32_t *__restrict__ pre,
-                                                  uint32_t *__restrict__ hist) {
+// State before digit d of the block's node; every thread of the block calls it.
+__device__ __forceinline__ void kd_state(const KdSel &Q, int64_t s, int d, bool first, KdStep &sh) {
+    if (threadIdx.x < 64) kd_step(Q, s, d, sh);
+    __syncthreads();
+    if (first && threadIdx.x == 0) {
+        Q.pre[d * Q.nsegmax + s] = sh.pre;
+        Q.need[d * Q.nsegmax + s] = sh.need;
+    }
+}
+
+// Histogram of the 8-bit digit d of the split keys that have the digits found
+// so far.  d = 0 begins with the split dimension (largest extent) and the
+// node's left count.  A block covers KD_LOCAL positions of one node.
+__global__ __launch_bounds__(KD_T) void k_kd_hist(KdState S, int64_t n, int nd, int lseg, int d,
+                                                  const uint32_t *__restrict__ ext, KdSel Q) {
     __shared__ uint32_t h[256];
+    __shared__ KdStep st;
     const int t = threadIdx.x;
     h[t] = 0u;
-    __syncthreads();
     const int64_t i0 = (int64_t)blockIdx.x * KD_LOCAL;
-    const int64_t s = i0 >> lseg;
-    const uint32_t *K = S.key[dsel[s]];
-    const uint32_t p = pre[s];
-    const uint32_t hm = sh >= 24 ? 0u : (0xffffffffu << (sh + 8));  // higher digits already fixed
+    const int64_t s = i0 >> lseg, a = s << lseg;
+    if (d == 0) {
+        if (t == 0) {
+            int best = 0;
+            float bext = -1.0f;
+            for (int c = 0; c < nd; ++c) {
+                const float e = fdekey(ext[(s * nd + c) * 2 + 1]) - fdekey(ext[(s * nd + c) * 2]);
+                if (e > bext) {
+                    bext = e;
+                    best = c;
+                }
+            }
+            st.dim = best;
+            st.pre = 0u;
+            st.need = (int32_t)(min(a + ((int64_t)1 << (lseg - 1)), n) - a);
+            if (i0 == a) {
+                Q.dsel[s] = (uint8_t)best;
+                Q.pre[s] = 0u;
+                Q.need[s] = st.need;
+            }
+        }
+        __syncthreads();
+    } else {
+        kd_state(Q, s, d, i0 == a, st);
+    }
+    const uint32_t *K = S.key[st.dim];
+    const uint32_t p = st.pre;
+    const int sh = 24 - 8 * d;
+    const uint32_t hm = d == 0 ? 0u : (0xffffffffu << (sh + 8));  // higher digits already fixed
     const int lane = t & 63;
 #pragma unroll
     for (int q = 0; q < KD_PER; ++q) {
@@ -183,63 +252,32 @@ __global__ __launch_bounds__(KD_T) void k_kd_hist(KdState S, int64_t n, int lseg
         }
     }
     __syncthreads();
-    if (h[t]) atomicAdd(hist + s * 256 + t, h[t]);
-}
-
-// Radix select step: the digit bin holding the node's remaining rank.  One
-// wave per node, four bins per lane and a wave prefix sum; the node's bins
-// are cleared for the next pass.
-__global__ __launch_bounds__(KD_T) void k_kd_select(int64_t n, int lseg, int64_t nseg, int sh,
-                                                    uint32_t *__restrict__ hist, uint32_t *__restrict__ pre,
-                                                    int32_t *__restrict__ need) {
-    const int lane = threadIdx.x & 63;
-    const int64_t s = (int64_t)blockIdx.x * (KD_T / 64) + (threadIdx.x >> 6);
-    if (s >= nseg || (s << lseg) >= n) return;
-    uint32_t *h = hist + s * 256;
-    const uint4 v = *(const uint4 *)(h + 4 * lane);
-    const uint32_t c4 = v.x + v.y + v.z + v.w;
-    uint32_t inc = c4;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)inc, off);
-        if (lane >= off) inc += y;
-    }
-    const uint32_t exc = inc - c4;
-    const uint32_t r = (uint32_t)need[s];
-    const uint64_t bm = ballot(exc < r && r <= inc);
-    const int L = bm ? __builtin_ctzll(bm) : 63;
-    if (lane == L) {
-        uint32_t rr = r - exc;
-        int b = 4 * lane;
-        if (rr > v.x) {
-            rr -= v.x;
-            ++b;
-            if (rr > v.y) {
-                rr -= v.y;
-                ++b;
-                if (rr > v.z) {
-                    rr -= v.z;
-                    ++b;
-                }
-            }
-        }
-        pre[s] |= (uint32_t)b << sh;
-        need[s] = (int32_t)rr;
-    }
-    *(uint4 *)(h + 4 * lane) = make_uint4(0u, 0u, 0u, 0u);
+    if (h[t]) atomicAdd(Q.hist + (d * Q.nsegmax + s) * 256 + t, h[t]);
 }
 
 // Per-block (below, equal) counts of the split keys against the node's
 // pivot, packed as below << 32 | equal.  A block covers KD_LOCAL positions
-// of one node.
-__global__ __launch_bounds__(KD_T) void k_kd_count(KdState S, int64_t n, int lseg, const uint8_t *__restrict__ dsel,
-                                                   const uint32_t *__restrict__ pre, uint64_t *__restrict__ blk) {
+// of one node.  The launch also prepares the next level: its extents (npair of
+// them; this level's were last read by the first digit's launch) and the other
+// set of histograms (of its 2^lnext nodes; lnext < 0: no next level).
+__global__ __launch_bounds__(KD_T) void k_kd_count(KdState S, int64_t n, int lseg, KdSel Q, uint64_t *__restrict__ blk,
+                                                   uint32_t *__restrict__ ext, int64_t npair,
+                                                   uint4 *__restrict__ clear, int lnext) {
     __shared__ uint32_t wb[KD_T / 64], we[KD_T / 64];
+    __shared__ KdStep st;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int64_t i0 = (int64_t)blockIdx.x * KD_LOCAL;
     const int64_t s = i0 >> lseg;
-    const uint32_t *K = S.key[dsel[s]];
-    const uint32_t p = pre[s];
+    for (int64_t i = (int64_t)blockIdx.x * KD_T + t; i < npair; i += (int64_t)gridDim.x * KD_T) {
+        ext[2 * i] = 0xffffffffu;
+        ext[2 * i + 1] = 0u;
+    }
+    const int64_t per = lnext < 0 ? 0 : (int64_t)64 << lnext;  // of one digit
+    for (int64_t i = (int64_t)blockIdx.x * KD_T + t; i < 4 * per; i += (int64_t)gridDim.x * KD_T)
+        clear[(i >> (lnext + 6)) * Q.nsegmax * 64 + (i & (per - 1))] = make_uint4(0u, 0u, 0u, 0u);
+    kd_state(Q, s, 4, i0 == s << lseg, st);
+    const uint32_t *K = S.key[st.dim];
+    const uint32_t p = st.pre;
     uint32_t nb = 0, ne = 0;
 #pragma unroll
     for (int q = 0; q < KD_PER; ++q) {
@@ -568,9 +606,8 @@ static inline int nblk(int64_t n, int b = KD_T) { return (int)((n + b - 1) / b);
 // histograms and the blocks' counts and prefixes.
 struct KdWork {
     KdState S;
-    uint32_t *ext, *pre, *hist;
-    int32_t *need;
-    uint8_t *dsel;
+    uint32_t *ext, *hist[2];  // (histograms: one set in use, one cleared for the next level)
+    KdSel sel;
     uint64_t *blk, *bpre;
     int ltot, lblk;
     bool global;
@@ -599,10 +636,11 @@ struct KdWork {
             S.id2 = (int32_t *)carve(sizeof(int32_t) * n);
             for (int d = 0; d < nd; ++d) S.key2[d] = (uint32_t *)carve(sizeof(uint32_t) * n);
             ext = (uint32_t *)carve(sizeof(uint32_t) * 2 * nd * nsegmax);
-            pre = (uint32_t *)carve(sizeof(uint32_t) * nsegmax);
-            need = (int32_t *)carve(sizeof(int32_t) * nsegmax);
-            dsel = (uint8_t *)carve((size_t)nsegmax);
-            hist = (uint32_t *)carve(sizeof(uint32_t) * 256 * nsegmax);
+            sel.nsegmax = nsegmax;
+            sel.pre = (uint32_t *)carve(5 * sizeof(uint32_t) * nsegmax);
+            sel.need = (int32_t *)carve(5 * sizeof(int32_t) * nsegmax);
+            sel.dsel = (uint8_t *)carve((size_t)nsegmax);
+            for (int i = 0; i < 2; ++i) hist[i] = (uint32_t *)carve(4 * sizeof(uint32_t) * 256 * nsegmax);
             blk = (uint64_t *)carve(sizeof(uint64_t) * nb);
             bpre = (uint64_t *)carve(sizeof(uint64_t) * nb);
         }
@@ -618,9 +656,8 @@ hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleaf
     KdWork W(work, nd, n, nleafp);
     KdState &Sh = W.S;
     const int ltot = W.ltot, lblk = W.lblk;
-    uint32_t *ext = W.ext, *pre = W.pre, *hist = W.hist;
-    int32_t *need = W.need;
-    uint8_t *dsel = W.dsel;
+    uint32_t *ext = W.ext;
+    KdSel Q = W.sel;
     uint64_t *blk = W.blk, *bpre = W.bpre;
     KdCoords C;
     memset(&C, 0, sizeof(C));
@@ -628,7 +665,9 @@ hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleaf
     hipLaunchKernelGGL(k_kd_init, dim3(nblk(n)), dim3(KD_T), 0, st, C, nd, n, Sh);
     if (W.global) {
         const int nb = nblk(n, KD_LOCAL);
-        hipLaunchKernelGGL(k_kd_zero, dim3(nblk(256 * W.nsegmax)), dim3(KD_T), 0, st, hist, (int64_t)256 * W.nsegmax);
+        // the first level's histograms; k_kd_count clears the others
+        hipLaunchKernelGGL(k_kd_zero, dim3(nblk(1024 * W.nsegmax)), dim3(KD_T), 0, st, W.hist[0],
+                           (int64_t)1024 * W.nsegmax);
         // root extents; deeper levels get theirs from the previous move
         hipLaunchKernelGGL(k_kd_ext_init, dim3(nblk(nd)), dim3(KD_T), 0, st, ext, (int64_t)nd);
         if (nd == 3)
@@ -637,27 +676,22 @@ hipError_t nbx_kd_order(const double *const *c, int nd, int64_t n, int32_t nleaf
             hipLaunchKernelGGL(k_kd_ext<6>, dim3(nb), dim3(KD_T), 0, st, Sh, n, ltot, ext);
         for (int lseg = ltot; lseg > lblk; --lseg) {
             const int64_t nseg = (int64_t)1 << (ltot - lseg);
-            hipLaunchKernelGGL(k_kd_dims, dim3(nblk(nseg)), dim3(KD_T), 0, st, ext, nd, n, lseg, nseg, dsel, pre,
-                               need);
             const bool next = lseg - 1 > lblk;
-            if (next)
-                hipLaunchKernelGGL(k_kd_ext_init, dim3(nblk(2 * nd * nseg)), dim3(KD_T), 0, st, ext,
-                                   (int64_t)2 * nd * nseg);
-            for (int sh = 24; sh >= 0; sh -= 8) {
-                // the select step leaves every bin it read at zero
-                hipLaunchKernelGGL(k_kd_hist, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, sh, dsel, pre, hist);
-                hipLaunchKernelGGL(k_kd_select, dim3(nblk(nseg, KD_T / 64)), dim3(KD_T), 0, st, n, lseg, nseg, sh,
-                                   hist, pre, need);
-            }
-            hipLaunchKernelGGL(k_kd_count, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, dsel, pre, blk);
+            const int set = (ltot - lseg) & 1;
+            Q.hist = W.hist[set];
+            for (int d = 0; d < 4; ++d)
+                hipLaunchKernelGGL(k_kd_hist, dim3(nb), dim3(KD_T), 0, st, Sh, n, nd, lseg, d, ext, Q);
+            hipLaunchKernelGGL(k_kd_count, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, Q, blk, ext,
+                               next ? (int64_t)2 * nd * nseg : 0, (uint4 *)W.hist[set ^ 1],
+                               next ? ltot - lseg + 1 : -1);
             hipLaunchKernelGGL(k_kd_bscan, dim3(1), dim3(KD_ST), 0, st, blk, (int64_t)nb, bpre);
             uint32_t *enext = next ? ext : nullptr;
             if (nd == 3)
-                hipLaunchKernelGGL(k_kd_move<3>, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, dsel, pre, need, bpre,
-                                   enext);
+                hipLaunchKernelGGL(k_kd_move<3>, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, Q.dsel, Q.pre + 4 * Q.nsegmax,
+                                   Q.need + 4 * Q.nsegmax, bpre, enext);
             else
-                hipLaunchKernelGGL(k_kd_move<6>, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, dsel, pre, need, bpre,
-                                   enext);
+                hipLaunchKernelGGL(k_kd_move<6>, dim3(nb), dim3(KD_T), 0, st, Sh, n, lseg, Q.dsel, Q.pre + 4 * Q.nsegmax,
+                                   Q.need + 4 * Q.nsegmax, bpre, enext);
             std::swap(Sh.id, Sh.id2);
             for (int d = 0; d < nd; ++d) std::swap(Sh.key[d], Sh.key2[d]);
         }
