@@ -464,9 +464,11 @@ static int build_tree(nbx_tree *t, const double *pos, const double *vel, const d
         if (t->nleafp > t->nleaf)
             hipLaunchKernelGGL(k_leafbox_pad, dim3(nblk(t->nleafp - t->nleaf)), dim3(256), 0, st, t->box, t->nleaf,
                                t->nleafp, nd);
-        for (int dep = t->depth - 1; dep >= 0; --dep)
-            hipLaunchKernelGGL(k_levelbox, dim3(nblk((int64_t)1 << dep)), dim3(256), 0, st, t->box, t->plane,
-                               1 << dep, 1 << dep, nd);
+        for (int dbot = t->depth; dbot > 0;) {
+            const int dtop = std::max(0, dbot - NBX_UP);
+            hipLaunchKernelGGL(k_levelbox, dim3(1 << dtop), dim3(256), 0, st, t->box, t->plane, dtop, dbot, nd);
+            dbot = dtop;
+        }
     }
     HIPCK(hipGetLastError());
     double rb[12];

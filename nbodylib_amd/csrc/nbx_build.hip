@@ -128,12 +128,8 @@ __global__ __launch_bounds__(256) void k_leafbox_pad(double *box, int32_t nleaf,
     }
 }
 
-// Internal nodes [first, first+count) of one depth: union of the two children.
-__global__ __launch_bounds__(256) void k_levelbox(double *__restrict__ box, float *__restrict__ plane, int32_t first,
-                                                  int32_t count, int nd) {
-    int32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= count) return;
-    int32_t nn = first + i;
+// Internal node nn: union of the two children.
+__device__ __forceinline__ void node_up(double *box, float *plane, int32_t nn, int nd) {
     const double *a = box + (size_t)(2 * nn) * 2 * nd;
     const double *b = a + 2 * nd;
     double *o = box + (size_t)nn * 2 * nd;
@@ -156,6 +152,18 @@ __global__ __launch_bounds__(256) void k_levelbox(double *__restrict__ box, floa
     }
     pl[nd] = empty ? 1.0f : (float)off;
     for (int d = nd + 1; d < plw; ++d) pl[d] = 0.0f;
+}
+// The nodes of depths [dtop, dbot), a block for each subtree under depth dtop
+// (at most NBX_UP levels, so the lowest has a node for each thread).  A launch
+// for each depth took longer to start than to run: 16 of them 73 us on 2M
+// particles, 32 us so.
+__global__ __launch_bounds__(256) void k_levelbox(double *box, float *plane, int dtop, int dbot, int nd) {
+    const int32_t r = (1 << dtop) + (int32_t)blockIdx.x;
+    for (int dep = dbot - 1; dep >= dtop; --dep) {
+        const int32_t cnt = 1 << (dep - dtop);
+        if ((int32_t)threadIdx.x < cnt) node_up(box, plane, (r << (dep - dtop)) + (int32_t)threadIdx.x, nd);
+        __syncthreads();  // the block's own boxes, read by it at the next depth
+    }
 }
 
 // the next FP32 value above f (f finite or -inf; +inf and NaN unchanged)

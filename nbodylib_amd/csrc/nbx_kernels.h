@@ -37,7 +37,8 @@ __global__ void k_bbox(CoordPtrs c, int64_t n, double *part);
 __global__ void k_bbox_end(const double *part, int nb, double *box);
 __global__ void k_gather_leaf(GatherArgs a);
 __global__ void k_leafbox_pad(double *box, int32_t nleaf, int32_t nleafp, int nd);
-__global__ void k_levelbox(double *box, float *plane, int32_t first, int32_t count, int nd);
+#define NBX_UP 9  // depths k_levelbox takes at once
+__global__ void k_levelbox(double *box, float *plane, int dtop, int dbot, int nd);
 __global__ void k_boxf(const double *box, float *boxf, int64_t count, int nd);
 
 // order (slot -> ID) of the implicit kd tree: midpoint splits along the
