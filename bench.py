@@ -138,25 +138,25 @@ def main():
         torch.cuda.synchronize()
         wall = time.perf_counter() - t0
         nb.prof_enable(False)
-        kname = "k_knn_mixed" if form == nb.FORM_MIXED else "k_knn_fp64"
-        kms, klaunch = nb.prof_get(kname)
+        kname, kms, klaunch = _search_time(nb, form)
         fbms, _ = nb.prof_get("k_knn_fallback")
         log(f"{label}: {wall / args.steps * 1e3:.2f} ms/step, {kname} {kms / max(klaunch, 1):.2f} ms/launch, "
             f"fallback {fbms / args.steps:.2f} ms/step, fallbacks {tree.last_fallbacks()}")
-        return tree, build_ms, wall, kms, klaunch
+        return tree, build_ms, wall, kname, kms, klaunch
 
     forms = args.forms.split(",")
-    plain_tree, plain_build_ms, plain_wall, plain_kms, plain_kl = run_form(nb.FORM_PLAIN, "plain-fp64")
+    plain_tree, plain_build_ms, plain_wall, plain_kn, plain_kms, plain_kl = run_form(nb.FORM_PLAIN, "plain-fp64")
     rho_plain = rho.clone()
-    headline = dict(form="plain-fp64", wall=plain_wall, kms=plain_kms, kl=plain_kl, build_ms=plain_build_ms)
+    headline = dict(form="plain-fp64", wall=plain_wall, kname=plain_kn, kms=plain_kms, kl=plain_kl,
+                    build_ms=plain_build_ms)
 
     mixed = None
     try:
         if "mixed" not in forms:
             raise nb.NbxError(-3, "mixed form not requested")
-        mixed_tree, mixed_build_ms, mixed_wall, mixed_kms, mixed_kl = run_form(nb.FORM_MIXED, "mixed")
+        mixed_tree, mixed_build_ms, mixed_wall, mixed_kn, mixed_kms, mixed_kl = run_form(nb.FORM_MIXED, "mixed")
         relerr = float(torch.max(torch.abs(rho / rho_plain - 1.0)))
-        mixed = dict(form="mixed", wall=mixed_wall, kms=mixed_kms, kl=mixed_kl, build_ms=mixed_build_ms,
+        mixed = dict(form="mixed", wall=mixed_wall, kname=mixed_kn, kms=mixed_kms, kl=mixed_kl, build_ms=mixed_build_ms,
                      rel=relerr, fallbacks=mixed_tree.last_fallbacks())
         headline = mixed
         del mixed_tree
@@ -187,7 +187,7 @@ def main():
     bytes_per_q = 48 + 4 * k
     kern_ms = headline["kms"] / max(headline["kl"], 1)
     achieved = bytes_per_q * n / (kern_ms / 1e3) / 1e9
-    kname = "k_knn_mixed" if headline["form"] == "mixed" else "k_knn_fp64"
+    kname = headline["kname"]
     traffic = None
     valu = None
     if os.path.exists(args.traffic):
@@ -320,6 +320,17 @@ class Timer:
         self.ms = self.a.elapsed_time(self.b)
 
 
+def _search_time(nb, form):
+    """(name, ms, launches) of the search kernel that ran: a precision-form call that the FP64 kernel serves faster
+    (few queries, k > 32) runs on that one."""
+    name = "k_knn_mixed"
+    ms, launches = nb.prof_get(name)
+    if form != nb.FORM_MIXED or launches == 0:
+        name = "k_knn_fp64"
+        ms, launches = nb.prof_get(name)
+    return name, ms, launches
+
+
 def _median(xs):
     xs = sorted(xs)
     return xs[len(xs) // 2]
@@ -375,8 +386,7 @@ def phase6d_section(args, steps, warmup):
                 t6.density(k, rho, hh)
             times.append(tm.ms)
         nb.prof_enable(False)
-        kname = "k_knn_mixed" if form == nb.FORM_MIXED else "k_knn_fp64"
-        kms, kl = nb.prof_get(kname)
+        kname, kms, kl = _search_time(nb, form)
         ms = _median(times)
         fb = t6.last_fallbacks()
         log(f"phase6d {label}: 6-D k={k} kNN + density {ms:.2f} ms ({kname} {kms / max(kl, 1):.2f} ms/launch, "
