@@ -104,23 +104,24 @@ __device__ __forceinline__ bool before(double da, int32_t ia, double db, int32_t
 }
 
 // Kept entries of the wave's query: position p = 64 e + lane, ascending in
-// (d2, ID); kth is the distance at position kh - 1, kid its ID and lim its key.
+// (d2, ID); kth, kslot: the entry at position kh - 1, lim: its key.  IDs decide
+// only between equal distances, and are looked up then.
 template <int E>
 struct WvKept {
     union Dbl {
         double d;
         int32_t w[2];
     } d[E];
-    int32_t id[E], slot[E];
+    int32_t slot[E];
     double kth;
-    int32_t kid;
+    int32_t kslot;
     uint32_t lim;
 };
 template <int E>
 struct WvShared {
     uint32_t stk[WV_LEVELS][NBX_WAVE];
     double d[NBX_WAVE * (E + 1)];
-    int32_t id[NBX_WAVE * (E + 1)], slot[NBX_WAVE * (E + 1)];
+    int32_t slot[NBX_WAVE * (E + 1)];
 };
 
 // (one unit above the distance's own key: a bound's last bits are free)
@@ -131,20 +132,23 @@ template <int E>
 __device__ __forceinline__ void wv_kth(WvKept<E> &k, int kh) {
     const int l = (kh - 1) & 63, at = (kh - 1) >> 6;
     double d = k.d[0].d;
-    int32_t i = k.id[0];
+    int32_t i = k.slot[0];
 #pragma unroll
     for (int e = 1; e < E; ++e) {
         d = at == e ? k.d[e].d : d;
-        i = at == e ? k.id[e] : i;
+        i = at == e ? k.slot[e] : i;
     }
     k.kth = lane_d(d, l);
-    k.kid = __builtin_amdgcn_readlane(i, l);
+    k.kslot = __builtin_amdgcn_readlane(i, l);
     k.lim = wv_lim(k.kth);
 }
 
+// ID of a kept entry; an empty one comes after all others
+__device__ __forceinline__ int32_t wv_id(const DevTree &T, int32_t slot) { return slot >= 0 ? T.perm[slot] : WV_NOID; }
+
 // Insert one entry (uniform values).
 template <int E>
-__device__ __forceinline__ void wv_insert(WvKept<E> &k, double d, int32_t id, int32_t slot, int lane) {
+__device__ __forceinline__ void wv_insert(const DevTree &T, WvKept<E> &k, double d, int32_t slot, int lane) {
     typename WvKept<E>::Dbl n;
     n.d = d;
     // (what leaves a block at its top enters the next one at its bottom)
@@ -152,24 +156,24 @@ __device__ __forceinline__ void wv_insert(WvKept<E> &k, double d, int32_t id, in
     for (int e = 0; e < E; ++e) {
         uint64_t less = ballot(k.d[e].d < n.d);
         const uint64_t same = ballot(k.d[e].d == n.d);
-        if (same) less |= ballot(k.d[e].d == n.d && k.id[e] < id);
+        if (same) {
+            const int32_t id = wv_id(T, slot), ki = wv_id(T, k.slot[e]);
+            less |= same & ballot(ki < id);
+        }
         const int p = __builtin_popcountll(less);
         if (p == NBX_WAVE) continue;
         const bool stay = lane < p;
         typename WvKept<E>::Dbl top;
         top.d = lane_d(k.d[e].d, NBX_WAVE - 1);
-        const int32_t tid = __builtin_amdgcn_readlane(k.id[e], NBX_WAVE - 1),
-                      tslot = __builtin_amdgcn_readlane(k.slot[e], NBX_WAVE - 1);
+        const int32_t tslot = __builtin_amdgcn_readlane(k.slot[e], NBX_WAVE - 1);
         auto put = [&](int32_t v, int32_t x) {
             const int32_t below = lane_below(v);
             return lane == p ? x : (stay ? v : below);
         };
         k.d[e].w[0] = put(k.d[e].w[0], n.w[0]);
         k.d[e].w[1] = put(k.d[e].w[1], n.w[1]);
-        k.id[e] = put(k.id[e], id);
         k.slot[e] = put(k.slot[e], slot);
         n = top;
-        id = tid;
         slot = tslot;
     }
 }
@@ -226,9 +230,12 @@ __device__ __forceinline__ uint32_t key_sort_row(uint32_t v, int lane) {
     v = key_merge<2>(key_pick<4>(v, dpp<0x141>(v), lane), lane);  // half a row
     return key_merge<4>(key_pick<8>(v, dpp<0x140>(v), lane), lane);  // a row
 }
-__device__ __forceinline__ uint32_t key_sort(uint32_t v, int lane) {
+__device__ __forceinline__ uint32_t key_sort_half(uint32_t v, int lane) {
     v = key_sort_row(v, lane);
-    v = key_merge<8>(key_pick<16>(v, (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x7c1f), lane), lane);  // lane ^ 31
+    return key_merge<8>(key_pick<16>(v, (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x7c1f), lane), lane);  // lane ^ 31
+}
+__device__ __forceinline__ uint32_t key_sort(uint32_t v, int lane) {
+    v = key_sort_half(v, lane);
     return key_merge<16>(key_pick<32>(v, key_reverse(v, lane), lane), lane);
 }
 
@@ -249,9 +256,10 @@ __device__ __forceinline__ void wv_exchange(D &d, int32_t &id, int32_t &slot, in
 // Merge 64 entries, one per lane in any order, into the kept ones, exactly:
 // for entries whose keys do not tell them apart.
 template <int E>
-__device__ __forceinline__ void wv_merge_exact(WvKept<E> &k, double nd, int32_t id, int32_t slot, int lane) {
+__device__ __forceinline__ void wv_merge_exact(const DevTree &T, WvKept<E> &k, double nd, int32_t slot, int lane) {
     typename WvKept<E>::Dbl d;
     d.d = nd;
+    int32_t id = wv_id(T, slot);
 #pragma unroll 1
     for (int n = 2; n <= NBX_WAVE; n <<= 1)
 #pragma unroll 1
@@ -260,11 +268,12 @@ __device__ __forceinline__ void wv_merge_exact(WvKept<E> &k, double nd, int32_t 
     // these go on, the larger stay in the block above
 #pragma unroll
     for (int e = E - 1; e >= 0; --e) {
-        const bool take = before(d.d, id, k.d[e].d, k.id[e]);
+        const int32_t ki = wv_id(T, k.slot[e]);
+        const bool take = before(d.d, id, k.d[e].d, ki);
         typename WvKept<E>::Dbl hd = take ? k.d[e] : d;
-        int32_t hi = take ? k.id[e] : id, hs = take ? k.slot[e] : slot;
+        int32_t hi = take ? ki : id, hs = take ? k.slot[e] : slot;
         d = take ? d : k.d[e];
-        id = take ? id : k.id[e];
+        id = take ? id : ki;
         slot = take ? slot : k.slot[e];
 #pragma unroll 1
         for (int j = 32; j > 0; j >>= 1) {
@@ -273,24 +282,22 @@ __device__ __forceinline__ void wv_merge_exact(WvKept<E> &k, double nd, int32_t 
         }
         if (e + 1 < E) {
             k.d[e + 1 < E ? e + 1 : 0] = hd;
-            k.id[e + 1 < E ? e + 1 : 0] = hi;
             k.slot[e + 1 < E ? e + 1 : 0] = hs;
         }
     }
     k.d[0] = d;
-    k.id[0] = id;
     k.slot[0] = slot;
 }
 
 // Merge cnt entries, staged from sh.d[0] on in any order, into the kept ones.
 template <int E>
-__device__ __forceinline__ void wv_merge(WvKept<E> &k, int cnt, int kh, WvShared<E> &sh, int lane) {
+__device__ __forceinline__ void wv_merge(const DevTree &T, WvKept<E> &k, int cnt, int kh, WvShared<E> &sh, int lane) {
     typedef WvKey<E> Key;
     __syncthreads();
     const bool in = lane < cnt;
     const bool empty = !(lane_d(k.d[0].d, 0) < NBX_MAXVALUE);
     uint32_t v = Key::of(in ? sh.d[lane] : 0.0, in, (uint32_t)lane), x[E], out = ~0u;
-    v = cnt <= 16 ? key_sort_row(v, lane) : key_sort(v, lane);
+    v = cnt <= 16 ? key_sort_row(v, lane) : cnt <= 32 ? key_sort_half(v, lane) : key_sort(v, lane);
 #pragma unroll
     for (int e = E - 1; e >= 0; --e) {
         const uint32_t kk = Key::of(k.d[e].d, k.d[e].d < NBX_MAXVALUE, (uint32_t)(NBX_WAVE * (e + 1) + lane));
@@ -315,18 +322,16 @@ __device__ __forceinline__ void wv_merge(WvKept<E> &k, int cnt, int kh, WvShared
     }
     if (!in) {
         sh.d[lane] = NBX_MAXVALUE;
-        sh.id[lane] = WV_NOID;
         sh.slot[lane] = -1;
     }
     if (tie) {
-        wv_merge_exact(k, sh.d[lane], sh.id[lane], sh.slot[lane], lane);
+        wv_merge_exact(T, k, sh.d[lane], sh.slot[lane], lane);
         __syncthreads();
         return;
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         sh.d[NBX_WAVE * (e + 1) + lane] = k.d[e].d;
-        sh.id[NBX_WAVE * (e + 1) + lane] = k.id[e];
         sh.slot[NBX_WAVE * (e + 1) + lane] = k.slot[e];
     }
     __syncthreads();
@@ -334,7 +339,6 @@ __device__ __forceinline__ void wv_merge(WvKept<E> &k, int cnt, int kh, WvShared
     for (int e = 0; e < E; ++e) {
         const uint32_t t = x[e] & (Key::TAGS - 1);
         k.d[e].d = sh.d[t];
-        k.id[e] = sh.id[t];
         k.slot[e] = sh.slot[t];
     }
     __syncthreads();
@@ -363,11 +367,10 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
         if (staged < WV_MERGE) {
             __syncthreads();
             for (int j = 0; j < staged; ++j)
-                wv_insert(k, readfirst_d(sh.d[j]), __builtin_amdgcn_readfirstlane(sh.id[j]),
-                          __builtin_amdgcn_readfirstlane(sh.slot[j]), lane);
+                wv_insert(T, k, readfirst_d(sh.d[j]), __builtin_amdgcn_readfirstlane(sh.slot[j]), lane);
             __syncthreads();
         } else {
-            wv_merge(k, staged, kh, sh, lane);
+            wv_merge(T, k, staged, kh, sh, lane);
         }
         wv_kth(k, kh);
         staged = 0;
@@ -431,13 +434,17 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
                 // (padding slots lie at 1e300, so their d2 is infinite)
                 uint64_t acc[2] = {ballot(d2[0] <= k.kth) & has, ballot(d2[1] <= k.kth) & has};
                 if (!(acc[0] | acc[1])) continue;
-                const int2 ids = *(const int2 *)((const char *)(T.perm + s0) + ls * 4u);
-                const int32_t id[2] = {ids.x, ids.y};
                 // equally far as the last kept: only a smaller ID counts; the
                 // query itself has d2 == 0
+                const uint64_t tie[2] = {acc[0] & ballot(d2[0] == k.kth), acc[1] & ballot(d2[1] == k.kth)};
+                if (tie[0] | tie[1]) {
+                    const int2 ids = *(const int2 *)((const char *)(T.perm + s0) + ls * 4u);
+                    const int32_t kid = wv_id(T, k.kslot);
+                    acc[0] &= ~tie[0] | ballot(ids.x < kid);
+                    acc[1] &= ~tie[1] | ballot(ids.y < kid);
+                }
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    acc[p] &= ballot(d2[p] < k.kth) | ballot(id[p] < k.kid);
                     if (exz) acc[p] &= ballot(d2[p] > 0.0);
                     const int cnt = __builtin_popcountll(acc[p]);
                     if (cnt == 0) continue;
@@ -446,7 +453,6 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
                         const int at = staged + __builtin_amdgcn_mbcnt_hi((uint32_t)(acc[p] >> 32),
                                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)acc[p], 0));
                         sh.d[at] = d2[p];
-                        sh.id[at] = id[p];
                         sh.slot[at] = sl + p;
                     }
                     staged += cnt;
@@ -494,11 +500,10 @@ __global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int first
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         k.d[e].d = NBX_MAXVALUE;
-        k.id[e] = WV_NOID;
         k.slot[e] = -1;
     }
     k.kth = NBX_MAXVALUE;
-    k.kid = WV_NOID;
+    k.kslot = -1;
     k.lim = wv_lim(k.kth);
 #pragma unroll
     for (int d = 0; d < ND; ++d) q[d] = q0[d];
@@ -534,10 +539,12 @@ __global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int first
             const double qvx = pts ? A.qv[0][qi] : T.x[3][qi], qvy = pts ? A.qv[1][qi] : T.x[4][qi],
                          qvz = pts ? A.qv[2][qi] : T.x[5][qi];
             __shared__ double sv[E * NBX_WAVE];
+            __shared__ int32_t di[E * NBX_WAVE];
             double *dv = sh.d;
-            int32_t *di = sh.id, *ss = sh.slot;
+            int32_t *ss = sh.slot;
             if (!bad) {
                 double v[E];
+                int32_t vi[E];
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
                     const int p = e * NBX_WAVE + lane;
@@ -545,7 +552,8 @@ __global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int first
                     const double vx = qvx - T.x[3][s], vy = qvy - T.x[4][s], vz = qvz - T.x[5][s];
                     v[e] = sqrt(vx * vx + vy * vy + vz * vz);
                     dv[p] = v[e];
-                    di[p] = k.id[e];
+                    vi[e] = T.perm[s];
+                    di[p] = vi[e];
                     sv[p] = v[e];  // (ranks of unordered values, NaN, may leave places unwritten)
                     ss[p] = s;
                 }
@@ -556,7 +564,7 @@ __global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int first
                     if (p >= kh) continue;
                     int r = 0;
                     for (int j = 0; j < kh; ++j)
-                        r += before(dv[j], di[j], v[e], k.id[e]) || (dv[j] == v[e] && di[j] == k.id[e] && j < p) ? 1 : 0;
+                        r += before(dv[j], di[j], v[e], vi[e]) || (dv[j] == v[e] && di[j] == vi[e] && j < p) ? 1 : 0;
                     sv[r] = v[e];
                     ss[r] = k.slot[e];
                 }
@@ -628,7 +636,7 @@ __global__ __launch_bounds__(64) void k_knn_wave(DevTree T, KnnArgs A, int first
         if (t < 0 || t >= A.kout) continue;
         const bool miss = !(k.d[e].d < NBX_MAXVALUE);
         const bool self = miss && A.miss_self;  // (a missing entry that names the query)
-        if (A.nn) A.nn[row * A.kout + t] = self ? (ids ? T.perm[qi] : qi) : miss ? -1 : (ids ? k.id[e] : k.slot[e]);
+        if (A.nn) A.nn[row * A.kout + t] = self ? (ids ? T.perm[qi] : qi) : miss ? -1 : (ids ? T.perm[k.slot[e]] : k.slot[e]);
         if (A.d2) A.d2[row * A.kout + t] = self ? 0.5 * NBX_MAXVALUE : k.d[e].d;
     }
 }
