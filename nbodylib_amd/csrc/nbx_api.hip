@@ -662,13 +662,18 @@ static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t s
 // ------------------------------------------------------------------ precision form
 // Which precision-form searches run on the FP64 kernel with a wave per query
 // (nbx_knn_wave.hip), whose neighbour sets, exact rows and densities are the
-// same.  Rows in key order come from the FP32 kernel alone.  Measured in ms,
-// FP32 lanes / FP64 waves: densities at k = 32 of 4096 particles 0.31 / 0.023,
-// 131072 0.44 / 0.26, 524288 0.74 / 1.02; k = 64 of 1M 3.7 / 2.7, rows 4.2 /
-// 2.1; 6-D at k = 32 524288 4.98 / 3.86, 1M 8.4 / 8.4, k = 64 18.2 / 11.3.
+// same.  Rows in key order come from the FP32 kernel alone.  The line moves with
+// k, whose insertions cost the lanes more.  Measured in ms, FP32 lanes / FP64
+// waves: densities of 0.2M particles k = 8 0.28 / 0.29, k = 32 0.48 / 0.37, of
+// 0.3M k = 20 0.45 / 0.48, k = 32 0.54 / 0.55; rows of 0.2M k = 4 0.26 / 0.22, of
+// 0.3M k = 8 0.31 / 0.33, k = 20 0.43 / 0.38, of 0.4M k = 32 0.56 / 0.55; k = 64
+// of 1M density 3.7 / 2.7, rows 4.2 / 2.1; 6-D 0.5M k = 32 4.98 / 3.9, 1M 8.4 /
+// 8.0, k = 64 18.2 / 11.
 static bool mixed_by_waves(const nbx_tree *t, const KnnArgs &A, int k, int64_t nq) {
-    if (A.nn && !A.d2 && !A.exact_rows) return false;
-    return k > 32 || nq <= (t->nd == 6 ? 1048576 : 262144);
+    const bool rows = A.d2 || A.exact_rows;
+    if (A.nn && !rows) return false;
+    if (k > 32) return true;
+    return nq <= (t->nd == 6 ? 1048576 : rows ? 163840 + 8192 * k : 131072 + 6144 * k);
 }
 
 // FP32 search with the FP64 certificate; queries whose certificate fails are
@@ -690,7 +695,7 @@ static hipError_t run_mixed(nbx_tree *t, KnnArgs A, int k, hipStream_t st, Works
     F.excl_zero = 1;
     if (waves && !ws) {
         t->last_fallbacks.store(nq);
-        return nbx_launch_knn(t->view(), F, (int)nq, st);
+        return nbx_launch_knn_wave(t->view(), F, (int)nq, st);
     }
     std::unique_ptr<ScratchLease> lease;
     if (!ws) {
@@ -706,7 +711,7 @@ static hipError_t run_mixed(nbx_tree *t, KnnArgs A, int k, hipStream_t st, Works
     if (!fb || !mwork) return hipErrorInvalidValue;
     if (waves) {  // (scratch that is too small is refused either way)
         t->last_fallbacks.store(nq);
-        return nbx_launch_knn(t->view(), F, (int)nq, st);
+        return nbx_launch_knn_wave(t->view(), F, (int)nq, st);
     }
     hipError_t e = hipSuccess;
     int32_t *cnt = fb + nfb;

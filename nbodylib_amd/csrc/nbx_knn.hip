@@ -597,14 +597,15 @@ static int knn_resident() {
 // Which kernel serves a search.  A lane per query shares each node and leaf
 // among 64 neighbours and wins for few kept entries over many queries; a wave
 // per query (nbx_knn_wave.hip) keeps its entries in registers and needs few
-// queries to fill the device.  Measured in ms, lanes / waves: 0.5M clustered
-// particles k = 8 0.70 / 0.61, periodic 0.73 / 0.81, density 0.69 / 0.78; 2.1M
-// k = 8 1.79 / 2.25, k = 20 3.79 / 2.90, k = 32 4.70 / 3.30; 8.4M k = 8 density
-// 6.4 / 12.2, k = 32 16.8 / 16.8.  Below 262144 queries the lanes leave CUs
-// idle (131072, k = 8: 0.30 / 0.15).
+// queries to fill the device.  Measured in ms, lanes / waves, density: 0.3M
+// clustered particles k = 1 0.24 / 0.38, k = 4 0.40 / 0.41, k = 8 0.51 / 0.42,
+// k = 17 0.69 / 0.46; 0.5M k = 4 0.49 / 0.68, k = 8 0.59 / 0.72, k = 17 0.77 /
+// 0.79; 1M k = 8 0.91 / 1.44, k = 17 1.24 / 1.60; with room for 33 entries in
+// the lanes' kernel, 2.1M k = 20 3.6 / 3.4, k = 32 4.4 / 3.7.  So the line moves
+// with the entries kept.
 #define KNN_KM 18
 bool nbx_knn_by_waves(int nd, int kh, int qsrc, bool listed, int64_t nqueries) {
-    return nd == 6 || kh > KNN_KM || qsrc == NBX_Q_POINTS || listed || nqueries <= 262144;
+    return nd == 6 || kh > KNN_KM || qsrc == NBX_Q_POINTS || listed || nqueries <= 163840 + 24576 * kh;
 }
 
 static const size_t KNN_CTR_BYTES = 8 * KNN_CTR_STRIDE * sizeof(int32_t);

@@ -345,6 +345,30 @@ __device__ __forceinline__ void wv_merge(const DevTree &T, WvKept<E> &k, int cnt
 }
 #define WV_MERGE 4  // accepted entries from which on a merge takes fewer instructions than insertions
 
+// Before anything is kept more particles are accepted than a merge takes at
+// once.  A distance that at least kh and at most a wave of them lie within,
+// found by bisection, leaves the rest out: they are not among the kh nearest.
+// A few compares instead of a second merge: 2.1M particles, density, k = 32
+// 3.86 -> 3.73 ms; 4096 particles 19 -> 17 us.
+#define WV_CUT 56  // kh up to which it is tried: a narrow target takes too many steps
+__device__ __forceinline__ void wv_cut(const double (&d2)[2], uint64_t (&acc)[2], int kh, int lane) {
+    float top = (acc[0] >> lane) & 1ULL ? (float)d2[0] : 0.0f;
+    top = fmaxf(top, (acc[1] >> lane) & 1ULL ? (float)d2[1] : 0.0f);
+    float lo = 0.0f, hi = __uint_as_float(~wave_umin(~__float_as_uint(top)));
+    for (int i = 0; i < 10; ++i) {
+        const float m = 0.5f * (lo + hi);
+        const uint64_t a = acc[0] & ballot(d2[0] <= (double)m), b = acc[1] & ballot(d2[1] <= (double)m);
+        const int c = __builtin_popcountll(a) + __builtin_popcountll(b);
+        if (c < kh) lo = m;
+        else if (c > NBX_WAVE) hi = m;
+        else {
+            acc[0] = a;
+            acc[1] = b;
+            return;
+        }
+    }
+}
+
 // The walk for one position q.  A node's key is its bound rounded to FP32
 // with the lane in the lowest bits: its least is the nearest node, and a node
 // whose key is above lim cannot hold a neighbour.
@@ -443,9 +467,15 @@ __device__ __forceinline__ void wv_walk(const DevTree &T, const double (&q)[ND],
                     acc[0] &= ~tie[0] | ballot(ids.x < kid);
                     acc[1] &= ~tie[1] | ballot(ids.y < kid);
                 }
+                if (exz) {
+                    acc[0] &= ballot(d2[0] > 0.0);
+                    acc[1] &= ballot(d2[1] > 0.0);
+                }
+                if (!(k.kth < NBX_MAXVALUE) && kh <= WV_CUT &&
+                    __builtin_popcountll(acc[0]) + __builtin_popcountll(acc[1]) > NBX_WAVE)
+                    wv_cut(d2, acc, kh, lane);
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    if (exz) acc[p] &= ballot(d2[p] > 0.0);
                     const int cnt = __builtin_popcountll(acc[p]);
                     if (cnt == 0) continue;
                     if (staged + cnt > NBX_WAVE) flush();

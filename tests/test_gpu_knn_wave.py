@@ -93,21 +93,22 @@ def test_phase_rows(gpu, n):
 @pytest.mark.parametrize("k", [1, 4, 5, 12, 13, 17, 18])
 @pytest.mark.parametrize("kind", ["clustered", "lattice"])
 def test_lane_per_query(gpu, kind, k):
-    """Past 262144 queries at most 18 kept entries are searched with a lane per
-    query; a list of the same particles still runs with a wave per query."""
+    """Past 606208 queries (fewer for fewer entries) at most 18 kept entries are
+    searched with a lane per query; a list of the same particles still runs with
+    a wave per query."""
     import torch
     import nbodylib_amd as nb
     from nbodylib_amd.device import DeviceTree
 
-    ax = np.arange(65.0)
+    ax = np.arange(85.0)
     if kind == "lattice":
         pos = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3)
         pos = pos[np.random.default_rng(1).permutation(len(pos))]
     else:
-        pos = datagen.clustered(262145 + 37, 1.0, nhalo=60, seed=5)[0]
+        pos = datagen.clustered(606208 + 37, 1.0, nhalo=60, seed=5)[0]
     n = len(pos)
     print(f"lane per query {kind} n={n} k={k}", flush=True)
-    period = 65.0 if kind == "lattice" else 1.0
+    period = 85.0 if kind == "lattice" else 1.0
     t = nb.KDTree(pos, kerntype=nb.KSPH, period=period)
     every = np.arange(n, dtype=np.int32)
     for per in (False, True):
