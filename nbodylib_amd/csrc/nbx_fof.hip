@@ -728,12 +728,18 @@ __global__ __launch_bounds__(256) void k_fof_begin(const int32_t *P, int64_t n, 
 }
 // Every particle's root, stored as its parent (no links are made any more;
 // the find stores nothing on its way, so no stale grandparent can follow).
-// Neighbouring slots mostly share a root, so the lanes whose root equals the
-// first such lane's are summed in the wave and counted with one atomic pair;
-// the rest count alone.
-__global__ __launch_bounds__(256) void k_fof_compress(int32_t *P, int64_t n, const int32_t *perm, int32_t *cnt,
-                                                      int32_t *minid) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// Neighbouring slots mostly share a root: the lanes of a wave that share one
+// are summed in the wave, for up to FOF_SUMS roots, and where the first of a
+// block's waves agree, as in the large halos, in the block, so that one
+// counter is not met by every wave of a halo.  Finishing 16.8M particles with
+// one root summed per wave 0.44 ms, in blocks 0.34, with four roots 0.23.
+#define FOF_CB 1024
+#define FOF_SUMS 4
+__global__ __launch_bounds__(FOF_CB) void k_fof_compress(int32_t *P, int64_t n, const int32_t *perm, int32_t *cnt,
+                                                         int32_t *minid) {
+    __shared__ int32_t wr[FOF_CB / NBX_WAVE], wn[FOF_CB / NBX_WAVE], wm[FOF_CB / NBX_WAVE];
+    const int64_t i = (int64_t)blockIdx.x * FOF_CB + threadIdx.x;
+    const int lane = threadIdx.x & 63, w = threadIdx.x / NBX_WAVE;
     const bool in = i < n;
     int32_t r = in ? P[i] : -1;
     if (in) {
@@ -741,23 +747,41 @@ __global__ __launch_bounds__(256) void k_fof_compress(int32_t *P, int64_t n, con
     }
     const bool add = in && r != i;
     if (add) P[i] = r;
-    const uint64_t act = ballot(add);
-    if (!act) return;
+    uint64_t rest = ballot(add);
     const int32_t id = add ? perm[i] : 0x7fffffff;
-    const int lead = __builtin_ctzll(act);
-    const int32_t r0 = __shfl(r, lead);
-    const bool same = add && r == r0;
-    const uint64_t m = ballot(same);
-    int32_t mn = same ? id : 0x7fffffff;
+    if (lane == 0) wr[w] = -1;
+    for (int s = 0; s < FOF_SUMS && rest; ++s) {
+        const int32_t r0 = __builtin_amdgcn_readlane(r, __builtin_ctzll(rest));
+        const bool same = add && r == r0;
+        const uint64_t m = ballot(same);
+        rest &= ~m;
+        int32_t mn = same ? id : 0x7fffffff;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mn = min(mn, __shfl_xor(mn, off));
-    if ((int)(threadIdx.x & 63) == lead) {
-        atomicAdd(cnt + r0, (int32_t)__popcll(m));
-        atomicMin(minid + r0, mn);
+        for (int off = 32; off > 0; off >>= 1) mn = min(mn, __shfl_xor(mn, off));
+        if (lane != 0) continue;
+        if (s == 0) {
+            wr[w] = r0;
+            wn[w] = __popcll(m);
+            wm[w] = mn;
+        } else {
+            atomicAdd(cnt + r0, (int32_t)__popcll(m));
+            atomicMin(minid + r0, mn);
+        }
     }
-    if (add && !same) {
+    if ((rest >> lane) & 1ULL) {
         atomicAdd(cnt + r, 1);
         atomicMin(minid + r, id);
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < FOF_CB / NBX_WAVE && wr[t] >= 0 && (t == 0 || wr[t - 1] != wr[t])) {
+        int32_t c = wn[t], mn = wm[t];
+        for (int v = t + 1; v < FOF_CB / NBX_WAVE && wr[v] == wr[t]; ++v) {
+            c += wn[v];
+            mn = min(mn, wm[v]);
+        }
+        atomicAdd(cnt + wr[t], c);
+        atomicMin(minid + wr[t], mn);
     }
 }
 // Groups of at least minnum members; every other root's label is 0.  A block
@@ -1043,7 +1067,8 @@ hipError_t nbx_fof_canonical(const DevTree &T, int32_t *P, int32_t minnum, int32
     {
         ProfScope ps("k_fof_finish", st);
         hipLaunchKernelGGL(k_fof_begin, dim3(nblk(n)), dim3(256), 0, st, P, n, T.perm, cnt, minid, ng);
-        hipLaunchKernelGGL(k_fof_compress, dim3(nblk(n)), dim3(256), 0, st, P, n, T.perm, cnt, minid);
+        hipLaunchKernelGGL(k_fof_compress, dim3((unsigned)((n + FOF_CB - 1) / FOF_CB)), dim3(FOF_CB), 0, st, P, n,
+                           T.perm, cnt, minid);
     }
     {
         hipLaunchKernelGGL(k_fof_collect, dim3((unsigned)((n + FOF_COLLECT - 1) / FOF_COLLECT)), dim3(256), 0, st, P, cnt,

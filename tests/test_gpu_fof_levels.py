@@ -65,3 +65,26 @@ def test_deeper_trees(gpu, n):
         raw, _ = ot.fof(b, 5)
         ol, og = oracle.fof_canonical(raw, 5)
         assert ng == og and np.array_equal(lab, ol)
+
+
+@pytest.mark.parametrize("size", [2, 3, 12, 13, 70, 5000])
+def test_group_sums(gpu, size):
+    """Sizes and smallest IDs where a wave of 64 particles holds more groups
+    than it sums, a few, and a part of one: n / size tight groups far apart."""
+    import nbodylib_amd as nb
+
+    n = 15000 // size * size
+    print(f"group sums size={size} n={n}", flush=True)
+    rng = np.random.default_rng(size)
+    ng = n // size
+    centre = np.stack(np.unravel_index(rng.permutation(8000)[:ng], (20, 20, 20)), -1).astype(float)
+    group = rng.permutation(np.repeat(np.arange(ng), size))  # members of a group all over the IDs
+    pos = centre[group] + rng.uniform(-0.01, 0.01, (n, 3))
+    lab, got = nb.KDTree(pos, kerntype=nb.KSPH).FOF(0.1, 2)
+    assert got == ng
+    # equal sizes: numbered by smallest member
+    first = np.full(ng, n)
+    np.minimum.at(first, group, np.arange(n))
+    want = np.empty(ng, dtype=np.int64)
+    want[np.argsort(first)] = np.arange(1, ng + 1)
+    assert np.array_equal(lab, want[group])
