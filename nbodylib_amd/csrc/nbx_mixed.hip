@@ -52,6 +52,7 @@
 typedef float fx8 __attribute__((ext_vector_type(8)));
 typedef const __attribute__((address_space(4))) fx8 *cf8ptr;
 
+#define MX_PLOG 5  // a wave's queries go to at most 32 waves
 #define MX_U 5.9604644775390625e-8  // 2^-24
 #define MX_DB 4               // neighbours gathered together in the density pass
 #define MX_EMPTY 0x7F7FFFFFu  // empty kept entry: the bits of FLT_MAX
@@ -798,7 +799,7 @@ __device__ __forceinline__ int verify_walk(const DevTree &T, const double *q, bo
 template <int ND, int KMAX, int MODE>
 __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, const double *ext, int32_t *fb_list,
                                          int32_t *fb_count, uint32_t *hk, float *cx, double *racc, uint32_t *sl,
-                                         uint32_t *slb, uint32_t *skc, int g, int lane) {
+                                         uint32_t *slb, uint32_t *skc, int g, int part, int plog, int lane) {
     constexpr bool GT = GShape<KMAX>::GT;
     constexpr uint32_t TM = GShape<KMAX>::TM;
     uint32_t *const kb = GT ? hk : skc;
@@ -822,14 +823,19 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
     asm volatile("" : "+s"(kh));
     const int k = kh - 1;
     const int qi = g * NBX_WAVE + lane;
-    const bool valid = qi < T.n;
+    const bool valid = qi < T.n && lane >> (6 - plog) == part;
     const int kres = T.kernres;
     MixCtx<ND> c;
-    // A lane past the end queries from the padding sentinel: node boxes
+    // A lane past the end, or of another part, queries from the padding sentinel: node boxes
     // bound real particles only, so every box bound from there is +inf and
     // the walk needs no activity test (the leaf code still masks the lane).
+    float qc[ND];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) c.q[d] = valid ? T.x[d][qi] : NBX_PAD_COORD;
+    for (int d = 0; d < ND; ++d) {
+        const double x = qi < T.n ? T.x[d][qi] : NBX_PAD_COORD;
+        qc[d] = (float)readfirst_d(x);  // the order of the walk is the whole wave's
+        c.q[d] = valid ? x : NBX_PAD_COORD;
+    }
     c.act = valid;
     c.self = qi;
     c.root = 0u;
@@ -843,9 +849,6 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
     if (lane == 0) vt[0] = (uint32_t)(2 * g);
     c.nvis = 0;
     c.fillkh = (GT && kh >= NBX_LEAF) ? kh : 0;
-    float qc[ND];
-#pragma unroll
-    for (int d = 0; d < ND; ++d) qc[d] = (float)readfirst_d(c.q[d]);
     mix_walk<ND, KMAX>(T, ext, c, qc, T.nleafp + 2 * g, hk, sl, cx, lane, gm);
 
     // ---------------------------------------------------------------- band
@@ -1099,7 +1102,7 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
         if (A.hout) A.hout[A.hout_by_id ? T.perm[qi] : qi] = hi;
     }
     __syncthreads();
-    if (sym && valid) unsafeAtomicAdd(A.rho + qi, racc_own + racc[lane]);
+    if (sym && (valid || (qi < T.n && racc[lane] != 0.0))) unsafeAtomicAdd(A.rho + qi, racc_own + racc[lane]);
 
     // ---------------------------------------------------------------- outputs
     if constexpr (MODE == MX_SPLINE) return;
@@ -1219,7 +1222,7 @@ __device__ __forceinline__ void mix_task(const DevTree &T, const KnnArgs &A, con
 template <int ND, int KMAX, int MODE>
 __global__ __launch_bounds__(64, ND == 6 && KMAX == 33 ? 4 : 1)
 void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list, int32_t *fb_count, uint32_t *scratch,
-                 int32_t *ctr) {
+                 int32_t *ctr, int plog) {
     __shared__ uint32_t hk[KMAX * NBX_WAVE];
     // one buffer for three uses at different times: the leaf copy (phase 2),
     // the compacted queries and their masks (6-D node tests and phase 1) and
@@ -1235,7 +1238,7 @@ void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list, int3
     // scalar base would be reloaded from its spill slot at every handle store
     asm volatile("" : "+v"(sl));
     uint32_t *slb = sl + KMAX * (NBX_WAVE / 2) + MX_V, *skc = slb + KMAX * NBX_WAVE;
-    const int nw = A.wcnt > 0 ? A.wcnt : (T.n + NBX_WAVE - 1) / NBX_WAVE;
+    const int nw = (A.wcnt > 0 ? A.wcnt : (T.n + NBX_WAVE - 1) / NBX_WAVE) << plog;
     const int x = blockIdx.x & 7, q8 = nw >> 3, r8 = nw & 7;
     for (int s = 0; s < 8; ++s) {
         const int y = (x + s) & 7;
@@ -1245,7 +1248,9 @@ void k_knn_mixed(DevTree T, KnnArgs A, const double *ext, int32_t *fb_list, int3
             if (lane == 0) t = atomicAdd(ctr + y * MX_CTR_STRIDE, 1);
             t = __builtin_amdgcn_readfirstlane(__shfl(t, 0));
             if (t >= ycnt) break;
-            mix_task<ND, KMAX, MODE>(T, A, ext, fb_list, fb_count, hk, cx, racc, sl, slb, skc, A.wbeg + ybeg + t, lane);
+            const int v = ybeg + t;
+            mix_task<ND, KMAX, MODE>(T, A, ext, fb_list, fb_count, hk, cx, racc, sl, slb, skc, A.wbeg + (v >> plog),
+                                     v & ((1 << plog) - 1), plog, lane);
         }
     }
 }
@@ -1300,9 +1305,20 @@ hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double
     const int km = A.kh <= 33 ? 33 : 65;
     const int mode = mx_mode(A);
     // densities and exact rows do not come together; the spline is 3-D; both keep at most 33
-    if ((mode != MX_TABLE && km > 33) || (mode == MX_EXACT && A.dens != NBX_DO_NONE) || (mode == MX_SPLINE && (T.nd != 3 || A.nn || A.d2)))
+    if ((mode != MX_TABLE && km > 33) || (mode == MX_EXACT && A.dens != NBX_DO_NONE) ||
+        (mode == MX_SPLINE && (T.nd != 3 || A.nn || A.d2)))
         return hipErrorInvalidValue;
     const int grid = mx_launch_grid(T.nd, km, mode);
+    // Few waves leave the device idle while each works through the union of
+    // its queries' neighbourhoods, so a wave's 64 queries are split among as
+    // many waves as there is room for.  The walk keeps the whole wave's order,
+    // so every lane meets its candidates as before and the rows are the same.
+    // Rows and density of 4096 clustered particles, k = 32, 0.26 -> 0.18 ms (a
+    // query per wave: 0.22), of 10001 0.40 -> 0.25, of 32768 0.37 -> 0.33, 6-D
+    // 1.65 -> 1.21; from 65536 on no difference in 3-D.
+    int plog = 0;
+    while (plog < MX_PLOG && ((int64_t)nw << (plog + 1)) <= grid) ++plog;
+    const int ngrid = (int)std::min<int64_t>(grid, (((int64_t)nw << plog) + 7) & ~(int64_t)7);
     const size_t nscr = (size_t)grid * MX_BLKW(km);
     const size_t need = nscr * sizeof(uint32_t) + 8 * MX_CTR_STRIDE * sizeof(int32_t);
     void *mem = work;
@@ -1319,8 +1335,8 @@ hipError_t nbx_launch_knn_mixed(const DevTree &T, const KnnArgs &A, const double
     {
         ProfScope ps("k_knn_mixed", st);
 #define MIXL(ND, KM, MODE)                                                                                       \
-    hipLaunchKernelGGL((k_knn_mixed<ND, KM, MODE>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, ext, fallback_list, \
-                       fallback_count, scr, ctr)
+    hipLaunchKernelGGL((k_knn_mixed<ND, KM, MODE>), dim3(ngrid), dim3(NBX_WAVE), 0, st, T, A, ext, fallback_list, \
+                       fallback_count, scr, ctr, plog)
         if (T.nd == 3) {
             if (km == 65) MIXL(3, 65, MX_TABLE);
             else if (mode == MX_TABLE) MIXL(3, 33, MX_TABLE);
