@@ -1108,11 +1108,12 @@ static int smooth_impl(nbx_tree *t, int32_t k, const double *rho_by_id, const do
     const bool need_disp = disp_out || moments;
     hipStream_t st = nullptr;
     int32_t *nn = nullptr;
-    double *rid = nullptr, *hid = nullptr, *mean = nullptr, *disp = nullptr, *mom = nullptr, *buf = nullptr;
+    double *rid = nullptr, *hid = nullptr, *hs = nullptr, *mean = nullptr, *disp = nullptr, *mom = nullptr, *buf = nullptr;
     SmoothRec *rec = nullptr;
     HIPCK(bufs.alloc(&nn, sizeof(int32_t) * (size_t)n * k));
     HIPCK(bufs.alloc(&rid, sizeof(double) * n));
     HIPCK(bufs.alloc(&hid, sizeof(double) * n));
+    HIPCK(bufs.alloc(&hs, sizeof(double) * n));
     HIPCK(bufs.alloc(&rec, sizeof(SmoothRec) * n));
     HIPCK(bufs.alloc(&mean, sizeof(double4) * n));
     if (need_disp) HIPCK(bufs.alloc(&disp, sizeof(SmoothSum) * n));
@@ -1122,7 +1123,8 @@ static int smooth_impl(nbx_tree *t, int32_t k, const double *rho_by_id, const do
     hipError_t e = hipSuccess;
     if (rc == NBX_OK) {
         if (rho_by_id) e = hipMemcpy(rid, rho_by_id, sizeof(double) * n, hipMemcpyHostToDevice);
-        if (e == hipSuccess) hipLaunchKernelGGL(k_smooth_pack, dim3(nblk(n)), dim3(256), 0, st, t->view(), rid, hid, rec);
+        if (e == hipSuccess) hipLaunchKernelGGL(k_smooth_pack, dim3(nblk(n)), dim3(256), 0, st, t->view(), rid, hid, rec,
+                                              hs);
         if (e == hipSuccess) {
             if (mean_in) e = upload_rows(t, mean_in, 3, buf, 4, mean);
             else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(4 * n)), dim3(256), 0, st, mean, 0.0, 4 * n);
@@ -1134,7 +1136,7 @@ static int smooth_impl(nbx_tree *t, int32_t k, const double *rho_by_id, const do
         if (e == hipSuccess && moments)
             hipLaunchKernelGGL(k_fill_f64, dim3(nblk(8 * n)), dim3(256), 0, st, mom, 0.0, 8 * n);
         if (e == hipSuccess) {
-            SmoothArgs A = {nn, k, rec, (double4 *)mean, (SmoothSum *)disp, (SmoothSum *)mom};
+            SmoothArgs A = {nn, k, rec, hs, (double4 *)mean, (SmoothSum *)disp, (SmoothSum *)mom};
             e = nbx_launch_smooth(t->view(), A, mean_in == nullptr, need_disp && disp_in == nullptr, st);
         }
         struct Out {

@@ -167,7 +167,7 @@ hipError_t nbx_point_order(const DevTree &T, const PointCoords &q, int64_t m, in
 
 // ------------------------------------------------------------------ smoothed velocities
 struct SmoothRec {
-    double4 x, v;  // position and mass / density; velocity and h
+    double4 x, v;  // position and mass; velocity and density
 };
 struct SmoothSum {
     double c[8];  // dispersion: xx xy xz yy yz zz; moments: skewness, kurtosis
@@ -177,11 +177,12 @@ struct SmoothArgs {
     const int32_t *nn;  // n x k neighbour slots, rows by slot
     int32_t k;
     const SmoothRec *rec;  // by slot
+    const double *h;       // by slot
     double4 *mean;         // smoothed velocity by slot; zeroed by the caller, as the sums below
     SmoothSum *disp;       // dispersion by slot, or null
     SmoothSum *mom;        // moments by slot, or null
 };
-__global__ void k_smooth_pack(DevTree T, const double *rho_by_id, const double *h_by_id, SmoothRec *rec);
+__global__ void k_smooth_pack(DevTree T, const double *rho_by_id, const double *h_by_id, SmoothRec *rec, double *h);
 __global__ void k_smooth_in(const double *rows, const int32_t *perm, int64_t n, int w, int ncomp, double *out);
 // with_mean / with_disp: compute those first (else A.mean / A.disp hold the
 // caller's); the moments run when A.mom is set.

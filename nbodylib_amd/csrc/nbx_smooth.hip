@@ -36,17 +36,18 @@ __device__ __forceinline__ double smooth_d2(const DevTree &T, const double *xi, 
     return s;
 }
 
-// Records by slot of what a particle gives: position and mass / density;
-// velocity and h.
+// Records by slot of what a particle gives: position and mass, velocity and
+// density; and its h.
 __global__ __launch_bounds__(256) void k_smooth_pack(DevTree T, const double *rho_by_id, const double *h_by_id,
-                                                     SmoothRec *rec) {
+                                                     SmoothRec *rec, double *h) {
     const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (s >= T.n) return;
     const int64_t id = T.perm[s];
     SmoothRec r;
-    r.x = make_double4(T.x[0][s], T.x[1][s], T.x[2][s], T.mass[s] / rho_by_id[id]);
-    r.v = make_double4(T.x[3][s], T.x[4][s], T.x[5][s], h_by_id[id]);
+    r.x = make_double4(T.x[0][s], T.x[1][s], T.x[2][s], T.mass[s]);
+    r.v = make_double4(T.x[3][s], T.x[4][s], T.x[5][s], rho_by_id[id]);
     rec[s] = r;
+    h[s] = h_by_id[id];
 }
 
 // Blocks of SM_B consecutive slots: a share for a particle of the same block
@@ -121,8 +122,8 @@ __global__ __launch_bounds__(SM_B) void k_smooth(DevTree T, SmoothArgs A, double
     for (int c = 0; c < NC; ++c) acc[c] = 0.0;
     const int k = A.k;
     const int32_t *row = A.nn + (valid ? i : 0) * k;
-    const double4 xi = A.rec[valid ? i : 0].x, vh = A.rec[valid ? i : 0].v;
-    const double vi[3] = {vh.x, vh.y, vh.z}, hi = vh.w, mi = xi.w;
+    const double4 xi = A.rec[valid ? i : 0].x, vr = A.rec[valid ? i : 0].v;
+    const double vi[3] = {vr.x, vr.y, vr.z}, hi = A.h[valid ? i : 0], mi = xi.w, rhoi = vr.w;
     const double norm = 1.0 / pow(hi, 3.0);
     double ui[3], si[3], pi[3];
     if (STAGE != SM_VEL) {
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(SM_B) void k_smooth(DevTree T, SmoothArgs A, double
             const double dx = xi.x - xj[u].x, dy = xi.y - xj[u].y, dz = xi.z - xj[u].z;
             const double rij = sqrt(dx * dx + dy * dy + dz * dz);
             const double w = 0.5 * wsm_at(rij, hi, T.kern, T.kernres) * norm;
-            const double tj = w * xj[u].w, ti = w * mi;
+            const double tj = w / vj[u].w * xj[u].w, ti = w / rhoi * mi;
             const double wj[3] = {vj[u].x, vj[u].y, vj[u].z};
             double v[NC];  // the neighbour's share
             if constexpr (STAGE == SM_VEL) {
