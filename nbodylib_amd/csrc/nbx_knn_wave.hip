@@ -30,10 +30,10 @@
 // the query's own entry is sorted out after something was accepted): 6-D, 0.5M,
 // k = 64 5.68 -> 5.4 ms.
 // Measured, a lane per query -> this: 4096 particles, k = 32, periodic 266 ->
-// 27 us; 100k positions among 1M particles 6.17 -> 0.59 ms; 2.1M clustered
-// particles, density at k = 32 4.5 -> 4.2 ms; 0.5M particles k = 64 3.8 ->
-// 1.05, k = 128 17.7 -> 2.1 ms; 6-D 0.5M k = 32 21.7 -> 4.2 ms, 2.1M k = 64
-// (from the FP32 form) 36 -> 23 ms.
+// 23 us; 100k positions among 1M particles 6.17 -> 0.52 ms; 2.1M clustered
+// particles, density at k = 32 4.5 -> 3.9 ms; 0.5M particles k = 64 3.8 -> 1.0,
+// k = 128 17.7 -> 2.0 ms; 6-D 0.5M k = 32 21.7 -> 3.9 ms, 2.1M k = 64 (from the
+// FP32 form) 36 -> 22 ms.
 #include <algorithm>
 
 #include "nbx_kernels.h"
