@@ -101,9 +101,9 @@ int nbx_tree_create(const nbx_params *p, const double *pos, const double *vel, c
 int nbx_tree_create_dev(const nbx_params *p, const double *pos_dev, const double *vel_dev, const double *mass_dev,
                         int64_t n, void *stream, nbx_tree **out);
 /* Replaces KDTree::~KDTree (KDTree.cxx:1340-1356); caller-side reorder is the
- * shim's job.  Waits for work still running on the device (as hipFree does),
- * so no launch on any stream may still be using the tree.  Its memory is kept
- * for the next tree (see below) or freed. */
+ * shim's job.  Waits for work still running on the tree's device (as hipFree
+ * does), whichever device is current, so no launch on any stream may still be
+ * using the tree.  Its memory is kept for the next tree (see above) or freed. */
 int nbx_tree_destroy(nbx_tree *t);
 /* slot -> ID map (host array of n).  The C++ shim uses it to reorder the
  * caller's Particle array as the reference does in BuildNodes. */

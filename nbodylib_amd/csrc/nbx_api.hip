@@ -84,6 +84,19 @@ static void drop_block(KeptBlocks &k, int dev, size_t i) {
     hipEventDestroy(b.used);
     hipFree(b.p);
 }
+// The current device is dev while this lives.
+struct OnDevice {
+    int was = -1;
+    explicit OnDevice(int dev) {
+        int cur = 0;
+        if (dev >= 0 && hipGetDevice(&cur) == hipSuccess && cur != dev && hipSetDevice(dev) == hipSuccess) was = cur;
+    }
+    ~OnDevice() {
+        if (was >= 0) hipSetDevice(was);
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+};
 // *got bytes (at least need) at *p, for work on st from now on
 static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) {
     *p = nullptr;
@@ -125,13 +138,14 @@ static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) 
     *got = bytes;
     return e;
 }
-// st: the stream of the block's last use
+// st: the stream of the block's last use, on the block's device (null: that
+// device's null stream, whichever device is current)
 static void block_put(void *p, size_t bytes, hipStream_t st) {
     if (!p) return;
-    int dev = 0;
+    int dev = -1;
     hipPointerAttribute_t at;
     if (hipPointerGetAttributes(&at, p) == hipSuccess) dev = at.device;
-    else dev = -1;
+    const OnDevice on(dev);
     hipEvent_t ev = nullptr;
     if (dev >= 0 && dev < NBX_MAX_DEVICES) {
         KeptBlocks &k = kept_blocks();
@@ -262,6 +276,7 @@ extern "C" int nbx_prof_get(const char *name, double *ms, int64_t *launches) {
 struct nbx_tree {
     nbx_params p;
     int64_t n;
+    int dev = -1;  // the device the tree was built on
     int nd;        // tree dimensionality (3 or 6)
     bool has_vel;  // TPHYS tree that also keeps sorted velocities (x[3..5])
     bool tvel;     // TVEL: the tree's coordinates are the velocities
@@ -362,10 +377,18 @@ static inline int nblk(int64_t n, int b = 256) { return (int)((n + b - 1) / b); 
 
 static void free_tree(nbx_tree *t) {
     if (!t) return;
-    // no stream may still be using the tree (hipFree used to wait for that)
-    if (t->mem || t->scr) hipDeviceSynchronize();
-    block_put(t->mem, t->mem_bytes, nullptr);
-    block_put(t->scr, t->scr_cap, nullptr);
+    // The blocks are handed to other streams of the tree's device next, so no
+    // work there may still be using them: wait for that device, not for the
+    // caller's.  Where the wait is refused (a capture in progress) they are
+    // freed instead of kept.
+    const OnDevice on(t->dev);
+    if (!(t->mem || t->scr) || hipDeviceSynchronize() == hipSuccess) {
+        block_put(t->mem, t->mem_bytes, nullptr);
+        block_put(t->scr, t->scr_cap, nullptr);
+    } else {
+        hipFree(t->mem);
+        hipFree(t->scr);
+    }
     if (t->scr_done) hipEventDestroy(t->scr_done);
     delete t;
 }
@@ -528,6 +551,7 @@ extern "C" int nbx_tree_create_dev(const nbx_params *p, const double *pos, const
     t->p = *p;
     if (t->p.recheck_rel <= 0) t->p.recheck_rel = 1e-5;
     t->n = n;
+    if (hipGetDevice(&t->dev) != hipSuccess) t->dev = -1;
     t->nd = p->treetype == NBX_TPHS ? 6 : 3;
     t->tvel = tvel;
     t->has_vel = (t->nd == 3 && !tvel && vel != nullptr);

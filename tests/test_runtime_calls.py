@@ -1,0 +1,31 @@
+"""What the library's host code asks of the HIP runtime, from the log of
+tests/cpp/fake_hip, which runs it over a runtime that runs nothing: devices,
+streams, events, allocations and launches, without a GPU."""
+import os
+import subprocess
+
+PROG = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "fake_hip")
+
+
+def log(*args):
+    r = subprocess.run([PROG, *map(str, args)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    return r.stdout.splitlines()
+
+
+def test_tree_freed_with_another_device_current():
+    """The tree of device 1 is freed with device 0 current: the wait and the
+    kept blocks' events belong to device 1, and device 0 is current again."""
+    got = log("other_device", 300000, 4)
+    assert "device_sync dev 1" in got
+    records = [x for x in got if x.startswith("record")]
+    assert records and all(x.startswith("record dev 1") for x in records)
+    assert "current dev 0" in got
+
+
+def test_tree_freed_during_a_capture():
+    """Where the device may not be waited for, nothing is kept: the blocks'
+    last uses are not known to have ended."""
+    got = log("other_device_capturing", 300000, 4)
+    assert sum(x.startswith("free dev 1") for x in got) == 2  # the tree's arrays and its scratch
+    assert not any(x.startswith("record") for x in got)
