@@ -17,15 +17,17 @@
  * these cases (KDCalcSmoothQuantities.cxx:205-207, :273-276,
  * PriorityQueue.h:49-53, KDTree.cxx:1096-1105).
  *
- * Scratch kept by a tree: the searches, the density passes and FOF take
- * their device temporaries from one block that the tree keeps from call to
- * call, so repeated calls allocate nothing after the first.
+ * Scratch kept by a tree: the density passes, the precision-form searches
+ * and FOF take their device temporaries from one block that the tree keeps
+ * from call to call, so repeated calls allocate nothing after the first.
  * The block grows to the largest need seen (searches: up to about 100 MB,
  * less for few queries, plus 4 bytes per particle in the precision form;
  * densities: 8 bytes per particle more; FOF: 16 bytes per particle and 24
  * per possible group of minnum members) and is freed by
  * nbx_tree_destroy.  Calls on one tree from several threads or streams take
  * turns with the block; each waits on the device for the previous one's use.
+ * The FP64 searches need none, or a block of their own (up to about 100 MB,
+ * from the kept memory below), and wait for nothing.
  *
  * Device memory kept by the library: blocks given back by trees and calls are
  * kept for later ones, at most 1/64 of the device's memory in all (4.5 GiB of

@@ -51,13 +51,16 @@ extern "C" int nbx_host_fail(int code, const char *msg) { return fail(code, msg)
 //    past that the oldest blocks are freed, and larger blocks are never kept.
 //    When an allocation fails every kept block is freed and it is tried again.
 //  * Streams: a block goes back with an event recorded on the stream that last
-//    used it, and the next user's stream waits for that event.
+//    used it, and the next user's stream waits for that event.  A block whose
+//    event has not come yet is given to the same stream only, so no stream
+//    waits for another.
 //  * Threads: one mutex around the lists.
 // Nothing here is called under stream capture (every caller synchronises).
 struct KeptBlock {
     void *p;
     size_t bytes;
     hipEvent_t used;
+    hipStream_t st;  // of the last use
 };
 #define NBX_MAX_DEVICES 64
 struct KeptBlocks {
@@ -109,9 +112,15 @@ static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) 
         std::lock_guard<std::mutex> lk(k.mu);
         std::vector<KeptBlock> &f = k.free[dev];
         size_t best = f.size();
-        for (size_t i = 0; i < f.size(); ++i)  // the smallest that fits, the latest of equals
-            if (f[i].bytes >= bytes && f[i].bytes <= bytes + bytes / 2 && (best == f.size() || f[i].bytes <= f[best].bytes))
-                best = i;
+        for (size_t i = 0; i < f.size(); ++i) {  // the smallest that fits, the latest of equals
+            if (f[i].bytes < bytes || f[i].bytes > bytes + bytes / 2) continue;
+            if (best < f.size() && f[i].bytes > f[best].bytes) continue;
+            if (f[i].st != st && hipEventQuery(f[i].used) != hipSuccess) {
+                (void)hipGetLastError();  // not ready is no error
+                continue;
+            }
+            best = i;
+        }
         if (best < f.size()) {
             const KeptBlock b = f[best];
             e = hipStreamWaitEvent(st, b.used, 0);
@@ -157,7 +166,7 @@ static void block_put(void *p, size_t bytes, hipStream_t st) {
         if (bytes <= k.limit[dev] && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) {
             if (hipEventRecord(ev, st) == hipSuccess) {
                 while (k.total[dev] + bytes > k.limit[dev]) drop_block(k, dev, 0);
-                k.free[dev].push_back({p, bytes, ev});
+                k.free[dev].push_back({p, bytes, ev, st});
                 k.total[dev] += bytes;
                 return;
             }
@@ -659,27 +668,29 @@ static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed, int32_t
     return dry.used;
 }
 
-// The FP64 search with its scratch from ws (as much of it as is left), or
-// from the tree's kept scratch when ws is null.
+// The FP64 search with its scratch from ws (as much of it as is left), or a
+// block of its own when ws is null: searches on several streams do not take
+// turns, as they would with the tree's one block.
 static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t st, Workspace *ws = nullptr) {
     if (nq <= 0) return hipSuccess;
     const bool listed = A.qsrc != NBX_Q_POINTS && A.qlist;
     size_t need = nbx_knn_scratch_bytes(t->nd, A.kh, A.qsrc, listed, nq);
     if (need == 0) return nbx_launch_knn(t->view(), A, nq, st);
     // under capture the launcher allocates for itself, as part of the graph: a
-    // replay must not meet later calls in the tree's block
+    // replay must not meet later calls in a block given back
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (!ws && st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
         return nbx_launch_knn(t->view(), A, nq, st);
-    std::unique_ptr<ScratchLease> lease;
-    if (!ws) {
-        lease.reset(new ScratchLease(t, need, st));
-        if (lease->err != hipSuccess) return lease->err;
-        ws = &lease->ws;
+    DevBufs own(st);
+    void *work = nullptr;
+    if (ws) {
+        need = std::min(need, ws->left());
+        work = ws->carve<void>(need);
+        if (!work) return hipErrorInvalidValue;
+    } else {
+        const hipError_t e = own.alloc(&work, need);
+        if (e != hipSuccess) return e;
     }
-    need = std::min(need, ws->left());
-    void *work = ws->carve<void>(need);
-    if (!work) return hipErrorInvalidValue;
     return nbx_launch_knn(t->view(), A, nq, st, work, need);
 }
 

@@ -231,6 +231,7 @@ int main(int argc, char **argv) {
         // a tree of device 1, searched on a stream there, freed with device 0 current
         hipSetDevice(1);
         nbx_tree *t = tree(n, 0, A);
+        nbx_density_dev(t, k, NBX_DENS_SYMMETRIC, 0, (double *)64, nullptr, A);
         nbx_knn_dev(t, k, NBX_KNN_NONPERIODIC, 0, OUT, nullptr, A);
         hipSetDevice(0);
         g_fail_sync = what != "other_device";

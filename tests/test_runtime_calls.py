@@ -29,3 +29,13 @@ def test_tree_freed_during_a_capture():
     got = log("other_device_capturing", 300000, 4)
     assert sum(x.startswith("free dev 1") for x in got) == 2  # the tree's arrays and its scratch
     assert not any(x.startswith("record") for x in got)
+
+
+def test_searches_on_two_streams():
+    """An FP64 search that needs scratch (a query per lane) does not wait for
+    one on another stream of the same tree, and a stream's later searches take
+    the memory of its earlier ones."""
+    got = log("two_streams", 300000, 4)
+    assert sum("k_knn" in x for x in got) == 3
+    assert not any(x.startswith(("wait", "host waits", "device_sync")) for x in got)
+    assert not any(x.startswith("malloc") for x in got[got.index("again"):])
