@@ -671,6 +671,11 @@ static size_t density_ws_bytes(const nbx_tree *t, int32_t k, bool mixed, int32_t
 // The FP64 search with its scratch from ws (as much of it as is left), or a
 // block of its own when ws is null: searches on several streams do not take
 // turns, as they would with the tree's one block.
+// Less scratch runs fewer workgroups of the kernel with a query per lane; with
+// less than a third of it a wave per query, which needs none, takes over.
+// Densities from the fixed scratch in ms, lanes / waves: with 0.49 of it (27.8M
+// particles) k = 1 22 / 39, k = 4 30 / 43, k = 18 47 / 50; with 0.30 (30M) 35 /
+// 42, 47 / 47, 74 / 54; with 0.005 (33.5M) 430 / 47, 580 / 52, 916 / 61.
 static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t st, Workspace *ws = nullptr) {
     if (nq <= 0) return hipSuccess;
     const bool listed = A.qsrc != NBX_Q_POINTS && A.qlist;
@@ -684,6 +689,7 @@ static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t s
     DevBufs own(st);
     void *work = nullptr;
     if (ws) {
+        if (ws->left() < need / 3) return nbx_launch_knn_wave(t->view(), A, nq, st);
         need = std::min(need, ws->left());
         work = ws->carve<void>(need);
         if (!work) return hipErrorInvalidValue;
@@ -1079,10 +1085,7 @@ extern "C" int nbx_knn_density_dev(nbx_tree *t, int32_t k, int32_t *nn_by_slot_d
 // device.  Every call on a GPU shares that GPU's copy: it clears what must
 // start at zero itself (fill kernels), and calls that overlap on one GPU race.
 #define NBX_NOALLOC_BYTES ((size_t)256 << 20)
-// Past the bytes that limit the tree's size, room for the FP64 search's
-// smallest scratch (8 workgroups, 1.03 MiB at k > 64).
-#define NBX_NOALLOC_ARRAY (NBX_NOALLOC_BYTES + ((size_t)2 << 20))
-static __device__ __align__(256) unsigned char scratch[NBX_NOALLOC_ARRAY];
+static __device__ __align__(256) unsigned char scratch[NBX_NOALLOC_BYTES];
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[NBX_MAX_DEVICES];  // per device: the address of `scratch` there
 
@@ -1115,7 +1118,7 @@ extern "C" int nbx_knn_density_noalloc(nbx_tree *t, int32_t k, int32_t *nn_by_sl
     void *base = nullptr;
     int rc = noalloc_scratch(&base);
     if (rc) return rc;
-    Workspace ws = {(char *)base, NBX_NOALLOC_ARRAY, 0};
+    Workspace ws = {(char *)base, NBX_NOALLOC_BYTES, 0};
     return density_impl(t, k, NBX_DENS_SYMMETRIC, 0, rho_by_id_dev, h_by_id_dev, nn_by_slot_dev, (hipStream_t)stream,
                         nullptr, &ws);
 }

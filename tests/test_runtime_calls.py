@@ -4,6 +4,8 @@ streams, events, allocations and launches, without a GPU."""
 import os
 import subprocess
 
+import pytest
+
 PROG = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "fake_hip")
 
 
@@ -39,3 +41,16 @@ def test_searches_on_two_streams():
     assert sum("k_knn" in x for x in got) == 3
     assert not any(x.startswith(("wait", "host waits", "device_sync")) for x in got)
     assert not any(x.startswith("malloc") for x in got[got.index("again"):])
+
+
+# 268.4 MB of fixed scratch, 8 bytes a particle of it for the densities, 94 MB
+# for the search at its best
+@pytest.mark.parametrize("n", [400000, 21000000, 27800000, 30000000, 33000000, 33554000])
+def test_noalloc_search_with_little_scratch(n):
+    """Once less than a third of the search's scratch is left, the search that
+    needs none runs instead of a few workgroups."""
+    got = log("noalloc", n, 8)
+    lanes = [int(x.split("grid ")[1].split()[0]) for x in got if "k_knnILi3E" in x]
+    waves = any("k_knn_wave" in x for x in got)
+    assert "rc 0" in got and not any(x.startswith("malloc") for x in got)
+    assert (lanes and min(lanes) >= 1360 and not waves) if n < 29600000 else (waves and not lanes)
