@@ -666,34 +666,55 @@ __device__ __forceinline__ void fof_task(const DevTree &T, const FofArgs &A, uin
     }
 }
 
-// Persistent linking kernel, one wave per workgroup.  Workgroup b stays on
-// XCD (b mod 8) and takes waves from that XCD's contiguous share of the tree
-// order through the XCD's counter, so the nodes and leaves a neighbourhood's
-// waves share are fetched into one XCD's L2; once its share is drained it
-// takes waves from the other XCDs' counters in turn, which evens out the
-// shares' unequal cost (dense halos).  Every ticket names one wave, so every
-// wave runs once; a workgroup exits when all eight counters are past their
-// shares' ends.
-// Against one workgroup per wave in launch order: 2.7 and 4.4 ms on 16.8M
-// clustered particles, 0.46 and 0.57 ms on 2M (the order that won while the
-// walk was a serial chain of box tests: 10.2 against 11.1 ms).  Registers are
-// held to 5 waves per SIMD in 3-D and 4 in 6-D: 2.80 -> 2.69 ms and FOF6d of
+// Linking, one wave per workgroup.  Registers are held to 5 waves per SIMD in
+// 3-D and 4 in 6-D: 2.80 -> 2.69 ms on 16.8M clustered particles and FOF6d of
 // 1.5M 0.63 -> 0.59 ms; one wave more spills (2.75 and 1.04 ms).
-#define FOF_CTR_STRIDE 16  // XCD counters 64 bytes apart
+#define FOF_BOUNDS(ND) __launch_bounds__(64, (ND) == 3 ? 5 : 4)
+// A workgroup for each wave, for up to twice as many waves as are resident.
+// The persistent form's tickets and ends cost it 60 to 140 us there, of a set
+// with few links most of the time.  In ms, persistent / each: 262144 particles
+// on a lattice, nothing linked, 0.19 / 0.09, uniform, b = 0.2 spacings, 0.20 /
+// 0.10, clustered 0.37 / 0.31; 636056: 0.24 / 0.12, 0.25 / 0.14, 0.42 / 0.40; of
+// more the clustered sets want the shares evened out: 1M 0.26 / 0.15, 0.28 /
+// 0.17, but 1.08 / 1.26.
 template <int ND, int MT>
-__global__ __launch_bounds__(64, ND == 3 ? 5 : 4) void k_fof(DevTree T, FofArgs A, uint8_t *conn, int32_t *ctr) {
+__global__ FOF_BOUNDS(ND) void k_fof_each(DevTree T, FofArgs A, uint8_t *conn) {
+    fof_task<ND, MT>(T, A, conn, xcd_wave(blockIdx.x, gridDim.x));
+}
+// Persistent form.  Workgroup b stays on XCD (b mod 8) and takes waves from
+// that XCD's contiguous share of the tree order through the XCD's counter, so
+// the nodes and leaves a neighbourhood's waves share are fetched into one XCD's
+// L2; once its share is drained it takes waves from the other XCDs' counters in
+// turn, which evens out the shares' unequal cost (dense halos).  Every ticket
+// names one wave, so every wave runs once; a workgroup drains its own share,
+// and exits at the first other counter, from the third on, that is past its
+// share's end.  (Atomics on a counter come one after another, 14 ns each, and
+// most of those that found a share drained were of workgroups that met seven
+// such.  To the end of all eight / stopping there: lattice of 1M 0.26 / 0.21 ms,
+// of 2.1M 0.32 / 0.27, clustered sets of 1M to 16.8M equal; stopping at the
+// first costs 16.8M 1.3%; reading a counter before adding to it made clustered
+// sets 7% slower.)
+// Against one workgroup per wave, in ms: 16.8M clustered particles 3.12 / 3.39,
+// 8M 1.48 / 1.57.
+#define FOF_CTR_STRIDE 16  // XCD counters 64 bytes apart
+#define FOF_TRIES 3
+template <int ND, int MT>
+__global__ FOF_BOUNDS(ND) void k_fof(DevTree T, FofArgs A, uint8_t *conn, int32_t *ctr) {
     const int nw = (T.n + NBX_WAVE - 1) / NBX_WAVE;
     const int x = blockIdx.x & 7, q8 = nw >> 3, r8 = nw & 7;
     for (int s = 0; s < 8; ++s) {
         const int y = (x + s) & 7;
         const int ybeg = y * q8 + (y < r8 ? y : r8), ycnt = q8 + (y < r8 ? 1 : 0);
+        bool got = false;
         for (;;) {
             int t = 0;
             if (threadIdx.x == 0) t = atomicAdd(ctr + y * FOF_CTR_STRIDE, 1);
             t = __builtin_amdgcn_readfirstlane(__shfl(t, 0));
             if (t >= ycnt) break;
             fof_task<ND, MT>(T, A, conn, ybeg + t);
+            got = true;
         }
+        if (s >= FOF_TRIES && !got) break;
     }
 }
 
@@ -998,12 +1019,15 @@ static void launch_fof_t(const DevTree &T, const FofArgs &A, uint8_t *conn, hipS
                                A.parent, conn, 1, T.nleafp - 1);
     }
     ProfScope ps("k_fof_link", st);
+    const int nw = (T.n + NBX_WAVE - 1) / NBX_WAVE, res = fof_grid<ND, MT>();
+    if (nw <= 2 * res) {
+        hipLaunchKernelGGL((k_fof_each<ND, MT>), dim3(nw), dim3(NBX_WAVE), 0, st, T, A, conn);
+        return;
+    }
     // the XCD queue counters sit after the node flags, 64-byte aligned
     int32_t *ctr = (int32_t *)(((uintptr_t)(conn + 2 * (int64_t)T.nleafp) + 63) & ~(uintptr_t)63);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, ctr, 0, (int64_t)(8 * FOF_CTR_STRIDE));
-    const int nw = (T.n + NBX_WAVE - 1) / NBX_WAVE, res = fof_grid<ND, MT>();
-    const int grid = nw < res ? (nw + 7) & ~7 : res;
-    hipLaunchKernelGGL((k_fof<ND, MT>), dim3(grid), dim3(NBX_WAVE), 0, st, T, A, conn, ctr);
+    hipLaunchKernelGGL((k_fof<ND, MT>), dim3(res), dim3(NBX_WAVE), 0, st, T, A, conn, ctr);
 }
 
 // Bytes of the parent array, node flags and queue counters that

@@ -251,6 +251,12 @@ int main(int argc, char **argv) {
         from = g_log.size();
         const int rc = nbx_knn_density_noalloc(t, k, OUT, (double *)64, (double *)64, A);
         note("rc %d", rc);
+    } else if (what == "fof") {
+        nbx_tree *t = tree(n, 0, A);
+        from = g_log.size();
+        int64_t ng = -1;
+        const int rc = nbx_fof_dev(t, 0.1, 2, OUT, &ng, A);
+        note("rc %d", rc);
     } else if (what == "build") {
         // n particles, form k, on a device of argv[4] GB
         if (argc > 4) g_total = (size_t)atoll(argv[4]) << 30;

@@ -54,3 +54,18 @@ def test_noalloc_search_with_little_scratch(n):
     waves = any("k_knn_wave" in x for x in got)
     assert "rc 0" in got and not any(x.startswith("malloc") for x in got)
     assert (lanes and min(lanes) >= 1360 and not waves) if n < 29600000 else (waves and not lanes)
+
+
+# the fake device holds 4096 workgroups of the linking kernel
+@pytest.mark.parametrize("n", [1, 64, 65, 262144, 524288, 524289, 4000000])
+def test_fof_without_counters(n):
+    """Up to two waves of particles per workgroup that fits, linking is a
+    workgroup for each wave, and no counters are cleared for it."""
+    got = log("fof", n)
+    assert "rc 0" in got
+    each = [x for x in got if "k_fof_each" in x]
+    if n <= 524288:
+        assert len(each) == 1 and f" grid {(n + 63) // 64} " in each[0]
+        assert not any("k_fill_i32" in x or "5k_fofI" in x for x in got)
+    else:
+        assert not each and sum("5k_fofI" in x for x in got) == 1
