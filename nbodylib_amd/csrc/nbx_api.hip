@@ -706,15 +706,15 @@ static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t s
 // same.  Rows in key order come from the FP32 kernel alone.  The line moves with
 // k, whose insertions cost the lanes more.  Measured in ms, FP32 lanes / FP64
 // waves: densities of 0.2M particles k = 8 0.28 / 0.29, k = 32 0.48 / 0.37, of
-// 0.3M k = 20 0.45 / 0.48, k = 32 0.54 / 0.55; rows of 0.2M k = 4 0.26 / 0.22, of
-// 0.3M k = 8 0.31 / 0.33, k = 20 0.43 / 0.38, of 0.4M k = 32 0.56 / 0.55; k = 64
-// of 1M density 3.7 / 2.7, rows 4.2 / 2.1; 6-D 0.5M k = 32 4.98 / 3.9, 1M 8.4 /
-// 8.0, k = 64 18.2 / 11.
+// 0.3M k = 20 0.45 / 0.48, k = 32 0.54 / 0.55 (uniform 0.55 / 0.58); rows of 0.2M
+// k = 4 0.26 / 0.22, of 0.3M k = 8 0.31 / 0.33, k = 20 0.43 / 0.38, of 0.4M k = 32
+// 0.56 / 0.55; k = 64 of 1M density 3.7 / 2.7, rows 4.2 / 2.1; 6-D 0.5M k = 32
+// 4.98 / 3.9, 1M 8.4 / 8.0, k = 64 18.2 / 11.
 static bool mixed_by_waves(const nbx_tree *t, const KnnArgs &A, int k, int64_t nq) {
     const bool rows = A.d2 || A.exact_rows;
     if (A.nn && !rows) return false;
     if (k > 32) return true;
-    return nq <= (t->nd == 6 ? 1048576 : rows ? 163840 + 8192 * k : 131072 + 6144 * k);
+    return nq <= (t->nd == 6 ? 1048576 : rows ? 163840 + 8192 * k : 131072 + 4608 * k);
 }
 
 // FP32 search with the FP64 certificate; queries whose certificate fails are

@@ -603,9 +603,16 @@ static int knn_resident() {
 // 0.79; 1M k = 8 0.91 / 1.44, k = 17 1.24 / 1.60; with room for 33 entries in
 // the lanes' kernel, 2.1M k = 20 3.6 / 3.4, k = 32 4.4 / 3.7.  So the line moves
 // with the entries kept.
+// Up to 7 entries it lies lower.  There a wave is slow on a lattice, where
+// nearly every merge meets equal distances: 262144 particles, density, lattice
+// k = 2 0.24 / 0.57, k = 4 0.26 / 0.58, k = 6 0.30 / 0.62 (k = 8 0.48 / 0.66);
+// uniform k = 4 0.28 / 0.38, k = 6 0.32 / 0.40; clustered k = 4 0.35 / 0.38, k =
+// 6 0.38 / 0.39, rows 0.34 / 0.28 and 0.39 / 0.29.  Of 195112: lattice k = 2
+// 0.32 / 0.46, clustered 0.26 / 0.29, rows 0.23 / 0.22.
 #define KNN_KM 18
 bool nbx_knn_by_waves(int nd, int kh, int qsrc, bool listed, int64_t nqueries) {
-    return nd == 6 || kh > KNN_KM || qsrc == NBX_Q_POINTS || listed || nqueries <= 163840 + 24576 * kh;
+    if (nd == 6 || kh > KNN_KM || qsrc == NBX_Q_POINTS || listed) return true;
+    return nqueries <= (kh <= 7 ? 139264 + 16384 * kh : 163840 + 24576 * kh);
 }
 
 static const size_t KNN_CTR_BYTES = 8 * KNN_CTR_STRIDE * sizeof(int32_t);

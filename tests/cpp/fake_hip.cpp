@@ -251,6 +251,12 @@ int main(int argc, char **argv) {
         from = g_log.size();
         const int rc = nbx_knn_density_noalloc(t, k, OUT, (double *)64, (double *)64, A);
         note("rc %d", rc);
+    } else if (what == "rows" || what == "density") {
+        nbx_tree *t = tree(n, argc > 4 ? atoi(argv[4]) : 0, A);
+        from = g_log.size();
+        const int rc = what == "rows" ? nbx_knn_dev(t, k, NBX_KNN_NONPERIODIC, 0, OUT, (double *)64, A)
+                                      : nbx_density_dev(t, k, NBX_DENS_SYMMETRIC, 0, (double *)64, nullptr, A);
+        note("rc %d", rc);
     } else if (what == "fof") {
         nbx_tree *t = tree(n, 0, A);
         from = g_log.size();

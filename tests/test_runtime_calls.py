@@ -69,3 +69,15 @@ def test_fof_without_counters(n):
         assert not any("k_fill_i32" in x or "5k_fofI" in x for x in got)
     else:
         assert not each and sum("5k_fofI" in x for x in got) == 1
+
+
+# sizes at which the other kernel was the slower one
+@pytest.mark.parametrize("what,n,k,form,kernel", [
+    ("rows", 262144, 4, 0, "5k_knnI"), ("rows", 262144, 5, 0, "5k_knnI"), ("density", 262144, 6, 0, "5k_knnI"),
+    ("rows", 262144, 7, 0, "5k_knnI"), ("density", 195112, 2, 0, "5k_knnI"), ("rows", 262144, 8, 0, "10k_knn_wave"),
+    ("rows", 110592, 1, 0, "10k_knn_wave"), ("density", 204800, 4, 0, "10k_knn_wave"),
+    ("density", 300000, 32, 1, "11k_knn_mixed"), ("density", 262144, 32, 1, "10k_knn_wave")])
+def test_search_kernel(what, n, k, form, kernel):
+    got = log(what, n, k, form)
+    assert "rc 0" in got
+    assert [x.split()[1][2:].startswith(kernel) for x in got if "k_knn" in x] == [True]
