@@ -322,9 +322,11 @@ int nbx_sph_density_adjoint_dev(const double *pos_dev, const double *mass_dev, c
  * list, [2] = how many of its n*k indices lie within their row's block of
  * 1024.  order: order_dev = the permutation (rank -> index) of pos's Morton
  * order; the ordered calls take NULL for the order of the arrays.  All take
- * device pointers; work is nbx_sph_work_bytes(n) bytes of device memory
- * (256-byte aligned), needed during the call only. */
+ * device pointers; work is nbx_sph_work_bytes(n) bytes of device memory (76 a
+ * particle), for the order and the forward nbx_sph_fwd_work_bytes(n) are enough
+ * (36 a particle), 256-byte aligned, needed during the call only. */
 int64_t nbx_sph_work_bytes(int64_t n);
+int64_t nbx_sph_fwd_work_bytes(int64_t n);
 int nbx_sph_list_check_dev(const int32_t *nbr_dev, int64_t n, int32_t k, int64_t *stats_dev, void *stream);
 int nbx_sph_order_dev(const double *pos_dev, int64_t n, int32_t *order_dev, void *work_dev, void *stream);
 int nbx_sph_density_fwd_ordered_dev(const double *pos_dev, const double *mass_dev, const int32_t *nbr_dev,

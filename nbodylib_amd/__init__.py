@@ -33,7 +33,7 @@ EXPORTS = [
     "nbx_tree_size", "nbx_tree_kernel", "nbx_knn", "nbx_knn_dev", "nbx_knn_points", "nbx_knn_targets", "nbx_knn_phase_points", "nbx_density_points", "nbx_veldensity_points", "nbx_veldensity_phys", "nbx_smooth_vel", "nbx_smooth_vel_moments", "nbx_smooth_local", "nbx_smooth_local_points", "nbx_density",
     "nbx_density_dev", "nbx_knn_density_dev", "nbx_knn_density_noalloc", "nbx_ball_points", "nbx_ball_points_many", "nbx_ball_mark", "nbx_fof", "nbx_fof_dev", "nbx_fof_criterion", "nbx_fof_criterion_dev", "nbx_fof_lists",
     "nbx_sph_density_fwd_dev", "nbx_sph_density_adjoint_dev", "nbx_sph_density_fwd_tree_dev",
-    "nbx_sph_density_adjoint_tree_dev", "nbx_sph_work_bytes", "nbx_sph_list_check_dev", "nbx_sph_order_dev",
+    "nbx_sph_density_adjoint_tree_dev", "nbx_sph_work_bytes", "nbx_sph_fwd_work_bytes", "nbx_sph_list_check_dev", "nbx_sph_order_dev",
     "nbx_sph_density_fwd_ordered_dev", "nbx_sph_density_adjoint_ordered_dev", "nbx_prof_enable", "nbx_prof_reset", "nbx_prof_get",
     "nbx_tree_last_fallbacks", "nbx_last_error",
 ]
@@ -105,6 +105,8 @@ def lib():
     L.nbx_sph_density_adjoint_dev.argtypes = [vp, vp, vp, i64, i32, vp, vp, vp, vp]
     L.nbx_sph_work_bytes.argtypes = [i64]
     L.nbx_sph_work_bytes.restype = i64
+    L.nbx_sph_fwd_work_bytes.argtypes = [i64]
+    L.nbx_sph_fwd_work_bytes.restype = i64
     L.nbx_sph_list_check_dev.argtypes = [vp, i64, i32, vp, vp]
     L.nbx_sph_order_dev.argtypes = [vp, i64, vp, vp, vp]
     L.nbx_sph_density_fwd_ordered_dev.argtypes = [vp, vp, vp, vp, i64, i32, vp, vp, vp, vp]

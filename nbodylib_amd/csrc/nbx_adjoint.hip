@@ -205,7 +205,7 @@ struct SphWork {
     double *g;     // dL/drho by rank
     double *acc;   // adjoint sums by rank, 4 per particle
     void *sort;
-    size_t sort_bytes, total;
+    size_t sort_bytes, fwd, total;  // fwd: what the order and the forward need
     SphWork(void *base, int64_t n) {
         char *at = (char *)base;
         auto carve = [&](size_t b) {
@@ -216,6 +216,7 @@ struct SphWork {
         bounds = (uint64_t *)carve(6 * sizeof(uint64_t));
         rank = (int32_t *)carve(sizeof(int32_t) * n);
         rec = (double4 *)carve(sizeof(double4) * n);
+        const size_t end_rec = (size_t)(at - (char *)base);
         g = (double *)carve(sizeof(double) * n);
         acc = (double *)carve(4 * sizeof(double) * n);
         // the sort's arrays are done with before the records are written
@@ -227,11 +228,13 @@ struct SphWork {
         nbx_sort_pairs_u32(nullptr, sort_bytes, key, key2, idx, rank, n, 3 * SPH_BITS, nullptr);
         sort = carve(sort_bytes);
         const size_t end_sort = (size_t)(at - (char *)base);
-        const size_t end_rec = (size_t)((char *)(acc + 4 * n) - (char *)base);
-        total = (end_sort > end_rec ? end_sort : end_rec) + 256;
+        const size_t end_acc = (size_t)((char *)(acc + 4 * n) - (char *)base);
+        fwd = (end_sort > end_rec ? end_sort : end_rec) + 256;
+        total = (end_sort > end_acc ? end_sort : end_acc) + 256;
     }
 };
 size_t nbx_sph_work_size(int64_t n) { return SphWork(nullptr, n).total; }
+size_t nbx_sph_fwd_work_size(int64_t n) { return SphWork(nullptr, n).fwd; }
 
 // Rows and columns are stepped without a division.  The waves of a block meet in LDS and blocks are few: with three atomics per
 // wave of 4096 blocks the pass took 582 us on 1M x 32, all of it atomics on
@@ -613,7 +616,7 @@ hipError_t nbx_launch_sph_fwd_ordered(const double *pos, const double *mass, con
     ProfScope ps("k_sph_fwd", st);
     hipLaunchKernelGGL(k_fill_f64, nb, dim3(256), 0, st, rho, 0.0, n);
     hipLaunchKernelGGL(k_sph_pack, nb, dim3(256), 0, st, pos, pos + n, pos + 2 * n, mass, (const double *)nullptr,
-                       (const int32_t *)nullptr, order, n, W.rec, W.g, W.rank);
+                       (const int32_t *)nullptr, order, n, W.rec, (double *)nullptr, W.rank);
 #define SPH_F(V, ORD)                                                                                                  \
     hipLaunchKernelGGL((k_sph_fwd_ordered<V, ORD>), blocks, dim3(ADJ_B), 0, st, W.rec, W.rank, order, nbr, n, k, rho, h)
     const bool v = sph_vec(nbr, k);

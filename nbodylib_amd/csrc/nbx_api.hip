@@ -1729,6 +1729,7 @@ extern "C" int nbx_sph_density_adjoint_dev(const double *pos, const double *mass
 
 // The same with the rows in a spatial order (for arrays in no such order).
 extern "C" int64_t nbx_sph_work_bytes(int64_t n) { return n < 1 ? 0 : (int64_t)nbx_sph_work_size(n); }
+extern "C" int64_t nbx_sph_fwd_work_bytes(int64_t n) { return n < 1 ? 0 : (int64_t)nbx_sph_fwd_work_size(n); }
 extern "C" int nbx_sph_list_check_dev(const int32_t *nbr, int64_t n, int32_t k, int64_t *stats, void *stream) {
     if (!nbr || !stats) return fail(NBX_ERR_ARG, "NULL argument");
     if (n < 1 || k < 1) return fail(NBX_ERR_ARG, "bad sizes");

@@ -221,11 +221,13 @@ hipError_t nbx_launch_sph_adj(const double *pos, const double *mass, const int32
 // A stored list over particles in an order of their own.  list_check: smallest
 // and largest entry and the number of entries within their row's block of
 // 1024 (stats: 3 int64 of device memory).  order: a permutation that brings
-// spatial neighbours together (work: nbx_sph_work_size).  The ordered forward
+// spatial neighbours together (work: nbx_sph_work_size, or nbx_sph_fwd_work_size
+// for the order and the forward alone).  The ordered forward
 // and adjoint take the rows in that order (null: as they lie); both outputs
 // are written.
 hipError_t nbx_launch_sph_list_check(const int32_t *nbr, int64_t n, int k, int64_t *stats, hipStream_t st);
 size_t nbx_sph_work_size(int64_t n);
+size_t nbx_sph_fwd_work_size(int64_t n);
 hipError_t nbx_launch_sph_order(const double *pos, int64_t n, int32_t *order, void *work, hipStream_t st);
 hipError_t nbx_launch_sph_fwd_ordered(const double *pos, const double *mass, const int32_t *nbr, const int32_t *order,
                                       int64_t n, int k, double *rho, double *h, void *work, hipStream_t st);

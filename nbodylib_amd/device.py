@@ -5,7 +5,8 @@ Positions/velocities are (3, n) float64 CUDA tensors (SoA), masses (n,).
 
 SPHDensity is the differentiation form: a torch.autograd.Function whose
 forward is the symmetric SPH density over a frozen neighbour list and whose
-backward is the hand-written adjoint kernel (nbx_sph_density_adjoint_dev).
+backward is the hand-written adjoint kernel
+(nbx_sph_density_adjoint_ordered_dev).
 """
 import ctypes
 
@@ -147,8 +148,21 @@ def _check_list(nbr, n):
     return local / nbr.numel()
 
 
-def _sph_work(pos):
-    return torch.empty(lib().nbx_sph_work_bytes(pos.shape[1]), dtype=torch.uint8, device=pos.device)
+def _sph_work(pos, size):
+    """Work memory for the packed kernels, or None where there is no room for it: the plain ones need none."""
+    try:
+        return torch.empty(size(pos.shape[1]), dtype=torch.uint8, device=pos.device)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def _sph_forward(pos, mass, nbr, order, work, rho, h):
+    n, k = pos.shape[1], nbr.shape[1]
+    if work is None:
+        _check(lib().nbx_sph_density_fwd_dev(_ptr(pos), _ptr(mass), _ptr(nbr), n, k, _ptr(rho), _ptr(h), _stream()))
+    else:
+        _check(lib().nbx_sph_density_fwd_ordered_dev(_ptr(pos), _ptr(mass), _ptr(nbr), _ptr(order), n, k, _ptr(rho),
+                                                     _ptr(h), _ptr(work), _stream()))
 
 
 def sph_density(pos, mass, nbr):
@@ -158,9 +172,8 @@ def sph_density(pos, mass, nbr):
     _need(mass, "mass", torch.float64, (n,))
     rho = torch.empty(n, dtype=torch.float64, device=pos.device)
     h = torch.empty(n, dtype=torch.float64, device=pos.device)
-    work = _sph_work(pos)
-    _check(lib().nbx_sph_density_fwd_ordered_dev(_ptr(pos), _ptr(mass), _ptr(nbr), None, n, nbr.shape[1], _ptr(rho),
-                                                 _ptr(h), _ptr(work), _stream()))
+    work = _sph_work(pos, lib().nbx_sph_fwd_work_bytes)
+    _sph_forward(pos, mass, nbr, None, work, rho, h)
     return rho, h
 
 
@@ -181,13 +194,12 @@ class SPHDensity(torch.autograd.Function):
         _need(pos, "pos", torch.float64, (3, n))
         _need(mass, "mass", torch.float64, (n,))
         rho = torch.empty(n, dtype=torch.float64, device=pos.device)
-        work = _sph_work(pos)
+        work = _sph_work(pos, lib().nbx_sph_fwd_work_bytes)
         order = None
-        if n >= _ORDER_MIN and local < 0.5:
+        if work is not None and n >= _ORDER_MIN and local < 0.5:
             order = torch.empty(n, dtype=torch.int32, device=pos.device)
             _check(lib().nbx_sph_order_dev(_ptr(pos), n, _ptr(order), _ptr(work), _stream()))
-        _check(lib().nbx_sph_density_fwd_ordered_dev(_ptr(pos), _ptr(mass), _ptr(nbr), _ptr(order), n, nbr.shape[1],
-                                                     _ptr(rho), None, _ptr(work), _stream()))
+        _sph_forward(pos, mass, nbr, order, work, rho, None)
         ctx.save_for_backward(pos, mass, nbr, order)
         return rho
 
@@ -198,9 +210,13 @@ class SPHDensity(torch.autograd.Function):
         g = g.contiguous().to(torch.float64)
         dpos = torch.empty_like(pos)
         dmass = torch.empty_like(mass)
-        work = _sph_work(pos)
-        _check(lib().nbx_sph_density_adjoint_ordered_dev(_ptr(pos), _ptr(mass), _ptr(nbr), _ptr(order), n, k, _ptr(g),
-                                                         _ptr(dpos), _ptr(dmass), _ptr(work), _stream()))
+        work = _sph_work(pos, lib().nbx_sph_work_bytes)
+        if work is None:
+            _check(lib().nbx_sph_density_adjoint_dev(_ptr(pos), _ptr(mass), _ptr(nbr), n, k, _ptr(g), _ptr(dpos),
+                                                     _ptr(dmass), _stream()))
+        else:
+            _check(lib().nbx_sph_density_adjoint_ordered_dev(_ptr(pos), _ptr(mass), _ptr(nbr), _ptr(order), n, k,
+                                                             _ptr(g), _ptr(dpos), _ptr(dmass), _ptr(work), _stream()))
         return dpos, dmass, None
 
 

@@ -1,0 +1,100 @@
+"""Work memory of the differentiation form over a stored list: no more than a
+call uses, and where there is no room for it the kernels
+that need none give the same results."""
+import pytest
+
+from nbodylib_amd import datagen
+
+pytestmark = pytest.mark.gpu
+
+
+def _set(n, k, shuffled=False):
+    import torch
+
+    import nbodylib_amd as nb
+    from nbodylib_amd.device import DeviceTree
+
+    p = torch.tensor(datagen.clustered(n, 1.0, nhalo=5, seed=n)[0].T.copy(), device="cuda")
+    m = torch.tensor(datagen.lognormal_masses(n, n), device="cuda")
+    t = DeviceTree(p, mass=m, kerntype=nb.KSPH)
+    nn = torch.empty((n, k), dtype=torch.int32, device="cuda")
+    d2 = torch.empty((n, k), dtype=torch.float64, device="cuda")
+    t.knn(k, nn, d2, variant=nb.KNN_NONPERIODIC, layout=nb.LAYOUT_BY_ID if shuffled else nb.LAYOUT_BY_SLOT)
+    if not shuffled:
+        o = t.order().long()
+        p, m = p[:, o].contiguous(), m[o].contiguous()
+    del t, d2
+    return p, m, nn
+
+
+def _peak(f):
+    """Most bytes of torch's that f held beyond what it found."""
+    import torch
+
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = f()
+    torch.cuda.synchronize()
+    return torch.cuda.max_memory_allocated() - before, out
+
+
+def test_forward_memory(gpu):
+    """Records and ranks, 36 bytes a particle, beside the two outputs."""
+    from nbodylib_amd.device import sph_density
+
+    n, k = 500000, 12
+    print(f"sph work n={n} k={k}", flush=True)
+    p, m, nn = _set(n, k)
+    got, _ = _peak(lambda: sph_density(p, m, nn))
+    assert got < (16 + 40) * n
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_no_room(gpu, shuffled):
+    import torch
+
+    from nbodylib_amd import device
+    from nbodylib_amd.device import SPHDensity, sph_density
+
+    n, k = 300000, 12
+    print(f"sph without work memory n={n} k={k} shuffled={shuffled}", flush=True)
+    p, m, nn = _set(n, k, shuffled)
+
+    def run():
+        rho, h = sph_density(p, m, nn)
+        pg, mg = p.clone().requires_grad_(), m.clone().requires_grad_()
+        r = SPHDensity.apply(pg, mg, nn)
+        r.backward(1.0 / r.detach())
+        return rho, h, r.detach(), pg.grad, mg.grad
+
+    want = run()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    sizes = []
+    real = device._sph_work
+
+    def counted(*a):
+        w = real(*a)
+        sizes.append(None if w is None else w.numel())
+        return w
+
+    device._sph_work = counted
+    try:
+        # the largest block of any pass, 10.8 MB, leaves no room for 10.8 MB more
+        hold = torch.empty(((64 << 20) - 8,), dtype=torch.uint8, device="cuda")
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (44 << 20)) / total)
+        fill = [torch.empty((8 << 20,), dtype=torch.uint8, device="cuda") for _ in range(2)]
+        got = run()
+        torch.cuda.synchronize()
+        del hold, fill
+    finally:
+        device._sph_work = real
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert None in sizes, sizes  # some call had to do without
+    assert torch.equal(got[1], want[1])
+    for a, b in zip(got, want):
+        assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
+    assert float((got[0] / want[0] - 1.0).abs().max()) < 1e-12
