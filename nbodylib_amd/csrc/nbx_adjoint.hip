@@ -375,20 +375,23 @@ hipError_t nbx_launch_sph_order(const double *pos, int64_t n, int32_t *order, vo
     return e;
 }
 
-// Records by rank, ranks by index, and with g the cotangents by rank.  No
-// order: rank and index are the same (rank is not written).  gidx: where the
-// cotangents of a rank are (null: at its index).
+// Records by rank, ranks by index, and with g (the adjoint) the cotangents by
+// rank and the sums cleared.  No order: rank and index are the same (rank is
+// not written).  gidx: where the cotangents of a rank are (null: at its index).
 __global__ __launch_bounds__(256) void k_sph_pack(const double *__restrict__ X, const double *__restrict__ Y,
                                                   const double *__restrict__ Z, const double *__restrict__ mass,
                                                   const double *__restrict__ g, const int32_t *__restrict__ gidx,
                                                   const int32_t *__restrict__ order, int64_t n, double4 *rec,
-                                                  double *gs, int32_t *rank) {
+                                                  double *gs, int32_t *rank, double4 *acc) {
     const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (s >= n) return;
     const int64_t i = order ? order[s] : s;
     rec[s] = make_double4(X[i], Y[i], Z[i], mass[i]);
     if (order) rank[i] = (int32_t)s;
-    if (g) gs[s] = g[gidx ? gidx[s] : i];
+    if (g) {
+        gs[s] = g[gidx ? gidx[s] : i];
+        acc[s] = make_double4(0.0, 0.0, 0.0, 0.0);
+    }
 }
 
 // G neighbours of a row from column j0 (their ranks; past the row's end: s).
@@ -616,7 +619,7 @@ hipError_t nbx_launch_sph_fwd_ordered(const double *pos, const double *mass, con
     ProfScope ps("k_sph_fwd", st);
     hipLaunchKernelGGL(k_fill_f64, nb, dim3(256), 0, st, rho, 0.0, n);
     hipLaunchKernelGGL(k_sph_pack, nb, dim3(256), 0, st, pos, pos + n, pos + 2 * n, mass, (const double *)nullptr,
-                       (const int32_t *)nullptr, order, n, W.rec, (double *)nullptr, W.rank);
+                       (const int32_t *)nullptr, order, n, W.rec, (double *)nullptr, W.rank, (double4 *)nullptr);
 #define SPH_F(V, ORD)                                                                                                  \
     hipLaunchKernelGGL((k_sph_fwd_ordered<V, ORD>), blocks, dim3(ADJ_B), 0, st, W.rec, W.rank, order, nbr, n, k, rho, h)
     const bool v = sph_vec(nbr, k);
@@ -629,9 +632,8 @@ hipError_t nbx_launch_sph_fwd_ordered(const double *pos, const double *mass, con
 void nbx_sph_adj_begin(const double *const *X, const double *mass, const int32_t *order, int64_t n, const double *g,
                        const int32_t *gidx, void *work, hipStream_t st) {
     SphWork W(work, n);
-    hipLaunchKernelGGL(k_fill_f64, dim3((unsigned)((4 * n + 255) / 256)), dim3(256), 0, st, W.acc, 0.0, 4 * n);
     hipLaunchKernelGGL(k_sph_pack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, X[0], X[1], X[2], mass, g, gidx,
-                       order, n, W.rec, W.g, W.rank);
+                       order, n, W.rec, W.g, W.rank, (double4 *)W.acc);
 }
 void nbx_sph_adj_rows(const int32_t *nbr, const int32_t *order, int64_t n, int64_t r0, int64_t nr, int k, void *work,
                       hipStream_t st) {

@@ -37,6 +37,7 @@ struct FakeEvent {
 static std::set<FakeEvent *> g_events;
 static std::vector<std::string> g_log;
 static bool g_fail_sync = false;
+static hipError_t g_last = hipSuccess;
 
 template <class... A>
 static void note(const char *f, A... a) {
@@ -100,6 +101,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shm, hipStream_t 
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t, hipStream_t st) {
     const uint64_t threads = (uint64_t)g.x * b.x;
     note("launch %s grid %u threads %llu stream %p", names()[f].c_str(), g.x, (unsigned long long)threads, (void *)st);
+    if (threads >> 32) g_last = hipErrorInvalidConfiguration;
     return threads >> 32 ? hipErrorInvalidConfiguration : hipSuccess;
 }
 hipError_t hipGetDevice(int *d) {
@@ -199,7 +201,11 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) {
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
 hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }
 hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
 hipError_t hipGetSymbolAddress(void **p, const void *) {
     static void *m = mmap(nullptr, (size_t)1 << 30, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     *p = m;
@@ -256,6 +262,10 @@ int main(int argc, char **argv) {
         from = g_log.size();
         const int rc = what == "rows" ? nbx_knn_dev(t, k, NBX_KNN_NONPERIODIC, 0, OUT, (double *)64, A)
                                       : nbx_density_dev(t, k, NBX_DENS_SYMMETRIC, 0, (double *)64, nullptr, A);
+        note("rc %d", rc);
+    } else if (what == "adjoint") {
+        double *const D = (double *)4096;
+        const int rc = nbx_sph_density_adjoint_ordered_dev(D, D, OUT, nullptr, n, k, D, D, D, D, A);
         note("rc %d", rc);
     } else if (what == "fof") {
         nbx_tree *t = tree(n, 0, A);

@@ -81,3 +81,11 @@ def test_search_kernel(what, n, k, form, kernel):
     got = log(what, n, k, form)
     assert "rc 0" in got
     assert [x.split()[1][2:].startswith(kernel) for x in got if "k_knn" in x] == [True]
+
+
+@pytest.mark.parametrize("n", [1000, (1 << 30) - 1, 1 << 30, (1 << 31) - 5000])
+def test_adjoint_of_many_particles(n):
+    """No launch of the adjoint has 2^32 threads, which none may have."""
+    got = log("adjoint", n, 4)
+    assert "rc 0" in got
+    assert all(int(x.split("threads ")[1].split()[0]) < 1 << 32 for x in got if x.startswith("launch"))
