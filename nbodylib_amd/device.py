@@ -148,6 +148,12 @@ def _check_list(nbr, n):
     return local / nbr.numel()
 
 
+# Records cost a launch more than they save up to this many list entries
+# (forward, plain and packed: 200 particles, k = 32 15.1 and 18.8 us; 300 17.6
+# and 18.8; 1000, k = 8 14.7 and 19.5; 600, k = 32 28.4 and 20.1).
+_RECORDS_MIN = 8192
+
+
 def _sph_work(pos, size):
     """Work memory for the packed kernels, or None where there is no room for it: the plain ones need none."""
     try:
@@ -172,7 +178,7 @@ def sph_density(pos, mass, nbr):
     _need(mass, "mass", torch.float64, (n,))
     rho = torch.empty(n, dtype=torch.float64, device=pos.device)
     h = torch.empty(n, dtype=torch.float64, device=pos.device)
-    work = _sph_work(pos, lib().nbx_sph_fwd_work_bytes)
+    work = _sph_work(pos, lib().nbx_sph_fwd_work_bytes) if n * nbr.shape[1] > _RECORDS_MIN else None
     _sph_forward(pos, mass, nbr, None, work, rho, h)
     return rho, h
 

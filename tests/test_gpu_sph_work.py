@@ -1,6 +1,7 @@
 """Work memory of the differentiation form over a stored list: no more than a
-call uses, and where there is no room for it the kernels
-that need none give the same results."""
+call uses, none for the smallest ones, and where there is no room for it the
+kernels that need none give the same results."""
+import numpy as np
 import pytest
 
 from nbodylib_amd import datagen
@@ -98,3 +99,28 @@ def test_no_room(gpu, shuffled):
     for a, b in zip(got, want):
         assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
     assert float((got[0] / want[0] - 1.0).abs().max()) < 1e-12
+
+
+@pytest.mark.parametrize("n,k", [(5, 4), (100, 32), (256, 32), (1024, 8), (257, 32), (1025, 8)])
+def test_small_lists(gpu, n, k):
+    """Up to 8192 entries no work memory, and the packed kernels' results."""
+    import torch
+
+    import nbodylib_amd as nb
+    from nbodylib_amd.device import _check, _ptr, _stream, lib, sph_density
+
+    print(f"sph small n={n} k={k}", flush=True)
+    p = torch.tensor(datagen.uniform(n, 1.0, n).T.copy(), device="cuda")
+    m = torch.tensor(datagen.lognormal_masses(n, n), device="cuda")
+    # no particle in its own row: as the last entry it would make h zero
+    rows = [(i + 1 + np.random.default_rng(i).permutation(n - 1)[:k]) % n for i in range(n)]
+    nn = torch.tensor(np.stack(rows).astype(np.int32), device="cuda")
+    held, (rho, h) = _peak(lambda: sph_density(p, m, nn))
+    out = 2 * ((8 * n + 511) // 512 * 512)  # (blocks of 512 bytes)
+    assert (held <= out) == (n * k <= 8192)
+    w = torch.empty(lib().nbx_sph_work_bytes(n), dtype=torch.uint8, device="cuda")
+    r2, h2 = torch.empty_like(rho), torch.empty_like(h)
+    _check(lib().nbx_sph_density_fwd_ordered_dev(_ptr(p), _ptr(m), _ptr(nn), None, n, k, _ptr(r2), _ptr(h2), _ptr(w),
+                                                 _stream()))
+    assert torch.equal(h, h2)
+    assert float((rho - r2).abs().max()) <= 1e-12 * float(r2.abs().max())
