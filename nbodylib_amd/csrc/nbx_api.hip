@@ -48,8 +48,9 @@ extern "C" int nbx_host_fail(int code, const char *msg) { return fail(code, msg)
 // unmapped fresh memory, and takes 1.86 ms with one block per tree and blocks
 // kept.
 //  * Bounded: at most 1/64 of the device's memory is kept (4.5 GiB of 288);
-//    past that the oldest blocks are freed, and larger blocks are never kept.
-//    When an allocation fails every kept block is freed and it is tried again.
+//    past that the oldest blocks are freed, and larger blocks are never kept,
+//    nor rounded up to a size class.  When an allocation fails every kept block
+//    is freed and it is tried again, as large as the need.
 //  * Streams: a block goes back with an event recorded on the stream that last
 //    used it, and the next user's stream waits for that event.  A block whose
 //    event has not come yet is given to the same stream only, so no stream
@@ -79,6 +80,14 @@ static size_t block_class(size_t bytes) {
     const size_t step = b >= (1 << 16) ? b >> 3 : b;  // eighths of a power of two from 64 KiB on
     return (bytes + step - 1) / step * step;
 }
+// most bytes kept on dev (k.mu held)
+static size_t keep_limit(KeptBlocks &k, int dev) {
+    if (k.limit[dev] == 0) {
+        size_t all = 0;
+        k.limit[dev] = hipDeviceTotalMem(&all, dev) == hipSuccess && all >= 64 ? all / 64 : 1;
+    }
+    return k.limit[dev];
+}
 static void drop_block(KeptBlocks &k, int dev, size_t i) {
     const KeptBlock b = k.free[dev][i];
     k.free[dev].erase(k.free[dev].begin() + i);
@@ -106,11 +115,13 @@ static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) 
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    const size_t bytes = block_class(need);
+    const size_t exact = (need + 4095) & ~(size_t)4095;
+    size_t bytes = block_class(need);
     if (dev >= 0 && dev < NBX_MAX_DEVICES) {
         KeptBlocks &k = kept_blocks();
         std::lock_guard<std::mutex> lk(k.mu);
         std::vector<KeptBlock> &f = k.free[dev];
+        if (bytes > keep_limit(k, dev)) bytes = exact;  // never kept
         size_t best = f.size();
         for (size_t i = 0; i < f.size(); ++i) {  // the smallest that fits, the latest of equals
             if (f[i].bytes < bytes || f[i].bytes > bytes + bytes / 2) continue;
@@ -141,6 +152,7 @@ static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) 
             std::lock_guard<std::mutex> lk(k.mu);
             while (!k.free[dev].empty()) drop_block(k, dev, 0);
         }
+        bytes = exact;
         e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) *p = nullptr;
@@ -159,13 +171,9 @@ static void block_put(void *p, size_t bytes, hipStream_t st) {
     if (dev >= 0 && dev < NBX_MAX_DEVICES) {
         KeptBlocks &k = kept_blocks();
         std::lock_guard<std::mutex> lk(k.mu);
-        if (k.limit[dev] == 0) {
-            size_t all = 0;
-            k.limit[dev] = hipDeviceTotalMem(&all, dev) == hipSuccess && all >= 64 ? all / 64 : 1;
-        }
-        if (bytes <= k.limit[dev] && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) {
+        if (bytes <= keep_limit(k, dev) && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) {
             if (hipEventRecord(ev, st) == hipSuccess) {
-                while (k.total[dev] + bytes > k.limit[dev]) drop_block(k, dev, 0);
+                while (k.total[dev] + bytes > keep_limit(k, dev)) drop_block(k, dev, 0);
                 k.free[dev].push_back({p, bytes, ev, st});
                 k.total[dev] += bytes;
                 return;

@@ -89,3 +89,15 @@ def test_adjoint_of_many_particles(n):
     got = log("adjoint", n, 4)
     assert "rc 0" in got
     assert all(int(x.split("threads ")[1].split()[0]) < 1 << 32 for x in got if x.startswith("launch"))
+
+
+def _build(n, form, gib=288):
+    got = [x for x in log("build", n, form, gib) if x.startswith("tree ")][0].split()
+    return int(got[1]), int(got[3]), int(got[5])  # made, most bytes at once, bytes held
+
+
+# need: the sum of the tree's arrays
+@pytest.mark.parametrize("n,form,need", [(2000000000, 0, 87516204768), (2000000000, 1, 124737430240)])
+def test_large_trees_are_not_rounded_up(n, form, need):
+    made, _, held = _build(n, form)
+    assert made and held < need + (16 << 20)
