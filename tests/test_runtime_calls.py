@@ -101,3 +101,18 @@ def _build(n, form, gib=288):
 def test_large_trees_are_not_rounded_up(n, form, need):
     made, _, held = _build(n, form)
     assert made and held < need + (16 << 20)
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("n", [200000000, 2000000000])
+def test_build_gives_its_work_memory_back_first(n, form):
+    """A build never holds the sort's work memory (32 bytes a particle and more)
+    beside the tree's arrays, only the order (4 bytes a particle)."""
+    made, peak, held = _build(n, form)
+    assert made and peak < held + 5 * n
+
+
+@pytest.mark.parametrize("gib,fits", [(131, True), (117, False)])
+def test_build_on_a_full_device(gib, fits):
+    """2e9 particles of the precision form: 124.7 GB of arrays and 8 of order."""
+    assert _build(2000000000, 1, gib)[0] == fits
