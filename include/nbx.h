@@ -32,7 +32,8 @@
  * Device memory kept by the library: blocks given back by trees and calls are
  * kept for later ones, at most 1/64 of the device's memory in all (4.5 GiB of
  * 288); what exceeds that is freed, and everything kept is freed when an
- * allocation fails.
+ * allocation of the library fails, or by nbx_trim_memory, which a program calls
+ * where another allocator of its process needs the memory.
  */
 #ifndef NBX_H
 #define NBX_H
@@ -107,6 +108,9 @@ int nbx_tree_create_dev(const nbx_params *p, const double *pos_dev, const double
  * does), whichever device is current, so no launch on any stream may still be
  * using the tree.  Its memory is kept for the next tree (see above) or freed. */
 int nbx_tree_destroy(nbx_tree *t);
+/* Frees the device memory kept for later trees and calls, on every device,
+ * once the work that last used it is done; returns the bytes. */
+int64_t nbx_trim_memory(void);
 /* slot -> ID map (host array of n).  The C++ shim uses it to reorder the
  * caller's Particle array as the reference does in BuildNodes. */
 int nbx_tree_order(nbx_tree *t, int32_t *slot_to_id);

@@ -29,7 +29,7 @@ NBX_OK = 0
 NBX_ERR_ARG, NBX_ERR_HIP, NBX_ERR_UNSUPPORTED, NBX_ERR_NOMEM, NBX_ERR_SEARCH = -1, -2, -3, -4, -5
 
 EXPORTS = [
-    "nbx_params_default", "nbx_tree_create", "nbx_tree_create_dev", "nbx_tree_destroy", "nbx_tree_order",
+    "nbx_params_default", "nbx_tree_create", "nbx_tree_create_dev", "nbx_tree_destroy", "nbx_trim_memory", "nbx_tree_order",
     "nbx_tree_size", "nbx_tree_kernel", "nbx_knn", "nbx_knn_dev", "nbx_knn_points", "nbx_knn_targets", "nbx_knn_phase_points", "nbx_density_points", "nbx_veldensity_points", "nbx_veldensity_phys", "nbx_smooth_vel", "nbx_smooth_vel_moments", "nbx_smooth_local", "nbx_smooth_local_points", "nbx_density",
     "nbx_density_dev", "nbx_knn_density_dev", "nbx_knn_density_noalloc", "nbx_ball_points", "nbx_ball_points_many", "nbx_ball_mark", "nbx_fof", "nbx_fof_dev", "nbx_fof_criterion", "nbx_fof_criterion_dev", "nbx_fof_lists",
     "nbx_sph_density_fwd_dev", "nbx_sph_density_adjoint_dev", "nbx_sph_density_fwd_tree_dev",
@@ -73,6 +73,8 @@ def lib():
     L.nbx_tree_create.argtypes = [P(Params), vp, vp, vp, i64, P(vp)]
     L.nbx_tree_create_dev.argtypes = [P(Params), vp, vp, vp, i64, vp, P(vp)]
     L.nbx_tree_destroy.argtypes = [vp]
+    L.nbx_trim_memory.argtypes = []
+    L.nbx_trim_memory.restype = i64
     L.nbx_tree_order.argtypes = [vp, vp]
     L.nbx_tree_size.argtypes = [vp]
     L.nbx_tree_size.restype = i64
@@ -511,6 +513,12 @@ def fof_lists(labels_by_id, slot_to_id, ngroups):
     head, nxt, tail, ln = (np.zeros(n, dtype=np.int32) for _ in range(4))
     _check(lib().nbx_fof_lists(_p(lab), _p(order), n, int(ngroups), _p(head), _p(nxt), _p(tail), _p(ln)))
     return head, nxt, tail, ln
+
+
+def trim_memory():
+    """Free the device memory the library keeps for later trees and calls (nbx_trim_memory), for another
+    allocator of the process, such as torch's; returns the bytes."""
+    return lib().nbx_trim_memory()
 
 
 def prof_enable(on=True):

@@ -50,7 +50,8 @@ extern "C" int nbx_host_fail(int code, const char *msg) { return fail(code, msg)
 //  * Bounded: at most 1/64 of the device's memory is kept (4.5 GiB of 288);
 //    past that the oldest blocks are freed, and larger blocks are never kept,
 //    nor rounded up to a size class.  When an allocation fails every kept block
-//    is freed and it is tried again, as large as the need.
+//    is freed and it is tried again, as large as the need; nbx_trim_memory frees
+//    them for the process's other allocations.
 //  * Streams: a block goes back with an event recorded on the stream that last
 //    used it, and the next user's stream waits for that event.  A block whose
 //    event has not come yet is given to the same stream only, so no stream
@@ -109,6 +110,19 @@ struct OnDevice {
     OnDevice(const OnDevice &) = delete;
     OnDevice &operator=(const OnDevice &) = delete;
 };
+// Every kept block of dev (-1: of all devices) back to the runtime; the bytes.
+int64_t nbx_drop_kept(int dev) {
+    KeptBlocks &k = kept_blocks();
+    std::lock_guard<std::mutex> lk(k.mu);
+    int64_t bytes = 0;
+    for (int d = 0; d < NBX_MAX_DEVICES; ++d) {
+        if (dev >= 0 && d != dev) continue;
+        bytes += (int64_t)k.total[d];
+        while (!k.free[d].empty()) drop_block(k, d, 0);
+    }
+    return bytes;
+}
+extern "C" int64_t nbx_trim_memory(void) { return nbx_drop_kept(-1); }
 // *got bytes (at least need) at *p, for work on st from now on
 static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) {
     *p = nullptr;
@@ -150,11 +164,7 @@ static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) 
     e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory && dev >= 0 && dev < NBX_MAX_DEVICES) {
         (void)hipGetLastError();
-        KeptBlocks &k = kept_blocks();
-        {
-            std::lock_guard<std::mutex> lk(k.mu);
-            while (!k.free[dev].empty()) drop_block(k, dev, 0);
-        }
+        nbx_drop_kept(dev);
         bytes = exact;
         e = hipMalloc(p, bytes);
     }

@@ -1107,7 +1107,11 @@ hipError_t nbx_fof_canonical(const DevTree &T, int32_t *P, int32_t minnum, int32
             size_t tb = 0;
             CK(nbx_sort_pairs_u64(nullptr, tb, keys, keys2, vals, vals2, hng, st));
             void *own = nullptr;
-            if (tb > W.sort_bytes) CK(hipMallocAsync(&own, tb, st));
+            if (tb > W.sort_bytes) {
+                e = hipMallocAsync(&own, tb, st);
+                if (e == hipErrorOutOfMemory && nbx_drop_kept(-1) > 0) e = hipMallocAsync(&own, tb, st);
+                CK(e);
+            }
             e = nbx_sort_pairs_u64(own ? own : tmp, tb, keys, keys2, vals, vals2, hng, st);
             if (own) hipFreeAsync(own, st);
             CK(e);

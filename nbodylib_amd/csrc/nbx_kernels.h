@@ -206,6 +206,10 @@ hipError_t nbx_launch_smooth_local(const DevTree &T, const LocalArgs &A, hipStre
 __global__ void k_smooth_out(const double *in, const int32_t *perm, int64_t n, int w, int from0, int ncomp, double *out);
 __global__ void k_gather_by_id(const double *by_id, const int32_t *perm, int64_t n, double *by_slot);
 
+// ------------------------------------------------------------------ memory
+// frees the kept device blocks of dev (-1: of all devices); the bytes
+int64_t nbx_drop_kept(int dev);
+
 // ------------------------------------------------------------------ small kernels
 __global__ void k_scatter_by_id(const double *src, const int32_t *perm, double *dst, int64_t n);
 __global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n);

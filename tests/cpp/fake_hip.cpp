@@ -263,6 +263,19 @@ int main(int argc, char **argv) {
         const int rc = what == "rows" ? nbx_knn_dev(t, k, NBX_KNN_NONPERIODIC, 0, OUT, (double *)64, A)
                                       : nbx_density_dev(t, k, NBX_DENS_SYMMETRIC, 0, (double *)64, nullptr, A);
         note("rc %d", rc);
+    } else if (what == "trim") {
+        // a tree on each device, one search's block still in use
+        for (int d = 0; d < 2; ++d) {
+            hipSetDevice(d);
+            nbx_tree_destroy(tree(n, 0, A));
+        }
+        nbx_tree *t = tree(n, 0, A);
+        nbx_knn_dev(t, k, NBX_KNN_NONPERIODIC, 0, OUT, nullptr, A);
+        const size_t before = g_used[0] + g_used[1];
+        from = g_log.size();
+        const int64_t got = nbx_trim_memory();
+        note("trimmed %lld freed %zu left %zu again %lld", (long long)got, before - g_used[0] - g_used[1], g_used[0],
+             (long long)nbx_trim_memory());
     } else if (what == "adjoint") {
         double *const D = (double *)4096;
         const int rc = nbx_sph_density_adjoint_ordered_dev(D, D, OUT, nullptr, n, k, D, D, D, D, A);

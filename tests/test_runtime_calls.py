@@ -116,3 +116,11 @@ def test_build_gives_its_work_memory_back_first(n, form):
 def test_build_on_a_full_device(gib, fits):
     """2e9 particles of the precision form: 124.7 GB of arrays and 8 of order."""
     assert _build(2000000000, 1, gib)[0] == fits
+
+
+def test_trim_memory():
+    """Everything kept goes back, on both devices, after the work that uses it."""
+    got = log("trim", 300000, 4)
+    f = [x for x in got if x.startswith("trimmed")][0].split()
+    assert int(f[1]) > 0 and f[1] == f[3] and f[5] == "0" and f[7] == "0"
+    assert "host waits for stream 0xa0" in got
