@@ -1137,11 +1137,6 @@ __global__ __launch_bounds__(256) void k_fill_f64(double *p, double v, int64_t n
     int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = v;
 }
-__global__ __launch_bounds__(256) void k_iota(int32_t *p, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = (int32_t)i;
-}
-
 // tree slots of the particles with the given IDs (-1 for an ID out of range)
 __global__ __launch_bounds__(256) void k_ids_to_slots(const int32_t *ids, const int32_t *inv, int64_t m,
                                                       int32_t *slots) {

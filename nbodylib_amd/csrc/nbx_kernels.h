@@ -89,9 +89,8 @@ struct KnnArgs {
     double *hout;       // as rho, or by ID with hout_by_id (nullable)
     int32_t hout_by_id;  // particle queries: hout[ID] rather than hout[slot]
     int32_t *err;       // set to 1 if a row has fewer than kh neighbours (densities, miss_self)
-    // nullable: the queries in the order the waves take them -- slots (FP64
-    // re-run of mixed-form fallbacks, lists of particles) or, for position
-    // queries, their indices
+    // nullable, particle queries: their slots in the order the waves take them
+    // (FP64 re-run of mixed-form fallbacks, lists of particles)
     const int32_t *qlist;
     // particle queries of a run of whole waves only: slots [64 wbeg, 64 (wbeg + wcnt)) (wcnt 0: every slot)
     int32_t wbeg, wcnt;
@@ -214,7 +213,6 @@ int64_t nbx_drop_kept(int dev);
 __global__ void k_scatter_by_id(const double *src, const int32_t *perm, double *dst, int64_t n);
 __global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n);
 __global__ void k_fill_f64(double *p, double v, int64_t n);
-__global__ void k_iota(int32_t *p, int64_t n);
 __global__ void k_ids_to_slots(const int32_t *ids, const int32_t *inv, int64_t m, int32_t *slots);
 
 // ------------------------------------------------------------------ adjoint

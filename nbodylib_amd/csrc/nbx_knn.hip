@@ -74,7 +74,6 @@ struct KnnCtx {
     double gm[KShape<KMAX>::G];
     int gp[KShape<KMAX>::G];
     bool act, exz;
-    int fill;  // kh while nothing is kept and a whole leaf fits (wave-uniform), else 0
 };
 
 // Largest of the S values of group g and its (first) position.
@@ -203,27 +202,6 @@ __device__ __forceinline__ void knn_leaf(const DevTree &T, const double *const (
         for (int d = 0; d < ND; ++d) cx[d * NBX_LEAF + lane] = st[d];
     }
     __syncthreads();
-    if (TIE == 0 && c.fill) {
-        // first leaf met with nothing kept: the accepted candidates take the
-        // positions in turn, and the group maxima are taken once at the end
-        c.fill = 0;
-        int cnt = 0;
-        for (int j = 0; j < NBX_LEAF; ++j) {
-            const double d2 = knn_d2<ND>(c.q, cx, j);
-            const bool in = ((mask >> j) & 1u) && d2 < c.kth && (!c.exz || d2 > 0.0);
-            if (in) {
-                HD(cnt) = d2;
-                SL(cnt) = base + j;
-            }
-            cnt += in ? 1 : 0;
-        }
-#pragma unroll
-        for (int g = 0; g < KShape<KMAX>::G; ++g)
-            group_max<KMAX>(hd, lane, g * KShape<KMAX>::S, c.gm[g], c.gp[g]);
-        knn_top<ND, KMAX>(c);
-        __syncthreads();
-        return;
-    }
     // as many steps as the lane with the most candidates needs (a counted
     // loop keeps the search state in place across steps)
     int nit = __popc(mask);
@@ -371,7 +349,6 @@ __device__ __forceinline__ void knn_task(const DevTree &T, const KnnArgs &A, dou
     c.exz = (QSRC == NBX_Q_SLOTS) && A.excl_zero;
     c.kth = NBX_MAXVALUE;
     c.lost = INFINITY;
-    c.fill = kh >= NBX_LEAF ? kh : 0;
     const int npass = (QSRC != NBX_Q_SLOTS && A.periodic) ? 8 : 1;
     uint32_t passes = 0;  // image passes the lane took part in
     auto pass_begin = [&](int pass, bool again, float(&qc)[ND]) -> bool {
