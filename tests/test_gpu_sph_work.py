@@ -52,15 +52,15 @@ def test_forward_memory(gpu):
     assert got < (16 + 40) * n
 
 
+@pytest.mark.parametrize("refused", [0, 1300000])  # work memory of every pass, or the backward's, which is larger
 @pytest.mark.parametrize("shuffled", [False, True])
-def test_no_room(gpu, shuffled):
+def test_no_room(gpu, monkeypatch, shuffled, refused):
     import torch
 
-    from nbodylib_amd import device
     from nbodylib_amd.device import SPHDensity, sph_density
 
-    n, k = 300000, 12
-    print(f"sph without work memory n={n} k={k} shuffled={shuffled}", flush=True)
+    n, k = 20000, 12
+    print(f"sph without work memory n={n} k={k} shuffled={shuffled} refused from {refused}", flush=True)
     p, m, nn = _set(n, k, shuffled)
 
     def run():
@@ -71,30 +71,19 @@ def test_no_room(gpu, shuffled):
         return rho, h, r.detach(), pg.grad, mg.grad
 
     want = run()
-    torch.cuda.synchronize()
-    torch.cuda.empty_cache()
-    total = torch.cuda.get_device_properties(0).total_memory
-    sizes = []
-    real = device._sph_work
+    real, sizes = torch.empty, []
 
-    def counted(*a):
-        w = real(*a)
-        sizes.append(None if w is None else w.numel())
-        return w
+    def full(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            sizes.append(size[0])
+            if size[0] >= refused:
+                raise torch.OutOfMemoryError("no room")
+        return real(*size, **kw)
 
-    device._sph_work = counted
-    try:
-        # the largest block of any pass, 10.8 MB, leaves no room for 10.8 MB more
-        hold = torch.empty(((64 << 20) - 8,), dtype=torch.uint8, device="cuda")
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (44 << 20)) / total)
-        fill = [torch.empty((8 << 20,), dtype=torch.uint8, device="cuda") for _ in range(2)]
-        got = run()
-        torch.cuda.synchronize()
-        del hold, fill
-    finally:
-        device._sph_work = real
-        torch.cuda.set_per_process_memory_fraction(1.0)
-    assert None in sizes, sizes  # some call had to do without
+    monkeypatch.setattr(torch, "empty", full)
+    got = run()
+    monkeypatch.undo()
+    assert len(sizes) == 3 and max(sizes) >= refused and (min(sizes) < refused) == (refused > 0)
     assert torch.equal(got[1], want[1])
     for a, b in zip(got, want):
         assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
