@@ -445,7 +445,8 @@ def phase6d_section(args, steps, warmup):
 def run_phase6d(args):
     r = phase6d_section(args, args.steps, args.warmup)
     _line(f"Mqueries/s 6-D kNN (k={r['k']}) + 6-D SPH density, N={r['n']}, precision form", r["mixed_mqps"],
-          "Mqueries/s", args, r["mixed_ms"], "f32+f64", r["workload"], dict(r, cpu_baseline=None))
+          "Mqueries/s", args, r["mixed_ms"], "f64" if "fp64" in r["roofline"]["kernel"] else "f32+f64",
+          r["workload"], dict(r, cpu_baseline=None))
 
 
 def _adjoint_pass(torch, nb, pos, mass, nbr, reps):

@@ -219,7 +219,8 @@ class KDTree:
         return tab
 
     def last_fallbacks(self):
-        """Precision form: queries of the last call re-run in FP64 (certificate failed)."""
+        """Precision form: queries of the last call searched in FP64: those whose FP32 certificate failed, or
+        all of them where the whole call runs in FP64 because that is faster."""
         v = ctypes.c_int64()
         _check(lib().nbx_tree_last_fallbacks(self._h, ctypes.byref(v)))
         return v.value

@@ -23,8 +23,9 @@
 //    entries took six times as many (0.5M queries, k = 32: 1.54 ms, and 0.77
 //    with keys).
 //  * No scratch, no counters: a call is one launch.
-// Vector issue bounds it: about 0.85k instructions a query at k = 32 in 3-D, of
-// which the merges are about half, 95% of the cycles busy.  So the common path
+// Vector issue bounds it: 892 instructions a query with the density at k = 32 in
+// 3-D (2.1M clustered particles; 972 of 16.8M), of which the merges are about
+// half, at 73 to 79% of the peak rate under the profiler.  So the common path
 // is kept short (the last few open nodes are taken without a minimum, a group's
 // leaves share one scalar base address, padding needs no test of its own and
 // the query's own entry is sorted out after something was accepted): 6-D, 0.5M,

@@ -87,8 +87,8 @@ class DeviceTree:
         _check(lib().nbx_knn_density_dev(self._h, k, _ptr(nn_out), _ptr(rho_out), _ptr(h_out), _stream()))
 
     def sph_density(self, k, rho_out, h_out=None, block_rows=1 << 22):
-        """Differentiation-form forward over the tree's own k-nearest lists, recomputed per block of
-        block_rows tree slots (nbx_sph_density_fwd_tree_dev); rho / h by ID."""
+        """Differentiation-form forward over the tree's own k-nearest lists, summed in the search
+        (nbx_sph_density_fwd_tree_dev; no list is made and block_rows is not read); rho / h by ID."""
         _need(rho_out, "rho_out", torch.float64, (self.n,))
         _need(h_out, "h_out", torch.float64, (self.n,))
         _check(lib().nbx_sph_density_fwd_tree_dev(self._h, k, int(block_rows), _ptr(rho_out), _ptr(h_out),

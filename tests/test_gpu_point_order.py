@@ -1,6 +1,6 @@
-"""Query points are taken in Morton order from 65 points on; rows still belong
-to the caller's points, for counts around a wave, points outside the box and
-coinciding points, in 3-D and in phase space."""
+"""Query points in any order: rows belong to the caller's points, for counts
+around a wave, points outside the box and coinciding points, in 3-D and in
+phase space."""
 import numpy as np
 import pytest
 
