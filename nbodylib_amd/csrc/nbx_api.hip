@@ -680,6 +680,17 @@ struct ScratchLease {
     ScratchLease &operator=(const ScratchLease &) = delete;
 };
 
+// The lease with full bytes or, where they cannot be had, with least.
+static std::unique_ptr<ScratchLease> lease_scratch(nbx_tree *t, size_t full, size_t least, hipStream_t st) {
+    std::unique_ptr<ScratchLease> l(new ScratchLease(t, full, st));
+    if (l->err == hipErrorOutOfMemory && least < full) {
+        (void)hipGetLastError();
+        l.reset();  // one at a time
+        l.reset(new ScratchLease(t, least, st));
+    }
+    return l;
+}
+
 // Bytes the fused kNN + density pass carves, in its order: densities by slot,
 // the error flag, the fallback list (precision form) and the search scratch.
 // kh: entries the FP64 search keeps (0: its scratch not counted).
@@ -721,9 +732,9 @@ static hipError_t run_plain(nbx_tree *t, const KnnArgs &A, int nq, hipStream_t s
         need = std::min(need, ws->left());
         work = ws->carve<void>(need);
         if (!work) return hipErrorInvalidValue;
-    } else {
-        const hipError_t e = own.alloc(&work, need);
-        if (e != hipSuccess) return e;
+    } else if (own.alloc(&work, need) != hipSuccess) {
+        (void)hipGetLastError();
+        return nbx_launch_knn_wave(t->view(), A, nq, st);  // slower, but it needs none
     }
     return nbx_launch_knn(t->view(), A, nq, st, work, need);
 }
@@ -1058,7 +1069,7 @@ static int density_impl(nbx_tree *t, int32_t k, int32_t variant, int32_t nsearch
     if (ws) {
         if (A.dens == NBX_DO_VELPHYS) return fail(NBX_ERR_UNSUPPORTED, "no workspace form of this density");
     } else {
-        lease.reset(new ScratchLease(t, density_ws_bytes(t, k, mixed, A.kh), st));
+        lease = lease_scratch(t, density_ws_bytes(t, k, mixed, A.kh), density_ws_bytes(t, k, mixed, 0), st);
         if (lease->err != hipSuccess) return hipfail(lease->err, "density scratch");
         ws = &lease->ws;
     }
@@ -1656,10 +1667,10 @@ static int sph_tree_fwd(nbx_tree *t, int32_t k, double *rho_id, double *h_id, hi
     if (rc) return rc;
     const int64_t n = t->n;
     const bool mixed = mixed_ok(t, k);
-    ScratchLease lease(t, density_ws_bytes(t, k, mixed, k), st);
-    if (lease.err != hipSuccess) return hipfail(lease.err, "differentiation form scratch");
-    double *rs = lease.ws.carve<double>(sizeof(double) * n);
-    int32_t *err = lease.ws.carve<int32_t>(sizeof(int32_t));
+    const auto lease = lease_scratch(t, density_ws_bytes(t, k, mixed, k), density_ws_bytes(t, k, mixed, 0), st);
+    if (lease->err != hipSuccess) return hipfail(lease->err, "differentiation form scratch");
+    double *rs = lease->ws.carve<double>(sizeof(double) * n);
+    int32_t *err = lease->ws.carve<int32_t>(sizeof(int32_t));
     if (!rs || !err) return fail(NBX_ERR_ARG, "scratch too small");
     hipLaunchKernelGGL(k_fill_f64, dim3(nblk(n)), dim3(256), 0, st, rs, 0.0, n);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, err, 0, (int64_t)1);
@@ -1669,7 +1680,7 @@ static int sph_tree_fwd(nbx_tree *t, int32_t k, double *rho_id, double *h_id, hi
     A.hout = h_id;
     A.hout_by_id = 1;
     A.err = err;
-    const hipError_t e = mixed ? run_mixed(t, A, k, st, &lease.ws) : run_plain(t, A, (int)n, st, &lease.ws);
+    const hipError_t e = mixed ? run_mixed(t, A, k, st, &lease->ws) : run_plain(t, A, (int)n, st, &lease->ws);
     if (e != hipSuccess) return hipfail(e, "differentiation form");
     hipLaunchKernelGGL(k_scatter_by_id, dim3(nblk(n)), dim3(256), 0, st, rs, t->perm, rho_id, n);
     return sph_tree_end(err, st);
@@ -1701,7 +1712,13 @@ static int sph_tree_adj(nbx_tree *t, int32_t k, int64_t block, const double *g_i
     Workspace ws = {nullptr, 0, 0};
     ws.cap = mixed ? 256 + sizeof(int32_t) * (block + 1) + 256 + nbx_mixed_scratch_bytes(t->nd, k + 1)
                    : 256 + nbx_knn_scratch_bytes(t->nd, k, NBX_Q_SLOTS, false, block);
-    HIPCK(bufs.alloc(&ws.base, ws.cap));
+    hipError_t we = bufs.alloc(&ws.base, ws.cap);
+    if (we == hipErrorOutOfMemory && !mixed) {  // (the search then does without)
+        (void)hipGetLastError();
+        ws = {nullptr, 0, 0};
+        we = hipSuccess;
+    }
+    HIPCK(we);
     for (int64_t r0 = 0; r0 < n; r0 += block) {
         const int64_t nr = std::min<int64_t>(block, n - r0);
         KnnArgs A = sph_tree_search(k);

@@ -276,6 +276,26 @@ int main(int argc, char **argv) {
         const int64_t got = nbx_trim_memory();
         note("trimmed %lld freed %zu left %zu again %lld", (long long)got, before - g_used[0] - g_used[1], g_used[0],
              (long long)nbx_trim_memory());
+    } else if (what == "full") {
+        // argv[4] bytes a particle are left beside the tree
+        nbx_tree *t = tree(n, 0, A);
+        nbx_trim_memory();
+        g_total = g_used[0] + (size_t)atoll(argv[4]) * n + (1 << 20);
+        from = g_log.size();
+        int rc = nbx_knn_dev(t, k, NBX_KNN_NONPERIODIC, 0, OUT, (double *)64, A);
+        note("rows rc %d", rc);
+        rc = nbx_density_dev(t, k, NBX_DENS_SYMMETRIC, 0, (double *)64, nullptr, A);
+        note("density rc %d", rc);
+        rc = nbx_sph_density_fwd_tree_dev(t, k, 0, (double *)64, nullptr, A);
+        note("spline rc %d", rc);
+        nbx_tree_destroy(t);
+        nbx_trim_memory();
+        g_total = (size_t)288 << 30;
+        t = tree(n, 0, A);
+        nbx_trim_memory();
+        g_total = g_used[0] + (size_t)(atoll(argv[4]) + 76 + 4 * k) * n + (1 << 20);
+        rc = nbx_sph_density_adjoint_tree_dev(t, k, 0, (double *)64, (double *)64, (double *)64, A);
+        note("adjoint rc %d", rc);
     } else if (what == "adjoint") {
         double *const D = (double *)4096;
         const int rc = nbx_sph_density_adjoint_ordered_dev(D, D, OUT, nullptr, n, k, D, D, D, D, A);

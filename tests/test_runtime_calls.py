@@ -124,3 +124,14 @@ def test_trim_memory():
     f = [x for x in got if x.startswith("trimmed")][0].split()
     assert int(f[1]) > 0 and f[1] == f[3] and f[5] == "0" and f[7] == "0"
     assert "host waits for stream 0xa0" in got
+
+
+def test_searches_on_a_full_device():
+    """8 bytes a particle, a density's own need, are enough for every FP64
+    call: where the lane search's scratch cannot be had, a wave per query runs."""
+    got = log("full", 1000000, 4, 8)
+    assert [x for x in got if " rc " in x] == ["rows rc 0", "density rc 0", "spline rc 0", "adjoint rc 0"]
+    assert sum("k_knn_wave" in x for x in got) == 4 and not any("5k_knnI" in x for x in got)
+    # with room for it the lane search runs
+    got = log("full", 1000000, 4, 200)
+    assert sum("5k_knnI" in x for x in got) == 4 and not any("k_knn_wave" in x for x in got)
