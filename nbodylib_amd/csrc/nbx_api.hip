@@ -1185,31 +1185,31 @@ static int smooth_impl(nbx_tree *t, int32_t k, const double *rho_by_id, const do
     const bool need_disp = disp_out || moments;
     hipStream_t st = nullptr;
     int32_t *nn = nullptr;
-    double *rid = nullptr, *hid = nullptr, *hs = nullptr, *mean = nullptr, *disp = nullptr, *mom = nullptr, *buf = nullptr;
-    SmoothRec *rec = nullptr;
+    double *rid = nullptr, *hs = nullptr, *mean = nullptr, *disp = nullptr, *mom = nullptr, *buf = nullptr;
     HIPCK(bufs.alloc(&nn, sizeof(int32_t) * (size_t)n * k));
     HIPCK(bufs.alloc(&rid, sizeof(double) * n));
-    HIPCK(bufs.alloc(&hid, sizeof(double) * n));
     HIPCK(bufs.alloc(&hs, sizeof(double) * n));
-    HIPCK(bufs.alloc(&rec, sizeof(SmoothRec) * n));
     HIPCK(bufs.alloc(&mean, sizeof(double4) * n));
     if (need_disp) HIPCK(bufs.alloc(&disp, sizeof(SmoothSum) * n));
     if (moments) HIPCK(bufs.alloc(&mom, sizeof(SmoothSum) * n));
+    // one buffer in turn for the caller's means and dispersions, the search's h
+    // and the records, and the outputs
     HIPCK(bufs.alloc(&buf, sizeof(double) * 9 * n));
-    int rc = density_impl(t, k, NBX_DENS_SYMMETRIC, 0, rid, hid, nn, st);
+    SmoothRec *rec = (SmoothRec *)buf;
+    double *hid = buf + 8 * n;
     hipError_t e = hipSuccess;
+    if (mean_in) e = upload_rows(t, mean_in, 3, buf, 4, mean);
+    if (e == hipSuccess && need_disp && disp_in) e = upload_rows(t, disp_in, 9, buf, 8, disp);
+    if (e != hipSuccess) return hipfail(e, "smoothed velocities");
+    int rc = density_impl(t, k, NBX_DENS_SYMMETRIC, 0, rid, hid, nn, st);
     if (rc == NBX_OK) {
         if (rho_by_id) e = hipMemcpy(rid, rho_by_id, sizeof(double) * n, hipMemcpyHostToDevice);
         if (e == hipSuccess) hipLaunchKernelGGL(k_smooth_pack, dim3(nblk(n)), dim3(256), 0, st, t->view(), rid, hid, rec,
                                               hs);
-        if (e == hipSuccess) {
-            if (mean_in) e = upload_rows(t, mean_in, 3, buf, 4, mean);
-            else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(4 * n)), dim3(256), 0, st, mean, 0.0, 4 * n);
-        }
-        if (e == hipSuccess && need_disp) {
-            if (disp_in) e = upload_rows(t, disp_in, 9, buf, 8, disp);
-            else hipLaunchKernelGGL(k_fill_f64, dim3(nblk(8 * n)), dim3(256), 0, st, disp, 0.0, 8 * n);
-        }
+        if (e == hipSuccess && !mean_in)
+            hipLaunchKernelGGL(k_fill_f64, dim3(nblk(4 * n)), dim3(256), 0, st, mean, 0.0, 4 * n);
+        if (e == hipSuccess && need_disp && !disp_in)
+            hipLaunchKernelGGL(k_fill_f64, dim3(nblk(8 * n)), dim3(256), 0, st, disp, 0.0, 8 * n);
         if (e == hipSuccess && moments)
             hipLaunchKernelGGL(k_fill_f64, dim3(nblk(8 * n)), dim3(256), 0, st, mom, 0.0, 8 * n);
         if (e == hipSuccess) {

@@ -214,13 +214,13 @@ hipError_t hipGetSymbolAddress(void **p, const void *) {
 const char *hipGetErrorString(hipError_t) { return "fake"; }
 }
 
-static nbx_tree *tree(int64_t n, int form, hipStream_t st) {
+static nbx_tree *tree(int64_t n, int form, hipStream_t st, bool vel = false) {
     nbx_params p;
     nbx_params_default(&p);
     p.form = form;
     nbx_tree *t = nullptr;
     // positions are only passed on
-    const int rc = nbx_tree_create_dev(&p, (double *)64, nullptr, nullptr, n, st, &t);
+    const int rc = nbx_tree_create_dev(&p, (double *)64, vel ? (double *)64 : nullptr, nullptr, n, st, &t);
     if (rc) note("create failed %d", rc);
     return t;
 }
@@ -276,6 +276,23 @@ int main(int argc, char **argv) {
         const int64_t got = nbx_trim_memory();
         note("trimmed %lld freed %zu left %zu again %lld", (long long)got, before - g_used[0] - g_used[1], g_used[0],
              (long long)nbx_trim_memory());
+    } else if (what == "smooth") {
+        // host arrays of this size are not copied
+        nbx_tree *t = tree(n, 0, A, true);
+        nbx_trim_memory();
+        const size_t base = g_peak = g_used[0];
+        from = g_log.size();
+        double *const H = (double *)64;
+        int rc = nbx_smooth_vel(t, k, nullptr, nullptr, H, nullptr);
+        note("mean rc %d peak %zu", rc, g_peak - base);
+        nbx_trim_memory();
+        g_peak = base;
+        rc = nbx_smooth_vel(t, k, nullptr, H, nullptr, H);
+        note("disp rc %d peak %zu", rc, g_peak - base);
+        nbx_trim_memory();
+        g_peak = base;
+        rc = nbx_smooth_vel_moments(t, k, nullptr, nullptr, H, H, H);
+        note("moments rc %d peak %zu", rc, g_peak - base);
     } else if (what == "full") {
         // argv[4] bytes a particle are left beside the tree
         nbx_tree *t = tree(n, 0, A);

@@ -135,3 +135,14 @@ def test_searches_on_a_full_device():
     # with room for it the lane search runs
     got = log("full", 1000000, 4, 200)
     assert sum("5k_knnI" in x for x in got) == 4 and not any("k_knn_wave" in x for x in got)
+
+
+def test_smoothed_velocities_memory():
+    """Beside the rows (4 k bytes a particle) and a density's 8: densities and h
+    16, means 32, dispersions 64, moments 64 and the buffer of the rest 72.  (The
+    blocks of 8 bytes a particle are small enough to be kept, and rounded up by
+    at most an eighth of 2^32.)"""
+    n, k = 500000000, 4
+    got = {x.split()[0]: x.split() for x in log("smooth", n, k) if " peak " in x}
+    for what, own in (("mean", 120), ("disp", 184), ("moments", 248)):
+        assert got[what][2] == "0" and int(got[what][4]) <= (4 * k + 8 + own) * n + 3 * (1 << 29) + (128 << 20), what
