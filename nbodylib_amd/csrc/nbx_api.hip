@@ -136,19 +136,17 @@ static hipError_t block_get(size_t need, hipStream_t st, void **p, size_t *got) 
         std::lock_guard<std::mutex> lk(k.mu);
         std::vector<KeptBlock> &f = k.free[dev];
         if (bytes > keep_limit(k, dev)) bytes = exact;  // never kept
-        // the smallest that fits, the latest of equals, of the stream's own;
-        // else of those whose use is over
+        // the smallest that fits, the latest of equals
         size_t best = f.size();
-        for (int others = 0; others < 2 && best == f.size(); ++others)
-            for (size_t i = 0; i < f.size(); ++i) {
-                if ((f[i].st != st) != (others == 1) || f[i].bytes < bytes || f[i].bytes > bytes + bytes / 2) continue;
-                if (best < f.size() && f[i].bytes > f[best].bytes) continue;
-                if (others && hipEventQuery(f[i].used) != hipSuccess) {
-                    (void)hipGetLastError();  // not ready is no error
-                    continue;
-                }
-                best = i;
+        for (size_t i = f.size(); i-- > 0;) {
+            if (f[i].bytes < bytes || f[i].bytes > bytes + bytes / 2) continue;
+            if (best < f.size() && f[i].bytes >= f[best].bytes) continue;
+            if (f[i].st != st && hipEventQuery(f[i].used) != hipSuccess) {
+                (void)hipGetLastError();  // not ready is no error
+                continue;
             }
+            best = i;
+        }
         if (best < f.size()) {
             const KeptBlock b = f[best];
             e = hipStreamWaitEvent(st, b.used, 0);
